@@ -978,12 +978,54 @@ void emit_phase_statements(const Routine& r, Printer& pr, const Phase& ph, int G
   }
 }
 
+// A window gather (Phase::window): the contraction tile of contract_any.h with the descriptor as a constant.
+// Grid: tiles x residues modulo the strides, dealt to the XCDs in contiguous ranges.  Returns the threads.
+uint64_t emit_window(const Routine& r, const Phase& ph, std::vector<std::string>& body) {
+  const GemmDesc& g = ph.gemm;
+  const bool f32 = g.a.prec != Prec::Bfloat16 || g.b.prec != Prec::Bfloat16;
+  // channels of c (n) of at most 32 take the narrow tile: half of a square one would be padding
+  const int BM = g.N <= 32 ? 128 : 64, BN = g.N <= 32 ? 32 : 64;
+  const bool bkc = g.b.k_stride[2] == 1 || g.b.row_stride[2] != 1;
+  // (A's rows are positions: their digits are kept per k-contiguous chunk)
+  const int64_t tm = (g.M + BM - 1) / BM, tn = (g.N + BN - 1) / BN, residues = ph.win_s[0] * ph.win_s[1];
+  std::ostringstream d;
+  auto three = [&](const int64_t (&x)[3]) { d << "{" << x[0] << ", " << x[1] << ", " << x[2] << "}"; };
+  auto two = [&](const int64_t (&x)[2]) { d << "{" << x[0] << ", " << x[1] << "}"; };
+  auto digits = [&](const int64_t (&e)[3], int n) {
+    unsigned m1, m2; int s1, s2;
+    digit_magic(e[1], m1, s1); digit_magic(e[2], m2, s2);
+    d << "{" << n << ", " << e[1] << ", " << e[2] << ", " << m1 << "u, " << m2 << "u, " << s1 << ", " << s2 << "}";
+  };
+  auto operand = [&](const GemmOperand& o) {
+    d << "{"; three(o.row_stride); d << ", "; three(o.k_stride); d << ", " << (o.prec == Prec::Bfloat16 ? 1 : 0) << "}";
+  };
+  d << "{" << g.M << ", " << g.N << ", " << g.K << ", ";
+  digits(g.m_ext, g.m_digits); d << ", "; digits(g.n_ext, g.n_digits); d << ", "; digits(g.k_ext, g.k_digits); d << ", ";
+  operand(g.a); d << ", "; operand(g.b); d << ", "; three(g.c.row_stride); d << ", "; three(g.c.k_stride);
+  d << ", 0, " << (g.accumulate ? 1 : 0) << ", 1, " << tm << ", " << tn << ", ";
+  two(ph.win_s); d << ", "; two(ph.win_taps); d << ", "; two(ph.win_lim); d << ", "; two(ph.win_pos); d << "}";
+  const std::string shape = std::to_string(BM) + ", " + std::to_string(BN) + ", true, " + (bkc ? "true" : "false") + ", " + (f32 ? "true" : "false");
+  const int64_t blocks = (tm * tn * residues + 7) / 8 * 8;
+  body.push_back("  constexpr OcnAnyDesc d_ = " + d.str() + ";");
+  body.push_back("  __shared__ __attribute__((aligned(16))) unsigned char smem_[ocn_any_smem<" + shape + ">()];");
+  body.push_back("  const int t_ = (int)(blockIdx.x % 8u) * " + std::to_string(blocks / 8) + " + (int)(blockIdx.x / 8u);");
+  body.push_back("  if (t_ >= " + std::to_string(tm * tn * residues) + ") return;");
+  body.push_back("  const int z_ = t_ / " + std::to_string(tm * tn) + ", q_ = t_ % " + std::to_string(tm * tn) + ", r0_ = z_ / " + std::to_string(ph.win_s[1]) +
+                 ", r1_ = z_ % " + std::to_string(ph.win_s[1]) + ";");
+  body.push_back("  ocn_any_tile<" + shape + ", true>(d_, " + r.node(g.a.node).ident + " + " + std::to_string(g.a.offset) + ", " + r.node(g.b.node).ident + " + " +
+                 std::to_string(g.b.offset) + " + r0_ * " + std::to_string(ph.win_b[0]) + " + r1_ * " + std::to_string(ph.win_b[1]) + ", " +
+                 r.node(g.c.node).ident + " + " + std::to_string(g.c.offset) + " + r0_ * " + std::to_string(ph.win_c[0]) + " + r1_ * " +
+                 std::to_string(ph.win_c[1]) + ", (void*)0, (float*)0, q_ / " + std::to_string(tn) + ", q_ % " + std::to_string(tn) + ", 0, r0_, r1_, smem_);");
+  return (uint64_t)blocks * 256;
+}
+
 }  // namespace
 
 GeneratedModule generate_module(const Routine& r, const Plan& plan) {
   GeneratedModule mod;
   std::ostringstream src;
   src << builtins_hip_source() << "\n";
+  for (auto& ph : plan.phases) if (ph.kind == Phase::Generic && ph.window) { src << contract_any_source() << "\n"; break; }
   int kidx = 0;
   for (size_t pi = 0; pi < plan.phases.size(); ++pi) {
     const Phase& ph = plan.phases[pi];
@@ -1221,7 +1263,10 @@ GeneratedModule generate_module(const Routine& r, const Plan& plan) {
     };
 
     uint64_t total_threads = 0;
-    if (!ph.serial_members.empty()) {
+    if (ph.window) {
+      total_threads = emit_window(r, ph, body);
+      pr.used_nodes.insert(ph.gemm.a.node); pr.used_nodes.insert(ph.gemm.b.node); pr.used_nodes.insert(ph.gemm.c.node);
+    } else if (!ph.serial_members.empty()) {
       // ---- the whole routine in one workgroup: phases in order, a barrier after each
       for (auto& kv : ph.serial_shadows) {
         const Node& sn = r.node(kv.first);

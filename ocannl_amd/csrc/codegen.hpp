@@ -34,6 +34,7 @@ struct GeneratedModule {
 };
 
 const char* builtins_hip_source();
+const char* contract_any_source();   // contract_any.h, for modules with a window-gather kernel
 
 GeneratedModule generate_module(const Routine& r, const Plan& plan);
 

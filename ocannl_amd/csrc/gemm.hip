@@ -522,6 +522,7 @@ bool dtl_operands_ok(const GemmArgs& a, bool akc, bool bkc) {
 }  // namespace
 
 const char* gemm_kernel_name(const GemmDesc& d) {
+  if (d.any) return contract_any_name(d);
   // the instantiation as a profiler prints it (without namespaces)
   static thread_local char buf[128];
   const bool af = d.a.prec == Prec::Single, bf = d.b.prec == Prec::Single;
@@ -539,11 +540,13 @@ const char* gemm_kernel_name(const GemmDesc& d) {
 }
 
 size_t gemm_workspace_bytes(const GemmDesc& d) {
+  if (d.any) return contract_any_workspace_bytes(d);
   const int sp = split_count(d);
   return sp > 1 ? (size_t)sp * (size_t)batch_count(d) * (size_t)d.M * (size_t)d.N * sizeof(float) : 0;
 }
 
 hipError_t launch_gemm(const GemmDesc& d, const GemmArgs& a_in, void* workspace, hipStream_t s, hipEvent_t ev) {
+  if (d.any) return launch_contract_any(d, a_in, workspace, s, ev);
   GemmArgs a = a_in;
   a.splits = split_count(d);
   a.ws = static_cast<float*>(workspace);

@@ -171,6 +171,8 @@ int64_t get_stride(const Strides& s, int sym) {
   return it == s.by_sym.end() ? 0 : it->second;
 }
 
+void choose_coop(const Routine& r, Phase& ph, const PlanOptions& opt);
+
 bool mfma_prec(Prec p) { return p == Prec::Single || p == Prec::Bfloat16; }
 
 // Recognises `for.. { c[L] := fma(a[A], b[B], c[L]) }` (either operand order; also
@@ -230,10 +232,6 @@ bool match_contraction(const Routine& r, Phase& ph, const PlanOptions& opt) {
     }
   };
   merge(batch, false); merge(ms, false); merge(ns, false); merge(ks, true);
-  // surplus M / N symbols become batch dimensions (the other operand is re-read: stride 0)
-  while (ms.size() > 1) { batch.push_back(ms.front()); ms.erase(ms.begin()); }
-  while (ns.size() > 1) { batch.push_back(ns.front()); ns.erase(ns.begin()); }
-  if (ks.size() > 1 || batch.size() > 3) return false;
   // The kernels store (or read-add-write) every (batch, m, n) cell from its own lane with no atomics:
   // distinct cells must be distinct elements of C.  An accumulation through overlapping windows
   // (the input gradient of a convolution: x_grad[stride * o + k] with stride < window) is not that,
@@ -248,63 +246,212 @@ bool match_contraction(const Routine& r, Phase& ph, const PlanOptions& opt) {
       reach += c.first * (c.second - 1);
     }
   }
+  auto total = [](const std::vector<Sym>& v) { int64_t n = 1; for (auto& s : v) n *= s.ext; return n; };
 
   GemmDesc g;
-  g.M = ms.empty() ? 1 : ms[0].ext;
-  g.N = ns.empty() ? 1 : ns[0].ext;
-  g.K = ks.empty() ? 1 : ks[0].ext;
   g.a.node = pa->node; g.a.prec = na.prec; g.a.offset = sa.offset; g.a.static_terms = sa.statics;
   g.b.node = pb->node; g.b.prec = nb.prec; g.b.offset = sb.offset; g.b.static_terms = sb.statics;
   g.c.node = set.node; g.c.prec = nc.prec; g.c.offset = sc.offset; g.c.static_terms = sc.statics;
-  g.a.s_row = ms.empty() ? 0 : ms[0].a;  g.a.s_k = ks.empty() ? 0 : ks[0].a;
-  g.b.s_row = ns.empty() ? 0 : ns[0].b;  g.b.s_k = ks.empty() ? 0 : ks[0].b;
-  g.c.s_row = ms.empty() ? 0 : ms[0].c;  g.c.s_k = ns.empty() ? 0 : ns[0].c;
-  g.nbatch = (int)batch.size();
-  for (int i = 0; i < g.nbatch; ++i) {
-    g.batch_ext[i] = batch[i].ext;
-    g.a.s_batch[i] = batch[i].a; g.b.s_batch[i] = batch[i].b; g.c.s_batch[i] = batch[i].c;
-  }
-  if (g.flops() < (double)opt.min_mfma_flops) return false;
-  if (g.M < 16 || g.N < 16 || g.K < 8) return false;   // matrix-vector shapes stay generic
-  {
-    int64_t nb = 1;   // the batch is the launch grid's z extent
-    for (int i = 0; i < g.nbatch; ++i) nb *= g.batch_ext[i];
-    if (nb > 65535) return false;
-  }
-
-  // C must be contiguous along N; if it is contiguous along M instead, compute the transpose.
-  if (g.c.s_k != 1) {
-    if (g.c.s_row != 1) return false;
-    std::swap(g.a, g.b);
-    std::swap(g.M, g.N);
-    std::swap(g.c.s_row, g.c.s_k);
-  }
-  // each operand: unit stride along K or along its row dimension; vector-load alignment
-  const bool f32_compute = g.a.prec == Prec::Single && g.b.prec == Prec::Single;
-  auto operand_ok = [&](const GemmOperand& o, int64_t rows) {
-    // staging moves 8-element (bf16 compute) or 4-element (fp32 compute) chunks
-    const int vec = f32_compute ? 4 : 8;
-    if (o.s_k != 1 && o.s_row != 1) return false;
-    const int64_t ld = o.s_k == 1 ? o.s_row : o.s_k;
-    if (rows > 1 && g.K > 1 && ld % vec) return false;
-    if (o.offset % vec) return false;
-    for (auto& t : o.static_terms) if (t.second % vec) return false;
-    for (int i = 0; i < g.nbatch; ++i) if (o.s_batch[i] % vec) return false;
-    const int64_t contig = o.s_k == 1 ? g.K : rows;
-    if (contig % vec) return false;
-    return true;
+  g.accumulate = !ph.fused_zero_init;
+  auto set_batch = [](GemmDesc& g, const std::vector<Sym>& batch) {
+    int64_t nb = 1;
+    g.nbatch = (int)batch.size();
+    for (int i = 0; i < g.nbatch; ++i) {
+      g.batch_ext[i] = batch[i].ext;
+      g.a.s_batch[i] = batch[i].a; g.b.s_batch[i] = batch[i].b; g.c.s_batch[i] = batch[i].c;
+      nb *= batch[i].ext;
+    }
+    return nb <= 65535;   // the batch is the launch grid's z extent
   };
-  if (!operand_ok(g.a, g.M) || !operand_ok(g.b, g.N)) return false;
-  {
+
+  // The kernels of gemm.hip: one symbol of each class, 16-byte chunks everywhere.
+  auto regular = [&](GemmDesc& g) {
+    std::vector<Sym> bt = batch, m1 = ms, n1 = ns;
+    // surplus M / N symbols become batch dimensions (the other operand is re-read: stride 0)
+    while (m1.size() > 1) { bt.push_back(m1.front()); m1.erase(m1.begin()); }
+    while (n1.size() > 1) { bt.push_back(n1.front()); n1.erase(n1.begin()); }
+    if (ks.size() > 1 || bt.size() > 3) return false;
+    g.M = total(m1); g.N = total(n1); g.K = total(ks);
+    g.a.s_row = m1.empty() ? 0 : m1[0].a;  g.a.s_k = ks.empty() ? 0 : ks[0].a;
+    g.b.s_row = n1.empty() ? 0 : n1[0].b;  g.b.s_k = ks.empty() ? 0 : ks[0].b;
+    g.c.s_row = m1.empty() ? 0 : m1[0].c;  g.c.s_k = n1.empty() ? 0 : n1[0].c;
+    if (!set_batch(g, bt)) return false;
+    if (g.flops() < (double)opt.min_mfma_flops) return false;
+    if (g.M < 16 || g.N < 16 || g.K < 8) return false;   // matrix-vector shapes stay generic
+    // C must be contiguous along N; if it is contiguous along M instead, compute the transpose.
+    if (g.c.s_k != 1) {
+      if (g.c.s_row != 1) return false;
+      std::swap(g.a, g.b);
+      std::swap(g.M, g.N);
+      std::swap(g.c.s_row, g.c.s_k);
+    }
+    // each operand: unit stride along K or along its row dimension; vector-load alignment
+    const bool f32_compute = g.a.prec == Prec::Single && g.b.prec == Prec::Single;
+    auto operand_ok = [&](const GemmOperand& o, int64_t rows) {
+      // staging moves 8-element (bf16 compute) or 4-element (fp32 compute) chunks
+      const int vec = f32_compute ? 4 : 8;
+      if (o.s_k != 1 && o.s_row != 1) return false;
+      const int64_t ld = o.s_k == 1 ? o.s_row : o.s_k;
+      if (rows > 1 && g.K > 1 && ld % vec) return false;
+      if (o.offset % vec) return false;
+      for (auto& t : o.static_terms) if (t.second % vec) return false;
+      for (int i = 0; i < g.nbatch; ++i) if (o.s_batch[i] % vec) return false;
+      const int64_t contig = o.s_k == 1 ? g.K : rows;
+      if (contig % vec) return false;
+      return true;
+    };
+    if (!operand_ok(g.a, g.M) || !operand_ok(g.b, g.N)) return false;
     const int vec = 4;
     if (g.c.s_row % vec || g.c.offset % vec || g.N % vec) return false;
     for (auto& t : g.c.static_terms) if (t.second % vec) return false;
     for (int i = 0; i < g.nbatch; ++i) if (g.c.s_batch[i] % vec) return false;
-  }
-  g.accumulate = !ph.fused_zero_init;
+    return true;
+  };
+
+  // Anything else of some size: up to three digits a class, any stride and offset (contract_any.h).
+  auto general = [&](GemmDesc& g) {
+    if (!opt.any_contractions) return false;
+    std::vector<Sym> bt = batch;
+    auto surplus = [&](std::vector<Sym>& v) { while (v.size() > 3) { bt.push_back(v.front()); v.erase(v.begin()); } };
+    surplus(ms); surplus(ns);
+    if (ks.size() > 3 || bt.size() > 3) return false;
+    g.M = total(ms); g.N = total(ns); g.K = total(ks);
+    if (!set_batch(g, bt)) return false;
+    if (g.flops() < (double)opt.min_mfma_flops) return false;
+    // (a vector-shaped result fills a sliver of a tile: a generated kernel with lanes sharing k does better)
+    if (std::min(g.M, g.N) < 8 || std::max(g.M, g.N) < 16 || g.K < 8) return false;
+    for (int id : {pa->node, pb->node, set.node}) if (r.node(id).num_elems() > (int64_t)0x3FFFFFFF) return false;   // 32-bit offsets
+    // A bf16 sum that a generated kernel would run in one thread is rounded after every addition, as the
+    // reference's is; one whose lanes share the sum is kept in fp32 and rounded once, as here.
+    if (nc.prec == Prec::Bfloat16) {
+      Phase alone = ph;
+      alone.kind = Phase::Generic;
+      choose_coop(r, alone, opt);
+      if (alone.coop_lanes <= 1) return false;
+    }
+    auto put = [](const std::vector<Sym>& v, int& digits, int64_t (&ext)[3], int64_t (&s1)[3], int64_t Sym::*f1, int64_t (&s2)[3], int64_t Sym::*f2) {
+      digits = std::max<int>(1, (int)v.size());
+      for (size_t i = 0; i < v.size(); ++i) {
+        const size_t at = 3 - v.size() + i;
+        ext[at] = v[i].ext; s1[at] = v[i].*f1; s2[at] = v[i].*f2;
+      }
+    };
+    put(ms, g.m_digits, g.m_ext, g.a.row_stride, &Sym::a, g.c.row_stride, &Sym::c);
+    put(ns, g.n_digits, g.n_ext, g.b.row_stride, &Sym::b, g.c.k_stride, &Sym::c);
+    put(ks, g.k_digits, g.k_ext, g.a.k_stride, &Sym::a, g.b.k_stride, &Sym::b);
+    // lanes store neighbouring n: put the class along which C is contiguous there
+    if (g.c.k_stride[2] != 1 && g.c.row_stride[2] == 1) {
+      std::swap(g.a, g.b);
+      std::swap(g.M, g.N);
+      std::swap(g.m_digits, g.n_digits);
+      std::swap(g.m_ext, g.n_ext);
+      std::swap(g.c.row_stride, g.c.k_stride);
+    }
+    g.any = true;
+    return true;
+  };
+  GemmDesc reg = g;
+  if (regular(reg)) g = reg;
+  else if (!general(g)) return false;
   ph.kind = Phase::Contraction;
   ph.gemm = g;
   ph.flops = g.flops();
+  return true;
+}
+
+// Phase::window: recognises the overlapping-window accumulation.  Conditions: c is fp32 (a bf16 sum is
+// rounded after every addition, in the order of the loops), every other axis of c and the positions cover
+// plain iterators, one loop symbol at most beside the positions in m, one channel symbol at least in k.
+bool match_window(const Routine& r, Phase& ph, const PlanOptions& opt) {
+  if (!opt.enable_mfma || !opt.any_contractions || ph.inner.size() != 1 || ph.inner[0]->kind != Stmt::Set) return false;
+  const Stmt& set = *ph.inner[0];
+  const Scalar& v = *set.value;
+  if (!(v.kind == Scalar::Tern && v.tern == Ternop::Fma)) return false;
+  const Scalar *pa = v.a.get(), *pb = v.b.get(), *pc = v.c.get();
+  if (pa->kind != Scalar::Get || pb->kind != Scalar::Get || pc->kind != Scalar::Get) return false;
+  if (pc->node != set.node || !same_indices(pc->idcs, set.idcs) || pa->node == set.node || pb->node == set.node) return false;
+  const Node& nc = r.node(set.node);
+  if (!mfma_prec(r.node(pa->node).prec) || !mfma_prec(r.node(pb->node).prec) || nc.prec != Prec::Single) return false;
+  std::map<int, int64_t> ext;
+  for (size_t i = 0; i < ph.par_syms.size(); ++i) { if (ph.par_from[i]) return false; ext[ph.par_syms[i]] = ph.par_ext[i]; }
+  for (size_t i = 0; i < ph.seq_syms.size(); ++i) { if (ph.seq_from[i]) return false; ext[ph.seq_syms[i]] = ph.seq_to[i] + 1; }
+  Strides sa = strides_of(r, pa->node, pa->idcs), sb = strides_of(r, pb->node, pb->idcs), sc = strides_of(r, set.node, set.idcs);
+  // the axes of c that are sums of two symbols: the one that a walks is the position, the other the tap
+  struct Win { int o, k; int64_t s, pos, step; };
+  std::vector<Win> wins;
+  std::set<int> special;
+  bool swapped = false;
+  for (size_t p = 0; p < set.idcs.size(); ++p) {
+    const AxisIndex& ax = set.idcs[p];
+    if (ax.kind == AxisIndex::Fixed) { if (ax.fixed != 0 || nc.dims[p] != 1) return false; continue; }
+    if (ax.kind == AxisIndex::Iter) { if (!ext.count(ax.sym) || ext[ax.sym] != nc.dims[p]) return false; continue; }
+    if (ax.kind != AxisIndex::Affine || ax.offset != 0 || ax.terms.size() != 2) return false;
+    Win w{-1, -1, 0, nc.dims[p], row_major_stride(nc, p)};
+    for (int q = 0; q < 2; ++q) {
+      // the tap has coefficient 1; with stride 1 both do, and the symbol of the earlier-named operand decides
+      const auto &to = ax.terms[q], &tk = ax.terms[1 - q];
+      if (tk.first != 1 || to.first < 1 || !ext.count(to.second) || !ext.count(tk.second)) continue;
+      const bool ab = get_stride(sa, to.second) > 0 && !get_stride(sb, to.second) && get_stride(sb, tk.second) > 0 && !get_stride(sa, tk.second);
+      const bool ba = get_stride(sb, to.second) > 0 && !get_stride(sa, to.second) && get_stride(sa, tk.second) > 0 && !get_stride(sb, tk.second);
+      // (a window slides over the larger extent; either reading is the same sum)
+      if (!(ab || ba) || (to.first == 1 && ext[to.second] < ext[tk.second])) continue;
+      if (!wins.empty() && ba != swapped) continue;
+      swapped = ba;
+      w.o = to.second; w.k = tk.second; w.s = to.first;
+      break;
+    }
+    if (w.o < 0 || w.s * (ext[w.o] - 1) + ext[w.k] > w.pos) return false;
+    special.insert(w.o); special.insert(w.k);
+    wins.push_back(w);
+  }
+  if (wins.empty() || wins.size() > 2 || special.size() != 2 * wins.size()) return false;
+  if (swapped) { std::swap(pa, pb); std::swap(sa, sb); }
+  if (!sa.statics.empty() || !sb.statics.empty() || !sc.statics.empty()) return false;
+  struct Sym { int64_t ext, a, b, c; };
+  std::vector<Sym> ms, ns, ks;
+  for (auto& kv : ext) {
+    if (special.count(kv.first) || kv.second == 1) continue;
+    Sym s{kv.second, get_stride(sa, kv.first), get_stride(sb, kv.first), get_stride(sc, kv.first)};
+    if (s.a < 0 || s.b < 0 || s.c < 0) return false;
+    if (s.c && s.a && !s.b) ms.push_back(s);
+    else if (s.c && s.b && !s.a) ns.push_back(s);
+    else if (!s.c && s.a && s.b) ks.push_back(s);
+    else return false;
+  }
+  if (ms.size() > 1 || ns.size() > 3 || ks.size() > 1) return false;
+  std::sort(ns.begin(), ns.end(), [](const Sym& x, const Sym& y) { return x.c > y.c; });
+  for (int id : {pa->node, pb->node, set.node}) if (r.node(id).num_elems() > (int64_t)0x3FFFFFFF) return false;
+  GemmDesc g;
+  g.any = true;
+  g.a.node = pa->node; g.a.prec = r.node(pa->node).prec; g.a.offset = sa.offset;
+  g.b.node = pb->node; g.b.prec = r.node(pb->node).prec; g.b.offset = sb.offset;
+  g.c.node = set.node; g.c.prec = nc.prec; g.c.offset = sc.offset;
+  g.m_digits = 3; g.k_digits = 3; g.n_digits = std::max<int>(1, (int)ns.size());
+  if (!ms.empty()) { g.m_ext[0] = ms[0].ext; g.a.row_stride[0] = ms[0].a; g.c.row_stride[0] = ms[0].c; }
+  if (!ks.empty()) { g.k_ext[2] = ks[0].ext; g.a.k_stride[2] = ks[0].a; g.b.k_stride[2] = ks[0].b; }
+  for (size_t i = 0; i < wins.size(); ++i) {
+    const Win& w = wins[i];
+    const size_t at = 2 - wins.size() + i;     // 0, 1 or just 1
+    const int64_t ka = get_stride(sa, w.o), kb = get_stride(sb, w.k);
+    ph.win_s[at] = w.s; ph.win_taps[at] = ext[w.k]; ph.win_lim[at] = ext[w.o]; ph.win_pos[at] = w.pos;
+    ph.win_c[at] = w.step; ph.win_b[at] = kb;
+    g.m_ext[1 + at] = (w.pos + w.s - 1) / w.s;
+    g.a.row_stride[1 + at] = ka; g.c.row_stride[1 + at] = w.s * w.step;
+    g.k_ext[at] = (ext[w.k] + w.s - 1) / w.s;
+    g.a.k_stride[at] = -ka; g.b.k_stride[at] = w.s * kb;
+  }
+  for (size_t i = 0; i < ns.size(); ++i) {
+    const size_t at = 3 - ns.size() + i;
+    g.n_ext[at] = ns[i].ext; g.b.row_stride[at] = ns[i].b; g.c.k_stride[at] = ns[i].c;
+  }
+  g.M = g.m_ext[0] * g.m_ext[1] * g.m_ext[2];
+  g.N = g.n_ext[0] * g.n_ext[1] * g.n_ext[2];
+  g.K = g.k_ext[0] * g.k_ext[1] * g.k_ext[2];
+  if (g.flops() < (double)opt.min_mfma_flops || g.M < 16 || g.K < 8 || g.M * g.K > (int64_t)1 << 40) return false;
+  ph.kind = Phase::Generic;
+  ph.window = true;
+  ph.gemm = g;
+  ph.flops = g.flops() * (double)ph.win_s[0] * (double)ph.win_s[1];
   return true;
 }
 
@@ -1017,7 +1164,7 @@ struct RowShape { std::vector<int64_t> outer; int64_t len = -1; };
 
 // Classifies `ph` as a member of a row group over `shape` (filling in what the shape leaves open).
 bool row_member(const Routine& r, Phase& ph, RowShape& shape, bool first) {
-  if (ph.kind != Phase::Generic || !ph.members.empty()) return false;
+  if (ph.kind != Phase::Generic || ph.window || !ph.members.empty()) return false;
   if (ph.inner.size() != 1 || ph.inner[0]->kind != Stmt::Set) return false;
   for (auto f : ph.par_from) if (f != 0) return false;
   for (auto f : ph.seq_from) if (f != 0) return false;
@@ -1226,6 +1373,15 @@ bool same_layout(const GemmOperand& x, const GemmOperand& y) {
   return true;
 }
 
+bool same_digits(const GemmDesc& x, const GemmDesc& y) {
+  if (x.any != y.any) return false;
+  if (!x.any) return true;
+  auto eq = [](const int64_t (&u)[3], const int64_t (&v)[3]) { return u[0] == v[0] && u[1] == v[1] && u[2] == v[2]; };
+  return x.m_digits == y.m_digits && x.n_digits == y.n_digits && x.k_digits == y.k_digits && eq(x.m_ext, y.m_ext) && eq(x.n_ext, y.n_ext) &&
+         eq(x.k_ext, y.k_ext) && eq(x.a.row_stride, y.a.row_stride) && eq(x.a.k_stride, y.a.k_stride) && eq(x.b.row_stride, y.b.row_stride) &&
+         eq(x.b.k_stride, y.b.k_stride) && eq(x.c.row_stride, y.c.row_stride) && eq(x.c.k_stride, y.c.k_stride);
+}
+
 void merge_contractions(Plan& plan, bool chain, int window = 1 << 30) {
   std::map<int, int> mirror_source;   // bf16 copy -> the tensor whose stores keep it in step
   for (auto& kv : plan.mirrors) mirror_source[kv.second] = kv.first;
@@ -1262,7 +1418,7 @@ void merge_contractions(Plan& plan, bool chain, int window = 1 << 30) {
       if (chain ? !g.group.empty() : !g.more.empty()) continue;
       if (chain) {
         // the kernels built for operand-pair lists: bf16 operands, fp32 result
-        if (g.a.prec != Prec::Bfloat16 || g.b.prec != Prec::Bfloat16 || g.c.prec != Prec::Single) continue;
+        if (g.any || g.a.prec != Prec::Bfloat16 || g.b.prec != Prec::Bfloat16 || g.c.prec != Prec::Single) continue;
       } else {
         // grouping pays where a launch alone leaves compute units idle or with one workgroup each
         double tiles = (double)((g.M + 127) / 128) * (double)((g.N + 127) / 128);
@@ -1278,7 +1434,7 @@ void merge_contractions(Plan& plan, bool chain, int window = 1 << 30) {
       if (!chain && (long)j - (long)i > (long)window) break;
       Phase& q = plan.phases[j];
       const GemmDesc& h = q.gemm;
-      bool candidate = q.kind == Phase::Contraction && h.group.empty() && h.more.empty() && h.epi_bias < 0 && h.epi_relu < 0 &&
+      bool candidate = q.kind == Phase::Contraction && same_digits(h, g) && h.group.empty() && h.more.empty() && h.epi_bias < 0 && h.epi_relu < 0 &&
                        g.epi_bias < 0 && g.epi_relu < 0 && h.M == g.M && h.N == g.N &&
                        h.K == g.K && h.nbatch == g.nbatch && same_layout(h.a, g.a) && same_layout(h.b, g.b) && same_layout(h.c, g.c);
       for (int b = 0; b < g.nbatch && candidate; ++b) candidate = h.batch_ext[b] == g.batch_ext[b];
@@ -1407,7 +1563,7 @@ void serialise_tiny(const Routine& r, Plan& plan) {
       for (auto e : ph.row_outer_ext) threads *= e;
       if (threads > 131072) return;
       iterations += (threads / 256 + 1) * (int64_t)ph.members.size();
-    } else if (ph.kind == Phase::Generic) {
+    } else if (ph.kind == Phase::Generic && !ph.window) {
       int64_t threads = ph.coop_lanes;
       for (auto e : ph.par_ext) threads *= e;
       int64_t work = 1;
@@ -1457,7 +1613,7 @@ void group_independent(const Routine& r, Plan& plan) {
   };
   auto sets_of = [&](const Phase& ph) {
     Sets s;
-    if (ph.kind != Phase::Generic || !ph.serial_members.empty() || !ph.parallel_members.empty() || ph.fused_x >= 0) return s;
+    if (ph.kind != Phase::Generic || !ph.serial_members.empty() || !ph.parallel_members.empty() || ph.fused_x >= 0 || ph.window) return s;
     if (ph.bytes > (double)(32 << 20)) return s;
     bool ok = true;
     if (ph.members.empty()) ok = add_accesses(ph, s);
@@ -1599,6 +1755,7 @@ struct Bf16Copies {
 
 void use_bf16_copies(Routine& r, Plan& plan, Phase& ph, Bf16Copies& copies, int* next_sym) {
   GemmDesc& g = ph.gemm;
+  if (g.any) return;   // (computes mixed products in fp32)
   if ((g.a.prec == Prec::Single) == (g.b.prec == Prec::Single)) return;   // all-fp32 stays exact fp32
   GemmOperand& op = g.a.prec == Prec::Single ? g.a : g.b;
   const Node src = r.node(op.node);
@@ -1831,7 +1988,7 @@ void fuse_row_contractions(Routine& r, Plan& plan, bool also_stored, int waves) 
       if (i < 0) continue;
       const Phase& P = plan.phases[i];
       const GemmDesc& g = P.gemm;
-      if (P.kind != Phase::Contraction || g.c.node != X || g.accumulate || !g.group.empty() || !g.more.empty() || g.c_copy >= 0) continue;
+      if (P.kind != Phase::Contraction || g.any || g.c.node != X || g.accumulate || !g.group.empty() || !g.more.empty() || g.c_copy >= 0) continue;
       if (g.a.prec != Prec::Bfloat16 || g.b.prec != Prec::Bfloat16 || g.a.s_k != 1 || g.b.s_k != 1) continue;
       if (g.K % 16 != 0 || g.K > 128 || g.N != G.row_len) continue;
       if (!g.a.static_terms.empty() || !g.b.static_terms.empty() || !g.c.static_terms.empty() || g.c.offset != 0) continue;
@@ -1944,7 +2101,7 @@ void fuse_row_projections(Routine& r, Plan& plan) {
     }
     for (size_t i = j + 1; i < plan.phases.size() && G.proj_y < 0; ++i) {
       const Phase& P = plan.phases[i];
-      if (P.kind != Phase::Contraction) continue;
+      if (P.kind != Phase::Contraction || P.gemm.any) continue;
       const GemmDesc& g = P.gemm;
       if (g.accumulate || !g.group.empty() || !g.more.empty() || g.epi_bias >= 0 || g.epi_relu >= 0) continue;
       if (P.inner.size() != 1 || P.inner[0]->kind != Stmt::Set) continue;
@@ -2146,7 +2303,7 @@ void fold_epilogues(Routine& r, Plan& plan) {
   for (size_t i = 0; i + 1 < plan.phases.size(); ++i) {
     Phase& P = plan.phases[i];
     GemmDesc& g = P.gemm;
-    if (P.kind != Phase::Contraction || !scratch.count(g.c.node) || g.accumulate || g.c_copy >= 0 || !g.group.empty() || !g.more.empty()) continue;
+    if (P.kind != Phase::Contraction || g.any || !scratch.count(g.c.node) || g.accumulate || g.c_copy >= 0 || !g.group.empty() || !g.more.empty()) continue;
     const int X = g.c.node;
     const Node xn = r.node(X);
     if (xn.prec != Prec::Bfloat16 || g.c.offset != 0 || !g.c.static_terms.empty()) continue;
@@ -2330,14 +2487,29 @@ Plan make_plan(Routine& r, const PlanOptions& requested) {
       }
     }
 
-    if (!match_contraction(r, ph, opt)) {
+    if (match_contraction(r, ph, opt)) {
+      set_contraction_bytes(ph);
+      if (opt.enable_bf16_copies) use_bf16_copies(r, plan, ph, copies, &next_sym);
+    } else if (match_window(r, ph, opt)) {
+      // the gather visits every element of the result once: a Zero_out ahead of it folds into it
+      const int target = ph.gemm.c.node;
+      for (int q = (int)plan.phases.size() - 1; q >= 0; --q) {
+        const Phase& prev = plan.phases[q];
+        if (prev.kind == Phase::Fill && prev.fill_node == target) {
+          ph.fused_zero_init = true;
+          plan.phases.erase(plan.phases.begin() + q);
+          copies.erased((size_t)q);
+          break;
+        }
+        if (phase_touches(prev, target)) break;
+      }
+      ph.gemm.accumulate = !ph.fused_zero_init;
+      account_bytes(r, ph);
+    } else {
       ph.kind = Phase::Generic;
       split_reduction(r, ph, opt, plan, &next_sym);
       choose_coop(r, ph, opt);
       account_bytes(r, ph);
-    } else {
-      set_contraction_bytes(ph);
-      if (opt.enable_bf16_copies) use_bf16_copies(r, plan, ph, copies, &next_sym);
     }
     ph.comments_before.swap(pending_comments);
     plan.phases.push_back(std::move(ph));

@@ -27,6 +27,8 @@ struct GemmOperand {
   int64_t s_row = 0;     // stride along M (A, C) or N (B)
   int64_t s_k = 0;       // stride along K (A, B); for C: stride along N
   int64_t s_batch[3] = {0, 0, 0};
+  // GemmDesc::any: strides of the row digits (m or n) and of the k digits; for C of the m and of the n digits
+  int64_t row_stride[3] = {0, 0, 0}, k_stride[3] = {0, 0, 0};
 };
 
 // C[batch, m, n] (+)= sum_k A[batch, m, k] * B[batch, n, k], all strides explicit.
@@ -36,6 +38,12 @@ struct GemmDesc {
   int nbatch = 0;
   int64_t batch_ext[3] = {1, 1, 1};
   bool accumulate = false;   // beta = 1: add into existing C (gradient accumulation `=+`)
+  // Set: extents or strides that the kernels of gemm.hip do not take; contract_any.hip runs it.  m, n and k are
+  // then numbers of up to three digits (the loop symbols of the class that do not merge, slowest first; unused
+  // leading digits have extent 1), s_row / s_k are not used, and a mixed product is computed in fp32.
+  bool any = false;
+  int m_digits = 1, n_digits = 1, k_digits = 1;
+  int64_t m_ext[3] = {1, 1, 1}, n_ext[3] = {1, 1, 1}, k_ext[3] = {1, 1, 1};
   // Independent contractions of the same shapes, strides and precisions (the q / k / v projections of
   // one input, their weight gradients) that ride in the same launch: {a, b, c} per extra member.  A
   // small contraction alone puts at most one workgroup on a compute unit; several together let
@@ -62,6 +70,13 @@ struct GemmDesc {
     return f;
   }
 };
+
+// Factor and shift of the quotient by `d` of a number below 2^31 (ocn_digit_div in contract_any.h).
+inline void digit_magic(int64_t d, unsigned& mul, int& sh) {
+  sh = 0;
+  while ((1ll << sh) < d) ++sh;
+  mul = (unsigned)((((1ull << sh) - (uint64_t)d) << 32) / (uint64_t)d + 1);
+}
 
 struct Phase {
   enum Kind { Generic, Fill, Contraction } kind = Generic;
@@ -130,6 +145,14 @@ struct Phase {
   int64_t proj_n = 0;
   int proj_kp = 1;                                      // parts of T that separate waves sum up (partial results meet in LDS)
   int proj_c_copy = -1;                                 // bf16 copy of an fp32 c, stored alongside
+  // Window gather (kind Generic, `window` set): an accumulation through overlapping windows
+  // `c[.., stride * o + k, ..] += a[.., o, ..] * b[.., k, ..]` (the input gradient of a convolution) turned
+  // round: every element of c gathers the taps k that reach it, so that no two workgroups meet on one, and
+  // the sum over taps and channels is a contraction for the matrix cores.  `gemm` holds it in digits: m =
+  // (rest, position, position), k = (tap, tap, channel), positions and taps counted in strides; c's and b's
+  // strides along them are per stride, win_c / win_b per single step.
+  bool window = false;
+  int64_t win_s[2] = {1, 1}, win_taps[2] = {1, 1}, win_lim[2] = {1, 1}, win_pos[2] = {1, 1}, win_c[2] = {0, 0}, win_b[2] = {0, 0};
   // Fill
   int fill_node = -1;
   // Contraction
@@ -149,6 +172,7 @@ struct Phase {
 struct PlanOptions {
   int64_t min_mfma_flops = 1 << 22;   // below this a contraction stays a generic kernel
   bool enable_mfma = true;
+  bool any_contractions = true;       // contractions of any extents and strides too (contract_any.hip)
   bool enable_coop = true;
   bool enable_row_groups = true;
   bool enable_serial_group = true;   // tiny routines as one single-workgroup kernel

@@ -147,6 +147,7 @@ PlanOptions parse_options(const char* options) {
     if (eq == std::string::npos) throw InvalidArgument("compile options: expected key=value, got '" + kv + "'");
     const std::string k = kv.substr(0, eq), v = kv.substr(eq + 1);
     if (k == "mfma") o.enable_mfma = v != "0";
+    else if (k == "any") o.any_contractions = v != "0";
     else if (k == "coop") o.enable_coop = v != "0";
     else if (k == "rows") o.enable_row_groups = v != "0";
     else if (k == "bf16_copies") o.enable_bf16_copies = v != "0";
@@ -186,6 +187,7 @@ std::vector<int> wide_access_nodes(const Plan& plan) {
   for (auto& ph : plan.phases) {
     if (ph.kind == Phase::Contraction) {
       const GemmDesc& g = ph.gemm;
+      if (g.any) continue;   // (loads of any element alignment)
       add(g.a.node); add(g.b.node); add(g.c.node); add(g.c_copy); add(g.epi_bias); add(g.epi_relu);
       for (auto& m : g.group) { add(m.a.node); add(m.b.node); add(m.c.node); add(m.c_copy); }
       for (auto& pr : g.more) { add(pr.first.node); add(pr.second.node); }

@@ -1,0 +1,130 @@
+"""Contractions of extents and strides that are not multiples of a vector or a tile, on the matrix cores:
+against a float64 recomputation from the same inputs.  Both operands bf16: products are exact and summed in
+fp32; an fp32 operand keeps all its bits (a mixed product is computed in fp32)."""
+import numpy as np
+import pytest
+
+from ocannl_amd import llir as L
+from ocannl_amd import workloads as W
+from parity import HipRun
+from test_gpu_contractions import _routine
+from test_gpu_conv import _conv
+
+pytestmark = pytest.mark.gpu
+
+
+def _values(rng, node):
+    return W.as_prec(rng.standard_normal(node.dims).astype(np.float32), node.prec)
+
+
+def _run(r, nodes, out, want, accumulate, k, seed=0):
+    """`want`: float64 inputs by name -> result without the accumulated-into values."""
+    rng = np.random.default_rng(seed)
+    init = {n.id: _values(rng, n) for n in nodes.values()}
+    hip = HipRun(r, init, "min_mfma_flops=1")
+    ks = [x for x in hip.code.kernels() if x["kind"] == "mfma"]
+    if not ks and nodes[out].prec == "bfloat16":   # a bf16 sum that one thread runs: rounded after every addition, left alone
+        return hip.close()
+    assert ks and all("contract_any" in x["name"] for x in ks), hip.code.kernels()
+    hip.step()
+    f = {name: W.to_float(init[n.id], n.prec).astype(np.float64) for name, n in nodes.items()}
+    ref = want(f) + (f[out] if accumulate else 0.0)
+    got = W.to_float(hip.get(nodes[out]), nodes[out].prec).astype(np.float64)
+    err = np.max(np.abs(got - ref)) / np.max(np.abs(ref))
+    tol = 2.0 ** -8 if nodes[out].prec == "bfloat16" else 2e-6 * max(1.0, np.sqrt(k) / 8)
+    assert err <= tol, (err, tol, ks[0]["name"])
+    hip.close()
+
+
+def _product(M, N, K, a_prec, b_prec, c_prec, a_kc, b_kc, accumulate, batch=0, seed=0):
+    r, A, B, C = _routine(M, N, K, a_prec, b_prec, c_prec, a_kc, b_kc, accumulate, batch)
+    t = lambda x, kc: x if kc else np.swapaxes(x, -1, -2)
+    _run(r, dict(a=A, b=B, c=C), "c", lambda f: t(f["a"], a_kc) @ np.swapaxes(t(f["b"], b_kc), -1, -2), accumulate, K, seed)
+
+
+@pytest.mark.parametrize("layout", [(True, True), (True, False), (False, True), (False, False)])
+@pytest.mark.parametrize("precs", [("bfloat16", "bfloat16", "single"), ("bfloat16", "bfloat16", "bfloat16"), ("single", "bfloat16", "single"),
+                                   ("bfloat16", "single", "bfloat16"), ("single", "single", "single")])
+def test_odd_extents(layout, precs):
+    for seed, (M, N, K) in enumerate(((65, 63, 67), (17, 9, 9), (129, 131, 31), (63, 65, 257))):
+        _product(M, N, K, *precs, *layout, accumulate=seed % 2 == 0, seed=seed)
+
+
+@pytest.mark.parametrize("layout", [(True, True), (False, False), (True, False)])
+@pytest.mark.parametrize("prec", ["bfloat16", "single"])
+def test_large_tiles_splits_and_batches(layout, prec):
+    _product(2049, 4099, 130, prec, prec, "single", *layout, accumulate=False, seed=1)      # 128 x 128 tiles
+    _product(33, 70, 4099, prec, prec, "single", *layout, accumulate=True, seed=2)          # K split
+    _product(71, 19, 2051, prec, prec, "bfloat16", *layout, accumulate=True, seed=3)
+    _product(99, 37, 45, prec, prec, "single", *layout, accumulate=False, batch=11, seed=4)
+
+
+@pytest.mark.parametrize("prec", ["bfloat16", "single"])
+@pytest.mark.parametrize("shape", [dict(b=3, oh=9, ow=7, ic=5, oc=17), dict(b=2, oh=16, ow=12, ic=8, oc=24), dict(b=5, oh=6, ow=11, ic=3, oc=19)])
+@pytest.mark.parametrize("stride,ksz", [(1, 3), (2, 3), (3, 2)])
+def test_convolution_windows(stride, ksz, shape, prec):
+    # y += x * w and w_grad += y_grad * x: rows and sums of several loop symbols that do not merge
+    full, n = _conv(stride, ksz, prec, **shape)
+    nests = [s for s in full.body if not isinstance(s, L.ZeroOut)]
+    names = ("x", "w", "y", "dy", "dw")
+    n["y"].prec = n["dw"].prec = "single"
+    nodes = {k: n[k] for k in names}
+    oh, ow = shape["oh"], shape["ow"]
+    window = lambda x, k1, k2: x[:, k1:k1 + stride * (oh - 1) + 1:stride, k2:k2 + stride * (ow - 1) + 1:stride, :]
+
+    def fwd(f):
+        return sum(np.einsum("bhwi,ci->bhwc", window(f["x"], k1, k2), f["w"][:, k1, k2, :]) for k1 in range(ksz) for k2 in range(ksz))
+
+    def dw(f):
+        out = np.zeros(n["dw"].dims)
+        for k1 in range(ksz):
+            for k2 in range(ksz):
+                out[:, k1, k2, :] = np.einsum("bhwc,bhwi->ci", f["dy"], window(f["x"], k1, k2))
+        return out
+
+    ins = lambda *k: {x: nodes[x] for x in k}
+    _run(L.Routine("conv_fwd", [nests[0]]), ins("x", "w", "y"), "y", fwd, True, ksz * ksz * shape["ic"])
+    _run(L.Routine("conv_dw", [nests[2]]), ins("x", "dy", "dw"), "dw", dw, True, shape["b"] * oh * ow)
+
+
+def test_slices_at_any_offset():
+    # the operands are slices that start at odd elements of larger tensors
+    L.reset_symbols(0)
+    M, N, K = 70, 41, 53
+    a = L.Node(1, "a", "bfloat16", (M + 1, K + 3)); b = L.Node(2, "b", "bfloat16", (K + 1, N + 2)); c = L.Node(3, "c", "single", (M, N + 1))
+    m, n, k = (L.fresh_symbol() for _ in range(3))
+    at = lambda s, o: L.Affine(((1, s),), o)
+    ci = (L.It(m), at(n, 1))
+    body = L.Set(c, ci, L.Ternop("fma", L.Get(a, (at(m, 1), at(k, 3))), L.Get(b, (at(k, 1), at(n, 1))), L.Get(c, ci)))
+    for sym, ext in ((k, K), (n, N), (m, M)):
+        body = L.For(sym, 0, ext - 1, [body])
+
+    def want(f):
+        out = np.zeros(c.dims)
+        out[:, 1:] = f["a"][1:, 3:] @ f["b"][1:, 1:N + 1]
+        return out
+    _run(L.Routine("slices", [body]), dict(a=a, b=b, c=c), "c", want, True, K)
+
+
+@pytest.mark.parametrize("prec", ["bfloat16", "single"])
+@pytest.mark.parametrize("shape", [dict(b=3, oh=9, ow=7, ic=5, oc=16), dict(b=2, oh=16, ow=12, ic=40, oc=24), dict(b=1, oh=6, ow=11, ic=3, oc=9)])
+@pytest.mark.parametrize("stride,ksz", [(1, 3), (2, 3), (2, 5), (3, 4)])
+@pytest.mark.parametrize("zeroed", [True, False])
+def test_overlapping_windows_are_gathered(stride, ksz, shape, prec, zeroed):
+    # x_grad[stride * o + k] += y_grad[o] * w[k]: turned round into a sum over the taps that reach a position
+    full, n = _conv(stride, ksz, prec, **shape)
+    n["dx"].prec = "single"
+    r = L.Routine("conv_dx", ([L.ZeroOut(n["dx"])] if zeroed else []) + [[s for s in full.body if not isinstance(s, L.ZeroOut)][1]])
+    rng = np.random.default_rng(stride)
+    init = {n[k].id: _values(rng, n[k]) for k in ("w", "dy", "dx")}
+    hip = HipRun(r, init, "min_mfma_flops=1")
+    assert [k["kind"] for k in hip.code.kernels()] == ["generated"] and "ocn_any_tile<" in hip.code.source().split('extern "C"')[1]
+    hip.step()
+    w, dy = (W.to_float(init[n[k].id], prec).astype(np.float64) for k in ("w", "dy"))
+    want = np.zeros(n["dx"].dims) if zeroed else init[n["dx"].id].astype(np.float64)
+    oh, ow = shape["oh"], shape["ow"]
+    for k1 in range(ksz):
+        for k2 in range(ksz):
+            want[:, k1:k1 + stride * (oh - 1) + 1:stride, k2:k2 + stride * (ow - 1) + 1:stride, :] += np.einsum("bhwc,ci->bhwi", dy, w[:, k1, k2, :])
+    assert np.max(np.abs(hip.get(n["dx"]) - want)) <= 4e-6 * np.max(np.abs(want))
+    hip.close()
