@@ -182,6 +182,14 @@ OCN_DEV uint4x32_t half_to_uint4x32(unsigned short x) { return ocn_u4(x, 0u, 0u,
 OCN_DEV uint4x32_t fp8_to_uint4x32(unsigned char x) { return ocn_u4(x, 0u, 0u, 0u); }
 
 // ---- lane-group combine used by cooperative reductions ------------------------------------------
+// Workgroup barrier that orders LDS only: loads and stores of global memory stay in flight across it (a
+// __syncthreads waits for every store to be acknowledged, most of a microsecond).
+OCN_DEV void ocn_lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 OCN_DEV float ocn_xshfl(float v, int m) { return __shfl_xor(v, m, 64); }
 OCN_DEV double ocn_xshfl(double v, int m) { return __shfl_xor(v, m, 64); }
 

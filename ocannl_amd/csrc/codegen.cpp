@@ -362,10 +362,10 @@ struct Printer {
     if (lanes > 64) {
       const std::string red = dbl ? "redd_" : "red_";
       out.push_back(ind + "if ((threadIdx.x & 63u) == 0) " + red + "[threadIdx.x >> 6] = " + var + ";");
-      out.push_back(ind + "__syncthreads();");
+      out.push_back(ind + "ocn_lds_barrier();");
       out.push_back(ind + var + " = " + combine_expr(accum, dbl, combine_expr(accum, dbl, red + "[0]", red + "[1]"),
                                                     combine_expr(accum, dbl, red + "[2]", red + "[3]")) + ";");
-      out.push_back(ind + "__syncthreads();");
+      out.push_back(ind + "ocn_lds_barrier();");
     }
   }
 
@@ -381,7 +381,8 @@ struct Printer {
                                idx_t + " " + sym + " = ";
       // a lane takes runs of four neighbouring positions, so that the unrolled loads and stores of a
       // unit-stride tensor combine into 16-byte (fp32) or 8-byte (bf16) accesses
-      return head + row_pos(lanes) + ";";
+      // (the last positions of a row that is not a multiple of the lanes are missing)
+      return head + row_pos(lanes) + ";" + (to + 1 < (int64_t)row_iters * lanes ? " if (" + sym + " > " + std::to_string(to) + ") continue;" : "");
     }
     return ind + "for (" + idx_t + " " + sym + " = " + std::to_string(from) + " + lane_; " + sym + " <= " + std::to_string(to) +
            "; " + sym + " += " + std::to_string(lanes) + ") {";
@@ -1200,7 +1201,7 @@ GeneratedModule generate_module(const Routine& r, const Plan& plan) {
         }
         if (QG > 64) body.push_back(pind + "__shared__ float red_[4]; __shared__ double redd_[4];");
         // short rows: everything the group produces stays in registers as well (no read-back)
-        const bool cached = q.row_len % QG == 0 && q.row_len / QG <= 16;
+        const bool cached = (q.row_len + QG - 1) / QG <= 16;
         if (cached) {
           pr.row_iters = (int)(q.row_len / QG);
           for (auto& m : q.members) {
@@ -1316,9 +1317,31 @@ GeneratedModule generate_module(const Routine& r, const Plan& plan) {
     } else {
       body.push_back(ind + "const uint64_t gtid_ = ((uint64_t)blockIdx.y * gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x;");
       total_threads = emit_points(ph, ind, "return");
+      for (auto& l : fetch) body.push_back(l);
+      for (auto& l : keep) body.push_back(l);
+      if (np) body.push_back(ind + "ocn_lds_barrier();");
+      std::set<int> lds_r, lds_w, mem_r, mem_w;   // touched since the last barrier / since the last full one
     }
 
     if (plan.debug_log) {
+        std::set<int> rd, wr, dyn;
+        if (q.kind == Phase::Fill) wr.insert(q.fill_node);
+        else if (q.members.empty()) touched_nodes(q.inner, rd, wr, dyn);
+        else for (auto& m : q.members) touched_nodes(m.inner, rd, wr, dyn);
+        std::set<int> rd_mem = dyn;
+        for (int n : rd) if (!pr.shadow_live.count(n)) rd_mem.insert(n);
+        auto meet = [](const std::set<int>& a, const std::set<int>& b) { for (int n : a) if (b.count(n)) return true; return false; };
+        std::set<int> rd_all = rd;
+        rd_all.insert(dyn.begin(), dyn.end());
+        if (meet(rd_mem, mem_w) || meet(wr, mem_w) || meet(wr, mem_r)) {
+          body.push_back(ind + "__syncthreads();");
+          lds_r.clear(); lds_w.clear(); mem_r.clear(); mem_w.clear();
+        } else if (meet(rd_all, lds_w) || meet(wr, lds_w) || meet(wr, lds_r)) {
+          body.push_back(ind + "ocn_lds_barrier();");
+          lds_r.clear(); lds_w.clear();
+        }
+        lds_r.insert(rd_all.begin(), rd_all.end()); lds_w.insert(wr.begin(), wr.end());
+        mem_r.insert(rd_mem.begin(), rd_mem.end()); mem_w.insert(wr.begin(), wr.end());
       // one thread runs the phase (the planner kept every loop sequential); the routine's top-level
       // comments since the previous phase come first, those after the last phase at the very end
       std::vector<std::string> head;
