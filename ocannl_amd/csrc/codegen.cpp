@@ -979,6 +979,23 @@ void emit_phase_statements(const Routine& r, Printer& pr, const Phase& ph, int G
   }
 }
 
+// Nodes that a block reads (`dyn`: through a run-time index) and writes.
+void touched_nodes(const Block& b, std::set<int>& rd, std::set<int>& wr, std::set<int>& dyn) {
+  std::function<void(const Scalar&)> sc = [&](const Scalar& s) {
+    if (s.kind == Scalar::Get || s.kind == Scalar::GetMerge) rd.insert(s.node);
+    if (s.kind == Scalar::GetDyn) dyn.insert(s.node);
+    if (s.kind == Scalar::LocalScope) touched_nodes(s.body, rd, wr, dyn);
+    if (s.a) sc(*s.a);
+    if (s.b) sc(*s.b);
+    if (s.c) sc(*s.c);
+  };
+  for (auto& s : b) {
+    if (s->kind == Stmt::Set || s->kind == Stmt::SetVec || s->kind == Stmt::ZeroOut) wr.insert(s->node);
+    if (s->value) sc(*s->value);
+    touched_nodes(s->body, rd, wr, dyn);
+  }
+}
+
 // A window gather (Phase::window): the contraction tile of contract_any.h with the descriptor as a constant.
 // Grid: tiles x residues modulo the strides, dealt to the XCDs in contiguous ranges.  Returns the threads.
 uint64_t emit_window(const Routine& r, const Phase& ph, std::vector<std::string>& body) {
@@ -1039,6 +1056,15 @@ GeneratedModule generate_module(const Routine& r, const Plan& plan) {
     std::vector<std::string> body;
     const std::string ind = "  ";
 
+    // threads that fit 31 bits decode their point in 32: quotients by constants cost a fifth of the 64-bit ones
+    std::string pt_t = "uint64_t", pt_u = "ull";
+    auto narrow_points = [&](uint64_t threads) { const bool n = threads < (1ull << 30); pt_t = n ? "uint32_t" : "uint64_t"; pt_u = n ? "u" : "ull"; };
+    auto phase_threads = [&](const Phase& q) {
+      uint64_t t = (uint64_t)q.coop_lanes;
+      for (auto e : (q.members.empty() ? q.par_ext : q.row_outer_ext)) t *= (uint64_t)e;
+      return t;
+    };
+    int serial_block = 256;   // workgroup size of a serial group
     int fused_block = 0;   // > 0: the kernel is a row group with a contraction prologue and wants this workgroup size
     // one phase for the thread (or loop iteration) identified by gtid_; `skip` leaves it
     auto emit_points = [&](const Phase& q, const std::string& pind, const std::string& skip) {
@@ -1046,9 +1072,9 @@ GeneratedModule generate_module(const Routine& r, const Plan& plan) {
       uint64_t QP = 1;
       if (QG > 1) {
         body.push_back(pind + "const uint32_t lane_ = (uint32_t)(gtid_ % " + std::to_string(QG) + "u);");
-        body.push_back(pind + "uint64_t pt_ = gtid_ / " + std::to_string(QG) + "u;");
+        body.push_back(pind + pt_t + " pt_ = (" + pt_t + ")(gtid_ / " + std::to_string(QG) + "u);");
       } else {
-        body.push_back(pind + "uint64_t pt_ = gtid_;");
+        body.push_back(pind + pt_t + " pt_ = (" + pt_t + ")gtid_;");
       }
       if (!q.members.empty() && q.fused_x >= 0) {
         // ---- row group with a contraction prologue: a workgroup owns 32 rows (consecutive along outer
@@ -1193,7 +1219,7 @@ GeneratedModule generate_module(const Routine& r, const Plan& plan) {
         body.push_back(pind + "if (pt_ >= " + std::to_string(QP) + "ull) " + skip + ";");
         const size_t n = q.row_outer_ext.size();
         for (int k = (int)n - 1; k >= 0; --k) {
-          const std::string ext = std::to_string(q.row_outer_ext[k]) + "ull";
+          const std::string ext = std::to_string(q.row_outer_ext[k]) + pt_u;
           std::string line = pind + "const " + pr.idx_t + " row" + std::to_string(k) + "_ = (" + pr.idx_t + ")(";
           if (k == 0) line += "pt_);";
           else line += "pt_ % " + ext + "); pt_ /= " + ext + ";";
@@ -1203,7 +1229,7 @@ GeneratedModule generate_module(const Routine& r, const Plan& plan) {
         // short rows: everything the group produces stays in registers as well (no read-back)
         const bool cached = (q.row_len + QG - 1) / QG <= 16;
         if (cached) {
-          pr.row_iters = (int)(q.row_len / QG);
+          pr.row_iters = (int)((q.row_len + QG - 1) / QG);
           for (auto& m : q.members) {
             const Stmt& st = *m.inner[0];
             if (pr.cache_name.count(st.node)) continue;
@@ -1250,7 +1276,7 @@ GeneratedModule generate_module(const Routine& r, const Plan& plan) {
         for (int k = (int)order.size() - 1; k >= 0; --k) {
           const size_t i = order[k];
           const std::string sy = sym_ident(q.par_syms[i]);
-          const std::string ext = std::to_string(q.par_ext[i]) + "ull";
+          const std::string ext = std::to_string(q.par_ext[i]) + pt_u;
           std::string line = pind + "const " + pr.idx_t + " " + sy + " = (" + pr.idx_t + ")(" + std::to_string(q.par_from[i]) + " + ";
           if (k == 0) line += "pt_);";
           else line += "pt_ % " + ext + "); pt_ /= " + ext + ";";
@@ -1268,62 +1294,36 @@ GeneratedModule generate_module(const Routine& r, const Plan& plan) {
       total_threads = emit_window(r, ph, body);
       pr.used_nodes.insert(ph.gemm.a.node); pr.used_nodes.insert(ph.gemm.b.node); pr.used_nodes.insert(ph.gemm.c.node);
     } else if (!ph.serial_members.empty()) {
-      // ---- the whole routine in one workgroup: phases in order, a barrier after each
+      // ---- the whole routine in one workgroup: phases in order.  Tensors shadowed in LDS from the start are read in
+      //      up front, all loads in flight together.  Between phases: nothing where the later one touches nothing
+      //      that the earlier ones since the last barrier stored (or stores nothing they touched); a barrier that
+      //      orders LDS where all that passes between them is shadowed; the full one only where memory is.
+      for (auto& q : ph.serial_members) if (q.kind != Phase::Fill && phase_threads(q) > (uint64_t)serial_block) serial_block = 512;
+      for (auto& q : ph.serial_members) if (q.kind != Phase::Fill && phase_threads(q) > 512) serial_block = 1024;
+      const std::string SB = std::to_string(serial_block) + "u";
+      std::vector<std::string> fetch, keep;
+      int np = 0;
       for (auto& kv : ph.serial_shadows) {
         const Node& sn = r.node(kv.first);
         pr.shadow[kv.first] = "sh_" + sn.ident;
         body.push_back(ind + "__shared__ " + c_typ(sn.prec) + " sh_" + sn.ident + "[" + std::to_string(sn.num_elems()) + "];");
-      }
-      for (size_t qi = 0; qi < ph.serial_members.size(); ++qi) {
-        const Phase& q = ph.serial_members[qi];
-        for (auto& kv : ph.serial_shadows) if (kv.second < (int)qi) pr.shadow_live.insert(kv.first);
-        body.push_back(ind + "/* " + q.label + " */");
-        if (q.kind == Phase::Fill) {
-          const Node& fn = r.node(q.fill_node);
-          pr.used_nodes.insert(q.fill_node);
-          Pair cv = convert_precision(Prec::Double, fn.prec);
-          const std::string zero = cv.first + "0" + cv.second;
-          std::string line = ind + "for (" + pr.idx_t + " z_ = threadIdx.x; z_ < " + std::to_string(fn.num_elems()) + "ull; z_ += 256u) ";
-          if (pr.shadow.count(q.fill_node)) line += "{ " + fn.ident + "[z_] = " + zero + "; " + pr.shadow.at(q.fill_node) + "[z_] = " + zero + "; }";
-          else line += fn.ident + "[z_] = " + zero + ";";
-          body.push_back(line);
-        } else {
-          uint64_t qt = (uint64_t)q.coop_lanes;
-          for (auto e : (q.members.empty() ? q.par_ext : q.row_outer_ext)) qt *= (uint64_t)e;
-          const uint64_t rounded = (qt + 255) / 256 * 256;
-          body.push_back(ind + "for (uint64_t gtid_ = threadIdx.x; gtid_ < " + std::to_string(rounded) + "ull; gtid_ += 256u) {");
-          emit_points(q, ind + "  ", "continue");
-          body.push_back(ind + "}");
+        if (kv.second >= 0) continue;
+        pr.used_nodes.insert(kv.first);
+        pr.shadow_live.insert(kv.first);
+        for (int64_t at = 0; at < sn.num_elems(); at += serial_block) {
+          const std::string v = "f" + std::to_string(np++) + "_", pos = "threadIdx.x + " + std::to_string(at) + "u";
+          const std::string guard = sn.num_elems() - at < serial_block ? "if (" + pos + " < " + std::to_string(sn.num_elems()) + "u) " : "";
+          fetch.push_back(ind + c_typ(sn.prec) + " " + v + " = 0; " + guard + v + " = " + sn.ident + "[" + pos + "];");
+          keep.push_back(ind + guard + "sh_" + sn.ident + "[" + pos + "] = " + v + ";");
         }
-        body.push_back(ind + "__syncthreads();");
       }
-      pr.shadow.clear(); pr.shadow_live.clear();
-      total_threads = 256;
-    } else if (!ph.parallel_members.empty()) {
-      // ---- independent phases side by side: every member owns a range of whole workgroups
-      body.push_back(ind + "const uint64_t g_ = ((uint64_t)blockIdx.y * gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x;");
-      uint64_t first = 0;
-      for (auto& q : ph.parallel_members) {
-        uint64_t qt = (uint64_t)q.coop_lanes;
-        for (auto e : (q.members.empty() ? q.par_ext : q.row_outer_ext)) qt *= (uint64_t)e;
-        const uint64_t end = first + (qt + 255) / 256 * 256;
-        body.push_back(ind + (first ? "else if" : "if") + " (g_ < " + std::to_string(end) + "ull) {  /* " + q.label + " */");
-        body.push_back(ind + "  const uint64_t gtid_ = g_ - " + std::to_string(first) + "ull;");
-        emit_points(q, ind + "  ", "return");
-        body.push_back(ind + "}");
-        first = end;
-      }
-      total_threads = first;
-    } else {
-      body.push_back(ind + "const uint64_t gtid_ = ((uint64_t)blockIdx.y * gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x;");
-      total_threads = emit_points(ph, ind, "return");
       for (auto& l : fetch) body.push_back(l);
       for (auto& l : keep) body.push_back(l);
       if (np) body.push_back(ind + "ocn_lds_barrier();");
       std::set<int> lds_r, lds_w, mem_r, mem_w;   // touched since the last barrier / since the last full one
-    }
-
-    if (plan.debug_log) {
+      for (size_t qi = 0; qi < ph.serial_members.size(); ++qi) {
+        const Phase& q = ph.serial_members[qi];
+        for (auto& kv : ph.serial_shadows) if (kv.second < (int)qi) pr.shadow_live.insert(kv.first);
         std::set<int> rd, wr, dyn;
         if (q.kind == Phase::Fill) wr.insert(q.fill_node);
         else if (q.members.empty()) touched_nodes(q.inner, rd, wr, dyn);
@@ -1342,6 +1342,51 @@ GeneratedModule generate_module(const Routine& r, const Plan& plan) {
         }
         lds_r.insert(rd_all.begin(), rd_all.end()); lds_w.insert(wr.begin(), wr.end());
         mem_r.insert(rd_mem.begin(), rd_mem.end()); mem_w.insert(wr.begin(), wr.end());
+        body.push_back(ind + "/* " + q.label + " */");
+        if (q.kind == Phase::Fill) {
+          const Node& fn = r.node(q.fill_node);
+          pr.used_nodes.insert(q.fill_node);
+          Pair cv = convert_precision(Prec::Double, fn.prec);
+          const std::string zero = cv.first + "0" + cv.second;
+          std::string line = ind + "for (" + pr.idx_t + " z_ = threadIdx.x; z_ < " + std::to_string(fn.num_elems()) + "ull; z_ += " + SB + ") ";
+          if (pr.shadow.count(q.fill_node)) line += "{ " + fn.ident + "[z_] = " + zero + "; " + pr.shadow.at(q.fill_node) + "[z_] = " + zero + "; }";
+          else line += fn.ident + "[z_] = " + zero + ";";
+          body.push_back(line);
+        } else {
+          const uint64_t qt = phase_threads(q), rounded = (qt + serial_block - 1) / serial_block * serial_block;
+          narrow_points(rounded);
+          body.push_back(ind + "for (" + pt_t + " gtid_ = threadIdx.x; gtid_ < " + std::to_string(rounded) + pt_u + "; gtid_ += " + SB + ") {");
+          emit_points(q, ind + "  ", "continue");
+          body.push_back(ind + "}");
+        }
+      }
+      pr.shadow.clear(); pr.shadow_live.clear();
+      total_threads = (uint64_t)serial_block;
+    } else if (!ph.parallel_members.empty()) {
+      // ---- independent phases side by side: every member owns a range of whole workgroups
+      uint64_t all = 0;
+      for (auto& q : ph.parallel_members) all += (phase_threads(q) + 255) / 256 * 256;
+      narrow_points(all);
+      body.push_back(ind + (pt_t == "uint32_t" ? "const uint32_t g_ = blockIdx.x * 256u + threadIdx.x;"
+                                               : "const uint64_t g_ = ((uint64_t)blockIdx.y * gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x;"));
+      uint64_t first = 0;
+      for (auto& q : ph.parallel_members) {
+        const uint64_t end = first + (phase_threads(q) + 255) / 256 * 256;
+        body.push_back(ind + (first ? "else if" : "if") + " (g_ < " + std::to_string(end) + pt_u + ") {  /* " + q.label + " */");
+        body.push_back(ind + "  const " + pt_t + " gtid_ = g_ - " + std::to_string(first) + pt_u + ";");
+        emit_points(q, ind + "  ", "return");
+        body.push_back(ind + "}");
+        first = end;
+      }
+      total_threads = first;
+    } else {
+      if (ph.fused_x < 0) narrow_points(phase_threads(ph));
+      body.push_back(ind + (pt_t == "uint32_t" ? "const uint32_t gtid_ = blockIdx.x * 256u + threadIdx.x;"
+                                               : "const uint64_t gtid_ = ((uint64_t)blockIdx.y * gridDim.x + blockIdx.x) * blockDim.x + threadIdx.x;"));
+      total_threads = emit_points(ph, ind, "return");
+    }
+
+    if (plan.debug_log) {
       // one thread runs the phase (the planner kept every loop sequential); the routine's top-level
       // comments since the previous phase come first, those after the last phase at the very end
       std::vector<std::string> head;
@@ -1355,7 +1400,7 @@ GeneratedModule generate_module(const Routine& r, const Plan& plan) {
     gk.name = r.name + "_k" + std::to_string(kidx++);
     gk.phase_index = (int)pi;
     gk.threads = total_threads;
-    gk.block = fused_block > 0 ? fused_block : 256;
+    gk.block = fused_block > 0 ? fused_block : ph.serial_members.empty() ? 256 : serial_block;
     std::vector<std::string> decls;
     for (int id : r.node_order) {
       if (!pr.used_nodes.count(id)) continue;

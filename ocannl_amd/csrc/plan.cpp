@@ -1510,18 +1510,22 @@ void choose_shadows(const Routine& r, Phase& g) {
     if (m.members.empty()) flat.push_back({&m, (int)q});
     else for (auto& sub : m.members) flat.push_back({&sub, (int)q});
   }
-  int64_t budget = 48 * 1024;
-  for (auto& kv : r.nodes) {
-    const Node& n = kv.second;
+  // (64 KB of static LDS in all, less the exchange arrays of lane groups; small tensors first)
+  int64_t budget = 60 * 1024;
+  std::vector<const Node*> by_size;
+  for (auto& kv : r.nodes) by_size.push_back(&kv.second);
+  std::stable_sort(by_size.begin(), by_size.end(), [](const Node* x, const Node* y) { return x->size_in_bytes() < y->size_in_bytes(); });
+  for (const Node* np : by_size) {
+    const Node& n = *np;
     if (n.mode == Mode::Virtual || n.prec == Prec::Uint4x32 || n.prec == Prec::Void) continue;
     const int64_t bytes = (int64_t)n.size_in_bytes();
     if (bytes > budget || bytes > 16 * 1024) continue;
-    int valid_after = -1;
-    bool ok = true;
+    int valid_after = -2;    // not touched yet
+    bool ok = true, pays = false;
     for (auto& f : flat) {
       const Phase& ph = *f.ph;
       if (ph.kind == Phase::Fill) {
-        if (ph.fill_node == n.id && valid_after < 0) valid_after = f.member;
+        if (ph.fill_node == n.id && valid_after == -2) valid_after = f.member;
         continue;
       }
       std::vector<Access> acc; bool w = false, fo = false; std::set<ScopeId> d;
@@ -1535,13 +1539,11 @@ void choose_shadows(const Routine& r, Phase& g) {
       }
       if (!touches) continue;
       if (vec) { ok = false; break; }
-      if (valid_after < 0) {
-        // the first touch has to store the whole tensor without reading it
-        if (!writes || reads || !writes_whole_node(r, ph, n.id)) { ok = false; break; }
-        valid_after = f.member;
-      }
+      // first touched by a store to all of it: valid from the next member on; else read in at the start
+      if (valid_after == -2) valid_after = writes && !reads && writes_whole_node(r, ph, n.id) ? f.member : -1;
+      if (reads && f.member > valid_after) pays = true;
     }
-    if (ok && valid_after >= 0 && valid_after + 1 < (int)g.serial_members.size()) {
+    if (ok && pays && valid_after >= -1) {
       g.serial_shadows[n.id] = valid_after;
       budget -= bytes;
     }
@@ -1581,6 +1583,15 @@ void serialise_tiny(const Routine& r, Plan& plan) {
   g.label = "whole routine, one workgroup";
   g.bytes = bytes;
   g.serial_members = std::move(plan.phases);
+  // The lanes that shared a sum hid the latency of memory; here the operands come from LDS, so a sum is shared
+  // only as far as the workgroup's (at most 1024) threads go round once.
+  for (auto& q : g.serial_members) {
+    if (q.kind != Phase::Generic) continue;
+    int64_t points = 1;
+    for (auto e : (q.members.empty() ? q.par_ext : q.row_outer_ext)) points *= e;
+    while (q.coop_lanes > 64 || (q.coop_lanes > 1 && points * q.coop_lanes > 1024 && (q.members.empty() || q.row_len <= 8 * q.coop_lanes))) q.coop_lanes /= 2;
+    if (q.coop_lanes == 1 && q.members.empty()) q.coop_scope = nullptr;
+  }
   choose_shadows(r, g);
   plan.phases.clear();
   plan.phases.push_back(std::move(g));
