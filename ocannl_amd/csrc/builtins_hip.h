@@ -190,8 +190,27 @@ OCN_DEV void ocn_lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-OCN_DEV float ocn_xshfl(float v, int m) { return __shfl_xor(v, m, 64); }
-OCN_DEV double ocn_xshfl(double v, int m) { return __shfl_xor(v, m, 64); }
+// The value of lane (own lane ^ m), m a power of two and a constant.  Through the data-parallel-primitive
+// modifiers and the row swaps, which take a few cycles and fold into the operation that follows; __shfl_xor
+// is a trip through LDS (address, permute, wait) per step, six in a row for a wave's sum.
+OCN_DEV unsigned ocn_xlane(unsigned v, int m) {
+  if (m == 1) return (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xF, 0xF, true);        // quad_perm [1,0,3,2]
+  if (m == 2) return (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xF, 0xF, true);        // quad_perm [2,3,0,1]
+  if (m == 4)                                                                                 // 7 - i, then i ^ 3
+    return (unsigned)__builtin_amdgcn_mov_dpp(__builtin_amdgcn_mov_dpp((int)v, 0x141, 0xF, 0xF, true), 0x1B, 0xF, 0xF, true);
+  if (m == 8) return (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x128, 0xF, 0xF, true);       // row_ror:8
+  if (m == 16) {   // odd rows of one copy against even rows of the other
+    const auto p = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    return (threadIdx.x & 16u) ? p[0] : p[1];
+  }
+  const auto p = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  return (threadIdx.x & 32u) ? p[0] : p[1];
+}
+OCN_DEV float ocn_xshfl(float v, int m) { return __uint_as_float(ocn_xlane(__float_as_uint(v), m)); }
+OCN_DEV double ocn_xshfl(double v, int m) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  return __longlong_as_double((long long)((unsigned long long)ocn_xlane((unsigned)(b >> 32), m) << 32 | ocn_xlane((unsigned)b, m)));
+}
 
 // ---- a contraction as the prologue of a row-wise kernel ---------------------------------------------
 // xs[32][T] = A[32][K] * B[T][K]^T for a workgroup of NW waves: bf16 operands, both unit-stride
