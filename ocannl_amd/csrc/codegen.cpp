@@ -1022,18 +1022,18 @@ uint64_t emit_window(const Routine& r, const Phase& ph, std::vector<std::string>
   operand(g.a); d << ", "; operand(g.b); d << ", "; three(g.c.row_stride); d << ", "; three(g.c.k_stride);
   d << ", 0, " << (g.accumulate ? 1 : 0) << ", 1, " << tm << ", " << tn << ", ";
   two(ph.win_s); d << ", "; two(ph.win_taps); d << ", "; two(ph.win_lim); d << ", "; two(ph.win_pos); d << "}";
-  const std::string shape = std::to_string(BM) + ", " + std::to_string(BN) + ", true, " + (bkc ? "true" : "false") + ", " + (f32 ? "true" : "false");
+  const std::string shape = std::to_string(BM) + ", " + std::to_string(BN) + ", true, " + (bkc ? "true" : "false") + ", ";
   const int64_t blocks = (tm * tn * residues + 7) / 8 * 8;
   body.push_back("  constexpr OcnAnyDesc d_ = " + d.str() + ";");
-  body.push_back("  __shared__ __attribute__((aligned(16))) unsigned char smem_[ocn_any_smem<" + shape + ">()];");
+  body.push_back("  __shared__ __attribute__((aligned(16))) unsigned char smem_[ocn_any_smem<" + shape + (f32 ? "true" : "false") + ">()];");
   body.push_back("  const int t_ = (int)(blockIdx.x % 8u) * " + std::to_string(blocks / 8) + " + (int)(blockIdx.x / 8u);");
   body.push_back("  if (t_ >= " + std::to_string(tm * tn * residues) + ") return;");
   body.push_back("  const int z_ = t_ / " + std::to_string(tm * tn) + ", q_ = t_ % " + std::to_string(tm * tn) + ", r0_ = z_ / " + std::to_string(ph.win_s[1]) +
                  ", r1_ = z_ % " + std::to_string(ph.win_s[1]) + ";");
-  body.push_back("  ocn_any_tile<" + shape + ", true>(d_, " + r.node(g.a.node).ident + " + " + std::to_string(g.a.offset) + ", " + r.node(g.b.node).ident + " + " +
+  body.push_back("  ocn_any_tile<" + shape + (g.a.prec == Prec::Bfloat16 ? "true, " : "false, ") + (g.b.prec == Prec::Bfloat16 ? "true" : "false") + ", true, 2>(d_, " + r.node(g.a.node).ident + " + " + std::to_string(g.a.offset) + ", " + r.node(g.b.node).ident + " + " +
                  std::to_string(g.b.offset) + " + r0_ * " + std::to_string(ph.win_b[0]) + " + r1_ * " + std::to_string(ph.win_b[1]) + ", " +
                  r.node(g.c.node).ident + " + " + std::to_string(g.c.offset) + " + r0_ * " + std::to_string(ph.win_c[0]) + " + r1_ * " +
-                 std::to_string(ph.win_c[1]) + ", (void*)0, (float*)0, q_ / " + std::to_string(tn) + ", q_ % " + std::to_string(tn) + ", 0, r0_, r1_, smem_);");
+                 std::to_string(ph.win_c[1]) + ", (void*)0, (float*)0, OcnAnyEpilogue{0, 0, 0}, q_ / " + std::to_string(tn) + ", q_ % " + std::to_string(tn) + ", 0, r0_, r1_, smem_);");
   return (uint64_t)blocks * 256;
 }
 

@@ -1,63 +1,13 @@
-// Library instances of the contraction tile for any extents and strides (contract_any.h) and their launch.
+// Contractions of any extents and strides: instances for bf16 operands, choice of the tile, launch.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cstdio>
 
-#include "contract_any.h"
-#include "gemm.hpp"
+#include "contract_any.hpp"
 
 namespace ocannl {
 namespace {
-
-struct AnyBatch {
-  int nbatch, batches, members;
-  int ext[3];
-  long a[3], b[3], c[3];      // element strides of the batch digits
-};
-struct AnyPtrs {
-  const void* a[4];
-  const void* b[4];
-  void* c[4];
-  void* c2[4];
-  float* ws;
-};
-
-// Batch entry z of the launch -> operands.
-__device__ __forceinline__ void any_operands(const OcnAnyDesc& d, const AnyBatch& q, const AnyPtrs& p, int z, const void*& a, const void*& b, void*& c,
-                                             void*& c2) {
-  const int g = q.members > 1 ? z / q.batches : 0;
-  int r = z - g * q.batches;
-  long ao = 0, bo = 0, co = 0;
-  if (q.nbatch > 2) { const int i = r % q.ext[2]; r /= q.ext[2]; ao += i * q.a[2]; bo += i * q.b[2]; co += i * q.c[2]; }
-  if (q.nbatch > 1) { const int i = r % q.ext[1]; r /= q.ext[1]; ao += i * q.a[1]; bo += i * q.b[1]; co += i * q.c[1]; }
-  if (q.nbatch > 0) { ao += r * q.a[0]; bo += r * q.b[0]; co += r * q.c[0]; }
-  a = g == 0 ? p.a[0] : g == 1 ? p.a[1] : g == 2 ? p.a[2] : p.a[3];
-  b = g == 0 ? p.b[0] : g == 1 ? p.b[1] : g == 2 ? p.b[2] : p.b[3];
-  c = g == 0 ? p.c[0] : g == 1 ? p.c[1] : g == 2 ? p.c[2] : p.c[3];
-  c2 = g == 0 ? p.c2[0] : g == 1 ? p.c2[1] : g == 2 ? p.c2[2] : p.c2[3];
-  a = static_cast<const char*>(a) + ao * (d.a.bf16 ? 2 : 4);
-  b = static_cast<const char*>(b) + bo * (d.b.bf16 ? 2 : 4);
-  c = static_cast<char*>(c) + co * (d.c_bf16 ? 2 : 4);
-  if (c2) c2 = static_cast<char*>(c2) + co * 2;
-}
-
-// Grid: x = tiles of all batch entries, padded to a multiple of eight and dealt so that each XCD (workgroup
-// ids go round robin) walks a contiguous range of them -- neighbouring tiles share panels through its L2;
-// y = K splits.
-template <int BM, int BN, bool A_KC, bool B_KC, bool F32>
-__global__ void __launch_bounds__(256) contract_any_kernel(const OcnAnyDesc d, const AnyBatch q, const AnyPtrs p) {
-  extern __shared__ __align__(16) unsigned char smem_any[];
-  const int per = gridDim.x / 8, tiles = d.tiles_m * d.tiles_n;
-  const int t = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
-  const int z = t / tiles, r = t - z * tiles;
-  if (z >= q.batches * q.members) return;
-  const void *a, *b;
-  void *c, *c2;
-  any_operands(d, q, p, z, a, b, c, c2);
-  float* const ws = d.splits > 1 ? p.ws + (long)z * d.splits * d.M * d.N : nullptr;
-  ocn_any_tile<BM, BN, A_KC, B_KC, F32, false>(d, a, b, c, c2, ws, r / d.tiles_n, r % d.tiles_n, (int)blockIdx.y, 0, 0, smem_any);
-}
 
 // Sums the K splits in index order and applies them to C.
 __global__ void __launch_bounds__(256) contract_any_reduce_kernel(const OcnAnyDesc d, const AnyBatch q, const AnyPtrs p) {
@@ -69,6 +19,7 @@ __global__ void __launch_bounds__(256) contract_any_reduce_kernel(const OcnAnyDe
   any_operands(d, q, p, z, a, b, c, c2);
   const float* ws = p.ws + (long)z * d.splits * cells + i;
   float v = 0.0f;
+#pragma unroll 16
   for (int s = 0; s < d.splits; ++s) v += ws[s * cells];
   const int m = (int)(i / d.N), n = (int)(i - (long)m * d.N);
   const long at = (long)ocn_digit_off(ocn_digits(d.dm, m), d.c_m) + ocn_digit_off(ocn_digits(d.dn, n), d.c_n);
@@ -94,6 +45,7 @@ OcnDigits digits_of(const int64_t (&ext)[3], int n) {
 }
 
 bool any_is_f32(const GemmDesc& d) { return d.a.prec != Prec::Bfloat16 || d.b.prec != Prec::Bfloat16; }
+bool any_mixed(const GemmDesc& d) { return d.a.prec != d.b.prec; }
 // k-contiguous (or contiguous along nothing), else row-contiguous
 bool any_kc(const GemmOperand& o) { return o.k_stride[2] == 1 || o.row_stride[2] != 1; }
 
@@ -106,47 +58,16 @@ long any_entries(const GemmDesc& d) {
 // 128 x 128 tiles when they fill the chip twice over, else 64 x 64 (128 x 32 or 32 x 128 when one extent is at most
 // 32: half of a square tile would be padding); K is split (never below 128 k a split) towards two workgroups
 // per compute unit when the tiles are fewer than one each.
-struct AnyShape { int bm, bn, splits; };
 AnyShape any_shape(const GemmDesc& d) {
   const long nb = any_entries(d);
   AnyShape s{64, 64, 1};
-  if (d.N <= 32) s = {128, 32, 1};
-  else if (d.M <= 32) s = {32, 128, 1};
-  else if (((d.M + 127) / 128) * ((d.N + 127) / 128) * nb >= 512) s = {128, 128, 1};
+  if (d.N <= 32 && !any_mixed(d)) s = {128, 32, 1};
+  else if (d.M <= 32 && !any_mixed(d)) s = {32, 128, 1};
+  else if (any_mixed(d)) s = {64, 64, 1};   // (the one tile built for a bf16 and an fp32 operand)
+  else if (d.M > 64 && d.N > 64 && ((d.M + 127) / 128) * ((d.N + 127) / 128) * nb >= 512) s = {128, 128, 1};
   const long tiles = ((d.M + s.bm - 1) / s.bm) * ((d.N + s.bn - 1) / s.bn) * nb;
-  if (tiles < 192) while ((long)s.splits * 2 * tiles <= 512 && d.K / (s.splits * 2) >= 128) s.splits *= 2;
+  if (tiles < 192 && d.epi_bias < 0 && d.epi_relu < 0) while ((long)s.splits * 2 * tiles <= 512 && d.K / (s.splits * 2) >= 128) s.splits *= 2;
   return s;
-}
-
-template <int BM, int BN, bool A_KC, bool B_KC, bool F32>
-hipError_t go(dim3 grid, const OcnAnyDesc& d, const AnyBatch& q, const AnyPtrs& p, hipStream_t s) {
-  constexpr int smem = ocn_any_smem<BM, BN, A_KC, B_KC, F32>();
-  if (smem > 65536) {
-    static thread_local bool configured = false;
-    if (!configured) {
-      hipError_t e = hipFuncSetAttribute((const void*)contract_any_kernel<BM, BN, A_KC, B_KC, F32>, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-      if (e != hipSuccess) return e;
-      configured = true;
-    }
-  }
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(contract_any_kernel<BM, BN, A_KC, B_KC, F32>), grid, dim3(256), smem, s, d, q, p);
-  return hipGetLastError();
-}
-
-template <int BM, int BN, bool F32>
-hipError_t launch_layout(bool akc, bool bkc, dim3 grid, const OcnAnyDesc& d, const AnyBatch& q, const AnyPtrs& p, hipStream_t s) {
-  if (akc && bkc) return go<BM, BN, true, true, F32>(grid, d, q, p, s);
-  if (akc) return go<BM, BN, true, false, F32>(grid, d, q, p, s);
-  if (bkc) return go<BM, BN, false, true, F32>(grid, d, q, p, s);
-  return go<BM, BN, false, false, F32>(grid, d, q, p, s);
-}
-
-template <bool F32>
-hipError_t launch_shape(const AnyShape& sh, bool akc, bool bkc, dim3 grid, const OcnAnyDesc& d, const AnyBatch& q, const AnyPtrs& p, hipStream_t s) {
-  if (sh.bn == 32) return launch_layout<128, 32, F32>(akc, bkc, grid, d, q, p, s);
-  if (sh.bm == 32) return launch_layout<32, 128, F32>(akc, bkc, grid, d, q, p, s);
-  if (sh.bm == 128) return launch_layout<128, 128, F32>(akc, bkc, grid, d, q, p, s);
-  return launch_layout<64, 64, F32>(akc, bkc, grid, d, q, p, s);
 }
 
 }  // namespace
@@ -155,7 +76,8 @@ const char* contract_any_name(const GemmDesc& d) {
   static thread_local char buf[96];
   const AnyShape s = any_shape(d);
   const char* tf[2] = {"false", "true"};
-  snprintf(buf, sizeof buf, "contract_any_kernel<%d, %d, %s, %s, %s>", s.bm, s.bn, tf[any_kc(d.a)], tf[any_kc(d.b)], tf[any_is_f32(d)]);
+  snprintf(buf, sizeof buf, "contract_any_kernel<%d, %d, %s, %s, %s, %s>", s.bm, s.bn, tf[any_kc(d.a)], tf[any_kc(d.b)], tf[d.a.prec == Prec::Bfloat16],
+           tf[d.b.prec == Prec::Bfloat16]);
   return buf;
 }
 
@@ -190,11 +112,16 @@ hipError_t launch_contract_any(const GemmDesc& g, const GemmArgs& in, void* work
   p.a[0] = in.a; p.b[0] = in.b; p.c[0] = in.c; p.c2[0] = in.c2;
   for (int i = 1; i < in.ngroups; ++i) { p.a[i] = in.a_more[i - 1]; p.b[i] = in.b_more[i - 1]; p.c[i] = in.c_more[i - 1]; p.c2[i] = in.c2_more[i - 1]; }
   p.ws = static_cast<float*>(workspace);
+  p.ep = {static_cast<const unsigned short*>(in.bias), static_cast<unsigned short*>(in.relu_out), in.relu_c};
   const long entries = (long)q.batches * q.members, tiles = (long)d.tiles_m * d.tiles_n * entries;
   if (tiles <= 0 || tiles > 0x3FFFFFFFL || entries > 65535 || in.npairs != 1 || (sh.splits > 1 && !p.ws)) return hipErrorInvalidValue;
   const dim3 grid((unsigned)((tiles + 7) / 8 * 8), (unsigned)sh.splits, 1);
   const bool akc = any_kc(g.a), bkc = any_kc(g.b), f32 = any_is_f32(g);
-  hipError_t e = f32 ? launch_shape<true>(sh, akc, bkc, grid, d, q, p, s) : launch_shape<false>(sh, akc, bkc, grid, d, q, p, s);
+  hipError_t e = f32 ? launch_any_f32(sh.bm, sh.bn, d.a.bf16, d.b.bf16, akc, bkc, grid, d, &q, &p, s)
+                 : sh.bn == 32 ? launch_layout<128, 32, true, true>(akc, bkc, grid, d, q, p, s)
+                 : sh.bm == 32 ? launch_layout<32, 128, true, true>(akc, bkc, grid, d, q, p, s)
+                 : sh.bm == 128 ? launch_layout<128, 128, true, true>(akc, bkc, grid, d, q, p, s)
+                                : launch_layout<64, 64, true, true>(akc, bkc, grid, d, q, p, s);
   if (e == hipSuccess && after_main) e = hipEventRecord(after_main, s);
   if (e != hipSuccess || sh.splits == 1) return e;
   const long cells = (long)d.M * d.N;
