@@ -76,8 +76,10 @@ const char* contract_any_name(const GemmDesc& d) {
   static thread_local char buf[96];
   const AnyShape s = any_shape(d);
   const char* tf[2] = {"false", "true"};
-  snprintf(buf, sizeof buf, "contract_any_kernel<%d, %d, %s, %s, %s, %s>", s.bm, s.bn, tf[any_kc(d.a)], tf[any_kc(d.b)], tf[d.a.prec == Prec::Bfloat16],
-           tf[d.b.prec == Prec::Bfloat16]);
+  if (!any_is_f32(d)) snprintf(buf, sizeof buf, "gemm_bf16_kernel_any<%d, %d, %s, %s>", s.bm, s.bn, tf[any_kc(d.a)], tf[any_kc(d.b)]);
+  else
+    snprintf(buf, sizeof buf, "gemm_f32_kernel_any<%d, %d, %s, %s, %s, %s>", s.bm, s.bn, tf[any_kc(d.a)], tf[any_kc(d.b)], tf[d.a.prec == Prec::Bfloat16],
+             tf[d.b.prec == Prec::Bfloat16]);
   return buf;
 }
 

@@ -50,7 +50,7 @@ __device__ __forceinline__ void any_operands(const OcnAnyDesc& d, const AnyBatch
 // ids go round robin) walks a contiguous range of them -- neighbouring tiles share panels through its L2;
 // y = K splits.
 template <int BM, int BN, bool A_KC, bool B_KC, bool ABF, bool BBF>
-__global__ void __launch_bounds__(256) contract_any_kernel(const OcnAnyDesc d, const AnyBatch q, const AnyPtrs p) {
+__device__ __forceinline__ void any_body(const OcnAnyDesc& d, const AnyBatch& q, const AnyPtrs& p) {
   extern __shared__ __align__(16) unsigned char smem_any[];
   const int per = gridDim.x / 8, tiles = d.tiles_m * d.tiles_n;
   const int t = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
@@ -63,18 +63,30 @@ __global__ void __launch_bounds__(256) contract_any_kernel(const OcnAnyDesc d, c
   ocn_any_tile<BM, BN, A_KC, B_KC, ABF, BBF, false, kAnyDepth>(d, a, b, c, c2, ws, p.ep, r / d.tiles_n, r % d.tiles_n, (int)blockIdx.y, 0, 0, smem_any);
 }
 
+template <int BM, int BN, bool A_KC, bool B_KC>
+__global__ void __launch_bounds__(256) gemm_bf16_kernel_any(const OcnAnyDesc d, const AnyBatch q, const AnyPtrs p) {
+  any_body<BM, BN, A_KC, B_KC, true, true>(d, q, p);
+}
+template <int BM, int BN, bool A_KC, bool B_KC, bool ABF, bool BBF>
+__global__ void __launch_bounds__(256) gemm_f32_kernel_any(const OcnAnyDesc d, const AnyBatch q, const AnyPtrs p) {
+  any_body<BM, BN, A_KC, B_KC, ABF, BBF>(d, q, p);
+}
+
 template <int BM, int BN, bool A_KC, bool B_KC, bool ABF, bool BBF>
 hipError_t go(dim3 grid, const OcnAnyDesc& d, const AnyBatch& q, const AnyPtrs& p, hipStream_t s) {
   constexpr int smem = ocn_any_smem<BM, BN, A_KC, B_KC, !(ABF && BBF)>();
+  void (*kernel)(OcnAnyDesc, AnyBatch, AnyPtrs);
+  if constexpr (ABF && BBF) kernel = gemm_bf16_kernel_any<BM, BN, A_KC, B_KC>;
+  else kernel = gemm_f32_kernel_any<BM, BN, A_KC, B_KC, ABF, BBF>;
   if (smem > 65536) {
     static thread_local bool configured = false;
     if (!configured) {
-      hipError_t e = hipFuncSetAttribute((const void*)contract_any_kernel<BM, BN, A_KC, B_KC, ABF, BBF>, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+      hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
       if (e != hipSuccess) return e;
       configured = true;
     }
   }
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(contract_any_kernel<BM, BN, A_KC, B_KC, ABF, BBF>), grid, dim3(256), smem, s, d, q, p);
+  hipLaunchKernelGGL(kernel, grid, dim3(256), smem, s, d, q, p);
   return hipGetLastError();
 }
 

@@ -521,6 +521,16 @@ bool dtl_operands_ok(const GemmArgs& a, bool akc, bool bkc) {
 
 }  // namespace
 
+// Fewer 128 x 128 tiles than compute units: the register-staged kernels leave some idle and hide no latency on the
+// rest, where 64 x 64 tiles of contract_any.hip put several workgroups on each.  Measured with both gradients, before ->
+// now: 1784 x 776 x 1000 bf16 67 -> 57 us, fp32 231 -> 141; 594 x 320 x 320 bf16 33 -> 26; 512 x 512 x 512 fp32
+// 129 -> 37.  From 256 tiles on the larger tile wins (8000 x 1000 x 1000 bf16: 122 against 173 us).
+bool gemm_prefers_any(const GemmDesc& d) {
+  if (d.any || !d.more.empty() || d.a.prec != d.b.prec) return false;
+  if (((d.M + 127) / 128) * ((d.N + 127) / 128) * batch_count(d) >= 256) return false;
+  return d.a.prec == Prec::Single || dtl_shape(d).bm == 0;
+}
+
 const char* gemm_kernel_name(const GemmDesc& d) {
   if (d.any) return contract_any_name(d);
   // the instantiation as a profiler prints it (without namespaces)

@@ -60,6 +60,9 @@ size_t gemm_workspace_bytes(const GemmDesc& desc);
 // Name of the instance launch_gemm would pick (for kernel_info and profiles).
 const char* gemm_kernel_name(const GemmDesc& desc);
 
+// Is this contraction, which the kernels of gemm.hip could take, faster as one of any shape (contract_any.hip)?
+bool gemm_prefers_any(const GemmDesc& desc);
+
 // contract_any.hip: the same for contractions with `desc.any` set (launch_gemm and its siblings forward to these).
 hipError_t launch_contract_any(const GemmDesc& desc, const GemmArgs& args, void* workspace, hipStream_t stream, hipEvent_t after_main);
 size_t contract_any_workspace_bytes(const GemmDesc& desc);

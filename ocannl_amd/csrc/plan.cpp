@@ -1,3 +1,4 @@
+#include "gemm.hpp"
 #include "plan.hpp"
 
 #include <algorithm>
@@ -2532,6 +2533,17 @@ Plan make_plan(Routine& r, const PlanOptions& requested) {
   if (opt.enable_coop && opt.enable_row_groups) group_rows(r, plan);
   if (opt.enable_mfma && opt.enable_coop && opt.enable_row_groups && opt.fuse_row_contractions) fuse_row_contractions(r, plan, opt.fuse_stored_rows, opt.row_tile_waves);
   if (opt.enable_mfma && opt.enable_coop && opt.enable_row_groups && opt.fuse_row_contractions && opt.fuse_row_projections) fuse_row_projections(r, plan);
+  if (opt.enable_mfma && opt.any_contractions) {
+    for (auto& ph : plan.phases) {
+      if (ph.kind != Phase::Contraction || !gemm_prefers_any(ph.gemm)) continue;
+      GemmDesc& g = ph.gemm;
+      auto digits = [](GemmOperand& o) { o.row_stride[2] = o.s_row; o.k_stride[2] = o.s_k; };
+      digits(g.a); digits(g.b); digits(g.c);
+      for (auto& m : g.group) { digits(m.a); digits(m.b); digits(m.c); }
+      g.m_ext[2] = g.M; g.n_ext[2] = g.N; g.k_ext[2] = g.K;
+      g.any = true;
+    }
+  }
   if (opt.enable_serial_group) serialise_tiny(r, plan);
   if (opt.enable_coop && opt.enable_parallel_groups) group_independent(r, plan);
   if (opt.enable_mfma && opt.side_queue && r.merge_node < 0) assign_side_queue(plan, opt.side_queue_generated);

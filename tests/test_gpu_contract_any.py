@@ -25,7 +25,7 @@ def _run(r, nodes, out, want, accumulate, k, seed=0):
     ks = [x for x in hip.code.kernels() if x["kind"] == "mfma"]
     if not ks and nodes[out].prec == "bfloat16":   # a bf16 sum that one thread runs: rounded after every addition, left alone
         return hip.close()
-    assert ks and all("contract_any" in x["name"] for x in ks), hip.code.kernels()
+    assert ks and all("_kernel_any" in x["name"] for x in ks), hip.code.kernels()
     hip.step()
     f = {name: W.to_float(init[n.id], n.prec).astype(np.float64) for name, n in nodes.items()}
     ref = want(f) + (f[out] if accumulate else 0.0)
