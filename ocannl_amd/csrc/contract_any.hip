@@ -56,8 +56,9 @@ long any_entries(const GemmDesc& d) {
 }
 
 // 128 x 128 tiles when they fill the chip twice over, else 64 x 64 (128 x 32 or 32 x 128 when one extent is at most
-// 32: half of a square tile would be padding); K is split (never below 128 k a split) towards two workgroups
-// per compute unit when the tiles are fewer than one each.
+// 32: half of a square tile would be padding).  K is split towards two workgroups per compute unit when the tiles
+// are fewer than one each and a split keeps a dozen K steps (about 0.3 us each, twice that in fp32): the launch that
+// sums the splits costs 4.5 us, which fewer steps do not give back.
 AnyShape any_shape(const GemmDesc& d) {
   const long nb = any_entries(d);
   AnyShape s{64, 64, 1};
@@ -66,7 +67,7 @@ AnyShape any_shape(const GemmDesc& d) {
   else if (any_mixed(d)) s = {64, 64, 1};   // (the one tile built for a bf16 and an fp32 operand)
   else if (d.M > 64 && d.N > 64 && ((d.M + 127) / 128) * ((d.N + 127) / 128) * nb >= 512) s = {128, 128, 1};
   const long tiles = ((d.M + s.bm - 1) / s.bm) * ((d.N + s.bn - 1) / s.bn) * nb;
-  if (tiles < 192 && d.epi_bias < 0 && d.epi_relu < 0) while ((long)s.splits * 2 * tiles <= 512 && d.K / (s.splits * 2) >= 128) s.splits *= 2;
+  if (tiles < 192 && d.epi_bias < 0 && d.epi_relu < 0) while ((long)s.splits * 2 * tiles <= 512 && d.K / (s.splits * 2) >= (any_is_f32(d) ? 384 : 768)) s.splits *= 2;
   return s;
 }
 
