@@ -384,8 +384,23 @@ struct Printer {
       // (the last positions of a row that is not a multiple of the lanes are missing)
       return head + row_pos(lanes) + ";" + (to + 1 < (int64_t)row_iters * lanes ? " if (" + sym + " > " + std::to_string(to) + ") continue;" : "");
     }
-    return ind + "for (" + idx_t + " " + sym + " = " + std::to_string(from) + " + lane_; " + sym + " <= " + std::to_string(to) +
+    return ind + (to - from + 1 > 2 * lanes ? "_Pragma(\"unroll 4\") " : "") + "for (" + idx_t + " " + sym + " = " + std::to_string(from) + " + lane_; " + sym + " <= " + std::to_string(to) +
            "; " + sym + " += " + std::to_string(lanes) + ") {";
+  }
+  // One loop over the whole range of several (`sym`, `from`, `to`; slowest first), shared by `lanes` lanes.
+  struct Loop { int sym; int64_t from, to; };
+  std::vector<std::string> flat_loop(const std::vector<Loop>& loops, int lanes, const std::string& ind) {
+    int64_t total = 1;
+    for (auto& l : loops) total *= l.to - l.from + 1;
+    std::vector<std::string> out;
+    out.push_back(ind + "_Pragma(\"unroll 4\") for (" + idx_t + " flat_ = lane_; flat_ < " + std::to_string(total) + "u; flat_ += " + std::to_string(lanes) + ") {");
+    std::string rest = "flat_";
+    for (size_t i = loops.size(); i-- > 0;) {
+      const std::string ext = std::to_string(loops[i].to - loops[i].from + 1) + "u";
+      out.push_back(ind + "  const " + idx_t + " " + sym_ident(loops[i].sym) + " = " + std::to_string(loops[i].from) + " + " + (i ? rest + " % " + ext : rest) + ";");
+      rest = "(" + rest + " / " + ext + ")";
+    }
+    return out;
   }
   // row group with a contraction prologue: reads of this node come from the LDS tile `xs_` that the
   // kernel computed itself: [row of the tile][row position]
@@ -642,7 +657,13 @@ struct Printer {
     Def d; d.scope = s.scope.scope;
     d.lines.push_back(ind + (dbl ? "double " : "float ") + part + " = " + neutral_literal(coop_accum, dbl) + ";");
     std::string ci = ind;
-    for (size_t i = 0; i < loops.size(); ++i) {
+    const bool flat = loops.size() > 1 && row_iters == 0 && coop_lanes > loops.back()->to - loops.back()->from + 1;
+    if (flat) {
+      std::vector<Loop> ls;
+      for (auto* l : loops) ls.push_back({l->sym, l->from, l->to});
+      for (auto& l : flat_loop(ls, coop_lanes, ci)) d.lines.push_back(l);
+      ci += "  ";
+    } else for (size_t i = 0; i < loops.size(); ++i) {
       const std::string sy = sym_ident(loops[i]->sym);
       if (i + 1 == loops.size())
         d.lines.push_back(row_loop(sy, loops[i]->from, loops[i]->to, coop_lanes, ci));
@@ -664,7 +685,7 @@ struct Printer {
       line = part + " = " + combine_expr(coop_accum, dbl, part, widen(e)) + ";";
     }
     with_defs(inner_defs, {line}, ci, d.lines);
-    for (size_t i = 0; i < loops.size(); ++i) { ci.resize(ci.size() - 2); d.lines.push_back(ci + "}"); }
+    for (size_t i = 0; i < (flat ? 1 : loops.size()); ++i) { ci.resize(ci.size() - 2); d.lines.push_back(ci + "}"); }
     group_reduce(part, coop_accum, dbl, coop_lanes, ind, d.lines);
     Pair narrow = convert_precision(accP, sp);
     d.lines.push_back(ind + c_typ(sp) + " " + scope_name(s.scope) + " = " + narrow.first + part + narrow.second + ";");
@@ -688,6 +709,30 @@ struct Printer {
     out.push_back(ind + "}");
   }
 
+  // The loads of a short loop body wait for one another's trip when the loop is left rolled: several iterations at
+  // a time, fewer where each costs a division or a transcendental.  Up to 32 trips the compiler unrolls whole by
+  // itself, and a factor would stop it (a step of 20-trip loops in LDS: 5.5 us so, 6.4 us with a factor of 8).
+  static bool has_loop(const Block& b) {
+    for (auto& s : b) {
+      if (s->kind == Stmt::For || has_loop(s->body)) return true;
+      if (s->value && has_loop(*s->value)) return true;
+    }
+    return false;
+  }
+  static bool has_loop(const Scalar& x) {
+    return (x.kind == Scalar::LocalScope && has_loop(x.body)) || (x.a && has_loop(*x.a)) || (x.b && has_loop(*x.b)) || (x.c && has_loop(*x.c));
+  }
+  static bool heavy(const Scalar& x) {
+    if (x.kind == Scalar::Un && x.un != Unop::Id && x.un != Unop::Neg && x.un != Unop::Relu) return true;
+    if (x.kind == Scalar::Bin && (x.bin == Binop::Div || x.bin == Binop::Pow || x.bin == Binop::Mod)) return true;
+    if (x.kind == Scalar::LocalScope) for (auto& s : x.body) if (s->value && heavy(*s->value)) return true;
+    return (x.a && heavy(*x.a)) || (x.b && heavy(*x.b)) || (x.c && heavy(*x.c));
+  }
+  std::string unroll_of(const Block& body, int64_t trips) const {
+    if (debug_log || trips <= 32 || body.size() != 1 || !body[0]->value || has_loop(body)) return "";
+    return std::string("_Pragma(\"unroll ") + (heavy(*body[0]->value) ? "2" : "8") + "\") ";
+  }
+
   void stmt(const Stmt& c, const std::string& ind, std::vector<std::string>& out) {
     switch (c.kind) {
       case Stmt::Comment:
@@ -696,7 +741,7 @@ struct Printer {
         break;
       case Stmt::For: {
         const std::string s = sym_ident(c.sym);
-        out.push_back(ind + "for (" + idx_t + " " + s + " = " + std::to_string(c.from) + "; " + s + " <= " +
+        out.push_back(ind + unroll_of(c.body, c.to - c.from + 1) + "for (" + idx_t + " " + s + " = " + std::to_string(c.from) + "; " + s + " <= " +
                       std::to_string(c.to) + "; ++" + s + ") {");
         if (debug_log) out.push_back(ind + "  " + log_call("index " + s + " = %d", {"(int)(" + s + ")"}));   // c_syntax.ml:458-465
         block(c.body, ind + "  ", out);
@@ -891,19 +936,27 @@ void emit_phase_statements(const Routine& r, Printer& pr, const Phase& ph, int G
     // one and the same element (not so for sums of symbols on an axis, convolution-style)
     for (auto& ix : set->idcs) for (int q : ph.seq_syms) if (ix.mentions(q)) is_reduction = false;
   }
+  const bool flat = G > 1 && ph.seq_syms.size() > 1 && !ph.coop_scope && pr.row_iters == 0 && G > ph.seq_to.back() - ph.seq_from.back() + 1;
   auto open_seq_loops = [&](std::string& cur_ind, bool coop_last) {
+    if (coop_last && flat) {
+      std::vector<Printer::Loop> ls;
+      for (size_t i = 0; i < ph.seq_syms.size(); ++i) ls.push_back({ph.seq_syms[i], ph.seq_from[i], ph.seq_to[i]});
+      for (auto& l : pr.flat_loop(ls, G, cur_ind)) body.push_back(l);
+      cur_ind += "  ";
+      return;
+    }
     for (size_t i = 0; i < ph.seq_syms.size(); ++i) {
       const std::string s = sym_ident(ph.seq_syms[i]);
       if (coop_last && i + 1 == ph.seq_syms.size())
         body.push_back(pr.row_loop(s, ph.seq_from[i], ph.seq_to[i], G, cur_ind));
       else
-        body.push_back(cur_ind + "for (" + pr.idx_t + " " + s + " = " + std::to_string(ph.seq_from[i]) + "; " + s + " <= " +
-                       std::to_string(ph.seq_to[i]) + "; ++" + s + ") {");
+        body.push_back(cur_ind + (i + 1 == ph.seq_syms.size() ? pr.unroll_of(ph.inner, ph.seq_to[i] - ph.seq_from[i] + 1) : "") + "for (" + pr.idx_t + " " + s + " = " +
+                       std::to_string(ph.seq_from[i]) + "; " + s + " <= " + std::to_string(ph.seq_to[i]) + "; ++" + s + ") {");
       cur_ind += "  ";
     }
   };
-  auto close_seq_loops = [&](std::string& cur_ind) {
-    for (size_t i = 0; i < ph.seq_syms.size(); ++i) { cur_ind.resize(cur_ind.size() - 2); body.push_back(cur_ind + "}"); }
+  auto close_seq_loops = [&](std::string& cur_ind, bool coop_last) {
+    for (size_t i = 0; i < (coop_last && flat ? 1 : ph.seq_syms.size()); ++i) { cur_ind.resize(cur_ind.size() - 2); body.push_back(cur_ind + "}"); }
   };
   const bool guard = lane0_store || ph.coop_scope;
   const std::string lane0 = guard && G > 1 ? "if (lane_ == 0) " : "";
@@ -933,7 +986,7 @@ void emit_phase_statements(const Routine& r, Printer& pr, const Phase& ph, int G
       lines.push_back("part_ = " + combine_expr(accum, dbl, "part_", widen(es)) + ";");
     }
     pr.with_defs(defs, lines, ci, body);
-    close_seq_loops(ci);
+    close_seq_loops(ci, true);
     pr.group_reduce("part_", accum, dbl, G, ind, body);
     const std::string lhs = n.ident + "[" + offset_str(set->idcs, n.dims) + "]";
     Pair narrow = convert_precision(accP, n.prec);
@@ -963,7 +1016,7 @@ void emit_phase_statements(const Routine& r, Printer& pr, const Phase& ph, int G
     std::string v = pr.scalar(n.prec, *set->value, ci + "  ", defs);
     pr.with_defs(defs, {"acc_ = " + v + ";"}, ci, body);
     pr.self_set = nullptr;
-    close_seq_loops(ci);
+    close_seq_loops(ci, false);
     body.push_back(ind + pr.store_line(set->node, lhs, "acc_", lane0));
     pr.coop_scope = nullptr;
   } else {
@@ -975,7 +1028,7 @@ void emit_phase_statements(const Routine& r, Printer& pr, const Phase& ph, int G
     pr.block(ph.inner, ci, body);
     pr.store_guard.clear();
     pr.coop_scope = nullptr;
-    close_seq_loops(ci);
+    close_seq_loops(ci, false);
   }
 }
 

@@ -555,7 +555,9 @@ void choose_scope_coop(const Routine& r, Phase& ph) {
   int64_t P = 1, R = 1;
   for (auto e : ph.par_ext) P *= e;
   for (const Stmt* l : loops) R *= l->to - l->from + 1;
-  const int64_t rext = loops.back()->to - loops.back()->from + 1;
+  // several loops with a short innermost one: the lanes share all of them as one range
+  const int64_t inner = loops.back()->to - loops.back()->from + 1;
+  const int64_t rext = loops.size() > 1 && inner < 64 ? R : inner;
   // one thread per point walks its own row: adjacent threads are a whole row apart, so sharing
   // the row between adjacent lanes is what makes the reads coalesce
   std::vector<Access> acc; bool f = false; std::set<ScopeId> d;
@@ -610,10 +612,12 @@ void choose_coop(const Routine& r, Phase& ph, const PlanOptions& opt) {
   const Stmt& set = *ph.inner[0];
   const Prec p = r.node(set.node).prec;
   if (!(p == Prec::Single || p == Prec::Double || p == Prec::Bfloat16 || p == Prec::Half)) return;
-  const int64_t rext = ph.seq_to.back() - ph.seq_from.back() + 1;
   int64_t P = 1, R = 1;
   for (auto e : ph.par_ext) P *= e;
   for (size_t i = 0; i < ph.seq_syms.size(); ++i) R *= ph.seq_to[i] - ph.seq_from[i] + 1;
+  // several loops with a short innermost one: the lanes share all of them as one range
+  const int64_t inner = ph.seq_to.back() - ph.seq_from.back() + 1;
+  const int64_t rext = ph.seq_syms.size() > 1 && inner < 64 && !ph.sums_partials ? R : inner;
   auto pow2_floor = [](int64_t x) { int64_t p2 = 1; while (p2 * 2 <= x) p2 *= 2; return p2; };
   if (ph.sums_partials) {
     // One thread per output would walk all the slices alone: a few thousand threads, each waiting on
