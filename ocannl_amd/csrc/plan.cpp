@@ -2370,6 +2370,18 @@ void fold_epilogues(Routine& r, Plan& plan) {
 
 }  // namespace
 
+// At least 16 launches (fewer do not win back what launching a graph costs) of about a microsecond of work or less on
+// average, at 2 TB/s and 200 TFLOP/s; longer kernels hide the host's time to launch the next.
+static bool many_short_launches(const Plan& plan) {
+  double us = 0;
+  for (auto& ph : plan.phases) {
+    if (ph.stream != 0) return false;
+    us += ph.bytes / 2e6;
+    if (ph.kind == Phase::Contraction) us += 2.0 * ph.gemm.M * ph.gemm.N * ph.gemm.K * ph.gemm.nbatch / 2e8;
+  }
+  return plan.phases.size() >= 16 && us < (double)plan.phases.size();
+}
+
 Plan make_plan(Routine& r, const PlanOptions& requested) {
   PlanOptions opt = requested;
   if (r.merge_node >= 0) {
@@ -2386,7 +2398,6 @@ Plan make_plan(Routine& r, const PlanOptions& requested) {
   Plan plan;
   plan.debug_log = opt.debug_log;
   plan.row_vec4 = opt.row_vec4;
-  plan.use_graphs = opt.use_graphs;
   plan.large_index = opt.large_models;
   for (auto& kv : r.nodes) if (kv.second.num_elems() > (int64_t)0x7FFFFFFF) plan.large_index = true;
   std::string label;
@@ -2551,6 +2562,7 @@ Plan make_plan(Routine& r, const PlanOptions& requested) {
   if (opt.enable_serial_group) serialise_tiny(r, plan);
   if (opt.enable_coop && opt.enable_parallel_groups) group_independent(r, plan);
   if (opt.enable_mfma && opt.side_queue && r.merge_node < 0) assign_side_queue(plan, opt.side_queue_generated);
+  plan.use_graphs = opt.graphs > 0 || (opt.graphs < 0 && many_short_launches(plan));
   return plan;
 }
 

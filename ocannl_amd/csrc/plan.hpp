@@ -112,8 +112,9 @@ struct Phase {
   // (dozens of launches of a few microseconds each would otherwise be pure launch latency).
   std::vector<Phase> serial_members;
   // Serial group: tensors whose first touch in the kernel is a store to all of their elements are
-  // shadowed in LDS (node -> index of the member that makes the shadow valid): later members read
-  // the shadow instead of waiting on global memory; every store still goes to global memory too.
+  // shadowed in LDS (node -> index of the member that makes the shadow valid, -1: read in at the
+  // start): later members read the shadow instead of waiting on global memory; every store still
+  // goes to global memory too.
   std::map<int, int> serial_shadows;
   // Parallel group (kind Generic, `parallel_members` non-empty): consecutive small phases that do not
   // depend on one another (the updates of many small parameters) run as ONE kernel in which every
@@ -189,11 +190,11 @@ struct PlanOptions {
   // measured on the transformer step the wide accesses were 5-8% slower than one position per lane
   // per unrolled iteration (these kernels are bound by the memory system, not by instruction count).
   bool row_vec4 = false;
-  // plain runs replay a captured HIP graph of the routine's kernels.  Off by default: measured on
-  // MI355X / ROCm 7.2 it pays only for a routine of about ten tiny kernels (half-moons step as ten
-  // launches: 40 -> 26 us); nine kernels of the char-MLP step went 36 -> 42 us and the 127 kernels of
-  // the transformer step 3.68 -> 3.73 ms.
-  bool use_graphs = false;
+  // Plain runs replay a captured HIP graph of the routine's kernels: 1 always, 0 never, -1 where it pays.  Launched
+  // one by one a kernel costs the host 3.2 us, replayed 1.1 us plus about 6 us per graph, so it pays for many kernels
+  // that each run for less than that: 48 kernels of a small transformer step 155 -> 103 us, nine of the char-MLP step
+  // 29.3 -> 29.0 us, 65 kernels of 8 us each 529 -> 533 us.
+  int graphs = -1;
   int group_window = 1 << 30;        // contractions share a launch only when at most this many phases apart
   // contractions off the critical path run on a second queue beside the rest (side_queue=1).  Off:
   // measured on the transformer step it gains 0.9 % (3.528 -> 3.495 ms), less than the step varies from

@@ -158,7 +158,7 @@ PlanOptions parse_options(const char* options) {
     else if (k == "side_queue") { o.side_queue = v != "0"; o.side_queue_generated = v == "2"; }
     else if (k == "debug_log") o.debug_log = v != "0";
     else if (k == "row_vec") o.row_vec4 = v != "0";
-    else if (k == "graphs") o.use_graphs = v != "0";
+    else if (k == "graphs") o.graphs = v != "0";
     else if (k == "group_window") o.group_window = std::stoi(v);
     else if (k == "epilogues") o.fuse_epilogues = v != "0";
     else if (k == "proj") o.fuse_row_projections = v != "0";
@@ -241,8 +241,7 @@ struct ocannl_hip_routine {
   // Replay: the kernel list of a plain run, captured once per combination of static-index values into
   // a HIP graph (fills recorded as kernels, the side queue as a branch) and launched as one unit from
   // then on: a routine of many short kernels stops paying a host call and a queue round trip per kernel.
-  std::map<std::vector<int64_t>, hipGraphExec_t> graphs;
-  bool warmed = false;               // one direct run first (it configures kernel attributes)
+  std::map<std::vector<int64_t>, hipGraphExec_t> graphs;   // null: run once with these values, directly
   int log_id = 0;                    // debug logging: prefix of this run's log lines (cuda_backend.ml:992-993)
   // Everything that names arena memory exists twice: [0] bound to the routine's own arena, [1] bound to
   // the library's static scratch array (valid when static_ok).
@@ -301,7 +300,7 @@ void destroy_routine(ocannl_hip_routine* rt) {
     if (kv.second.second) (void)hipEventDestroy(kv.second.second);
   }
   if (!rt->side_events.empty()) (void)hipStreamSynchronize(rt->dev->side_stream);
-  for (auto& kv : rt->graphs) (void)hipGraphExecDestroy(kv.second);
+  for (auto& kv : rt->graphs) if (kv.second) (void)hipGraphExecDestroy(kv.second);
   for (auto e : rt->profile_events) (void)hipEventDestroy(e);
   if (rt->module) (void)hipModuleUnload(rt->module);
   if (rt->scratch) { (void)hipFree(rt->scratch); rt->dev->scratch_used -= rt->scratch_bytes; }
@@ -310,9 +309,11 @@ void destroy_routine(ocannl_hip_routine* rt) {
 }
 
 // `v` = 0: the routine's own arena; 1: the library's static scratch array, with fills as kernels
-// and no call that allocates (no events: kernel_ms must be null and bracketing is off).
-void enqueue(ocannl_hip_routine& rt, float* kernel_ms, int cap, int v = 0, bool capturing = false) {
+// and no call that allocates (no events: kernel_ms must be null and bracketing is off).  `capture`: a stream in
+// capture to record into, in place of the device's.
+void enqueue(ocannl_hip_routine& rt, float* kernel_ms, int cap, int v = 0, hipStream_t capture = nullptr) {
   ocannl_hip_device& dev = *rt.dev;
+  const hipStream_t main = capture ? capture : dev.stream;
   dev.make_current();
   const Routine& r = rt.code->r;
   // static indices: range check, then publish (cuda_backend.ml:1015-1030)
@@ -374,7 +375,7 @@ void enqueue(ocannl_hip_routine& rt, float* kernel_ms, int cap, int v = 0, bool 
       hip_check(hipEventCreate(&e), "hipEventCreate");
       rt.timing_events.push_back(e);
     }
-    hip_check(hipEventRecord(rt.timing_events[0], dev.stream), "hipEventRecord");
+    hip_check(hipEventRecord(rt.timing_events[0], main), "hipEventRecord");
   }
   // The side queue is used by plain runs over the routine's own arena; per-kernel timing and the
   // static-scratch variant keep everything in order on the main queue.
@@ -384,16 +385,16 @@ void enqueue(ocannl_hip_routine& rt, float* kernel_ms, int cap, int v = 0, bool 
     auto& l = rt.launches[li];
     const Phase& ph = rt.code->plan.phases[l.phase];
     const bool on_side = two_queues && ph.stream == 1;
-    hipStream_t stream = on_side ? dev.side_stream : dev.stream;
+    hipStream_t stream = on_side ? dev.side_stream : main;
     if (on_side) {
       auto& ev = rt.side_events.at((int)li);
-      hip_check(hipEventRecord(ev.first, dev.stream), "hipEventRecord");
+      hip_check(hipEventRecord(ev.first, main), "hipEventRecord");
       hip_check(hipStreamWaitEvent(dev.side_stream, ev.first, 0), "hipStreamWaitEvent");
     } else if (two_queues) {
       int need = -1;
       for (int p : ph.wait_for) need = std::max(need, p);
       if (need > joined) {   // (the side queue runs in order: its latest phase stands for the earlier ones)
-        hip_check(hipStreamWaitEvent(dev.stream, rt.side_events.at(need).second, 0), "hipStreamWaitEvent");
+        hip_check(hipStreamWaitEvent(main, rt.side_events.at(need).second, 0), "hipStreamWaitEvent");
         joined = need;
       }
     }
@@ -407,11 +408,11 @@ void enqueue(ocannl_hip_routine& rt, float* kernel_ms, int cap, int v = 0, bool 
       hip_check(hipEventRecord(rt.profile_events[rt.profile_used], stream), "hipEventRecord");
     }
     if (ph.kind == Phase::Fill) {
-      if (v == 0 && !capturing) {
-        hip_check(hipMemsetAsync(l.fill_ptr[0], 0, l.fill_bytes, dev.stream), "hipMemsetAsync");
+      if (v == 0 && !capture) {
+        hip_check(hipMemsetAsync(l.fill_ptr[0], 0, l.fill_bytes, main), "hipMemsetAsync");
       } else {
         const uint64_t n16 = l.fill_bytes / 16 + 1;   // one thread per 16-byte store; the first block's 256 threads also cover the <= 15 head and tail bytes
-        hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)((n16 + 255) / 256)), dim3(256), 0, dev.stream,
+        hipLaunchKernelGGL(fill_zero_kernel, dim3((unsigned)((n16 + 255) / 256)), dim3(256), 0, main,
                            static_cast<unsigned char*>(l.fill_ptr[v]), l.fill_bytes);
         hip_check(hipGetLastError(), "fill_zero_kernel");
       }
@@ -457,7 +458,7 @@ void enqueue(ocannl_hip_routine& rt, float* kernel_ms, int cap, int v = 0, bool 
       hip_check(hipEventRecord(rt.side_events.at((int)li).second, dev.side_stream), "hipEventRecord");
       last_side = (int)li;
     }
-    if (timed) hip_check(hipEventRecord(rt.timing_events[li + 1], dev.stream), "hipEventRecord");
+    if (timed) hip_check(hipEventRecord(rt.timing_events[li + 1], main), "hipEventRecord");
     if (bracket) {
       if (ph.kind != Phase::Contraction)
         hip_check(hipEventRecord(rt.profile_events[rt.profile_used + 1], stream), "hipEventRecord");
@@ -465,9 +466,9 @@ void enqueue(ocannl_hip_routine& rt, float* kernel_ms, int cap, int v = 0, bool 
     }
   }
   // whatever follows on the main queue (the caller's copies, the next run) comes after the side queue's work
-  if (last_side > joined) hip_check(hipStreamWaitEvent(dev.stream, rt.side_events.at(last_side).second, 0), "hipStreamWaitEvent");
+  if (last_side > joined) hip_check(hipStreamWaitEvent(main, rt.side_events.at(last_side).second, 0), "hipStreamWaitEvent");
   if (timed) {
-    hip_check(hipStreamSynchronize(dev.stream), "hipStreamSynchronize");
+    hip_check(hipStreamSynchronize(main), "hipStreamSynchronize");
     for (size_t li = 0; li < rt.launches.size(); ++li)
       hip_check(hipEventElapsedTime(&kernel_ms[li], rt.timing_events[li], rt.timing_events[li + 1]), "hipEventElapsedTime");
   }
@@ -995,41 +996,51 @@ int ocannl_hip_routine_set_static(ocannl_hip_routine* rt, int symbol, int64_t va
   });
 }
 
-// A plain run, replayed from a captured graph when it can be: several kernels, no merge buffer (bound
-// at launch), no event bracketing, no device printing, and a graph for this combination of static indices
-// (at most kMaxGraphs of them are kept; beyond that, and on the very first run, the kernels are
-// launched one by one).
+// A plain run, replayed from a captured graph when it can be: several kernels, no merge buffer (bound at launch), no
+// event bracketing, no device printing, and a graph for this combination of static indices.  A combination is captured
+// when it comes for the second time (at most kMaxGraphs are remembered, the first of each run kernel by kernel, which
+// also configures kernel attributes), so that indices that never come again cost no capture.  The capture has a stream
+// of its own: what other threads enqueue on the device's meanwhile is not recorded, and a caller that is capturing the
+// device's stream gets the kernels themselves.
 static void run_plain(ocannl_hip_routine& rt) {
   constexpr size_t kMaxGraphs = 128;
   const auto& plan = rt.code->plan;
   bool bracketing = false;
   for (char m : rt.profile_mask) bracketing = bracketing || m;
   const bool graphable = plan.use_graphs && rt.launches.size() >= 2 && rt.code->r.merge_node < 0 && !bracketing && !plan.debug_log;
-  if (!graphable || !rt.warmed) { enqueue(rt, nullptr, 0); rt.warmed = true; return; }
+  if (!graphable) { enqueue(rt, nullptr, 0); return; }
   std::vector<int64_t> key;
   for (auto& s : rt.code->r.statics) key.push_back(rt.statics[s.sym]);
   auto it = rt.graphs.find(key);
   ocannl_hip_device& dev = *rt.dev;
-  if (it == rt.graphs.end()) {
-    if (rt.graphs.size() >= kMaxGraphs) { enqueue(rt, nullptr, 0); return; }
-    dev.make_current();
-    hip_check(hipStreamBeginCapture(dev.stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
+  dev.make_current();
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  hip_check(hipStreamIsCapturing(dev.stream, &status), "hipStreamIsCapturing");
+  if (it == rt.graphs.end() || status != hipStreamCaptureStatusNone) {
+    enqueue(rt, nullptr, 0);
+    if (it == rt.graphs.end() && rt.graphs.size() < kMaxGraphs) rt.graphs.emplace(key, nullptr);
+    return;
+  }
+  if (!it->second) {
+    hipStream_t stream = nullptr;
+    hip_check(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking), "hipStreamCreateWithFlags");
+    struct Guard { hipStream_t s; ~Guard() { (void)hipStreamDestroy(s); } } guard{stream};
+    hip_check(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
     hipGraph_t graph = nullptr;
     try {
-      enqueue(rt, nullptr, 0, 0, true);
+      enqueue(rt, nullptr, 0, 0, stream);
     } catch (...) {
-      (void)hipStreamEndCapture(dev.stream, &graph);
+      (void)hipStreamEndCapture(stream, &graph);
       if (graph) (void)hipGraphDestroy(graph);
       throw;
     }
-    hip_check(hipStreamEndCapture(dev.stream, &graph), "hipStreamEndCapture");
+    hip_check(hipStreamEndCapture(stream, &graph), "hipStreamEndCapture");
     hipGraphExec_t exec = nullptr;
     hipError_t e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
     (void)hipGraphDestroy(graph);
     hip_check(e, "hipGraphInstantiate");
-    it = rt.graphs.emplace(key, exec).first;
+    it->second = exec;
   }
-  dev.make_current();
   hip_check(hipGraphLaunch(it->second, dev.stream), "hipGraphLaunch");
 }
 

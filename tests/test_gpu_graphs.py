@@ -1,8 +1,8 @@
 """Replay of a routine's kernel list from a captured HIP graph (one graph per combination of static-index
 values; fills recorded as kernels, never as memsets; the side queue as a branch of the graph): every
 replay has to leave exactly what launching the kernels one by one leaves (`graphs=0`), step after step,
-with reads of results and synchronisations of the program's own between the replays.  (`graphs=1`; the
-default is off: on this ROCm the replay pays only for routines of about ten tiny kernels.)"""
+with reads of results and synchronisations of the program's own between the replays.  (`graphs=1`; by
+default only routines of many short kernels are replayed.)"""
 import numpy as np
 import pytest
 
@@ -13,9 +13,9 @@ from parity import HipRun
 pytestmark = pytest.mark.gpu
 
 
-def _same_after_every_step(w, steps, statics_of, names, options=None):
+def _same_after_every_step(w, steps, statics_of, names, options=None, how="graphs=1"):
     opt = (options + ";" if options else "")
-    replay, direct = HipRun(w.routine, w.init, opt + "graphs=1"), HipRun(w.routine, w.init, opt + "graphs=0")
+    replay, direct = HipRun(w.routine, w.init, opt + how), HipRun(w.routine, w.init, opt + "graphs=0")
     for step in range(steps):
         st = statics_of(step)
         replay.step(st); direct.step(st)
@@ -58,3 +58,10 @@ def test_attention_replayed_and_bad_static_index_still_refused():
         h.step({sym: m.statics["batch_n"].range})   # out of range: refused, nothing captured or launched
     h.step({sym: 2})
     h.close()
+
+
+@pytest.mark.parametrize("layers", [1, 3])   # dozens of short kernels: replayed without being asked for
+def test_many_short_kernels_replayed_by_default(layers):
+    w = W.transformer(batch=2, seq=17, d_model=36, heads=2, d_ff=68, layers=layers, vocab=65, prec="single", grad_prec="single", lr=0.05)
+    assert len(B.compile(w.routine).kernels()) >= 16
+    _same_after_every_step(w, 6, lambda s: None, ("loss", "w_q_l0", "w_out", "b_ffn1_l0"), how="")
