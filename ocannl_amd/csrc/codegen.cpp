@@ -1123,7 +1123,7 @@ GeneratedModule generate_module(const Routine& r, const Plan& plan) {
     auto emit_points = [&](const Phase& q, const std::string& pind, const std::string& skip) {
       const int QG = q.coop_lanes;
       uint64_t QP = 1;
-      if (QG > 1) {
+      if (QG > 1 || !q.members.empty()) {   // (a row group names its lane even where it is the only one)
         body.push_back(pind + "const uint32_t lane_ = (uint32_t)(gtid_ % " + std::to_string(QG) + "u);");
         body.push_back(pind + pt_t + " pt_ = (" + pt_t + ")(gtid_ / " + std::to_string(QG) + "u);");
       } else {
