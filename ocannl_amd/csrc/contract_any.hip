@@ -3,6 +3,7 @@
 
 #include <algorithm>
 #include <cstdio>
+#include <cstdlib>
 
 #include "contract_any.hpp"
 
@@ -72,6 +73,22 @@ AnyShape any_shape(const GemmDesc& d) {
 }
 
 }  // namespace
+
+// Offsets by row and by k are computed apart, each in an int, and added in 64 bits; 2^30 leaves room for a tile and a
+// K step past the end.  Batch strides are 64 bits wide and may be anything.
+bool contract_any_fits(const GemmDesc& d) {
+  constexpr int64_t kLimit = (int64_t)1 << 30;
+  auto reach = [&](const int64_t (&ext)[3], const int64_t (&stride)[3], int64_t n, int64_t s) {
+    if (!d.any) return (n - 1) * std::abs(s);
+    int64_t r = 0;
+    for (int i = 0; i < 3; ++i) r += (ext[i] - 1) * std::abs(stride[i]);
+    return r;
+  };
+  if (d.M > kLimit || d.N > kLimit || d.K > kLimit) return false;
+  return reach(d.m_ext, d.a.row_stride, d.M, d.a.s_row) <= kLimit && reach(d.k_ext, d.a.k_stride, d.K, d.a.s_k) <= kLimit &&
+         reach(d.n_ext, d.b.row_stride, d.N, d.b.s_row) <= kLimit && reach(d.k_ext, d.b.k_stride, d.K, d.b.s_k) <= kLimit &&
+         reach(d.m_ext, d.c.row_stride, d.M, d.c.s_row) + reach(d.n_ext, d.c.k_stride, d.N, d.c.s_k) <= kLimit;
+}
 
 const char* contract_any_name(const GemmDesc& d) {
   static thread_local char buf[96];

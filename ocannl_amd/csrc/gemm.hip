@@ -526,7 +526,7 @@ bool dtl_operands_ok(const GemmArgs& a, bool akc, bool bkc) {
 // now: 1784 x 776 x 1000 bf16 67 -> 57 us, fp32 231 -> 141; 594 x 320 x 320 bf16 33 -> 26; 512 x 512 x 512 fp32
 // 129 -> 37.  From 256 tiles on the larger tile wins (8000 x 1000 x 1000 bf16: 122 against 173 us).
 bool gemm_prefers_any(const GemmDesc& d) {
-  if (d.any || !d.more.empty() || d.a.prec != d.b.prec) return false;
+  if (d.any || !d.more.empty() || d.a.prec != d.b.prec || !contract_any_fits(d)) return false;
   if (((d.M + 127) / 128) * ((d.N + 127) / 128) * batch_count(d) >= 256) return false;
   return d.a.prec == Prec::Single || dtl_shape(d).bm == 0;
 }

@@ -349,7 +349,7 @@ bool match_contraction(const Routine& r, Phase& ph, const PlanOptions& opt) {
       std::swap(g.c.row_stride, g.c.k_stride);
     }
     g.any = true;
-    return true;
+    return contract_any_fits(g);
   };
   GemmDesc reg = g;
   if (regular(reg)) g = reg;
@@ -401,7 +401,8 @@ bool match_window(const Routine& r, Phase& ph, const PlanOptions& opt) {
       w.o = to.second; w.k = tk.second; w.s = to.first;
       break;
     }
-    if (w.o < 0 || w.s * (ext[w.o] - 1) + ext[w.k] > w.pos) return false;
+    // (a stride beyond the axis, which one position may have, would leave more residues than positions)
+    if (w.o < 0 || w.s > w.pos || w.s * (ext[w.o] - 1) + ext[w.k] > w.pos) return false;
     special.insert(w.o); special.insert(w.k);
     wins.push_back(w);
   }
@@ -448,7 +449,7 @@ bool match_window(const Routine& r, Phase& ph, const PlanOptions& opt) {
   g.M = g.m_ext[0] * g.m_ext[1] * g.m_ext[2];
   g.N = g.n_ext[0] * g.n_ext[1] * g.n_ext[2];
   g.K = g.k_ext[0] * g.k_ext[1] * g.k_ext[2];
-  if (g.flops() < (double)opt.min_mfma_flops || g.M < 16 || g.K < 8 || g.M * g.K > (int64_t)1 << 40) return false;
+  if (g.flops() < (double)opt.min_mfma_flops || g.M < 16 || g.K < 8 || !contract_any_fits(g)) return false;
   ph.kind = Phase::Generic;
   ph.window = true;
   ph.gemm = g;
