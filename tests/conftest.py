@@ -17,6 +17,6 @@ def pytest_configure(config):
 
 @pytest.fixture(scope="session")
 def reference_root():
-    if not os.path.isdir(REFERENCE):
+    if not os.path.isdir(os.path.join(REFERENCE, "arrayjit")):
         pytest.skip("reference tree not present on this machine")
     return REFERENCE
