@@ -389,6 +389,13 @@ struct Printer {
   }
   // One loop over the whole range of several (`sym`, `from`, `to`; slowest first), shared by `lanes` lanes.
   struct Loop { int sym; int64_t from, to; };
+  // Where the lanes outnumber the innermost loop.  The one counter is as wide as the kernel's offsets (32 bits), and its
+  // last step goes past the range: a range that this could wrap stays nested, one counter a loop.
+  bool flattens(const std::vector<Loop>& loops, int lanes) const {
+    double total = 1;
+    for (auto& l : loops) total *= (double)(l.to - l.from + 1);
+    return loops.size() > 1 && row_iters == 0 && lanes > loops.back().to - loops.back().from + 1 && total <= (double)(1ll << 31);
+  }
   std::vector<std::string> flat_loop(const std::vector<Loop>& loops, int lanes, const std::string& ind) {
     int64_t total = 1;
     for (auto& l : loops) total *= l.to - l.from + 1;
@@ -657,10 +664,10 @@ struct Printer {
     Def d; d.scope = s.scope.scope;
     d.lines.push_back(ind + (dbl ? "double " : "float ") + part + " = " + neutral_literal(coop_accum, dbl) + ";");
     std::string ci = ind;
-    const bool flat = loops.size() > 1 && row_iters == 0 && coop_lanes > loops.back()->to - loops.back()->from + 1;
+    std::vector<Loop> ls;
+    for (auto* l : loops) ls.push_back({l->sym, l->from, l->to});
+    const bool flat = flattens(ls, coop_lanes);
     if (flat) {
-      std::vector<Loop> ls;
-      for (auto* l : loops) ls.push_back({l->sym, l->from, l->to});
       for (auto& l : flat_loop(ls, coop_lanes, ci)) d.lines.push_back(l);
       ci += "  ";
     } else for (size_t i = 0; i < loops.size(); ++i) {
@@ -936,12 +943,12 @@ void emit_phase_statements(const Routine& r, Printer& pr, const Phase& ph, int G
     // one and the same element (not so for sums of symbols on an axis, convolution-style)
     for (auto& ix : set->idcs) for (int q : ph.seq_syms) if (ix.mentions(q)) is_reduction = false;
   }
-  const bool flat = G > 1 && ph.seq_syms.size() > 1 && !ph.coop_scope && pr.row_iters == 0 && G > ph.seq_to.back() - ph.seq_from.back() + 1;
+  std::vector<Printer::Loop> seq;
+  for (size_t i = 0; i < ph.seq_syms.size(); ++i) seq.push_back({ph.seq_syms[i], ph.seq_from[i], ph.seq_to[i]});
+  const bool flat = G > 1 && !ph.coop_scope && pr.flattens(seq, G);
   auto open_seq_loops = [&](std::string& cur_ind, bool coop_last) {
     if (coop_last && flat) {
-      std::vector<Printer::Loop> ls;
-      for (size_t i = 0; i < ph.seq_syms.size(); ++i) ls.push_back({ph.seq_syms[i], ph.seq_from[i], ph.seq_to[i]});
-      for (auto& l : pr.flat_loop(ls, G, cur_ind)) body.push_back(l);
+      for (auto& l : pr.flat_loop(seq, G, cur_ind)) body.push_back(l);
       cur_ind += "  ";
       return;
     }

@@ -340,3 +340,24 @@ def test_a_recomputed_contraction_reads_the_stored_relu_output_instead():
     loops = lambda code: len(re.findall(r"for \(uint32_t i\d+ = 0; i\d+ <= 127; \+\+i\d+\) \{\s*v\d+_ffn1", code.source()))
     assert loops(B.compile(w.routine, "reuse=0")) >= 1
     assert loops(B.compile(w.routine)) == 0
+
+
+@pytest.mark.parametrize("inlined", [False, True])
+def test_one_counter_over_nested_loops_does_not_wrap(inlined):
+    # lanes outnumber the inner loop and share both through one 32-bit counter -- unless
+    # the range is within a step of 2^32, where the counter would never pass its end
+    def source(n):
+        L.reset_symbols(0)
+        a, b, out = L.Node(1, "a", "single", (n,)), L.Node(2, "b", "single", (40,)), L.Node(3, "out", "single", (3,))
+        tmp = L.Node(4, "tmp", "single", (3,), mode="virtual")
+        p, i, j = (L.fresh_symbol() for _ in range(3))
+        term = lambda acc: L.Binop("max", acc, L.Binop("mul", L.Get(a, (L.It(i),)), L.Get(b, (L.It(j),))))
+        if inlined:
+            v = L.Scope(tmp, L.fresh_symbol())
+            scope = L.LocalScope(v, [L.SetLocal(v, L.Const(float("-inf"))), L.For(i, 0, n - 1, [L.For(j, 0, 39, [L.SetLocal(v, term(L.GetLocal(v)))])])])
+            body = L.For(p, 0, 2, [L.Set(out, (L.It(p),), scope)])
+        else:
+            body = L.For(p, 0, 2, [L.For(i, 0, n - 1, [L.For(j, 0, 39, [L.Set(out, (L.It(p),), term(L.Get(out, (L.It(p),))))])])])
+        return B.compile(L.Routine("nested", [body]), "serial=0").source()
+    assert "flat_ < 40000u" in source(1000)
+    assert "flat_ < " not in source(1 << 27)
