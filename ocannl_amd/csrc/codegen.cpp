@@ -307,6 +307,7 @@ struct Printer {
   // row-position values, a scalar every lane holds for per-row values) and later reads of it
   // inside the group use that instead of memory.
   bool row_vec4 = false;                    // see row_loop
+  bool row_arrays = true;                   // row_iters > 0: something per position is kept in registers, indexed by `it_`
   int row_iters = 0;                        // > 0: loops over the row position run `it_` = 0..row_iters-1, unrolled
   std::map<int, std::string> cache_name;    // node -> register expression
   std::set<int> cache_defined;              // nodes whose cache holds the current value
@@ -376,6 +377,10 @@ struct Printer {
   }
   // header of a loop over the row position shared by `lanes` lanes
   std::string row_loop(const std::string& sym, int64_t from, int64_t to, int lanes, const std::string& ind) {
+    // (nothing indexed by `it_`: the loop over the positions themselves, whole; the compiler finds the bound)
+    if (row_iters > 0 && from == 0 && !row_arrays)
+      return ind + "_Pragma(\"unroll" + (row_iters > 8 ? " 4" : "") + "\") for (" + idx_t + " " + sym + " = lane_; " + sym + " <= " + std::to_string(to) + "; " + sym + " += " +
+             std::to_string(lanes) + ") {";
     if (row_iters > 0 && from == 0) {
       const std::string head = ind + "_Pragma(\"unroll\") for (uint32_t it_ = 0; it_ < " + std::to_string(row_iters) + "; ++it_) { const " +
                                idx_t + " " + sym + " = ";
@@ -1270,7 +1275,7 @@ GeneratedModule generate_module(const Routine& r, const Plan& plan) {
                          (q.proj_c_copy >= 0 ? r.node(q.proj_c_copy).ident + " + (" + co + ")" : std::string("(unsigned short*)0")) + ");");
         }
         pr.lds_node = -1;
-        pr.row_iters = 0; pr.cache_name.clear(); pr.cache_defined.clear();
+        pr.row_iters = 0; pr.row_arrays = true; pr.cache_name.clear(); pr.cache_defined.clear();
         return (uint64_t)(QP * (uint64_t)fused_block);
       }
       if (!q.members.empty()) {
@@ -1290,6 +1295,7 @@ GeneratedModule generate_module(const Routine& r, const Plan& plan) {
         const bool cached = (q.row_len + QG - 1) / QG <= 16;
         if (cached) {
           pr.row_iters = (int)((q.row_len + QG - 1) / QG);
+          pr.row_arrays = q.row_len % QG == 0;
           for (auto& m : q.members) {
             const Stmt& st = *m.inner[0];
             if (pr.cache_name.count(st.node)) continue;
@@ -1298,6 +1304,7 @@ GeneratedModule generate_module(const Routine& r, const Plan& plan) {
             for (auto& ix : st.idcs) if (ix.kind == AxisIndex::Iter && ix.sym == m.row_sym && m.row_role == Phase::RowPointwise) per_position = true;
             const std::string base = "c" + std::to_string(st.node) + "_";
             if (per_position) {
+              pr.row_arrays = true;
               body.push_back(pind + c_typ(wn.prec) + " " + base + "[" + std::to_string(pr.row_iters) + "];");
               pr.cache_name[st.node] = base + "[it_]";
             } else {
@@ -1326,7 +1333,7 @@ GeneratedModule generate_module(const Routine& r, const Plan& plan) {
           pr.skip_store.clear();
           body.push_back(pind + "}");
         }
-        pr.row_iters = 0; pr.cache_name.clear(); pr.cache_defined.clear();
+        pr.row_iters = 0; pr.row_arrays = true; pr.cache_name.clear(); pr.cache_defined.clear();
       } else {
         // --- point decode: the symbol with the smallest stride in the first written array varies
         //     fastest across adjacent threads (coalesced stores)
