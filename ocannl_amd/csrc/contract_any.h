@@ -304,7 +304,15 @@ __device__ __forceinline__ void ocn_any_tile(const OcnAnyDesc& d, const void* a,
   const int wm = (wave / GN) * WM, wn = (wave % GN) * WN, m0 = tm * BM, n0 = tn * BN;
   const int steps = (d.K + BK - 1) / BK, per = (steps + d.splits - 1) / d.splits;
   const int kbeg = split * per * BK;
-  const int kend = kbeg + per * BK < d.K ? kbeg + per * BK : d.K;
+  int kend = kbeg + per * BK < d.K ? kbeg + per * BK : d.K;
+  if constexpr (WIN) {
+    // a residue that no tap has (an axis of fewer taps than its step) sums nothing and reads nothing: `b` is then where
+    // the tap would be, past the weights as they are stored
+    if (r0 >= d.win_taps[0] || r1 >= d.win_taps[1]) {
+      if (d.accumulate) return;
+      kend = kbeg;
+    }
+  }
   const int ksteps = kend > kbeg ? (kend - kbeg + BK - 1) / BK : 0;
   const bool ra = ocn_any_regular<A_KC, F32>(d.a, d.dm, d.dk, d.M), rb = ocn_any_regular<B_KC, F32>(d.b, d.dn, d.dk, d.N);
   const bool edge_a = m0 + BM > d.M, edge_b = n0 + BN > d.N;

@@ -1,8 +1,14 @@
 """What the planner hands to the contraction tile for any shape, and what that tile reads; no GPU needed."""
+import os
+import re
+import subprocess
+
+import numpy as np
 import pytest
 
 from ocannl_amd import backend as B
 from ocannl_amd import llir as L
+from ocannl_amd import workloads as W
 
 
 def _product(M, N, K, prec="single", a_kc=True, b_kc=True):
@@ -57,3 +63,72 @@ def test_a_window_step_beyond_its_axis_is_not_gathered():
         return B.compile(L.Routine("window", [body]), "min_mfma_flops=1").source().split('extern "C"')[1]
     assert "ocn_any_tile<" in source(2, 5)
     assert "ocn_any_tile<" not in source(1 << 20, 1)
+
+
+# ---- the window gather, run on the host --------------------------------------------------------------
+
+CLANG = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin", "clang++")
+
+
+def _on_the_host(tmp_path, code, values):
+    """The one kernel of `code` in a host program (host_workgroup.h): the tensors by name, as it leaves them."""
+    source = code.source()
+    tile, kernel = source[source.index("template <bool C, typename A"):], source[source.index('extern "C" __global__'):]
+    name, params = re.match(r'extern "C" __global__ void __launch_bounds__\(256\) (\w+)\(([^)]*)\)', kernel).groups()
+    types, names = zip(*(p.replace("__restrict__", "").split("*") for p in params.split(",")))
+    names = [n.strip() for n in names]
+    call = ", ".join(f"({t.strip()}*)p[{i}]" for i, t in enumerate(types))
+    (tmp_path / "kernel.cpp").write_text(f'#include "host_workgroup.h"\n{tile}\nvoid host_kernel(void** p) {{ {name}({call}); }}\n')
+    subprocess.run([CLANG, "-std=c++17", "-O1", "-w", "-ffp-contract=off", "-I", os.path.dirname(os.path.abspath(__file__)), "kernel.cpp", "-o", "kernel"],
+                   cwd=tmp_path, check=True)
+    arrays = [np.ascontiguousarray(values[n]) for n in names]
+    (tmp_path / "tensors").write_bytes(b"".join(a.tobytes() for a in arrays))
+    blocks = 8 * int(re.search(r"blockIdx.x % 8u\) \* (\d+)", kernel).group(1))
+    subprocess.run([tmp_path / "kernel", str(blocks), tmp_path / "tensors"] + [str(a.nbytes) for a in arrays], check=True, timeout=120, stdout=subprocess.DEVNULL)
+    raw, out, at = (tmp_path / "tensors").read_bytes(), {}, 0
+    for n, a in zip(names, arrays):
+        out[n] = np.frombuffer(raw, a.dtype, a.size, at).reshape(a.shape)
+        at += a.nbytes
+    return out
+
+
+def input_gradient(taps, stride, prec, taps_first, b=2, oh=5, ow=4, ic=32, oc=32, zeroed=True):
+    """x_grad[b, s1 * o1 + k1, s2 * o2 + k2, i] += y_grad[b, o1, o2, c] * w[c, k1, k2, i], the weights stored in that
+    order or as [k1, k2, i, c]; and the same from float64 values by name, the taps that reach a position and no others."""
+    L.reset_symbols(0)
+    (kh, kw), (s1, s2) = taps, stride
+    w = L.Node(1, "w", prec, (kh, kw, ic, oc) if taps_first else (oc, kh, kw, ic)); dy = L.Node(2, "dy", prec, (b, oh, ow, oc))
+    dx = L.Node(3, "dx", "single", (b, s1 * (oh - 1) + kh, s2 * (ow - 1) + kw, ic))
+    bb, o1, o2, c, k1, k2, i = syms = [L.fresh_symbol() for _ in range(7)]
+    at = (L.It(bb), L.Affine(((s1, o1), (1, k1)), 0), L.Affine(((s2, o2), (1, k2)), 0), L.It(i))
+    wi = (L.It(k1), L.It(k2), L.It(i), L.It(c)) if taps_first else (L.It(c), L.It(k1), L.It(k2), L.It(i))
+    body = [L.Set(dx, at, L.Ternop("fma", L.Get(dy, (L.It(bb), L.It(o1), L.It(o2), L.It(c))), L.Get(w, wi), L.Get(dx, at)))]
+    for sym, ext in reversed(list(zip(syms, (b, oh, ow, oc, kh, kw, ic)))):
+        body = [L.For(sym, 0, ext - 1, body)]
+
+    def want(f):
+        out = np.zeros(dx.dims) if zeroed else f["dx"].copy()
+        weights = f["w"].transpose(3, 0, 1, 2) if taps_first else f["w"]
+        for r in range(kh):
+            for s in range(kw):
+                at = out[:, r:r + s1 * (oh - 1) + 1:s1, s:s + s2 * (ow - 1) + 1:s2, :]
+                for k in range(oc):   # (term by term: a library product may move a NaN where no term has one)
+                    at += f["dy"][..., k, None] * weights[k, r, s, :]
+        return out
+    return L.Routine("dx", ([L.ZeroOut(dx)] if zeroed else []) + body), (w, dy, dx), want
+
+
+@pytest.mark.skipif(not os.path.exists(CLANG), reason="needs the ROCm compiler")
+@pytest.mark.parametrize("prec", ["single", "bfloat16"])
+@pytest.mark.parametrize("taps,stride,ic", [((3, 3), (2, 1), 32), ((1, 3), (2, 2), 32), ((3, 1), (2, 2), 40), ((2, 3), (3, 2), 5), ((1, 4), (4, 3), 5)])
+def test_window_gathers_stay_inside_their_operands(taps, stride, ic, prec, tmp_path):
+    # a residue of the step that no tap has reads no weights: behind them lies a page that may not be touched
+    for taps_first in (True, False):
+        r, nodes, want = input_gradient(taps, stride, prec, taps_first, ic=ic, oc=ic, zeroed=taps_first)
+        code = B.compile(r, "min_mfma_flops=1")
+        assert "ocn_any_tile<" in code.source().split('extern "C"')[1]
+        rng = np.random.default_rng(ic)
+        init = {n.ident: W.as_prec(rng.standard_normal(n.dims).astype(np.float32), n.prec) for n in nodes}
+        ref = want({n.ident: W.to_float(init[n.ident], n.prec).astype(np.float64) for n in nodes})
+        # fp32 sums of at most 9 x 40 terms: their rounding is below 2^-24 a term, of the size of the largest result
+        assert np.max(np.abs(_on_the_host(tmp_path, code, init)["dx"] - ref)) <= 4e-6 * np.max(np.abs(ref))

@@ -7,6 +7,7 @@ import pytest
 from ocannl_amd import llir as L
 from ocannl_amd import workloads as W
 from parity import HipRun
+from test_contract_any_cpu import input_gradient
 from test_gpu_contractions import _routine
 from test_gpu_conv import _conv
 
@@ -127,4 +128,21 @@ def test_overlapping_windows_are_gathered(stride, ksz, shape, prec, zeroed):
         for k2 in range(ksz):
             want[:, k1:k1 + stride * (oh - 1) + 1:stride, k2:k2 + stride * (ow - 1) + 1:stride, :] += np.einsum("bhwc,ci->bhwi", dy, w[:, k1, k2, :])
     assert np.max(np.abs(hip.get(n["dx"]) - want)) <= 4e-6 * np.max(np.abs(want))
+    hip.close()
+
+
+@pytest.mark.parametrize("prec", ["bfloat16", "single"])
+@pytest.mark.parametrize("taps,stride,ic", [((3, 3), (2, 1), 32), ((1, 3), (2, 2), 32), ((3, 1), (2, 2), 40), ((2, 3), (3, 2), 5), ((1, 4), (4, 3), 5)])
+@pytest.mark.parametrize("taps_first", [True, False])
+@pytest.mark.parametrize("zeroed", [True, False])
+def test_windows_of_any_taps_steps_and_weight_layout(taps, stride, ic, prec, taps_first, zeroed):
+    # steps that some residues of an axis have no tap for: those positions are zeros, or stay as they were
+    r, nodes, want = input_gradient(taps, stride, prec, taps_first, b=3, oh=9, ow=7, ic=ic, oc=ic, zeroed=zeroed)
+    rng = np.random.default_rng(ic)
+    init = {n.id: _values(rng, n) for n in nodes}
+    hip = HipRun(r, init, "min_mfma_flops=1")
+    assert "ocn_any_tile<" in hip.code.source().split('extern "C"')[1]
+    hip.step()
+    ref = want({n.ident: W.to_float(init[n.id], n.prec).astype(np.float64) for n in nodes})
+    assert np.max(np.abs(hip.get(nodes[2]) - ref)) <= 4e-6 * np.max(np.abs(ref))
     hip.close()
