@@ -508,8 +508,39 @@ __device__ __forceinline__ void ocn_any_tile(const OcnAnyDesc& d, const void* a,
       });
     }
   };
-  if constexpr (WIN) finish(No{});
-  else if (d.splits > 1) {
+  if constexpr (WIN) {
+    // A position that a tap does not reach multiplied that tap's weights by zero, which is no term of its sum: it turned
+    // NaN if one of them was infinite or NaN.  What has come out as NaN is summed again, one cell at a time, from its own
+    // terms (nothing, where the weights are finite), and is NaN only if that sum is.
+    static_assert(16 * TM * TN <= 32, "a bit a cell");
+    unsigned again = 0;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) again |= (unsigned)((__float_as_uint(acc[i][j][e]) & 0x7FFFFFFFu) > 0x7F800000u) << ((i * TN + j) * 16 + e);
+    if (d.accumulate) cells(No{}, [&](int j, int i, int, int e, int, int at) __attribute__((always_inline)) { acc[i][j][e] += cf[at]; });
+    cells(No{}, [&](int j, int i, int, int e, int, int at) __attribute__((always_inline)) { if (!(again >> ((i * TN + j) * 16 + e) & 1u)) cf[at] = acc[i][j][e]; });
+    for (; again; again &= again - 1) {
+      const int cell = __builtin_ctz(again), e = cell & 15, j = (cell >> 4) % TN, i = (cell >> 4) / TN;
+      const int n = n0 + wn + j * 32 + (lane & 31), m = m0 + wm + i * 32 + (lane >> 5) * 4 + (e >> 2) * 8 + (e & 3);
+      if (m >= d.M || n >= d.N) continue;
+      const OcnDigitVal md = ocn_digits(d.dm, m), nd = ocn_digits(d.dn, n);
+      if (d.win_s[0] * md.d1 + r0 >= d.win_pos[0] || d.win_s[1] * md.d2 + r1 >= d.win_pos[1]) continue;
+      float v = 0.0f;
+      for (int t0 = 0; d.win_s[0] * t0 + r0 < d.win_taps[0]; ++t0) {
+        if ((unsigned)(md.d1 - t0) >= (unsigned)d.win_lim[0]) continue;
+        for (int t1 = 0; d.win_s[1] * t1 + r1 < d.win_taps[1]; ++t1) {
+          if ((unsigned)(md.d2 - t1) >= (unsigned)d.win_lim[1]) continue;
+          long at_a = (long)ocn_digit_off(md, d.a.row) + ocn_digit_off({t0, t1, 0}, d.a.k), at_b = (long)ocn_digit_off(nd, d.b.row) + ocn_digit_off({t0, t1, 0}, d.b.k);
+          for (int k = 0; k < d.dk.e2; ++k, at_a += d.a.k[2], at_b += d.b.k[2]) v = __builtin_fmaf(SA::one(a, ABF, at_a), SB::one(b, BBF, at_b), v);
+        }
+      }
+      const int at = ocn_digit_off(md, d.c_m) + ocn_digit_off(nd, d.c_n);
+      cf[at] = d.accumulate ? v + cf[at] : v;
+    }
+  } else if (d.splits > 1) {
     float* const w = ws + (long)split * d.M * d.N;
     cells(Yes{}, [&](int j, int i, int n, int e, int m, int) __attribute__((always_inline)) { w[m * d.N + n] = acc[i][j][e]; });
   } else if (d.dm.n == 1) finish(Yes{});

@@ -132,3 +132,38 @@ def test_window_gathers_stay_inside_their_operands(taps, stride, ic, prec, tmp_p
         ref = want({n.ident: W.to_float(init[n.ident], n.prec).astype(np.float64) for n in nodes})
         # fp32 sums of at most 9 x 40 terms: their rounding is below 2^-24 a term, of the size of the largest result
         assert np.max(np.abs(_on_the_host(tmp_path, code, init)["dx"] - ref)) <= 4e-6 * np.max(np.abs(ref))
+
+
+def _same_numbers(got, want, tol):
+    """The same infinities and NaNs in the same places, and the rest within `tol` of the largest."""
+    got = got.astype(np.float64)
+    finite = np.isfinite(want)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[~finite & ~np.isnan(want)], want[~finite & ~np.isnan(want)])
+    assert 0 < finite.sum() < want.size and np.max(np.abs(got[finite] - want[finite])) <= tol * np.max(np.abs(want[finite]))
+
+
+def non_finite(nodes, seed):
+    """Values for the nodes, an infinity or a NaN in some of the weights and gradients."""
+    rng = np.random.default_rng(seed)
+    init = {}
+    for n in nodes:
+        v = rng.standard_normal(n.dims).astype(np.float32)
+        if n.ident != "dx":
+            for x in (np.inf, -np.inf, np.nan):
+                v.flat[rng.integers(v.size, size=2)] = x
+        init[n.ident] = W.as_prec(v, n.prec)
+    with np.errstate(invalid="ignore"):
+        return init, {n.ident: W.to_float(init[n.ident], n.prec).astype(np.float64) for n in nodes}
+
+
+@pytest.mark.skipif(not os.path.exists(CLANG), reason="needs the ROCm compiler")
+@pytest.mark.parametrize("prec", ["single", "bfloat16"])
+@pytest.mark.parametrize("taps,stride,ic", [((3, 3), (1, 1), 33), ((3, 2), (2, 1), 40), ((5, 3), (2, 2), 5)])
+@pytest.mark.parametrize("zeroed", [True, False])
+def test_a_weight_counts_only_where_its_tap_reaches(taps, stride, ic, prec, zeroed, tmp_path):
+    # 0 x infinity is NaN: a gathered position outside of a tap's reach has no such term
+    r, nodes, want = input_gradient(taps, stride, prec, not zeroed, ic=ic, oc=8, zeroed=zeroed)
+    init, values = non_finite(nodes, ic)
+    with np.errstate(invalid="ignore"):
+        ref = want(values)
+    _same_numbers(_on_the_host(tmp_path, B.compile(r, "min_mfma_flops=1"), init)["dx"], ref, 4e-6)

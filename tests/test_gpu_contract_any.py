@@ -7,7 +7,7 @@ import pytest
 from ocannl_amd import llir as L
 from ocannl_amd import workloads as W
 from parity import HipRun
-from test_contract_any_cpu import input_gradient
+from test_contract_any_cpu import _same_numbers, input_gradient, non_finite
 from test_gpu_contractions import _routine
 from test_gpu_conv import _conv
 
@@ -145,4 +145,18 @@ def test_windows_of_any_taps_steps_and_weight_layout(taps, stride, ic, prec, tap
     hip.step()
     ref = want({n.ident: W.to_float(init[n.id], n.prec).astype(np.float64) for n in nodes})
     assert np.max(np.abs(hip.get(nodes[2]) - ref)) <= 4e-6 * np.max(np.abs(ref))
+    hip.close()
+
+
+@pytest.mark.parametrize("prec", ["bfloat16", "single"])
+@pytest.mark.parametrize("taps,stride,ic", [((3, 3), (1, 1), 33), ((3, 2), (2, 1), 40), ((5, 3), (2, 2), 5), ((3, 3), (1, 1), 64)])
+@pytest.mark.parametrize("zeroed", [True, False])
+def test_a_weight_counts_only_where_its_tap_reaches(taps, stride, ic, prec, zeroed):
+    r, nodes, want = input_gradient(taps, stride, prec, not zeroed, oh=9, ow=7, ic=ic, oc=16, zeroed=zeroed)
+    init, values = non_finite(nodes, ic)
+    hip = HipRun(r, {n.id: init[n.ident] for n in nodes}, "min_mfma_flops=1")
+    hip.step()
+    with np.errstate(invalid="ignore"):
+        ref = want(values)
+    _same_numbers(hip.get(nodes[2]), ref, 4e-6)
     hip.close()
