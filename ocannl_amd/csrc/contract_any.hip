@@ -90,6 +90,13 @@ bool contract_any_fits(const GemmDesc& d) {
          reach(d.m_ext, d.c.row_stride, d.M, d.c.s_row) + reach(d.n_ext, d.c.k_stride, d.N, d.c.s_k) <= kLimit;
 }
 
+int64_t contract_any_area(const GemmDesc& d, bool& alone) {
+  const AnyShape s = any_shape(d);
+  const int64_t groups = (int64_t)((d.M + s.bm - 1) / s.bm) * ((d.N + s.bn - 1) / s.bn) * any_entries(d) * s.splits;
+  alone = groups <= 256;
+  return (groups + 255) / 256 * s.bm * s.bn / s.splits;
+}
+
 const char* contract_any_name(const GemmDesc& d) {
   static thread_local char buf[96];
   const AnyShape s = any_shape(d);

@@ -522,13 +522,28 @@ bool dtl_operands_ok(const GemmArgs& a, bool akc, bool bkc) {
 }  // namespace
 
 // Fewer 128 x 128 tiles than compute units: the register-staged kernels leave some idle and hide no latency on the
-// rest, where 64 x 64 tiles of contract_any.hip put several workgroups on each.  Measured with both gradients, before ->
-// now: 1784 x 776 x 1000 bf16 67 -> 57 us, fp32 231 -> 141; 594 x 320 x 320 bf16 33 -> 26; 512 x 512 x 512 fp32
-// 129 -> 37.  From 256 tiles on the larger tile wins (8000 x 1000 x 1000 bf16: 122 against 173 us).
+// rest, where 64 x 64 tiles of contract_any.hip put several workgroups on each; but they split K further, and the
+// smaller tile reads twice the operands per product.  Compared is what a compute unit goes through, area of C by k, a
+// stage of the smaller tile costing more by what was measured for it: 12 and 25 % in fp32 with one and both operands
+// row-contiguous (fragments of four reads), 8 % in bf16 with both, and 15 % where no unit holds a second workgroup.  On
+// the other side stand the register-staged kernel's longer start and the launch that sums its splits: 2.5 M, 13 us in
+// fp32, 4 in bf16.  Measured over 9 shapes of C of 16 to 192 tiles, K of 256 to 16384 and the operand layouts, one
+// product, register-staged against small tile: 1000 x 1000, both row-contiguous: K = 1024 fp32 50 against 33 us, bf16
+// 18 against 12; 2048 fp32 52 against 59, bf16 21 against 20; 8192 fp32 157 against 225, bf16 44 against 66.  From 256
+// tiles on the larger tile wins (8000 x 1000 x 1000 bf16, both gradients too: 122 against 173 us).
 bool gemm_prefers_any(const GemmDesc& d) {
   if (d.any || !d.more.empty() || d.a.prec != d.b.prec || !contract_any_fits(d)) return false;
-  if (((d.M + 127) / 128) * ((d.N + 127) / 128) * batch_count(d) >= 256) return false;
-  return d.a.prec == Prec::Single || dtl_shape(d).bm == 0;
+  const int64_t t128 = (int64_t)((d.M + 127) / 128) * ((d.N + 127) / 128) * batch_count(d);
+  if (t128 >= 256) return false;
+  const bool f32 = d.a.prec == Prec::Single;
+  if (!f32 && dtl_shape(d).bm != 0) return false;
+  const TileConfig c = tile_config(d);
+  const int64_t staged = (t128 * c.splits + 255) / 256 * 128 * (c.narrow ? 64 : 128) / c.splits;
+  bool alone;
+  const int64_t small = contract_any_area(d, alone);
+  const int lines = !a_kcontig(d) + !b_kcontig(d);
+  const int extra = (alone ? 15 : 0) + (f32 ? (lines == 2 ? 25 : 12 * lines) : lines == 2 ? 8 : 0);
+  return (double)small * (100 + extra) / 100 * d.K <= (double)staged * d.K + 2.5e6;
 }
 
 const char* gemm_kernel_name(const GemmDesc& d) {

@@ -66,6 +66,9 @@ bool gemm_prefers_any(const GemmDesc& desc);
 // contract_any.hip: the same for contractions with `desc.any` set (launch_gemm and its siblings forward to these).
 // Do the extents and the element offsets within one batch entry fit the 32-bit arithmetic of contract_any.h?
 bool contract_any_fits(const GemmDesc& desc);
+// Elements of C, padding included, that a compute unit works on per k with the workgroups dealt out evenly and K split as
+// it would be; `alone`: no unit gets a second workgroup.
+int64_t contract_any_area(const GemmDesc& desc, bool& alone);
 hipError_t launch_contract_any(const GemmDesc& desc, const GemmArgs& args, void* workspace, hipStream_t stream, hipEvent_t after_main);
 size_t contract_any_workspace_bytes(const GemmDesc& desc);
 const char* contract_any_name(const GemmDesc& desc);

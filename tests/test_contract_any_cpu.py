@@ -29,10 +29,20 @@ def _matrix_kernels(r):
 @pytest.mark.parametrize("layout", [(True, True), (False, False)])
 @pytest.mark.parametrize("prec", ["single", "bfloat16"])
 def test_operands_beyond_32_bit_offsets_keep_the_64_bit_kernels(layout, prec):
-    # the tile's element offsets within one batch entry are ints: 2^20 * 1008 elements fit, 2^22 * 1008 do not
-    assert "kernel_any<" in _matrix_kernels(_product(1008, 1008, 1 << 20, prec, *layout))[0]
-    name, = _matrix_kernels(_product(1008, 1008, 1 << 22, prec, *layout))
+    # the tile's element offsets within one batch entry are ints: 2^21 * 264 elements fit, 2^23 * 264 do not
+    assert "kernel_any<" in _matrix_kernels(_product(264, 264, 1 << 21, prec, *layout))[0]
+    name, = _matrix_kernels(_product(264, 264, 1 << 23, prec, *layout))
     assert "kernel_any<" not in name
+
+
+@pytest.mark.parametrize("prec", ["single", "bfloat16"])
+@pytest.mark.parametrize("shape,layout,small", [((1000, 1000, 1024), (False, False), True), ((1000, 1000, 8192), (False, False), False),
+                                                ((1000, 1000, 8192), (True, True), False), ((264, 264, 8192), (False, False), True),
+                                                ((2040, 1528, 8192), (True, True), True), ((1784, 776, 8192), (False, False), False)])
+def test_small_tiles_where_they_go_through_less(shape, layout, small, prec):
+    # a long sum over few tiles: the register-staged kernels split it further and re-read less
+    name, = _matrix_kernels(_product(*shape, prec, *layout))
+    assert ("kernel_any<64, 64" in name) == small
 
 
 def test_sums_of_more_terms_than_32_bits_count_are_left_alone():
