@@ -6,7 +6,7 @@ import pytest
 
 from ocannl_amd import llir as L
 from ocannl_amd import workloads as W
-from parity import HipRun
+from parity import HipRun, OracleRun
 from test_contract_any_cpu import _same_numbers, input_gradient, non_finite
 from test_gpu_contractions import _routine
 from test_gpu_conv import _conv
@@ -24,7 +24,11 @@ def _run(r, nodes, out, want, accumulate, k, seed=0):
     init = {n.id: _values(rng, n) for n in nodes.values()}
     hip = HipRun(r, init, "min_mfma_flops=1")
     ks = [x for x in hip.code.kernels() if x["kind"] == "mfma"]
-    if not ks and nodes[out].prec == "bfloat16":   # a bf16 sum that one thread runs: rounded after every addition, left alone
+    if not ks and nodes[out].prec == "bfloat16":
+        # a sum that one thread runs, rounded after every addition: left alone, and the checker's bits
+        checker = OracleRun(r, init)
+        hip.step(); checker.step()
+        assert np.array_equal(hip.get(nodes[out]).ravel(), np.asarray(checker.get(nodes[out])).ravel())
         return hip.close()
     assert ks and all("_kernel_any" in x["name"] for x in ks), hip.code.kernels()
     hip.step()
