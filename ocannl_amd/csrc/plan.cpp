@@ -2378,7 +2378,7 @@ static bool many_short_launches(const Plan& plan) {
   for (auto& ph : plan.phases) {
     if (ph.stream != 0) return false;
     us += ph.bytes / 2e6;
-    if (ph.kind == Phase::Contraction) us += 2.0 * ph.gemm.M * ph.gemm.N * ph.gemm.K * ph.gemm.nbatch / 2e8;
+    if (ph.kind == Phase::Contraction) us += ph.gemm.flops() / 2e8;
   }
   return plan.phases.size() >= 16 && us < (double)plan.phases.size();
 }
