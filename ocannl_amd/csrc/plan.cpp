@@ -1784,12 +1784,12 @@ void use_bf16_copies(Routine& r, Plan& plan, Phase& ph, Bf16Copies& copies, int*
     if (!stale) copy = it->second;
   }
   if (copy < 0) {
-    // a mirror is kept in step by generated stores and zero fills only: once a contraction has
-    // written the tensor it no longer stands for it
+    // a mirror is kept in step by generated stores and zero fills only: once a contraction or a window gather (the
+    // contraction tile in a generated kernel) has written the tensor it no longer stands for it
     auto m = plan.mirrors.find(src.id);
     if (m != plan.mirrors.end()) {
       bool in_step = true;
-      for (auto& q : plan.phases) in_step &= !(q.kind == Phase::Contraction && q.gemm.c.node == src.id);
+      for (auto& q : plan.phases) in_step &= !((q.kind == Phase::Contraction || q.window) && q.gemm.c.node == src.id);
       if (in_step) copy = m->second;
     }
   }
@@ -1805,7 +1805,7 @@ void use_bf16_copies(Routine& r, Plan& plan, Phase& ph, Bf16Copies& copies, int*
       if (!phase_writes(w, src.id)) continue;
       any = true;
       if (w.kind == Phase::Fill) { fills.push_back(q); whole = true; }
-      else if (w.kind == Phase::Generic && w.members.empty() && w.serial_members.empty()) whole |= writes_whole_node(r, w, src.id);
+      else if (w.kind == Phase::Generic && !w.window && w.members.empty() && w.serial_members.empty()) whole |= writes_whole_node(r, w, src.id);
       else all_generated = false;
     }
     mirror = any && all_generated && whole && src.mode != Mode::Virtual && !src.read_only;

@@ -75,6 +75,38 @@ def test_a_window_step_beyond_its_axis_is_not_gathered():
     assert "ocn_any_tile<" not in source(1 << 20, 1)
 
 
+def gathered_then_multiplied(late):
+    """dx := r; dx += windows of dy * w; out := h^T dx, h in bf16 (so that the product reads dx rounded); with `late` the
+    product also runs ahead of the windows, into first."""
+    L.reset_symbols(0)
+    b, o, taps, ic, g = 4, 16, 3, 32, 32
+    p = o + taps - 1
+    w = L.Node(1, "w", "bfloat16", (ic, taps, ic)); dy = L.Node(2, "dy", "bfloat16", (b, o, ic)); r = L.Node(3, "r", "single", (b, p, ic))
+    h = L.Node(4, "h", "bfloat16", (b, p, g)); dx = L.Node(5, "dx", "single", (b, p, ic)); out = L.Node(6, "out", "single", (g, ic)); first = L.Node(7, "first", "single", (g, ic))
+
+    def nest(exts, stmt):
+        syms = [L.fresh_symbol() for _ in exts]
+        body = [stmt(*(L.It(s) for s in syms), *syms)]
+        for s, e in reversed(list(zip(syms, exts))):
+            body = [L.For(s, 0, e - 1, body)]
+        return body
+    product = lambda c: [L.ZeroOut(c)] + nest((g, ic, b, p), lambda m, n, k, l, *_: L.Set(c, (m, n), L.Ternop("fma", L.Get(h, (k, l, m)), L.Get(dx, (k, l, n)), L.Get(c, (m, n)))))
+    at = lambda syms: (L.It(syms[0]), L.Affine(((1, syms[1]), (1, syms[2])), 0), L.It(syms[4]))
+    body = nest((b, p, ic), lambda i, j, k, *_: L.Set(dx, (i, j, k), L.Get(r, (i, j, k)))) + (product(first) if late else [])
+    body += nest((b, o, taps, ic, ic), lambda bb, oo, k, c, i, *s: L.Set(dx, at(s), L.Ternop("fma", L.Get(dy, (bb, oo, c)), L.Get(w, (c, k, i)), L.Get(dx, at(s)))))
+    return L.Routine("gathered", body + product(out)), dict(w=w, dy=dy, r=r, h=h, dx=dx, out=out, **({"first": first} if late else {}))
+
+
+@pytest.mark.parametrize("late", [False, True])
+def test_a_bf16_copy_is_made_after_the_window_gather_that_writes_its_tensor(late):
+    # (the copy that generated stores keep in step: the gather stores the tensor alone)
+    r, _ = gathered_then_multiplied(late)
+    code = B.compile(r, "min_mfma_flops=1")
+    kernels = re.findall(r'extern "C" __global__ void[^(]*\(256\) \w+\(([^)]*)\) \{(.*?)\n\}\n', code.source(), re.S)
+    gather = [i for i, (_, body) in enumerate(kernels) if "ocn_any_tile<" in body]
+    assert len(gather) == 1 and any("bf" in params and "_dx" in params for params, _ in kernels[gather[0] + 1:])
+
+
 # ---- the window gather, run on the host --------------------------------------------------------------
 
 CLANG = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin", "clang++")

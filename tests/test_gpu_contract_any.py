@@ -7,7 +7,7 @@ import pytest
 from ocannl_amd import llir as L
 from ocannl_amd import workloads as W
 from parity import HipRun, OracleRun
-from test_contract_any_cpu import _same_numbers, input_gradient, non_finite
+from test_contract_any_cpu import _same_numbers, gathered_then_multiplied, input_gradient, non_finite
 from test_gpu_contractions import _routine
 from test_gpu_conv import _conv
 
@@ -163,4 +163,22 @@ def test_a_weight_counts_only_where_its_tap_reaches(taps, stride, ic, prec, zero
     with np.errstate(invalid="ignore"):
         ref = want(values)
     _same_numbers(hip.get(nodes[2]), ref, 4e-6)
+    hip.close()
+
+
+@pytest.mark.parametrize("late", [False, True])
+def test_a_product_reads_what_the_window_gather_left(late):
+    r, n = gathered_then_multiplied(late)
+    rng = np.random.default_rng(5)
+    init = {x.id: _values(rng, x) for x in n.values()}
+    hip = HipRun(r, init, "min_mfma_flops=1")
+    hip.step()
+    f = {k: W.to_float(init[x.id], x.prec).astype(np.float64) for k, x in n.items()}
+    rounded = lambda x: W.to_float(W.as_prec(x.astype(np.float32), "bfloat16"), "bfloat16").astype(np.float64)
+    times_h = lambda x: np.einsum("bpg,bpi->gi", f["h"], rounded(x))
+    dx = f["r"].copy()
+    for k in range(3):
+        dx[:, k:k + 16] += np.einsum("boc,ci->boi", f["dy"], f["w"][:, k])
+    for name, want in (("dx", dx), ("out", times_h(hip.get(n["dx"]).astype(np.float64)))) + ((("first", times_h(f["r"])),) if late else ()):
+        assert np.max(np.abs(hip.get(n[name]) - want)) <= 4e-6 * np.max(np.abs(want)), name
     hip.close()
