@@ -17,7 +17,8 @@ __global__ void __launch_bounds__(256) contract_any_reduce_kernel(const OcnAnyDe
   const int z = blockIdx.y;
   const void *a, *b;
   void *c, *c2;
-  any_operands(d, q, p, z, a, b, c, c2);
+  unsigned short* relu_out;   // (a folded layer is never split)
+  any_operands(d, q, p, z, a, b, c, c2, relu_out);
   const float* ws = p.ws + (long)z * d.splits * cells + i;
   float v = 0.0f;
 #pragma unroll 16

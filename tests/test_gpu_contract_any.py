@@ -182,3 +182,30 @@ def test_a_product_reads_what_the_window_gather_left(late):
     for name, want in (("dx", dx), ("out", times_h(hip.get(n["dx"]).astype(np.float64)))) + ((("first", times_h(f["r"])),) if late else ()):
         assert np.max(np.abs(hip.get(n[name]) - want)) <= 4e-6 * np.max(np.abs(want)), name
     hip.close()
+
+
+@pytest.mark.parametrize("shape", [(3, 72, 40, 72), (5, 136, 72, 200), (2, 24, 200, 64)])
+@pytest.mark.parametrize("one_statement", [False, True])
+def test_bias_and_relu_of_every_batch_entry(shape, one_statement):
+    # y[z, b, o] := (the inlined product) + bias[o]; relu(y), stored by the contraction itself, per batch entry
+    from ocannl_amd.frontend import Graph, make_routine
+    Z, M, N, K = shape
+    L.reset_symbols(0)
+    g = Graph("bfloat16", "single")
+    x = g.input("x", ("z", "b", "i"), (Z, M, K)); w = g.param("w", ("z", "o", "i"), (Z, N, K)); bias = g.param("bias", ("o",), (N,))
+    y = g.add(g.einsum(w, x, ("z", "b", "o"), ident="wx"), bias, ("z", "b", "o"), ident="y")
+    relu = g.unary("relu", y, ident="relu")
+    r = make_routine(g, "layers", g.forward(relu), outputs=[relu.value] if one_statement else [y.value, relu.value], **({"inline": "visits"} if one_statement else {}))
+    rng = np.random.default_rng(M)
+    init = {t.value.id: W.as_prec((rng.standard_normal(t.value.dims) / np.sqrt(K if t is w else 1)).astype(np.float32), "bfloat16") for t in (x, w, bias)}
+    folded, apart = HipRun(r, init, "min_mfma_flops=1"), HipRun(r, init, "min_mfma_flops=1;epilogues=0;fused=0")
+    assert [k["name"][:20] for k in folded.code.kernels()] == ["gemm_bf16_kernel_any"] and len(apart.code.kernels()) > 1
+    folded.step(); apart.step()
+    f = {t: W.to_float(init[t.value.id], "bfloat16").astype(np.float64) for t in (x, w, bias)}
+    want = np.einsum("zbi,zoi->zbo", f[x], f[w]) + f[bias]
+    for t, ref in ([] if one_statement else [(y, want)]) + [(relu, np.maximum(want, 0))]:
+        got = folded.get(t.value)
+        assert np.array_equal(got, apart.get(t.value)), t.value.ident
+        # (the product is rounded, and its sum with the bias again: 2^-9 of either, of at most the largest)
+        assert np.max(np.abs(W.to_float(got, "bfloat16") - ref)) <= 2.0 ** -7 * np.max(np.abs(want))
+    folded.close(); apart.close()
