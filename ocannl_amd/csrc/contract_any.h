@@ -13,13 +13,17 @@
 // of the register-staged kernels (gemm_common.hpp): rows padded by 16 bytes for a k-contiguous operand,
 // [k][row] with ds_read_b64_tr_b16 fragments for a row-contiguous bf16 one.
 //
-// What bounds it: latency of a K step (load, LDS, barrier), with several workgroups per compute unit to hide it;
-// address arithmetic comes next (up to two quotients per chunk and step).  As generated kernels, one thread or
-// lane group per element of C, these contractions ran at the rate of scalar loads.  Measured, before -> now:
-// b=1777 i=1001 o=771 bf16, forward and both gradients, 4192 -> 101 us; attention scores and their product with
-// V over 197 positions, 96 heads, 438 + 569 -> 14 + 12 us; a 3 x 3 convolution of 64 x 32 x 32 positions,
-// 32 -> 64 channels in fp32, forward 314 -> 66 us, weight gradient 2106 -> 94 us, input gradient (which only
-// the batch and channel axes kept apart: 2048 threads) 28 500 -> 43 us.
+// What bounds it: latency of a K step (load, LDS, barrier), about a microsecond, with one or two workgroups per compute
+// unit to hide it: matrix cores busy 4 to 5 % and about 5 TB/s out of L2 on the bf16 products of 1777 x 1001 x 771, no
+// bank conflicts; in fp32, whose products take sixteen times as long, the matrix cores are busy 26 to 39 %.  Rows at odd
+// elements, and the row-contiguous fp32 fragments of four reads, cost more (the last two launches of the dense layer, the
+// weight gradient of the convolution).  Kernel trace, as generated kernels with one thread or lane group per element of C
+// -> as tiles: the dense layer above, forward and both gradients, 4192 -> 16 + 21 + 25 us; attention scores and their
+// product with V over 197 positions, 96 heads, 438 + 569 -> 12 + 9 us; a 3 x 3 convolution of 64 x 32 x 32 positions, 32 ->
+// 64 channels in fp32, forward 314 -> 36 us, weight gradient 2106 -> 64 us with its summing launch, input gradient (which
+// only the batch and channel axes kept apart: 2048 threads) 28 500 -> 50 us.
+//
+// Offsets within a batch entry are ints: contract_any_fits (contract_any.hip) says what may come here.
 #pragma once
 
 template <bool C, typename A, typename B> struct ocn_if { using type = A; };

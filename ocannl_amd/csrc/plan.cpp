@@ -323,7 +323,9 @@ bool match_contraction(const Routine& r, Phase& ph, const PlanOptions& opt) {
     if (std::min(g.M, g.N) < 8 || std::max(g.M, g.N) < 16 || g.K < 8) return false;
     for (int id : {pa->node, pb->node, set.node}) if (r.node(id).num_elems() > (int64_t)0x3FFFFFFF) return false;   // 32-bit offsets
     // A bf16 sum that a generated kernel would run in one thread is rounded after every addition, as the
-    // reference's is; one whose lanes share the sum is kept in fp32 and rounded once, as here.
+    // reference's is; one whose lanes share the sum is kept in fp32 and rounded once, as here.  So the tile takes
+    // what lanes would share and leaves the rest its numbers.  (Contractions of regular shape round once whatever
+    // their layout: 64 x 64 x 64 with both operands row-contiguous does, 65 x 63 x 67 is a serial sum.)
     if (nc.prec == Prec::Bfloat16) {
       Phase alone = ph;
       alone.kind = Phase::Generic;

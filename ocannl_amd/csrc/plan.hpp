@@ -191,9 +191,11 @@ struct PlanOptions {
   // per unrolled iteration (these kernels are bound by the memory system, not by instruction count).
   bool row_vec4 = false;
   // Plain runs replay a captured HIP graph of the routine's kernels: 1 always, 0 never, -1 where it pays.  Launched
-  // one by one a kernel costs the host 3.2 us, replayed 1.1 us plus about 6 us per graph, so it pays for many kernels
-  // that each run for less than that: 48 kernels of a small transformer step 155 -> 103 us, nine of the char-MLP step
-  // 29.3 -> 29.0 us, 65 kernels of 8 us each 529 -> 533 us.
+  // one by one a kernel costs the host 2.4 to 3.2 us, replayed 1.1 us plus about 6 us per graph, so it pays for many
+  // kernels that each run for less than that: 48 kernels of a small transformer step 121 -> 104 us; nine of the char-MLP
+  // step 23.1 -> 29.2 us (30.7 -> 28.9 where the caller sets the next batch ahead of each step: its host time is then the
+  // longer part either way); 65 kernels of 8 us each 527 -> 532 us; transformer steps of 32 to 179 kernels of 4 to 16 us
+  // each within 2 % either way.
   int graphs = -1;
   int group_window = 1 << 30;        // contractions share a launch only when at most this many phases apart
   // contractions off the critical path run on a second queue beside the rest (side_queue=1).  Off:
