@@ -283,10 +283,11 @@ __device__ __forceinline__ void ocn_any_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// Folded consumers of a bf16 result (GemmArgs): a bias by column, relu into a second tensor or in place.
+// Folded consumers of a bf16 result (GemmArgs): a bias by column, relu into a second tensor or in place.  The second
+// tensor is laid out as C and found from where C's element is, in every batch entry.
 struct OcnAnyEpilogue {
   const unsigned short* bias;
-  unsigned short* relu_out;
+  long relu_from_c;           // bytes; 0: none
   int relu_c;
 };
 
@@ -499,7 +500,7 @@ __device__ __forceinline__ void ocn_any_tile(const OcnAnyDesc& d, const void* a,
         cf[at] = acc[i][j][e];
         if (c2) static_cast<unsigned short*>(c2)[at] = to_bf16(acc[i][j][e]);
       });
-    } else if (!d.accumulate && !ep.bias && !ep.relu_out && !ep.relu_c)
+    } else if (!d.accumulate && !ep.bias && !ep.relu_from_c && !ep.relu_c)
       cells(single, [&](int j, int i, int, int e, int, int at) __attribute__((always_inline)) { ch[at] = to_bf16(acc[i][j][e]); });
     else {
       if (d.accumulate) cells(single, [&](int j, int i, int, int e, int, int at) __attribute__((always_inline)) { acc[i][j][e] += __uint_as_float((unsigned)ch[at] << 16); });
@@ -507,7 +508,7 @@ __device__ __forceinline__ void ocn_any_tile(const OcnAnyDesc& d, const void* a,
         unsigned short x = to_bf16(acc[i][j][e]);
         if (ep.bias) x = to_bf16(__uint_as_float((unsigned)x << 16) + __uint_as_float((unsigned)ep.bias[n] << 16));
         const unsigned short y = (x & 0x8000u) || (x & 0x7FFFu) > 0x7F80u ? (unsigned short)0 : x;   // fmaxf(0, x)
-        if (ep.relu_out) ep.relu_out[at] = y;
+        if (ep.relu_from_c) *reinterpret_cast<unsigned short*>(reinterpret_cast<char*>(ch + at) + ep.relu_from_c) = y;
         ch[at] = ep.relu_c ? y : x;
       });
     }

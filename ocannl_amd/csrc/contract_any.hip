@@ -17,8 +17,7 @@ __global__ void __launch_bounds__(256) contract_any_reduce_kernel(const OcnAnyDe
   const int z = blockIdx.y;
   const void *a, *b;
   void *c, *c2;
-  unsigned short* relu_out;   // (a folded layer is never split)
-  any_operands(d, q, p, z, a, b, c, c2, relu_out);
+  any_operands(d, q, p, z, a, b, c, c2);
   const float* ws = p.ws + (long)z * d.splits * cells + i;
   float v = 0.0f;
 #pragma unroll 16
@@ -141,7 +140,7 @@ hipError_t launch_contract_any(const GemmDesc& g, const GemmArgs& in, void* work
   p.a[0] = in.a; p.b[0] = in.b; p.c[0] = in.c; p.c2[0] = in.c2;
   for (int i = 1; i < in.ngroups; ++i) { p.a[i] = in.a_more[i - 1]; p.b[i] = in.b_more[i - 1]; p.c[i] = in.c_more[i - 1]; p.c2[i] = in.c2_more[i - 1]; }
   p.ws = static_cast<float*>(workspace);
-  p.ep = {static_cast<const unsigned short*>(in.bias), static_cast<unsigned short*>(in.relu_out), in.relu_c};
+  p.ep = {static_cast<const unsigned short*>(in.bias), in.relu_out ? static_cast<const char*>(in.relu_out) - static_cast<const char*>(in.c) : 0, in.relu_c};
   const long entries = (long)q.batches * q.members, tiles = (long)d.tiles_m * d.tiles_n * entries;
   if (tiles <= 0 || tiles > 0x3FFFFFFFL || entries > 65535 || in.npairs != 1 || (sh.splits > 1 && !p.ws)) return hipErrorInvalidValue;
   const dim3 grid((unsigned)((tiles + 7) / 8 * 8), (unsigned)sh.splits, 1);

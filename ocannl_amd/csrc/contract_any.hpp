@@ -30,7 +30,7 @@ constexpr int kAnyDepth = 2;
 
 // Batch entry z of the launch -> operands.
 __device__ __forceinline__ void any_operands(const OcnAnyDesc& d, const AnyBatch& q, const AnyPtrs& p, int z, const void*& a, const void*& b, void*& c,
-                                             void*& c2, unsigned short*& relu_out) {
+                                             void*& c2) {
   const int g = q.members > 1 ? z / q.batches : 0;
   int r = z - g * q.batches;
   long ao = 0, bo = 0, co = 0;
@@ -45,7 +45,6 @@ __device__ __forceinline__ void any_operands(const OcnAnyDesc& d, const AnyBatch
   b = static_cast<const char*>(b) + bo * (d.b.bf16 ? 2 : 4);
   c = static_cast<char*>(c) + co * (d.c_bf16 ? 2 : 4);
   if (c2) c2 = static_cast<char*>(c2) + co * 2;
-  relu_out = p.ep.relu_out ? p.ep.relu_out + co : nullptr;
 }
 
 // Grid: x = tiles of all batch entries, padded to a multiple of eight and dealt so that each XCD (workgroup
@@ -60,10 +59,9 @@ __device__ __forceinline__ void any_body(const OcnAnyDesc& d, const AnyBatch& q,
   if (z >= q.batches * q.members) return;
   const void *a, *b;
   void *c, *c2;
-  OcnAnyEpilogue ep = p.ep;
-  any_operands(d, q, p, z, a, b, c, c2, ep.relu_out);
+  any_operands(d, q, p, z, a, b, c, c2);
   float* const ws = d.splits > 1 ? p.ws + (long)z * d.splits * d.M * d.N : nullptr;
-  ocn_any_tile<BM, BN, A_KC, B_KC, ABF, BBF, false, kAnyDepth>(d, a, b, c, c2, ws, ep, r / d.tiles_n, r % d.tiles_n, (int)blockIdx.y, 0, 0, smem_any);
+  ocn_any_tile<BM, BN, A_KC, B_KC, ABF, BBF, false, kAnyDepth>(d, a, b, c, c2, ws, p.ep, r / d.tiles_n, r % d.tiles_n, (int)blockIdx.y, 0, 0, smem_any);
 }
 
 template <int BM, int BN, bool A_KC, bool B_KC>
