@@ -309,14 +309,13 @@ __device__ __forceinline__ void ocn_any_tile(const OcnAnyDesc& d, const void* a,
   const int wm = (wave / GN) * WM, wn = (wave % GN) * WN, m0 = tm * BM, n0 = tn * BN;
   const int steps = (d.K + BK - 1) / BK, per = (steps + d.splits - 1) / d.splits;
   const int kbeg = split * per * BK;
-  int kend = kbeg + per * BK < d.K ? kbeg + per * BK : d.K;
+  const int kend = kbeg + per * BK < d.K ? kbeg + per * BK : d.K;
+  // a residue that no tap has (an axis of fewer taps than its step) sums nothing and reads nothing: `b` is then where
+  // the tap would be, past the weights as they are stored
+  bool none = false;
   if constexpr (WIN) {
-    // a residue that no tap has (an axis of fewer taps than its step) sums nothing and reads nothing: `b` is then where
-    // the tap would be, past the weights as they are stored
-    if (r0 >= d.win_taps[0] || r1 >= d.win_taps[1]) {
-      if (d.accumulate) return;
-      kend = kbeg;
-    }
+    none = r0 >= d.win_taps[0] || r1 >= d.win_taps[1];
+    if (none && d.accumulate) return;
   }
   const int ksteps = kend > kbeg ? (kend - kbeg + BK - 1) / BK : 0;
   const bool ra = ocn_any_regular<A_KC, F32>(d.a, d.dm, d.dk, d.M), rb = ocn_any_regular<B_KC, F32>(d.b, d.dn, d.dk, d.N);
@@ -448,7 +447,8 @@ __device__ __forceinline__ void ocn_any_tile(const OcnAnyDesc& d, const void* a,
       multiply(n & 1);
     }
   };
-  if (ra && rb) {
+  if (none) {
+  } else if (ra && rb) {
     if (d.dk.n == 1) pipeline(Yes{}); else pipeline(No{});
   } else {
     if (ksteps > 0) gather(qa[0], qb[0], 0);
@@ -534,8 +534,10 @@ __device__ __forceinline__ void ocn_any_tile(const OcnAnyDesc& d, const void* a,
       const OcnDigitVal md = ocn_digits(d.dm, m), nd = ocn_digits(d.dn, n);
       if (d.win_s[0] * md.d1 + r0 >= d.win_pos[0] || d.win_s[1] * md.d2 + r1 >= d.win_pos[1]) continue;
       float v = 0.0f;
+#pragma unroll 1
       for (int t0 = 0; d.win_s[0] * t0 + r0 < d.win_taps[0]; ++t0) {
         if ((unsigned)(md.d1 - t0) >= (unsigned)d.win_lim[0]) continue;
+#pragma unroll 1
         for (int t1 = 0; d.win_s[1] * t1 + r1 < d.win_taps[1]; ++t1) {
           if ((unsigned)(md.d2 - t1) >= (unsigned)d.win_lim[1]) continue;
           long at_a = (long)ocn_digit_off(md, d.a.row) + ocn_digit_off({t0, t1, 0}, d.a.k), at_b = (long)ocn_digit_off(nd, d.b.row) + ocn_digit_off({t0, t1, 0}, d.b.k);
