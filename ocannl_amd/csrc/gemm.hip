@@ -531,12 +531,14 @@ bool dtl_operands_ok(const GemmArgs& a, bool akc, bool bkc) {
 // product, register-staged against small tile: 1000 x 1000, both row-contiguous: K = 1024 fp32 50 against 33 us, bf16
 // 18 against 12; 2048 fp32 52 against 59, bf16 21 against 20; 8192 fp32 157 against 225, bf16 44 against 66.  From 256
 // tiles on the larger tile wins (8000 x 1000 x 1000 bf16, both gradients too: 122 against 173 us).
-bool gemm_prefers_any(const GemmDesc& d) {
+// A workspace that would take the routine beyond the static scratch array, where the small tile's does not, is no choice.
+bool gemm_prefers_any(const GemmDesc& d, uint64_t room) {
   if (d.any || !d.more.empty() || d.a.prec != d.b.prec || !contract_any_fits(d)) return false;
   const int64_t t128 = (int64_t)((d.M + 127) / 128) * ((d.N + 127) / 128) * batch_count(d);
   if (t128 >= 256) return false;
   const bool f32 = d.a.prec == Prec::Single;
   if (!f32 && dtl_shape(d).bm != 0) return false;
+  if (gemm_workspace_bytes(d) > room && contract_any_workspace_bytes(d) <= room) return true;
   const TileConfig c = tile_config(d);
   const int64_t staged = (t128 * c.splits + 255) / 256 * 128 * (c.narrow ? 64 : 128) / c.splits;
   bool alone;

@@ -60,8 +60,9 @@ size_t gemm_workspace_bytes(const GemmDesc& desc);
 // Name of the instance launch_gemm would pick (for kernel_info and profiles).
 const char* gemm_kernel_name(const GemmDesc& desc);
 
-// Is this contraction, which the kernels of gemm.hip could take, faster as one of any shape (contract_any.hip)?
-bool gemm_prefers_any(const GemmDesc& desc);
+// Is this contraction, which the kernels of gemm.hip could take, faster as one of any shape (contract_any.hip)?  `room`:
+// bytes of workspace that keep the routine's scratch within what ocannl_hip_routine_run_static_scratch has.
+bool gemm_prefers_any(const GemmDesc& desc, uint64_t room);
 
 // contract_any.hip: the same for contractions with `desc.any` set (launch_gemm and its siblings forward to these).
 // Do the extents and the element offsets within one batch entry fit the 32-bit arithmetic of contract_any.h?

@@ -1,4 +1,5 @@
 #include "gemm.hpp"
+#include "ocannl_hip.h"
 #include "plan.hpp"
 
 #include <algorithm>
@@ -2552,8 +2553,12 @@ Plan make_plan(Routine& r, const PlanOptions& requested) {
   if (opt.enable_mfma && opt.enable_coop && opt.enable_row_groups && opt.fuse_row_contractions) fuse_row_contractions(r, plan, opt.fuse_stored_rows, opt.row_tile_waves);
   if (opt.enable_mfma && opt.enable_coop && opt.enable_row_groups && opt.fuse_row_contractions && opt.fuse_row_projections) fuse_row_projections(r, plan);
   if (opt.enable_mfma && opt.any_contractions) {
+    uint64_t local = 0;   // (as link lays out the arena)
+    for (auto& kv : r.nodes) if (kv.second.mode == Mode::Local) local += ((uint64_t)kv.second.size_in_bytes() + 255) / 256 * 256;
+    constexpr uint64_t limit = OCANNL_HIP_STATIC_SCRATCH_BYTES;
+    const uint64_t room = local <= limit ? limit - local : ~0ull;
     for (auto& ph : plan.phases) {
-      if (ph.kind != Phase::Contraction || !gemm_prefers_any(ph.gemm)) continue;
+      if (ph.kind != Phase::Contraction || !gemm_prefers_any(ph.gemm, room)) continue;
       GemmDesc& g = ph.gemm;
       auto digits = [](GemmOperand& o) { o.row_stride[2] = o.s_row; o.k_stride[2] = o.s_k; };
       digits(g.a); digits(g.b); digits(g.c);

@@ -45,6 +45,21 @@ def test_small_tiles_where_they_go_through_less(shape, layout, small, prec):
     assert ("kernel_any<64, 64" in name) == small
 
 
+@pytest.mark.parametrize("local_mib,small", [(0, False), (8, True), (31, True), (40, False)])
+def test_a_workspace_does_not_take_a_routine_beyond_the_static_scratch(local_mib, small):
+    # 1000 x 1000 x 8192 staged: eight splits, 30.5 of 32 MiB; beside local tensors that leave less the small tile, which
+    # needs none, keeps the routine runnable without an allocation (beyond 32 MiB it is not, either way)
+    r = _product(1000, 1000, 8192, "single", False, False)
+    if local_mib:
+        i, n = L.fresh_symbol(), local_mib << 18
+        src, local, out = L.Node(4, "src", "single", (n,)), L.Node(5, "local", "single", (n,), mode="local"), L.Node(6, "out", "single", (n,))
+        at = (L.It(i),)
+        copy = lambda d, s: L.For(i, 0, n - 1, [L.Set(d, at, L.Unop("neg", L.Get(s, at)))])
+        r.body.extend([copy(local, src), copy(out, local)])
+    name, = _matrix_kernels(r)
+    assert ("kernel_any<64, 64" in name) == small
+
+
 def test_sums_of_more_terms_than_32_bits_count_are_left_alone():
     # k in two digits over operands of few elements: x[i + j] * w[i + j], 2^31 terms and more
     def names(I, J):
