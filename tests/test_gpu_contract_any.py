@@ -25,10 +25,10 @@ def _run(r, nodes, out, want, accumulate, k, seed=0):
     hip = HipRun(r, init, "min_mfma_flops=1")
     ks = [x for x in hip.code.kernels() if x["kind"] == "mfma"]
     if not ks and nodes[out].prec == "bfloat16":
-        # a sum that one thread runs, rounded after every addition: left alone, and the checker's bits
-        checker = OracleRun(r, init)
-        hip.step(); checker.step()
-        assert np.array_equal(hip.get(nodes[out]).ravel(), np.asarray(checker.get(nodes[out])).ravel())
+        # a sum that one thread runs, rounded after every addition: left alone, and the oracle's bits
+        oracle = OracleRun(r, init)
+        hip.step(); oracle.step()
+        assert np.array_equal(hip.get(nodes[out]).ravel(), np.asarray(oracle.get(nodes[out])).ravel())
         return hip.close()
     assert ks and all("_kernel_any" in x["name"] for x in ks), hip.code.kernels()
     hip.step()

@@ -41,7 +41,7 @@ def test_row_lengths(q, k, d):
 @pytest.mark.parametrize("opts", ["serial=0", None])
 @pytest.mark.parametrize("q,k,d", [(7, 63, 9), (9, 99, 7), (197, 197, 16), (2, 1003, 8), (64, 1025, 5)])
 def test_row_lengths_in_bf16(q, k, d, opts):
-    # Against the checker in fp32 on the same values: 2e-2 in the Frobenius norm as every bf16 routine, and no element
+    # Against the oracle in fp32 on the same values: 2e-2 in the Frobenius norm as every bf16 routine, and no element
     # further off than 2^-5 of the tensor's largest -- scores, exponentials, weights and their gradients carry up to
     # sixteen roundings of 2^-9, and a gradient is a sum of few terms that cancel, so its own row sets no scale.
     w, wr = (W.attention(b=1, h=2, q=q, k=k, d=d, prec=p, grad_prec="single") for p in ("bfloat16", "single"))
