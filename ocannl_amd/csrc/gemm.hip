@@ -19,7 +19,7 @@
 //   * v_mfma_f32_32x32x16_bf16, each wavefront owns a (BM/2) x (BN/2) sub-tile;
 //   * workgroup ids are remapped so that each XCD (ids are dealt round-robin over 8 XCDs) works on
 //     a compact band of tiles and shares B/A panels through its own L2.
-// fp32 compute uses v_mfma_f32_32x32x2_f32 with the same staging.
+// fp32 operands: gemm_f32.hip.
 #include <hip/hip_runtime.h>
 
 #include <cstdio>
@@ -33,6 +33,8 @@ namespace ocannl {
 
 // gemm_dtl.hip: the direct-to-LDS instance of that shape (one of those dtl_shape() names).
 hipError_t launch_gemm_dtl(int bm, int bn, int bk, int ns, bool akc, bool bkc, const GemmArgs& a, hipStream_t s, hipEvent_t ev);
+// gemm_f32.hip: fp32 operands, 256 x 256 (big) or 128 x 128 tiles.
+hipError_t launch_gemm_f32(bool big, bool akc, bool bkc, const GemmArgs& a, hipStream_t s, hipEvent_t ev);
 
 namespace {
 
@@ -269,147 +271,8 @@ gemm_bf16_kernel(const GemmArgs g) {
                    reinterpret_cast<float*>(smem) + wave * ((kAT + kBT) / 4));
 }
 
-// ---- fp32 compute -------------------------------------------------------------------------------
-// v_mfma_f32_32x32x2_f32: a lane supplies one float of its row per instruction; instruction q of a
-// group of four multiplies k = q (lanes 0-31) and k = 4 + q (lanes 32-63) of an 8-k sub-step -- A
-// and B use the same assignment, so the sum is complete.
-//   K-contiguous operand:   LDS [row][k], row stride kBKf + kPadf: a lane reads its four k with one
-//     ds_read_b128.
-//   row-contiguous operand: LDS [k][row] as it lies in memory, row stride ROWS + kPadTf: a lane
-//     reads its four k with four ds_read_b32 (lanes of a half read 32 consecutive floats; the two
-//     halves sit 4 k-rows = 32 banks apart): no transposition anywhere.
-constexpr int kPadTf = 8;
-
-template <int ROWS, bool KC>
-constexpr int lds_tile_floats() { return KC ? ROWS * (kBKf + kPadf) : kBKf * (ROWS + kPadTf); }
-
-template <int ROWS, bool KC>
-struct StagerF {
-  static constexpr int kChunks = ROWS * (kBKf / 4) / kThreads;   // 16-byte chunks per thread
-  static constexpr int kPerLine = KC ? kBKf / 4 : ROWS / 4;      // chunks per contiguous line
-  static constexpr int kLineStride = KC ? kBKf + kPadf : ROWS + kPadTf;
-  f32x4 regs[kChunks];
-
-  __device__ __forceinline__ void load(const float* base, long ld, long row0, long k0, long rows, long K, int tid) {
-#pragma unroll
-    for (int j = 0; j < kChunks; ++j) {
-      const int c = tid + kThreads * j;
-      const long line = c / kPerLine, pos = (c % kPerLine) * 4;
-      f32x4 v = {0, 0, 0, 0};
-      if (KC) { if (row0 + line < rows && k0 + pos < K) v = *reinterpret_cast<const f32x4*>(base + (row0 + line) * ld + k0 + pos); }
-      else    { if (k0 + line < K && row0 + pos < rows) v = *reinterpret_cast<const f32x4*>(base + (k0 + line) * ld + row0 + pos); }
-      regs[j] = v;
-    }
-  }
-
-  __device__ __forceinline__ void store(float* lds, int tid) const {
-#pragma unroll
-    for (int j = 0; j < kChunks; ++j) {
-      const int c = tid + kThreads * j;
-      *reinterpret_cast<f32x4*>(lds + (c / kPerLine) * kLineStride + (c % kPerLine) * 4) = regs[j];
-    }
-  }
-};
-
-template <int BM, int BN, bool A_KC, bool B_KC>
-__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, BM >= 256 ? 1 : 2)))
-gemm_f32_kernel(const GemmArgs g) {
-  constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 32, TN = WN / 32;
-  constexpr int kAT = lds_tile_floats<BM, A_KC>(), kBT = lds_tile_floats<BN, B_KC>();
-  constexpr int kAS = StagerF<BM, A_KC>::kLineStride, kBS = StagerF<BN, B_KC>::kLineStride;
-  extern __shared__ __align__(16) unsigned short smem[];
-  float* fsm = reinterpret_cast<float*>(smem);
-  float* const As0 = fsm;
-  float* const Bs0 = fsm + 2 * kAT;
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm0 = (wave >> 1) * WM, wn0 = (wave & 1) * WN;
-  const long tiles_m = (g.M + BM - 1) / BM, tiles_n = (g.N + BN - 1) / BN;
-  long tmi, tni, wg, zz;
-  int nx;
-  place_workgroup(g, wg, zz, nx);
-  tile_of_block(wg, tiles_m, tiles_n, g.xcd_m, nx, tmi, tni);
-  const long m0 = tmi * BM, n0 = tni * BN;
-  long ao, bo, co;
-  const void *abase, *bbase;
-  void *cbase, *c2base;
-  decode_batch(g, decode_group(g, zz, abase, bbase, cbase, c2base), ao, bo, co);
-  const float* A = static_cast<const float*>(abase) + ao;
-  const float* B = static_cast<const float*>(bbase) + bo;
-  const long lda = A_KC ? g.a_row : g.a_k, ldb = B_KC ? g.b_row : g.b_k;
-
-  f32x16 acc[TM][TN];
-  static_for<TM>([&](auto ic) OCN_LAMBDA_INLINE {
-    static_for<TN>([&](auto jc) OCN_LAMBDA_INLINE {
-      static_for<16>([&](auto ec) OCN_LAMBDA_INLINE { acc[decltype(ic)::value][decltype(jc)::value][decltype(ec)::value] = 0.0f; });
-    });
-  });
-
-  StagerF<BM, A_KC> sa;
-  StagerF<BN, B_KC> sb;
-  // split-K: blockIdx.y owns a contiguous range of K steps
-  const long all_steps = (g.K + kBKf - 1) / kBKf;
-  const long per_split = (all_steps + g.splits - 1) / g.splits;
-  const long kbeg = (long)blockIdx.y * per_split * kBKf;
-  const long kend = (kbeg + per_split * kBKf) < g.K ? (kbeg + per_split * kBKf) : g.K;
-  sa.load(A, lda, m0, kbeg, g.M, kend, tid);
-  sb.load(B, ldb, n0, kbeg, g.N, kend, tid);
-  sa.store(As0, tid);
-  sb.store(Bs0, tid);
-  __syncthreads();
-
-  const long ksteps = kend > kbeg ? (kend - kbeg + kBKf - 1) / kBKf : 0;
-  for (long ks = 0; ks < ksteps; ++ks) {
-    const int cur = ks & 1;
-    const bool more = ks + 1 < ksteps;
-    if (more) {
-      sa.load(A, lda, m0, kbeg + (ks + 1) * kBKf, g.M, kend, tid);
-      sb.load(B, ldb, n0, kbeg + (ks + 1) * kBKf, g.N, kend, tid);
-    }
-    const float* as = As0 + cur * kAT + (A_KC ? (wm0 + (lane & 31)) * kAS + (lane >> 5) * 4 : (lane >> 5) * 4 * kAS + wm0 + (lane & 31));
-    const float* bs = Bs0 + cur * kBT + (B_KC ? (wn0 + (lane & 31)) * kBS + (lane >> 5) * 4 : (lane >> 5) * 4 * kBS + wn0 + (lane & 31));
-#pragma unroll
-    for (int kk = 0; kk < kBKf / 8; ++kk) {
-      f32x4 af[TM], bf[TN];
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        if (A_KC) af[i] = *reinterpret_cast<const f32x4*>(as + i * 32 * kAS + kk * 8);
-        else {
-          const float* p = as + kk * 8 * kAS + i * 32;
-          af[i] = f32x4{p[0], p[kAS], p[2 * kAS], p[3 * kAS]};
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        if (B_KC) bf[j] = *reinterpret_cast<const f32x4*>(bs + j * 32 * kBS + kk * 8);
-        else {
-          const float* p = bs + kk * 8 * kBS + j * 32;
-          bf[j] = f32x4{p[0], p[kBS], p[2 * kBS], p[3 * kBS]};
-        }
-      }
-      static_for<4>([&](auto qc) OCN_LAMBDA_INLINE {
-        static_for<TM>([&](auto ic) OCN_LAMBDA_INLINE {
-          static_for<TN>([&](auto jc) OCN_LAMBDA_INLINE {
-            constexpr int q = decltype(qc)::value, i = decltype(ic)::value, j = decltype(jc)::value;
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[i][q], bf[j][q], acc[i][j], 0, 0, 0);
-          });
-        });
-      });
-    }
-    if (more) {
-      sa.store(As0 + (cur ^ 1) * kAT, tid);
-      sb.store(Bs0 + (cur ^ 1) * kBT, tid);
-    }
-    __syncthreads();
-  }
-
-  epilogue<TM, TN>(g, cbase, c2base, acc, m0 + wm0, n0 + wn0, co, lane, fsm + wave * ((kAT + kBT) / 2));
-}
-
 template <int BM, int BN, bool A_KC, bool B_KC>
 constexpr size_t bf16_smem() { return 2ull * (lds_tile_elems<BM, A_KC>() + lds_tile_elems<BN, B_KC>()) * sizeof(unsigned short); }
-template <int BM, int BN, bool A_KC, bool B_KC>
-constexpr size_t f32_smem() { return 2ull * (lds_tile_floats<BM, A_KC>() + lds_tile_floats<BN, B_KC>()) * sizeof(float); }
 
 // Tile grids of one launch along z: batch entries times grouped contractions.
 long batch_count(const GemmDesc& d) {
@@ -467,14 +330,6 @@ hipError_t launch_bf16_layout(bool akc, bool bkc, const GemmArgs& a, hipStream_t
   if (akc && !bkc) return launch(gemm_bf16_kernel<BM, BN, AT, BT, true, false, PF, CHAIN>, bf16_smem<BM, BN, true, false>(), BM, BN, a, s, ev);
   if (!akc && bkc) return launch(gemm_bf16_kernel<BM, BN, AT, BT, false, true, PF, CHAIN>, bf16_smem<BM, BN, false, true>(), BM, BN, a, s, ev);
   return launch(gemm_bf16_kernel<BM, BN, AT, BT, false, false, PF, CHAIN>, bf16_smem<BM, BN, false, false>(), BM, BN, a, s, ev);
-}
-
-template <int BM, int BN>
-hipError_t launch_f32_layout(bool akc, bool bkc, const GemmArgs& a, hipStream_t s, hipEvent_t ev) {
-  if (akc && bkc) return launch(gemm_f32_kernel<BM, BN, true, true>, f32_smem<BM, BN, true, true>(), BM, BN, a, s, ev);
-  if (akc && !bkc) return launch(gemm_f32_kernel<BM, BN, true, false>, f32_smem<BM, BN, true, false>(), BM, BN, a, s, ev);
-  if (!akc && bkc) return launch(gemm_f32_kernel<BM, BN, false, true>, f32_smem<BM, BN, false, true>(), BM, BN, a, s, ev);
-  return launch(gemm_f32_kernel<BM, BN, false, false>, f32_smem<BM, BN, false, false>(), BM, BN, a, s, ev);
 }
 
 bool a_kcontig(const GemmDesc& d) { return d.a.s_k == 1 || d.K == 1; }
@@ -557,7 +412,7 @@ const char* gemm_kernel_name(const GemmDesc& d) {
   const char* tf[2] = {"false", "true"};
   const DtlShape ds = dtl_shape(d);
   if (af && bf)
-    snprintf(buf, sizeof buf, "gemm_f32_kernel<%d, %d, %s, %s>", tile, tile, tf[a_kcontig(d)], tf[b_kcontig(d)]);
+    snprintf(buf, sizeof buf, "gemm_f32_kernel<%d, %d, 2, 2, %s, %s>", tile, tile, tf[a_kcontig(d)], tf[b_kcontig(d)]);
   else if (ds.bm)   // (operands that turn out misaligned at launch take the register-staged kernel instead)
     snprintf(buf, sizeof buf, "gemm_bf16_dtl_kernel<%d, %d, %d, %d, %s, %s>", ds.bm, ds.bn, ds.bk, ds.ns, tf[a_kcontig(d)], tf[b_kcontig(d)]);
   else
@@ -604,7 +459,7 @@ hipError_t launch_gemm(const GemmDesc& d, const GemmArgs& a_in, void* workspace,
     }
   }
   const bool af = d.a.prec == Prec::Single, bf = d.b.prec == Prec::Single;
-  if (af && bf) return big ? launch_f32_layout<256, 256>(akc, bkc, a, s, ev) : launch_f32_layout<128, 128>(akc, bkc, a, s, ev);
+  if (af && bf) return launch_gemm_f32(big, akc, bkc, a, s, ev);
   if (a.npairs > 1 && (af || bf)) return hipErrorInvalidValue;   // chains: bf16 operands only
   if (!af && !bf) {
     const DtlShape ds = dtl_shape(d);

@@ -34,8 +34,6 @@ __device__ __forceinline__ void static_for(F&& f) {
 constexpr int kThreads = 256;
 constexpr int kBK = 64;        // K elements per stage (bf16 compute)
 constexpr int kPad = 8;        // bf16 elements of row padding (16 bytes)
-constexpr int kBKf = 32;       // K elements per stage (fp32 compute)
-constexpr int kPadf = 4;       // floats of row padding (16 bytes)
 
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
@@ -450,7 +448,7 @@ __global__ void __launch_bounds__(256) splitk_reduce_kernel(const GemmArgs g) {
 // Launches `kernel` over the tile grid of `a` (x: tiles, y: K splits, z: members x batch entries) and,
 // after a K split, the reduction pass.
 template <typename K>
-hipError_t launch(K kernel, size_t smem, int BM, int BN, GemmArgs a, hipStream_t s, hipEvent_t after_main) {
+hipError_t launch(K kernel, size_t smem, int BM, int BN, GemmArgs a, hipStream_t s, hipEvent_t after_main, int threads = kThreads) {
   static thread_local const void* configured[128];
   static thread_local int n_configured = 0;
   bool done = false;
@@ -468,7 +466,7 @@ hipError_t launch(K kernel, size_t smem, int BM, int BN, GemmArgs a, hipStream_t
   nb *= a.ngroups;
   if (tiles <= 0 || tiles > 0x7FFFFFFFL || nb <= 0 || nb > 65535) return hipErrorInvalidValue;
   if (a.splits > 1 && (!a.ws || a.N % 4 != 0)) return hipErrorInvalidValue;   // (the reduction pass adds four columns per thread)
-  hipLaunchKernelGGL(kernel, dim3((unsigned)tiles, (unsigned)a.splits, (unsigned)nb), dim3(kThreads), smem, s, a);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)tiles, (unsigned)a.splits, (unsigned)nb), dim3((unsigned)threads), smem, s, a);
   hipError_t e = hipGetLastError();
   if (e == hipSuccess && after_main) e = hipEventRecord(after_main, s);
   if (e != hipSuccess || a.splits <= 1) return e;

@@ -425,3 +425,37 @@ def test_relu_of_the_biased_product_in_one_statement_is_folded_too(shape):
     assert np.array_equal(zf, two.get(z2.value))
     assert np.any(W.to_float(zf, "bfloat16") > 0) and np.any(W.to_float(zf, "bfloat16") == 0)
     folded.close(); apart.close(); two.close()
+
+
+@pytest.mark.parametrize("a_kc,b_kc", [(True, True), (True, False), (False, True), (False, False)])
+@pytest.mark.parametrize("M,N,K", [(512, 512, 512), (1020, 516, 36), (4096, 4096, 512), (4100, 4092, 520)])
+@pytest.mark.parametrize("what", ["tiny", "special"])
+def test_f32_products_outside_the_split_range(M, N, K, a_kc, b_kc, what):
+    """fp32 operands are multiplied as sums of three bf16 values; values whose parts are none (below 2^-102), and
+    infinities, NaN and values above the largest bf16, give what fp32 products give."""
+    if M > 2000 and (a_kc, b_kc) in ((True, False), (False, True)):
+        pytest.skip("large tiles: the two uniform layouts")
+    r, A, B, C = _routine(M, N, K, "single", "single", "single", a_kc, b_kc, False)
+    rng = np.random.default_rng(3)
+    a, b = rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((N, K)).astype(np.float32)
+    if what == "tiny":
+        a[: M // 2] *= np.float32(2.0 ** -118)          # the other half of the tiles' rows is ordinary
+        b *= np.float32(2.0 ** 30)
+        b[:, K // 2:] = 1.0                              # (whose mid and lo parts are zero)
+    else:
+        b[:, :4] = 1.0
+        a[3, 1], a[M - 1, 0], a[M // 2, 2], b[N - 2, K - 1] = np.inf, -np.inf, np.nan, np.float32(3.4e38)
+        a[:, K - 1] = rng.choice(np.float32([0.5, 0.25]), M)
+    hip = HipRun(r, {1: np.ascontiguousarray(a if a_kc else a.T), 2: np.ascontiguousarray(b if b_kc else b.T)}, "min_mfma_flops=1;any=0")
+    assert hip.code.kernels()[-1]["name"].startswith("gemm_f32_kernel<"), hip.code.kernels()
+    hip.step()
+    got = hip.get(C).astype(np.float64)
+    hip.close()
+    with np.errstate(all="ignore"):
+        want = a.astype(np.float64) @ b.astype(np.float64).T
+        size = np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64).T
+    fine = np.isfinite(want)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[~fine & ~np.isnan(want)], want[~fine & ~np.isnan(want)])
+    # K roundings of fp32, each of half a unit of a partial sum that is no larger than `size`
+    err = np.abs(got[fine] - want[fine]) / size[fine]
+    assert err.max() <= K * 2.0 ** -24, err.max()
