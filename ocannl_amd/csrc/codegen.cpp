@@ -1,4 +1,5 @@
 #include "codegen.hpp"
+#include "gemm.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -1066,6 +1067,8 @@ void touched_nodes(const Block& b, std::set<int>& rd, std::set<int>& wr, std::se
 uint64_t emit_window(const Routine& r, const Phase& ph, std::vector<std::string>& body) {
   const GemmDesc& g = ph.gemm;
   const bool f32 = g.a.prec != Prec::Bfloat16 || g.b.prec != Prec::Bfloat16;
+  const std::string precs = std::string(g.a.prec == Prec::Bfloat16 ? "true, " : "false, ") + (g.b.prec == Prec::Bfloat16 ? "true" : "false");
+  const std::string parts = f32 && g.K >= kPartsFrom ? "true" : "false";
   // channels of c (n) of at most 32 take the narrow tile: half of a square one would be padding
   const int BM = g.N <= 32 ? 128 : 64, BN = g.N <= 32 ? 32 : 64;
   const bool bkc = g.b.k_stride[2] == 1 || g.b.row_stride[2] != 1;
@@ -1090,12 +1093,12 @@ uint64_t emit_window(const Routine& r, const Phase& ph, std::vector<std::string>
   const std::string shape = std::to_string(BM) + ", " + std::to_string(BN) + ", true, " + (bkc ? "true" : "false") + ", ";
   const int64_t blocks = (tm * tn * residues + 7) / 8 * 8;
   body.push_back("  constexpr OcnAnyDesc d_ = " + d.str() + ";");
-  body.push_back("  __shared__ __attribute__((aligned(16))) unsigned char smem_[ocn_any_smem<" + shape + (f32 ? "true" : "false") + ">()];");
+  body.push_back("  __shared__ __attribute__((aligned(16))) unsigned char smem_[ocn_any_smem<" + shape + precs + ", " + parts + ">()];");
   body.push_back("  const int t_ = (int)(blockIdx.x % 8u) * " + std::to_string(blocks / 8) + " + (int)(blockIdx.x / 8u);");
   body.push_back("  if (t_ >= " + std::to_string(tm * tn * residues) + ") return;");
   body.push_back("  const int z_ = t_ / " + std::to_string(tm * tn) + ", q_ = t_ % " + std::to_string(tm * tn) + ", r0_ = z_ / " + std::to_string(ph.win_s[1]) +
                  ", r1_ = z_ % " + std::to_string(ph.win_s[1]) + ";");
-  body.push_back("  ocn_any_tile<" + shape + (g.a.prec == Prec::Bfloat16 ? "true, " : "false, ") + (g.b.prec == Prec::Bfloat16 ? "true" : "false") + ", true, 2>(d_, " + r.node(g.a.node).ident + " + " + std::to_string(g.a.offset) + ", " + r.node(g.b.node).ident + " + " +
+  body.push_back("  ocn_any_tile<" + shape + precs + ", true, 2, " + parts + ">(d_, " + r.node(g.a.node).ident + " + " + std::to_string(g.a.offset) + ", " + r.node(g.b.node).ident + " + " +
                  std::to_string(g.b.offset) + " + r0_ * " + std::to_string(ph.win_b[0]) + " + r1_ * " + std::to_string(ph.win_b[1]) + ", " +
                  r.node(g.c.node).ident + " + " + std::to_string(g.c.offset) + " + r0_ * " + std::to_string(ph.win_c[0]) + " + r1_ * " +
                  std::to_string(ph.win_c[1]) + ", (void*)0, (float*)0, OcnAnyEpilogue{0, 0, 0}, q_ / " + std::to_string(tn) + ", q_ % " + std::to_string(tn) + ", 0, r0_, r1_, smem_);");

@@ -13,15 +13,19 @@
 // of the register-staged kernels (gemm_common.hpp): rows padded by 16 bytes for a k-contiguous operand,
 // [k][row] with ds_read_b64_tr_b16 fragments for a row-contiguous bf16 one.
 //
-// What bounds it: latency of a K step (load, LDS, barrier), about a microsecond, with one or two workgroups per compute
-// unit to hide it: matrix cores busy 4 to 5 % and about 5 TB/s out of L2 on the bf16 products of 1777 x 1001 x 771, no
-// bank conflicts; in fp32, whose products take sixteen times as long, the matrix cores are busy 26 to 39 %.  Rows at odd
-// elements, and the row-contiguous fp32 fragments of four reads, cost more (the last two launches of the dense layer, the
-// weight gradient of the convolution).  Kernel trace, as generated kernels with one thread or lane group per element of C
-// -> as tiles: the dense layer above, forward and both gradients, 4192 -> 16 + 21 + 25 us; attention scores and their
-// product with V over 197 positions, 96 heads, 438 + 569 -> 12 + 9 us; a 3 x 3 convolution of 64 x 32 x 32 positions, 32 ->
-// 64 channels in fp32, forward 314 -> 36 us, weight gradient 2106 -> 64 us with its summing launch, input gradient (which
-// only the batch and channel axes kept apart: 2048 threads) 28 500 -> 50 us.
+// What bounds it: in bf16 what the tiles read out of L2.  64 of K of a 64 x 64 tile take 0.29 us where every compute unit has
+// one, 0.56 us with two: 14 TB/s, the rate at which tiles reach LDS in every kernel here; alone on a unit the latency of a
+// step (0.27 us).  Start, stores and launch are 4.5 to 6 us.  Rows at odd elements cost 1.2 to 1.5 times as much.  With
+// fp32 operands in parts 1.0 us (two: 1.9): LDS, a kilobyte of fragments for every 32 cycles of products of a wavefront's
+// 32 x 32 cells, beside the 130 vector instructions that split 16 values; 128 x 128 tiles 0.72 us per 64 x 64 cells.
+// 1777 x 771 x 1001, k-contiguous: bf16 15.6 us with a loop that waited for all of its loads in every turn, 14.4 now; fp32
+// 40.2 us on the fp32 instructions, 32.3 in parts; both row-contiguous 16.9 -> 15.9 and 49.9 -> 35.7.  4001 x 4003 x 1001 in
+// fp32 (128 x 128 tiles) 313 -> 196 us; the convolution below with both gradients 137 -> 117 us.
+// Kernel trace, as generated kernels with one thread or lane group per element of C -> as tiles, first version: a dense
+// layer of 1777 x 1001 -> 771, forward and both gradients, 4192 -> 16 + 21 + 25 us; attention scores and their product with V
+// over 197 positions, 96 heads, 438 + 569 -> 12 + 9 us; a 3 x 3 convolution of 64 x 32 x 32 positions, 32 -> 64 channels in
+// fp32, forward 314 -> 36 us, weight gradient 2106 -> 64 us with its summing launch, input gradient (which only the batch
+// and channel axes kept apart: 2048 threads) 28 500 -> 50 us.
 //
 // Offsets within a batch entry are ints: contract_any_fits (contract_any.hip) says what may come here.
 #pragma once
@@ -79,24 +83,41 @@ __device__ __forceinline__ OcnDigitVal ocn_digits(const OcnDigits& d, int x) {
 }
 __device__ __forceinline__ int ocn_digit_off(const OcnDigitVal& v, const int (&s)[3]) { return v.d0 * s[0] + v.d1 * s[1] + v.d2 * s[2]; }
 
-// ROWS x BK tile of one operand: global -> registers -> LDS, 256 threads.  F32: fp32 in LDS (bf16 sources are
-// widened, exactly), chunks of 4; else bf16 in LDS, chunks of 8.  WIN: see OcnAnyDesc (1: this is A, 2: B).
+// How an operand lies in LDS: bf16, both operands being bf16 (chunks of 8); else in chunks of 4, as the three bf16 parts
+// of its fp32 values, each in a plane of its own, or as its bf16 values beside an operand in parts; or, where parts do
+// not do (see ocn_any_tile), as fp32, a bf16 source widened.
+constexpr int kOcnBf16 = 0, kOcnWhole = 1, kOcnParts = 2, kOcnPart = 3;
+
+// Two values rounded to bf16 (to nearest even), x in the low half.
+__device__ __forceinline__ unsigned ocn_bf16_pair(float x, float y) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{x, y}), bf16x2));
+}
+
+// ROWS x BK tile of one operand: global -> registers -> LDS, 256 threads.  WIN: see OcnAnyDesc (1: this is A, 2: B).
+// Planes of parts have no padding: the 16-byte pieces of a line change places so that the lanes of a fragment read meet
+// all banks (k-contiguous: by row, so that 16 rows do; else by k-line, so that the four k-lines of a transposing read do).
 //
 // A regular operand (see ocn_any_regular) is fetched without a branch, so that the loads of several steps stay in
 // flight and each is waited for by count: rows past the end are clamped to the last one (their results are
 // never stored), a chunk that runs past the end of its row or of K starts early and is shifted into place on the
 // way to LDS, k past the end and positions outside a window are zeroed there.  Irregular operands (a run of
 // memory that is not whole chunks) are gathered element by element, clamped and zeroed the same way.
-template <int ROWS, bool KC, bool F32, int WIN>
+template <int ROWS, bool KC, int MODE, int WIN, int BKE>
 struct OcnAnyStage {
-  static constexpr int V = F32 ? 4 : 8, BK = F32 ? 32 : 64;
+  static constexpr bool F32 = MODE == kOcnWhole || MODE == kOcnParts;   // registers hold fp32
+  static constexpr bool PLANES = MODE == kOcnParts || MODE == kOcnPart;
+  static constexpr int V = MODE == kOcnBf16 ? 8 : 4, BK = BKE;
   static constexpr int PER = KC ? BK / V : ROWS / V;             // chunks per contiguous line
   static constexpr int CH = ROWS * BK / V / 256;                 // chunks per thread
   static constexpr int LINES = 256 / PER;                        // lines one pass of the workgroup covers
-  static constexpr int PAD = F32 ? (KC ? 4 : 8) : (KC ? 8 : 32);
+  static constexpr int PAD = PLANES ? 0 : F32 ? (KC ? 4 : 8) : (KC ? 8 : 32);
   static constexpr int STRIDE = (KC ? BK : ROWS) + PAD;          // LDS elements per line
-  static constexpr int ELEMS = (KC ? ROWS : BK) * STRIDE;
-  using Elem = typename ocn_if<F32, float, unsigned short>::type;
+  static constexpr int PLANE = (KC ? ROWS : BK) * STRIDE, ELEMS = (MODE == kOcnParts ? 3 : 1) * PLANE;
+  using Elem = typename ocn_if<MODE == kOcnWhole, float, unsigned short>::type;
+  static constexpr int RP = KC ? 128 / BK : 1, PPR = KC ? BK / 8 : 1;   // planes: rows per 256 bytes, pieces per row
+  static_assert(!PLANES || LINES % (KC ? RP * PPR : 4) == 0, "one place for all chunks of a thread");
   union Chunk { ocn_u32x4 u; ocn_f32x4 f; unsigned short h[8]; float s[4]; };
   // what one step fetches; mask: chunks that count; an fp32 tile of a bf16 source is widened on the way to LDS (touching
   // the values any earlier would wait for them), unless it was gathered
@@ -105,8 +126,10 @@ struct OcnAnyStage {
   int off[KC ? CH : 1];       // KC: row offset of each chunk; else the offset of this thread's rows (chunk start)
   int u0[WIN == 1 ? CH : 1], u1[WIN == 1 ? CH : 1];
   int shift;                  // !KC: elements by which the chunk starts early (0 .. V)
+  unsigned tiny;              // parts: least 2 |bits| - 1 stored so far (zero: the largest unsigned)
 
   __device__ __forceinline__ void init(const OcnAnyOperand& o, const OcnDigits& dr, int row0, int rows, int tid) {
+    tiny = ~0u;
     if constexpr (KC) {
       shift = 0;
 #pragma unroll
@@ -127,8 +150,8 @@ struct OcnAnyStage {
     return bf ? __uint_as_float((unsigned)static_cast<const unsigned short*>(p)[i] << 16) : static_cast<const float*>(p)[i];
   }
   static __device__ __forceinline__ void whole(Chunk& c, const void* p, bool bf, long i) {
-    if constexpr (!F32) __builtin_memcpy(&c.u, static_cast<const unsigned short*>(p) + i, 16);
-    else if (bf) { ocn_u32x2 t; __builtin_memcpy(&t, static_cast<const unsigned short*>(p) + i, 8); c.u = ocn_u32x4{t.x, t.y, 0, 0}; }
+    if constexpr (MODE == kOcnBf16) __builtin_memcpy(&c.u, static_cast<const unsigned short*>(p) + i, 16);
+    else if (MODE == kOcnPart || bf) { ocn_u32x2 t; __builtin_memcpy(&t, static_cast<const unsigned short*>(p) + i, 8); c.u = ocn_u32x4{t.x, t.y, 0, 0}; }
     else __builtin_memcpy(&c.f, static_cast<const float*>(p) + i, 16);
   }
   static __device__ __forceinline__ void widen(Chunk& c) {
@@ -236,9 +259,15 @@ struct OcnAnyStage {
     return c;
   }
 
+  // where a thread's first chunk goes in a plane
+  static __device__ __forceinline__ int place(int tid) {
+    const int line = tid / PER, c = tid % PER;
+    const int turn = KC ? (line / RP) & (PPR - 1) : ROWS >= 128 ? (line & 3) << 2 : ROWS == 64 ? (line >> 1 & 1) << 2 : 0;
+    return line * STRIDE + ((c >> 1) ^ turn) * 8 + (c & 1) * 4;
+  }
   // `edge`: rows of the tile run past the end; TAIL: so may k
   template <bool TAIL, bool WIDEN>
-  __device__ __forceinline__ void store(const Set& s, Elem* lds, int tid, bool edge) const {
+  __device__ __forceinline__ void store(const Set& s, Elem* lds, int tid, bool edge) {
 #pragma unroll
     for (int j = 0; j < CH; ++j) {
       Chunk c = s.c[j];
@@ -246,9 +275,46 @@ struct OcnAnyStage {
       if constexpr (!KC) { if (edge) c = shifted(c, shift); }
       if constexpr (KC && TAIL) c = shifted(c, s.down);
       if constexpr (WIN != 0 || TAIL) { if (!(s.mask >> j & 1u)) c.u = ocn_u32x4{0, 0, 0, 0}; }
-      *reinterpret_cast<ocn_u32x4*>(lds + (tid / PER + j * LINES) * STRIDE + (tid % PER) * V) = c.u;
+      if constexpr (!PLANES) *reinterpret_cast<ocn_u32x4*>(lds + (tid / PER + j * LINES) * STRIDE + (tid % PER) * V) = c.u;
+      else {
+        Elem* const to = lds + place(tid) + j * LINES * STRIDE;
+        put<0>(c, to);
+        if constexpr (MODE == kOcnParts) { put<1>(c, to); put<2>(c, to); }
+      }
     }
   }
+  // part P of a chunk to its plane; what is left of the values stays in the chunk
+  template <int P>
+  __device__ __forceinline__ void put(Chunk& c, Elem* to) {
+    if constexpr (MODE == kOcnPart) *reinterpret_cast<ocn_u32x2*>(to) = ocn_u32x2{c.u.x, c.u.y};
+    else {
+      ocn_f32x4& r = c.f;
+      if constexpr (P == 0) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) { const unsigned t = (__float_as_uint(r[q]) << 1) - 1u; tiny = t < tiny ? t : tiny; }
+      }
+      const unsigned x = ocn_bf16_pair(r.x, r.y), y = ocn_bf16_pair(r.z, r.w);
+      *reinterpret_cast<ocn_u32x2*>(to + P * PLANE) = ocn_u32x2{x, y};
+      if constexpr (P < 2) r = ocn_f32x4{r.x - __uint_as_float(x << 16), r.y - __uint_as_float(x & 0xFFFF0000u), r.z - __uint_as_float(y << 16), r.w - __uint_as_float(y & 0xFFFF0000u)};
+    }
+  }
+  // the store of a whole step in pieces, to go between matrix instructions: ready() first, then units 0 .. UNITS - 1
+  static constexpr int UNITS = CH * (MODE == kOcnParts ? 3 : 1);
+  __device__ __forceinline__ void ready(Set& s, bool edge) const {
+    if constexpr (!KC) {
+      if (edge) {
+#pragma unroll
+        for (int j = 0; j < CH; ++j) s.c[j] = shifted(s.c[j], shift);
+      }
+    }
+  }
+  template <int U>
+  __device__ __forceinline__ void unit(Set& s, Elem* lds, int tid) {
+    constexpr int J = U / (UNITS / CH), P = U % (UNITS / CH);
+    if constexpr (WIN != 0 && P == 0) { if (!(s.mask >> J & 1u)) s.c[J].u = ocn_u32x4{0, 0, 0, 0}; }
+    put<P>(s.c[J], lds + place(tid) + J * LINES * STRIDE);
+  }
+  static __device__ __forceinline__ ocn_bf16x8 part(const Elem* plane, int row, int kk, int lane);
 };
 
 // Whole chunks only: along k (KC) or along the rows, memory runs in multiples of a chunk.
@@ -268,11 +334,38 @@ __device__ __forceinline__ ocn_bf16x8 ocn_any_tr(const unsigned short* at_lane, 
   return __builtin_bit_cast(ocn_bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
-template <int BM, int BN, bool A_KC, bool B_KC, bool F32>
-constexpr int ocn_any_smem() {
-  return 2 * (OcnAnyStage<BM, A_KC, F32, 0>::ELEMS + OcnAnyStage<BN, B_KC, F32, 0>::ELEMS) * (F32 ? 4 : 2);
+// fragment (32 rows from `row`, 16 k from kk * 16) out of a plane
+template <int ROWS, bool KC, int MODE, int WIN, int BKE>
+__device__ __forceinline__ ocn_bf16x8 OcnAnyStage<ROWS, KC, MODE, WIN, BKE>::part(const Elem* plane, int row, int kk, int lane) {
+  if constexpr (KC) return *reinterpret_cast<const ocn_bf16x8*>(plane + (row + (lane & 31)) * STRIDE + ((kk * 2 + (lane >> 5)) ^ (((lane & 31) / RP) & (PPR - 1))) * 8);
+  else {
+    const int p = lane & 15, turn = ROWS >= 128 ? (p >> 2) * 32 : ROWS == 64 ? (p >> 3) * 32 : 0;
+    return ocn_any_tr(plane + (kk * 16 + (lane >> 5) * 8 + (p >> 2)) * STRIDE + ((row + ((lane >> 4) & 1) * 16 + (p & 3) * 4) ^ turn), STRIDE);
+  }
 }
 
+template <bool ABF, bool BBF, bool PARTS> struct OcnAnyModes {
+  static constexpr int A = ABF && BBF ? kOcnBf16 : !PARTS ? kOcnWhole : ABF ? kOcnPart : kOcnParts;
+  static constexpr int B = ABF && BBF ? kOcnBf16 : !PARTS ? kOcnWhole : BBF ? kOcnPart : kOcnParts;
+};
+// k of a step: parts of 128 x 128 tiles take half as much, so that two workgroups share a compute unit's LDS
+template <int BM, int BN, bool ABF, bool BBF, bool PARTS>
+constexpr int ocn_any_bk() { return ABF && BBF ? 64 : PARTS && BM == 128 && BN == 128 ? 16 : 32; }
+template <int BM, int BN, bool A_KC, bool B_KC, bool ABF, bool BBF, bool PARTS>
+constexpr int ocn_any_smem() {
+  constexpr int BK = ocn_any_bk<BM, BN, ABF, BBF, PARTS>();
+  using M = OcnAnyModes<ABF, BBF, PARTS>;
+  using SA = OcnAnyStage<BM, A_KC, M::A, 0, BK>;
+  using SB = OcnAnyStage<BN, B_KC, M::B, 0, BK>;
+  return 2 * (int)sizeof(typename SA::Elem) * (SA::ELEMS + SB::ELEMS);
+}
+
+template <int I> struct OcnAnyInt { static constexpr int value = I; };
+// f(0), f(1), ..  f(N - 1) with compile-time numbers
+template <int N, int I = 0, typename F>
+__device__ __forceinline__ void ocn_any_each(F&& f) {
+  if constexpr (I < N) { f(OcnAnyInt<I>{}); ocn_any_each<N, I + 1>(f); }
+}
 struct OcnAnyNo { static constexpr bool value = false; };
 struct OcnAnyYes { static constexpr bool value = true; };
 
@@ -295,16 +388,25 @@ struct OcnAnyEpilogue {
 // columns, 1 x 4 for tiles of 32 rows).  a, b, c, c2: operands at the batch entry; ws: with splits, where partial
 // sums of this entry go ([split][M][N] fp32).  c2: a bf16 tensor of C's layout that receives the rounded fp32
 // result, or null.  PF: steps of K in flight in registers ahead of the one being multiplied.
-template <int BM, int BN, bool A_KC, bool B_KC, bool ABF, bool BBF, bool WIN, int PF>
+//
+// PARTS: an fp32 operand is multiplied as the sum of three bf16 values, which it is exactly, on the bf16 matrix cores: six of the
+// nine products of two such operands (the others are below 2^-24 of the whole), all three with a bf16 operand.  Tiles
+// with values below 2^-102, whose third part may be no normal bf16, or with results that are not finite (an infinity
+// has no remainder) are multiplied again with fp32 instructions.
+template <int BM, int BN, bool A_KC, bool B_KC, bool ABF, bool BBF, bool WIN, int PF, bool PARTS>
 __device__ __forceinline__ void ocn_any_tile(const OcnAnyDesc& d, const void* a, const void* b, void* c, void* c2, float* ws, const OcnAnyEpilogue& ep,
                                              int tm, int tn, int split, int r0, int r1, unsigned char* smem) {
   constexpr bool F32 = !(ABF && BBF);
-  using SA = OcnAnyStage<BM, A_KC, F32, WIN ? 1 : 0>;
-  using SB = OcnAnyStage<BN, B_KC, F32, WIN ? 2 : 0>;
+  constexpr int BK = ocn_any_bk<BM, BN, ABF, BBF, PARTS>();
+  using SA = OcnAnyStage<BM, A_KC, OcnAnyModes<ABF, BBF, PARTS>::A, WIN ? 1 : 0, BK>;
+  using SB = OcnAnyStage<BN, B_KC, OcnAnyModes<ABF, BBF, PARTS>::B, WIN ? 2 : 0, BK>;
+  using WA = OcnAnyStage<BM, A_KC, kOcnWhole, WIN ? 1 : 0, 32>;
+  using WB = OcnAnyStage<BN, B_KC, kOcnWhole, WIN ? 2 : 0, 32>;
   using Elem = typename SA::Elem;
-  constexpr int BK = SA::BK, GN = BN == 32 ? 1 : BM == 32 ? 4 : 2, GM = 4 / GN, WM = BM / GM, WN = BN / GN, TM = WM / 32, TN = WN / 32;
+  constexpr int GN = BN == 32 ? 1 : BM == 32 ? 4 : 2, GM = 4 / GN, WM = BM / GM, WN = BN / GN, TM = WM / 32, TN = WN / 32;
   Elem* const as = reinterpret_cast<Elem*>(smem);
-  Elem* const bs = as + 2 * SA::ELEMS;
+  Elem* const bs = as + SA::ELEMS;
+  constexpr int STAGE = SA::ELEMS + SB::ELEMS;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = (wave / GN) * WM, wn = (wave % GN) * WN, m0 = tm * BM, n0 = tn * BN;
   const int steps = (d.K + BK - 1) / BK, per = (steps + d.splits - 1) / d.splits;
@@ -348,9 +450,38 @@ __device__ __forceinline__ void ocn_any_tile(const OcnAnyDesc& d, const void* a,
   using Yes = OcnAnyYes;
   using No = OcnAnyNo;
   const int p16 = lane & 15;
-  auto multiply = [&](int cur) __attribute__((always_inline)) {
-    const Elem* const ap = as + cur * SA::ELEMS;
-    const Elem* const bp = bs + cur * SB::ELEMS;
+  // a step of fp32 operands
+  auto whole = [&](const float* fa, const float* fb) __attribute__((always_inline)) {
+    // v_mfma_f32_32x32x2_f32: instruction q of four multiplies k = q (lanes 0-31) and k = 4 + q (lanes 32-63)
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+      ocn_f32x4 af[TM], bf[TN];
+      const int k = kk * 8 + (lane >> 5) * 4;
+#pragma unroll
+      for (int i = 0; i < TM; ++i) {
+        const int row = wm + i * 32 + (lane & 31);
+        if constexpr (A_KC) af[i] = *reinterpret_cast<const ocn_f32x4*>(fa + row * WA::STRIDE + k);
+        else { const float* q = fa + k * WA::STRIDE + row; af[i] = ocn_f32x4{q[0], q[WA::STRIDE], q[2 * WA::STRIDE], q[3 * WA::STRIDE]}; }
+      }
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const int row = wn + j * 32 + (lane & 31);
+        if constexpr (B_KC) bf[j] = *reinterpret_cast<const ocn_f32x4*>(fb + row * WB::STRIDE + k);
+        else { const float* q = fb + k * WB::STRIDE + row; bf[j] = ocn_f32x4{q[0], q[WB::STRIDE], q[2 * WB::STRIDE], q[3 * WB::STRIDE]}; }
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[i][q], bf[j][q], acc[i][j], 0, 0, 0);
+    }
+  };
+  // The products of a step; `units`: how many pieces of the next step's stores there are, `unit(i)` is piece i.  They go
+  // evenly between the products and are pinned there: a wavefront alone on its SIMD hides nothing else.
+  auto multiply = [&](int cur, auto units, auto unit) __attribute__((always_inline)) {
+    const Elem* const ap = as + cur * STAGE;
+    const Elem* const bp = bs + cur * STAGE;
     // all fragments of the step first: with few waves per SIMD nothing else would hide their latency
     if constexpr (!F32) {
       ocn_bf16x8 af[BK / 16][TM], bf[BK / 16][TN];
@@ -375,40 +506,40 @@ __device__ __forceinline__ void ocn_any_tile(const OcnAnyDesc& d, const void* a,
 #pragma unroll
           for (int j = 0; j < TN; ++j)
             acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[kk][i], bf[kk][j], acc[i][j], 0, 0, 0);
-    } else {
-      // v_mfma_f32_32x32x2_f32: instruction q of four multiplies k = q (lanes 0-31) and k = 4 + q (lanes 32-63)
-      ocn_f32x4 af[BK / 8][TM], bf[BK / 8][TN];
+    } else if constexpr (!PARTS) whole(ap, bp);
+    else {
+      constexpr int NA = SA::ELEMS / SA::PLANE, NB = SB::ELEMS / SB::PLANE;
+      ocn_bf16x8 af[BK / 16][NA][TM], bf[BK / 16][NB][TN];
 #pragma unroll
-      for (int kk = 0; kk < BK / 8; ++kk) {
+      for (int kk = 0; kk < BK / 16; ++kk) {
 #pragma unroll
-        for (int i = 0; i < TM; ++i) {
-          const int row = wm + i * 32 + (lane & 31), k = kk * 8 + (lane >> 5) * 4;
-          if constexpr (A_KC) af[kk][i] = *reinterpret_cast<const ocn_f32x4*>(ap + row * SA::STRIDE + k);
-          else { const Elem* q = ap + k * SA::STRIDE + row; af[kk][i] = ocn_f32x4{q[0], q[SA::STRIDE], q[2 * SA::STRIDE], q[3 * SA::STRIDE]}; }
-        }
+        for (int p = 0; p < NA; ++p)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          const int row = wn + j * 32 + (lane & 31), k = kk * 8 + (lane >> 5) * 4;
-          if constexpr (B_KC) bf[kk][j] = *reinterpret_cast<const ocn_f32x4*>(bp + row * SB::STRIDE + k);
-          else { const Elem* q = bp + k * SB::STRIDE + row; bf[kk][j] = ocn_f32x4{q[0], q[SB::STRIDE], q[2 * SB::STRIDE], q[3 * SB::STRIDE]}; }
-        }
+          for (int i = 0; i < TM; ++i) af[kk][p][i] = SA::part(ap + p * SA::PLANE, wm + i * 32, kk, lane);
+#pragma unroll
+        for (int p = 0; p < NB; ++p)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) bf[kk][p][j] = SB::part(bp + p * SB::PLANE, wn + j * 32, kk, lane);
       }
       __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int kk = 0; kk < BK / 8; ++kk)
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-          for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(af[kk][i][q], bf[kk][j][q], acc[i][j], 0, 0, 0);
+      constexpr int NQ = NA * NB == 9 ? 6 : 3, ALL = BK / 16 * NQ * TM * TN, U = decltype(units)::value;
+      ocn_any_each<ALL>([&](auto mc) __attribute__((always_inline)) {
+        constexpr int m = decltype(mc)::value, kk = m / (NQ * TM * TN), q = m / (TM * TN) % NQ, i = m / TN % TM, j = m % TN;
+        // small products first: parts 0 2, 2 0, 1 1, 0 1, 1 0, 0 0, or 2, 1, 0 of the operand that has three
+        constexpr int pa = NQ == 6 ? (q == 1 ? 2 : q == 2 || q == 4 ? 1 : 0) : NA == 3 ? 2 - q : 0;
+        constexpr int pb = NQ == 6 ? (q == 0 ? 2 : q == 2 || q == 3 ? 1 : 0) : NB == 3 ? 2 - q : 0;
+        ocn_any_each<U>([&](auto uc) __attribute__((always_inline)) { if constexpr (decltype(uc)::value * ALL / U == m) unit(uc); });
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[kk][pa][i], bf[kk][pb][j], acc[i][j], 0, 0, 0);
+        if constexpr (U > 0) __builtin_amdgcn_sched_barrier(0);
+      });
     }
   };
+  using None = OcnAnyInt<0>;
+  auto nothing = [](auto) __attribute__((always_inline)) {};
   auto put = [&](const typename SA::Set& x, const typename SB::Set& y, int buf, auto tail, auto fetched) __attribute__((always_inline)) {
-    constexpr bool T = decltype(tail)::value, R = decltype(fetched)::value && F32;
-    sa.template store<T, R && ABF>(x, as + buf * SA::ELEMS, tid, edge_a);
-    sb.template store<T, R && BBF>(y, bs + buf * SB::ELEMS, tid, edge_b);
+    constexpr bool T = decltype(tail)::value, R = decltype(fetched)::value && F32 && !PARTS;
+    sa.template store<T, R && ABF>(x, as + buf * STAGE, tid, edge_a);
+    sb.template store<T, R && BBF>(y, bs + buf * STAGE, tid, edge_b);
   };
 
   // Regular operands.  At step t its tile is in LDS buffer t & 1 and those of the next PF - 1 steps are on their way
@@ -428,23 +559,45 @@ __device__ __forceinline__ void ocn_any_tile(const OcnAnyDesc& d, const void* a,
     if (n > 0) {
       put(qa[0], qb[0], 0, No{}, Yes{});
       ocn_any_barrier();
-      for (int t = 0; t < n; t += PF) {
+      // (no branch in a turn of the loop: a path on which a set is not stored would make the next one wait for every load)
+      int t = 0;
+      for (; t + PF <= n; t += PF) {
 #pragma unroll
         for (int p = 0; p < PF; ++p) {
-          if (t + p >= n) break;
           fetch(qa[p], qb[p], at(t + p + PF), No{}, single);
-          __builtin_amdgcn_sched_barrier(0);
-          multiply((t + p) & 1);
-          __builtin_amdgcn_sched_barrier(0);
-          if (t + p + 1 < n) put(qa[(p + 1) % PF], qb[(p + 1) % PF], (t + p + 1) & 1, No{}, Yes{});
+          typename SA::Set& na = qa[(p + 1) % PF];
+          typename SB::Set& nb = qb[(p + 1) % PF];
+          const int to = (t + p + 1) & 1;
+          if constexpr (F32 && PARTS) {
+            sa.ready(na, edge_a);
+            sb.ready(nb, edge_b);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply((t + p) & 1, OcnAnyInt<SA::UNITS + SB::UNITS>{}, [&](auto uc) __attribute__((always_inline)) {
+              constexpr int u = decltype(uc)::value;
+              if constexpr (u < SA::UNITS) sa.template unit<u>(na, as + to * STAGE, tid);
+              else sb.template unit<u - SA::UNITS>(nb, bs + to * STAGE, tid);
+            });
+          } else {
+            __builtin_amdgcn_sched_barrier(0);
+            multiply((t + p) & 1, None{}, nothing);
+            __builtin_amdgcn_sched_barrier(0);
+            put(na, nb, to, No{}, Yes{});
+          }
           ocn_any_barrier();
         }
+      }
+#pragma unroll
+      for (int p = 0; p + 1 < PF; ++p) {
+        if (t + p >= n) break;
+        multiply((t + p) & 1, None{}, nothing);
+        if (t + p + 1 < n) put(qa[(p + 1) % PF], qb[(p + 1) % PF], (t + p + 1) & 1, No{}, Yes{});
+        ocn_any_barrier();
       }
     }
     if (n < ksteps) {
       put(ta, tb, n & 1, Yes{}, Yes{});
       ocn_any_barrier();
-      multiply(n & 1);
+      multiply(n & 1, None{}, nothing);
     }
   };
   if (none) {
@@ -456,9 +609,54 @@ __device__ __forceinline__ void ocn_any_tile(const OcnAnyDesc& d, const void* a,
     ocn_any_barrier();
     for (int t = 0; t < ksteps; ++t) {
       if (t + 1 < ksteps) gather(qa[0], qb[0], t + 1);
-      multiply(t & 1);
+      multiply(t & 1, None{}, nothing);
       if (t + 1 < ksteps) put(qa[0], qb[0], (t + 1) & 1, No{}, No{});
       ocn_any_barrier();
+    }
+  }
+
+  if constexpr (F32 && PARTS) {
+    float nan = 0.0f;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) nan = __builtin_fmaf(acc[i][j][e], 0.0f, nan);
+    constexpr unsigned kTiny = 25u << 24;   // of 2^-102
+    if (__syncthreads_or(nan != nan || sa.tiny < kTiny || sb.tiny < kTiny)) {
+      WA wa; WB wb;
+      wa.init(d.a, d.dm, m0, d.M, tid);
+      wb.init(d.b, d.dn, n0, d.N, tid);
+      if (!(ra && rb)) wa.shift = wb.shift = 0;
+      float* const fa = reinterpret_cast<float*>(smem);
+      float* const fb = fa + WA::ELEMS;
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+#pragma unroll 1
+      for (int k0 = kbeg; k0 < kend; k0 += 32) {
+        typename WA::Set xa;
+        typename WB::Set xb;
+        if (ra && rb) {
+          wa.template fetch<ABF, true, false>(xa, d, d.a, a, k0, kend, tid, r0, r1);
+          wb.template fetch<BBF, true, false>(xb, d, d.b, b, k0, kend, tid, r0, r1);
+          ocn_any_barrier();
+          wa.template store<true, ABF>(xa, fa, tid, edge_a);
+          wb.template store<true, BBF>(xb, fb, tid, edge_b);
+        } else {
+          wa.template gather<ABF>(xa, d, d.a, d.dm, a, m0, d.M, k0, kend, tid, r0, r1);
+          wb.template gather<BBF>(xb, d, d.b, d.dn, b, n0, d.N, k0, kend, tid, r0, r1);
+          ocn_any_barrier();
+          wa.template store<true, false>(xa, fa, tid, edge_a);
+          wb.template store<true, false>(xb, fb, tid, edge_b);
+        }
+        ocn_any_barrier();
+        whole(fa, fb);
+      }
     }
   }
 

@@ -63,11 +63,11 @@ long any_entries(const GemmDesc& d) {
 // through 4096 x 4096, four splits: 13.6 us).
 AnyShape any_shape(const GemmDesc& d) {
   const long nb = any_entries(d);
-  AnyShape s{64, 64, 1};
-  if (d.N <= 32 && !any_mixed(d)) s = {128, 32, 1};
-  else if (d.M <= 32 && !any_mixed(d)) s = {32, 128, 1};
-  else if (any_mixed(d)) s = {64, 64, 1};   // (the one tile built for a bf16 and an fp32 operand)
-  else if (d.M > 64 && d.N > 64 && ((d.M + 127) / 128) * ((d.N + 127) / 128) * nb >= 512) s = {128, 128, 1};
+  AnyShape s{64, 64, 1, any_is_f32(d) && d.K >= kPartsFrom};
+  if (any_mixed(d)) {}   // (the one tile built for a bf16 and an fp32 operand)
+  else if (d.N <= 32) { s.bm = 128; s.bn = 32; }
+  else if (d.M <= 32) { s.bm = 32; s.bn = 128; }
+  else if (d.M > 64 && d.N > 64 && ((d.M + 127) / 128) * ((d.N + 127) / 128) * nb >= 512) s.bm = s.bn = 128;
   const long tiles = ((d.M + s.bm - 1) / s.bm) * ((d.N + s.bn - 1) / s.bn) * nb;
   if (tiles < 192 && d.epi_bias < 0 && d.epi_relu < 0) while ((long)s.splits * 2 * tiles <= 512 && d.K / (s.splits * 2) >= (any_is_f32(d) ? 384 : 768)) s.splits *= 2;
   return s;
@@ -102,10 +102,9 @@ const char* contract_any_name(const GemmDesc& d) {
   static thread_local char buf[96];
   const AnyShape s = any_shape(d);
   const char* tf[2] = {"false", "true"};
-  if (!any_is_f32(d)) snprintf(buf, sizeof buf, "gemm_bf16_kernel_any<%d, %d, %s, %s>", s.bm, s.bn, tf[any_kc(d.a)], tf[any_kc(d.b)]);
-  else
-    snprintf(buf, sizeof buf, "gemm_f32_kernel_any<%d, %d, %s, %s, %s, %s>", s.bm, s.bn, tf[any_kc(d.a)], tf[any_kc(d.b)], tf[d.a.prec == Prec::Bfloat16],
-             tf[d.b.prec == Prec::Bfloat16]);
+  const char *ak = tf[any_kc(d.a)], *bk = tf[any_kc(d.b)], *ab = tf[d.a.prec == Prec::Bfloat16], *bb = tf[d.b.prec == Prec::Bfloat16];
+  if (!any_is_f32(d)) snprintf(buf, sizeof buf, "gemm_bf16_kernel_any<%d, %d, %s, %s>", s.bm, s.bn, ak, bk);
+  else snprintf(buf, sizeof buf, "gemm_f32_kernel_any<%d, %d, %s, %s, %s, %s, %s>", s.bm, s.bn, ak, bk, ab, bb, tf[s.parts]);
   return buf;
 }
 
@@ -145,11 +144,11 @@ hipError_t launch_contract_any(const GemmDesc& g, const GemmArgs& in, void* work
   if (tiles <= 0 || tiles > 0x3FFFFFFFL || entries > 65535 || in.npairs != 1 || (sh.splits > 1 && !p.ws)) return hipErrorInvalidValue;
   const dim3 grid((unsigned)((tiles + 7) / 8 * 8), (unsigned)sh.splits, 1);
   const bool akc = any_kc(g.a), bkc = any_kc(g.b), f32 = any_is_f32(g);
-  hipError_t e = f32 ? launch_any_f32(sh.bm, sh.bn, d.a.bf16, d.b.bf16, akc, bkc, grid, d, &q, &p, s)
-                 : sh.bn == 32 ? launch_layout<128, 32, true, true>(akc, bkc, grid, d, q, p, s)
-                 : sh.bm == 32 ? launch_layout<32, 128, true, true>(akc, bkc, grid, d, q, p, s)
-                 : sh.bm == 128 ? launch_layout<128, 128, true, true>(akc, bkc, grid, d, q, p, s)
-                                : launch_layout<64, 64, true, true>(akc, bkc, grid, d, q, p, s);
+  hipError_t e = f32 ? launch_any_f32(sh.bm, sh.bn, sh.parts, d.a.bf16, d.b.bf16, akc, bkc, grid, d, &q, &p, s)
+                 : sh.bn == 32 ? launch_layout<128, 32, true, true, false>(akc, bkc, grid, d, q, p, s)
+                 : sh.bm == 32 ? launch_layout<32, 128, true, true, false>(akc, bkc, grid, d, q, p, s)
+                 : sh.bm == 128 ? launch_layout<128, 128, true, true, false>(akc, bkc, grid, d, q, p, s)
+                                : launch_layout<64, 64, true, true, false>(akc, bkc, grid, d, q, p, s);
   if (e == hipSuccess && after_main) e = hipEventRecord(after_main, s);
   if (e != hipSuccess || sh.splits == 1) return e;
   const long cells = (long)d.M * d.N;

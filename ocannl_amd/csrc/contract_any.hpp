@@ -23,9 +23,8 @@ struct AnyPtrs {
   OcnAnyEpilogue ep;
 };
 
-// K steps in flight ahead (ocn_any_tile): measured with 1, 2, 3 and 4, more than two gained nothing.  A step lasts 0.9 us
-// then (1777 x 771 x 1001 in bf16: 16 steps, 16.4 us; 1.5 us where rows start at odd elements), of which neither L2 (6 TB/s
-// of the 13 it delivers to the direct-to-LDS kernel) nor the matrix cores (5 %) is the bound
+// K steps in flight ahead (ocn_any_tile): three gained nothing (1777 x 771 x 1001 in bf16, forward and both gradients: 56.3
+// us with two, 58.2 with three)
 constexpr int kAnyDepth = 2;
 
 // Batch entry z of the launch -> operands.
@@ -50,7 +49,7 @@ __device__ __forceinline__ void any_operands(const OcnAnyDesc& d, const AnyBatch
 // Grid: x = tiles of all batch entries, padded to a multiple of eight and dealt so that each XCD (workgroup
 // ids go round robin) walks a contiguous range of them -- neighbouring tiles share panels through its L2;
 // y = K splits.
-template <int BM, int BN, bool A_KC, bool B_KC, bool ABF, bool BBF>
+template <int BM, int BN, bool A_KC, bool B_KC, bool ABF, bool BBF, bool PARTS>
 __device__ __forceinline__ void any_body(const OcnAnyDesc& d, const AnyBatch& q, const AnyPtrs& p) {
   extern __shared__ __align__(16) unsigned char smem_any[];
   const int per = gridDim.x / 8, tiles = d.tiles_m * d.tiles_n;
@@ -61,24 +60,24 @@ __device__ __forceinline__ void any_body(const OcnAnyDesc& d, const AnyBatch& q,
   void *c, *c2;
   any_operands(d, q, p, z, a, b, c, c2);
   float* const ws = d.splits > 1 ? p.ws + (long)z * d.splits * d.M * d.N : nullptr;
-  ocn_any_tile<BM, BN, A_KC, B_KC, ABF, BBF, false, kAnyDepth>(d, a, b, c, c2, ws, p.ep, r / d.tiles_n, r % d.tiles_n, (int)blockIdx.y, 0, 0, smem_any);
+  ocn_any_tile<BM, BN, A_KC, B_KC, ABF, BBF, false, kAnyDepth, PARTS>(d, a, b, c, c2, ws, p.ep, r / d.tiles_n, r % d.tiles_n, (int)blockIdx.y, 0, 0, smem_any);
 }
 
 template <int BM, int BN, bool A_KC, bool B_KC>
 __global__ void __launch_bounds__(256) gemm_bf16_kernel_any(const OcnAnyDesc d, const AnyBatch q, const AnyPtrs p) {
-  any_body<BM, BN, A_KC, B_KC, true, true>(d, q, p);
+  any_body<BM, BN, A_KC, B_KC, true, true, false>(d, q, p);
 }
-template <int BM, int BN, bool A_KC, bool B_KC, bool ABF, bool BBF>
+template <int BM, int BN, bool A_KC, bool B_KC, bool ABF, bool BBF, bool PARTS>
 __global__ void __launch_bounds__(256) gemm_f32_kernel_any(const OcnAnyDesc d, const AnyBatch q, const AnyPtrs p) {
-  any_body<BM, BN, A_KC, B_KC, ABF, BBF>(d, q, p);
+  any_body<BM, BN, A_KC, B_KC, ABF, BBF, PARTS>(d, q, p);
 }
 
-template <int BM, int BN, bool A_KC, bool B_KC, bool ABF, bool BBF>
+template <int BM, int BN, bool A_KC, bool B_KC, bool ABF, bool BBF, bool PARTS>
 hipError_t go(dim3 grid, const OcnAnyDesc& d, const AnyBatch& q, const AnyPtrs& p, hipStream_t s) {
-  constexpr int smem = ocn_any_smem<BM, BN, A_KC, B_KC, !(ABF && BBF)>();
+  constexpr int smem = ocn_any_smem<BM, BN, A_KC, B_KC, ABF, BBF, PARTS>();
   void (*kernel)(OcnAnyDesc, AnyBatch, AnyPtrs);
   if constexpr (ABF && BBF) kernel = gemm_bf16_kernel_any<BM, BN, A_KC, B_KC>;
-  else kernel = gemm_f32_kernel_any<BM, BN, A_KC, B_KC, ABF, BBF>;
+  else kernel = gemm_f32_kernel_any<BM, BN, A_KC, B_KC, ABF, BBF, PARTS>;
   if (smem > 65536) {
     static thread_local bool configured = false;
     if (!configured) {
@@ -91,20 +90,19 @@ hipError_t go(dim3 grid, const OcnAnyDesc& d, const AnyBatch& q, const AnyPtrs& 
   return hipGetLastError();
 }
 
-template <int BM, int BN, bool ABF, bool BBF>
+template <int BM, int BN, bool ABF, bool BBF, bool PARTS>
 hipError_t launch_layout(bool akc, bool bkc, dim3 grid, const OcnAnyDesc& d, const AnyBatch& q, const AnyPtrs& p, hipStream_t s) {
-  if (akc && bkc) return go<BM, BN, true, true, ABF, BBF>(grid, d, q, p, s);
-  if (akc) return go<BM, BN, true, false, ABF, BBF>(grid, d, q, p, s);
-  if (bkc) return go<BM, BN, false, true, ABF, BBF>(grid, d, q, p, s);
-  return go<BM, BN, false, false, ABF, BBF>(grid, d, q, p, s);
+  if (akc && bkc) return go<BM, BN, true, true, ABF, BBF, PARTS>(grid, d, q, p, s);
+  if (akc) return go<BM, BN, true, false, ABF, BBF, PARTS>(grid, d, q, p, s);
+  if (bkc) return go<BM, BN, false, true, ABF, BBF, PARTS>(grid, d, q, p, s);
+  return go<BM, BN, false, false, ABF, BBF, PARTS>(grid, d, q, p, s);
 }
 
-struct AnyShape { int bm, bn, splits; };
+struct AnyShape { int bm, bn, splits; bool parts; };
 
 }  // namespace
 
 // contract_any_f32.hip
-hipError_t launch_any_f32(int bm, int bn, bool a_bf16, bool b_bf16, bool akc, bool bkc, dim3 grid, const OcnAnyDesc& d, const void* q, const void* p,
+hipError_t launch_any_f32(int bm, int bn, bool parts, bool a_bf16, bool b_bf16, bool akc, bool bkc, dim3 grid, const OcnAnyDesc& d, const void* q, const void* p,
                           hipStream_t s);
-
 }  // namespace ocannl

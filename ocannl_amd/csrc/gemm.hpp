@@ -64,6 +64,11 @@ const char* gemm_kernel_name(const GemmDesc& desc);
 // bytes of workspace that keep the routine's scratch within what ocannl_hip_routine_run_static_scratch has.
 bool gemm_prefers_any(const GemmDesc& desc, uint64_t room);
 
+// Least K at which an fp32 operand of a contraction of any shape is multiplied in bf16 parts: below, what parts save is less
+// than what they cost, a vote on whether to multiply again (260 x 132 x 16 4.4 us as fp32, 5.2 in parts; 1023 x 1023 x 198
+// 9.4, 9.5).
+constexpr int64_t kPartsFrom = 129;
+
 // contract_any.hip: the same for contractions with `desc.any` set (launch_gemm and its siblings forward to these).
 // Do the extents and the element offsets within one batch entry fit the 32-bit arithmetic of contract_any.h?
 bool contract_any_fits(const GemmDesc& desc);

@@ -68,6 +68,22 @@ template <typename V> static V host_transposed(const void* at) {
 template <typename C> static C host_mfma_f32(float a, float b, C c) { return host_mfma(&a, &b, 1, c); }
 #define __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, x, y, z) host_mfma_f32(a, b, c)
 #define __builtin_amdgcn_ds_read_tr16_b64_v4i16(p) host_transposed<s16x4>((const void*)(p))
+// fp32 -> bf16 bits, to nearest even
+static inline unsigned short host_bf16(float x) {
+  const unsigned u = __float_as_uint(x);
+  return (unsigned short)(x != x ? u >> 16 | 0x40 : (u + 0x7FFF + (u >> 16 & 1)) >> 16);
+}
+template <typename T, typename V> static T host_bf16_pair(V v) { T t; t[0] = host_bf16(v[0]); t[1] = host_bf16(v[1]); return t; }
+#define __builtin_convertvector(v, T) host_bf16_pair<T>(v)
+static int host_votes[2][256];
+static int __syncthreads_or(int x) {
+  const int t = host_turn, s = host_step[t]++ & 1;
+  host_votes[s][t] = x;
+  host_yield();
+  int any = 0;
+  for (int i = 0; i < 256; ++i) any |= host_votes[s][i];
+  return any;
+}
 #define __builtin_amdgcn_readfirstlane(x) (x)
 #define __builtin_amdgcn_fence(...) ((void)0)
 #define __builtin_amdgcn_sched_barrier(x) ((void)0)

@@ -209,3 +209,43 @@ def test_bias_and_relu_of_every_batch_entry(shape, one_statement):
         # (the product is rounded, and its sum with the bias again: 2^-9 of either, of at most the largest)
         assert np.max(np.abs(W.to_float(got, "bfloat16") - ref)) <= 2.0 ** -7 * np.max(np.abs(want))
     folded.close(); apart.close()
+
+
+def _forms(kernels):
+    return [k["name"].split("<")[0] for k in kernels if k["kind"] == "mfma"]
+
+
+@pytest.mark.parametrize("layout", [(True, True), (False, False), (True, False)])
+@pytest.mark.parametrize("precs", [("single", "single"), ("single", "bfloat16"), ("bfloat16", "single")])
+@pytest.mark.parametrize("M,N,K", [(70, 66, 131), (1031, 1099, 150), (30, 9000, 150), (2049, 4099, 135)])
+@pytest.mark.parametrize("what", ["tiny", "special"])
+def test_values_that_three_bf16_parts_do_not_cover(M, N, K, precs, layout, what):
+    """Values below 2^-102, infinities, NaN and values above the largest bf16 give what fp32 products give."""
+    if (M > 2000 and precs != ("single", "single")) or (M == 30 and "bfloat16" in precs):
+        pytest.skip("tiles of fp32 operands only")
+    r, A, B, C = _routine(M, N, K, *precs, "single", *layout, False)
+    rng = np.random.default_rng(4)
+    a, b = rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((N, K)).astype(np.float32)
+    if what == "tiny":
+        x, y = (a, b) if precs[0] == "single" else (b, a)
+        x[: len(x) // 2] *= np.float32(2.0 ** -118)
+        y *= np.float32(2.0 ** 30)
+        y[:, K // 2:] = 1.0                      # (whose mid and lo parts are zero)
+    else:
+        b[:, :4] = 1.0
+        a[3, 1], a[M - 1, 0], a[M // 2, 2], b[N - 2, K - 1] = np.inf, -np.inf, np.nan, np.float32(3.3e38)
+        a[:, K - 1] = rng.choice(np.float32([0.5, 0.25]), M)
+    a, b = (W.to_float(W.as_prec(x, p), p) for x, p in ((a, precs[0]), (b, precs[1])))
+    t = lambda x, kc, p: W.as_prec(np.ascontiguousarray(x if kc else x.T), p)
+    hip = HipRun(r, {1: t(a, layout[0], precs[0]), 2: t(b, layout[1], precs[1])}, "min_mfma_flops=1;bf16_copies=0")
+    assert all("_kernel_any" in f for f in _forms(hip.code.kernels())), hip.code.kernels()
+    hip.step()
+    got = hip.get(C).astype(np.float64)
+    hip.close()
+    with np.errstate(all="ignore"):
+        want = a.astype(np.float64) @ b.astype(np.float64).T
+        size = np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64).T
+    fine = np.isfinite(want)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[~fine & ~np.isnan(want)], want[~fine & ~np.isnan(want)])
+    # K roundings of fp32, each of half a unit of a partial sum that is no larger than `size`
+    assert (np.abs(got[fine] - want[fine]) / size[fine]).max() <= K * 2.0 ** -24
