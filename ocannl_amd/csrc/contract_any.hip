@@ -50,10 +50,49 @@ bool any_mixed(const GemmDesc& d) { return d.a.prec != d.b.prec; }
 // k-contiguous (or contiguous along nothing), else row-contiguous
 bool any_kc(const GemmOperand& o) { return o.k_stride[2] == 1 || o.row_stride[2] != 1; }
 
+// Whole chunks of memory along k or along the rows, as DirectOperand takes them.
+bool any_regular(const GemmDesc& d) {
+  auto operand = [&](const GemmOperand& o, int64_t rows, const int64_t (&ext)[3], int digits) {
+    if (any_kc(o)) return o.k_stride[2] == 1 && (d.k_digits == 1 || d.k_ext[2] % (o.prec == Prec::Bfloat16 ? 8 : 4) == 0);
+    return o.row_stride[2] == 1 && rows >= 2 && (digits == 1 || ext[2] % 2 == 0);
+  };
+  return operand(d.a, d.M, d.m_ext, d.m_digits) && operand(d.b, d.N, d.n_ext, d.n_digits);
+}
+
 long any_entries(const GemmDesc& d) {
   long nb = 1 + (long)d.group.size();
   for (int i = 0; i < d.nbatch; ++i) nb *= d.batch_ext[i];
   return nb;
+}
+
+// Do 32 x 32 tiles whose wavefronts share K and read their operands straight from memory (contract_direct.hip) take it, and
+// in how many splits?  They read twice the operands per product that 64 x 64 tiles do and cost 5 us + 6.5 ns a k in fp32
+// (4.2 + 3 in bf16) where a compute unit has one of them, against 6 + 16 (4.5 + 5): so up to one tile a unit, and up to
+// two in fp32 where an operand is row-contiguous.  594 x 320, start -> now, both row-contiguous: K = 320 fp32 11.8 -> 7.4
+// us, bf16 6.1 -> 5.6; K = 1001 20.1 -> 11.2 and 10.6 -> 7.1; 594 x 640 x 1001 (380 tiles) fp32 21.3 -> 16.4, bf16 10.6 ->
+// 9.6 but x 320 6.2 -> 6.9.  Two k-contiguous bf16 operands touch 32 rows with every load and lose from K = 320 on (5.4 ->
+// 5.7); rows at odd elements, which the vector memory path takes apart, at once (K = 1001 9.5 -> 12.9).  Short sums are all
+// start (K = 27 fp32 4.4 -> 4.8) and beyond 4096 the traffic tells (594 x 320 x 4096 bf16, k-contiguous 13.7 -> 17.9).
+// Members of a grouped launch that are few enough by themselves for four of them to fit are taken however many there are:
+// grouped or apart, they are then summed in the same order.  A split has to give back the launch that sums the splits.
+int direct_splits(const GemmDesc& d) {
+  const long t32 = ((d.M + 31) / 32) * ((d.N + 31) / 32) * any_entries(d);
+  const bool f32 = any_is_f32(d), both_kc = any_kc(d.a) && any_kc(d.b);
+  const long members = 1 + (long)d.group.size();
+  if (d.K <= 64 || d.K > 4096 || !any_regular(d)) return 0;
+  if (t32 > (f32 && !both_kc ? 512 : 256) && t32 / members > (f32 ? 128 : 64)) return 0;
+  if (!f32 && both_kc && d.K > 256) return 0;
+  auto odd = [&](const GemmOperand& o) {
+    int64_t all = o.offset;
+    for (auto& t : o.static_terms) all |= t.second;
+    for (int i = 0; i < d.nbatch; ++i) all |= o.s_batch[i];
+    for (int i = 0; i < 3; ++i) all |= o.row_stride[i];
+    return o.prec == Prec::Bfloat16 && any_kc(o) && (all & 1);
+  };
+  if (odd(d.a) || odd(d.b)) return 0;
+  int splits = 1;
+  if (d.epi_bias < 0 && d.epi_relu < 0) while (splits * 2 * t32 <= 512 && d.K / (splits * 2) >= (f32 ? 768 : 1536)) splits *= 2;
+  return splits;
 }
 
 // 128 x 128 tiles when they fill the chip twice over, else 64 x 64 (128 x 32 or 32 x 128 when one extent is at most
@@ -61,9 +100,9 @@ long any_entries(const GemmDesc& d) {
 // are fewer than one each and a split keeps a dozen K steps: fewer do not give back the launch that sums the splits, 4 to
 // 5 us (17 such launches in a bf16 transformer block of odd extents at 128 of K a split: 569 us, 551 without them; 64 rows
 // through 4096 x 4096, four splits: 13.6 us).
-AnyShape any_shape(const GemmDesc& d) {
+AnyShape staged_shape(const GemmDesc& d) {
   const long nb = any_entries(d);
-  AnyShape s{64, 64, 1, any_is_f32(d) && d.K >= kPartsFrom};
+  AnyShape s{64, 64, 1, any_is_f32(d) && d.K >= kPartsFrom, false};
   if (any_mixed(d)) {}   // (the one tile built for a bf16 and an fp32 operand)
   else if (d.N <= 32) { s.bm = 128; s.bn = 32; }
   else if (d.M <= 32) { s.bm = 32; s.bn = 128; }
@@ -71,6 +110,11 @@ AnyShape any_shape(const GemmDesc& d) {
   const long tiles = ((d.M + s.bm - 1) / s.bm) * ((d.N + s.bn - 1) / s.bn) * nb;
   if (tiles < 192 && d.epi_bias < 0 && d.epi_relu < 0) while ((long)s.splits * 2 * tiles <= 512 && d.K / (s.splits * 2) >= (any_is_f32(d) ? 384 : 768)) s.splits *= 2;
   return s;
+}
+
+AnyShape any_shape(const GemmDesc& d) {
+  if (const int splits = direct_splits(d)) return {32, 32, splits, false, true};
+  return staged_shape(d);
 }
 
 }  // namespace
@@ -91,8 +135,10 @@ bool contract_any_fits(const GemmDesc& d) {
          reach(d.m_ext, d.c.row_stride, d.M, d.c.s_row) + reach(d.n_ext, d.c.k_stride, d.N, d.c.s_k) <= kLimit;
 }
 
+bool contract_any_direct(const GemmDesc& d) { return direct_splits(d) > 0; }
+
 int64_t contract_any_area(const GemmDesc& d, bool& alone) {
-  const AnyShape s = any_shape(d);
+  const AnyShape s = staged_shape(d);
   const int64_t groups = (int64_t)((d.M + s.bm - 1) / s.bm) * ((d.N + s.bn - 1) / s.bn) * any_entries(d) * s.splits;
   alone = groups <= 256;
   return (groups + 255) / 256 * s.bm * s.bn / s.splits;
@@ -103,7 +149,8 @@ const char* contract_any_name(const GemmDesc& d) {
   const AnyShape s = any_shape(d);
   const char* tf[2] = {"false", "true"};
   const char *ak = tf[any_kc(d.a)], *bk = tf[any_kc(d.b)], *ab = tf[d.a.prec == Prec::Bfloat16], *bb = tf[d.b.prec == Prec::Bfloat16];
-  if (!any_is_f32(d)) snprintf(buf, sizeof buf, "gemm_bf16_kernel_any<%d, %d, %s, %s>", s.bm, s.bn, ak, bk);
+  if (s.direct) snprintf(buf, sizeof buf, "gemm_%s_kernel_any_direct<%s, %s, %s, %s>", any_is_f32(d) ? "f32" : "bf16", ak, bk, ab, bb);
+  else if (!any_is_f32(d)) snprintf(buf, sizeof buf, "gemm_bf16_kernel_any<%d, %d, %s, %s>", s.bm, s.bn, ak, bk);
   else snprintf(buf, sizeof buf, "gemm_f32_kernel_any<%d, %d, %s, %s, %s, %s, %s>", s.bm, s.bn, ak, bk, ab, bb, tf[s.parts]);
   return buf;
 }
@@ -144,7 +191,8 @@ hipError_t launch_contract_any(const GemmDesc& g, const GemmArgs& in, void* work
   if (tiles <= 0 || tiles > 0x3FFFFFFFL || entries > 65535 || in.npairs != 1 || (sh.splits > 1 && !p.ws)) return hipErrorInvalidValue;
   const dim3 grid((unsigned)((tiles + 7) / 8 * 8), (unsigned)sh.splits, 1);
   const bool akc = any_kc(g.a), bkc = any_kc(g.b), f32 = any_is_f32(g);
-  hipError_t e = f32 ? launch_any_f32(sh.bm, sh.bn, sh.parts, d.a.bf16, d.b.bf16, akc, bkc, grid, d, &q, &p, s)
+  hipError_t e = sh.direct ? launch_direct(akc, bkc, grid, d, &q, &p, s)
+                 : f32 ? launch_any_f32(sh.bm, sh.bn, sh.parts, d.a.bf16, d.b.bf16, akc, bkc, grid, d, &q, &p, s)
                  : sh.bn == 32 ? launch_layout<128, 32, true, true, false>(akc, bkc, grid, d, q, p, s)
                  : sh.bm == 32 ? launch_layout<32, 128, true, true, false>(akc, bkc, grid, d, q, p, s)
                  : sh.bm == 128 ? launch_layout<128, 128, true, true, false>(akc, bkc, grid, d, q, p, s)

@@ -98,11 +98,14 @@ hipError_t launch_layout(bool akc, bool bkc, dim3 grid, const OcnAnyDesc& d, con
   return go<BM, BN, false, false, ABF, BBF, PARTS>(grid, d, q, p, s);
 }
 
-struct AnyShape { int bm, bn, splits; bool parts; };
+struct AnyShape { int bm, bn, splits; bool parts, direct; };
 
 }  // namespace
 
 // contract_any_f32.hip
 hipError_t launch_any_f32(int bm, int bn, bool parts, bool a_bf16, bool b_bf16, bool akc, bool bkc, dim3 grid, const OcnAnyDesc& d, const void* q, const void* p,
                           hipStream_t s);
+// contract_direct.hip: 32 x 32 tiles of regular operands
+hipError_t launch_direct(bool akc, bool bkc, dim3 grid, const OcnAnyDesc& d, const void* q, const void* p, hipStream_t s);
+
 }  // namespace ocannl

@@ -376,6 +376,14 @@ bool dtl_operands_ok(const GemmArgs& a, bool akc, bool bkc) {
 
 }  // namespace
 
+void as_any_shape(GemmDesc& g) {
+  auto digits = [](GemmOperand& o) { o.row_stride[2] = o.s_row; o.k_stride[2] = o.s_k; };
+  digits(g.a); digits(g.b); digits(g.c);
+  for (auto& m : g.group) { digits(m.a); digits(m.b); digits(m.c); }
+  g.m_ext[2] = g.M; g.n_ext[2] = g.N; g.k_ext[2] = g.K;
+  g.any = true;
+}
+
 // Fewer 128 x 128 tiles than compute units: the register-staged kernels leave some idle and hide no latency on the
 // rest, where 64 x 64 tiles of contract_any.hip put several workgroups on each; but they split K further, and the
 // smaller tile reads twice the operands per product.  Compared is what a compute unit goes through, area of C by k, a
@@ -387,12 +395,16 @@ bool dtl_operands_ok(const GemmArgs& a, bool akc, bool bkc) {
 // 18 against 12; 2048 fp32 52 against 59, bf16 21 against 20; 8192 fp32 157 against 225, bf16 44 against 66.  From 256
 // tiles on the larger tile wins (8000 x 1000 x 1000 bf16, both gradients too: 122 against 173 us).
 // A workspace that would take the routine beyond the static scratch array, where the small tile's does not, is no choice.
+// Few enough tiles for contract_direct.hip: that, whatever the layout (512 x 512 x 1024 in fp32 12 us, 30 on 64 x 64 tiles).
 bool gemm_prefers_any(const GemmDesc& d, uint64_t room) {
   if (d.any || !d.more.empty() || d.a.prec != d.b.prec || !contract_any_fits(d)) return false;
   const int64_t t128 = (int64_t)((d.M + 127) / 128) * ((d.N + 127) / 128) * batch_count(d);
   if (t128 >= 256) return false;
   const bool f32 = d.a.prec == Prec::Single;
   if (!f32 && dtl_shape(d).bm != 0) return false;
+  GemmDesc few = d;
+  as_any_shape(few);
+  if (contract_any_direct(few) && contract_any_workspace_bytes(few) <= room) return true;
   if (gemm_workspace_bytes(d) > room && contract_any_workspace_bytes(d) <= room) return true;
   const TileConfig c = tile_config(d);
   const int64_t staged = (t128 * c.splits + 255) / 256 * 128 * (c.narrow ? 64 : 128) / c.splits;

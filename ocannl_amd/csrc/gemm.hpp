@@ -63,6 +63,8 @@ const char* gemm_kernel_name(const GemmDesc& desc);
 // Is this contraction, which the kernels of gemm.hip could take, faster as one of any shape (contract_any.hip)?  `room`:
 // bytes of workspace that keep the routine's scratch within what ocannl_hip_routine_run_static_scratch has.
 bool gemm_prefers_any(const GemmDesc& desc, uint64_t room);
+// Makes it one of any shape: extents and strides as digits.
+void as_any_shape(GemmDesc& desc);
 
 // Least K at which an fp32 operand of a contraction of any shape is multiplied in bf16 parts: below, what parts save is less
 // than what they cost, a vote on whether to multiply again (260 x 132 x 16 4.4 us as fp32, 5.2 in parts; 1023 x 1023 x 198
@@ -72,9 +74,11 @@ constexpr int64_t kPartsFrom = 129;
 // contract_any.hip: the same for contractions with `desc.any` set (launch_gemm and its siblings forward to these).
 // Do the extents and the element offsets within one batch entry fit the 32-bit arithmetic of contract_any.h?
 bool contract_any_fits(const GemmDesc& desc);
-// Elements of C, padding included, that a compute unit works on per k with the workgroups dealt out evenly and K split as
+// Elements of C, padding included, that a compute unit works on per k in staged tiles, with the workgroups dealt out evenly and K split as
 // it would be; `alone`: no unit gets a second workgroup.
 int64_t contract_any_area(const GemmDesc& desc, bool& alone);
+// Is it few enough tiles for contract_direct.hip?
+bool contract_any_direct(const GemmDesc& desc);
 hipError_t launch_contract_any(const GemmDesc& desc, const GemmArgs& args, void* workspace, hipStream_t stream, hipEvent_t after_main);
 size_t contract_any_workspace_bytes(const GemmDesc& desc);
 const char* contract_any_name(const GemmDesc& desc);

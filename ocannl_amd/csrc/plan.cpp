@@ -2559,12 +2559,7 @@ Plan make_plan(Routine& r, const PlanOptions& requested) {
     const uint64_t room = local <= limit ? limit - local : ~0ull;
     for (auto& ph : plan.phases) {
       if (ph.kind != Phase::Contraction || !gemm_prefers_any(ph.gemm, room)) continue;
-      GemmDesc& g = ph.gemm;
-      auto digits = [](GemmOperand& o) { o.row_stride[2] = o.s_row; o.k_stride[2] = o.s_k; };
-      digits(g.a); digits(g.b); digits(g.c);
-      for (auto& m : g.group) { digits(m.a); digits(m.b); digits(m.c); }
-      g.m_ext[2] = g.M; g.n_ext[2] = g.N; g.k_ext[2] = g.K;
-      g.any = true;
+      as_any_shape(ph.gemm);
     }
   }
   if (opt.enable_serial_group) serialise_tiny(r, plan);

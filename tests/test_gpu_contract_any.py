@@ -215,6 +215,14 @@ def _forms(kernels):
     return [k["name"].split("<")[0] for k in kernels if k["kind"] == "mfma"]
 
 
+@pytest.mark.parametrize("layout", [(True, True), (False, False), (True, False), (False, True)])
+@pytest.mark.parametrize("precs", [("bfloat16", "bfloat16", "single"), ("single", "single", "single"), ("single", "bfloat16", "single"), ("bfloat16", "single", "single")])
+@pytest.mark.parametrize("M,N,K,batch", [(40, 30, 66, 0), (33, 18, 97, 5), (16, 8, 127, 0), (70, 66, 200, 7), (34, 130, 3100, 0)])
+def test_few_tiles_share_k_among_wavefronts(M, N, K, batch, precs, layout):
+    # one step of K for some wavefronts and none for others, a partial step, rows past the end, batch entries, K splits
+    _product(M, N, K, *precs, *layout, accumulate=K % 2 == 0, batch=batch, seed=K)
+
+
 @pytest.mark.parametrize("layout", [(True, True), (False, False), (True, False)])
 @pytest.mark.parametrize("precs", [("single", "single"), ("single", "bfloat16"), ("bfloat16", "single")])
 @pytest.mark.parametrize("M,N,K", [(70, 66, 131), (1031, 1099, 150), (30, 9000, 150), (2049, 4099, 135)])
