@@ -240,13 +240,6 @@ __device__ __forceinline__ void store_tile_row(f32x16 (&acc)[TN], void* origin, 
   unsigned short* const base2 = static_cast<unsigned short*>(origin2);
   const unsigned col = lane & 31, rb = (lane >> 5) * 4;
   const unsigned loff = rb * (unsigned)ld + col;
-  // Pin the tiles to accumulation registers up to this point: without it the register allocator
-  // may move all accumulators of the block into ordinary registers right after the main loop and
-  // spill most of them.
-  static_assert(TN == 1 || TN == 2 || TN == 4, "tile rows of 1, 2 or 4 tiles");
-  if constexpr (TN == 1) asm volatile("" : "+a"(acc[0]));
-  else asm volatile("" : "+a"(acc[0]), "+a"(acc[1]));
-  if constexpr (TN == 4) asm volatile("" : "+a"(acc[2]), "+a"(acc[3]));
   float old[ACC ? TN : 1][16];
   if (ACC) {
     static_for<TN>([&](auto jc) OCN_LAMBDA_INLINE {
@@ -295,10 +288,6 @@ __device__ __forceinline__ void store_tile_row_wide(f32x16 (&acc)[TN], float* st
                                                     void* origin2 = nullptr, const unsigned short* bias = nullptr,
                                                     unsigned short* relu_out = nullptr, bool relu_c = false) {
   constexpr int CW = TN * 32, LS = CW + 4;
-  static_assert(TN == 1 || TN == 2 || TN == 4, "tile rows of 1, 2 or 4 tiles");
-  if constexpr (TN == 1) asm volatile("" : "+a"(acc[0]));
-  else asm volatile("" : "+a"(acc[0]), "+a"(acc[1]));
-  if constexpr (TN == 4) asm volatile("" : "+a"(acc[2]), "+a"(acc[3]));
   float* const wr = stage + ((lane >> 5) * 4) * LS + (lane & 31);
   static_for<TN>([&](auto jc) OCN_LAMBDA_INLINE {
     static_for<16>([&](auto ec) OCN_LAMBDA_INLINE {
@@ -359,8 +348,9 @@ __device__ __forceinline__ void store_tile_row_wide(f32x16 (&acc)[TN], float* st
 // registers (hoisting all 256 accumulator reads above one up-front branch spills them).
 // `stage`: this wave's own LDS area of at least 32 * (TN * 32 + 4) floats, free once the main loop
 // has passed its last barrier.
-template <int TM, int TN>
-__device__ __forceinline__ void epilogue(const GemmArgs& g, void* cbase, void* c2base, f32x16 (&acc)[TM][TN], long m, long n, long co, int lane,
+// `rows(i, row)`: makes row i of tiles in ordinary registers.
+template <int TM, int TN, typename Rows>
+__device__ __forceinline__ void epilogue(const GemmArgs& g, void* cbase, void* c2base, Rows&& rows, long m, long n, long co, int lane,
                                          float* stage) {
   const long rows_left = g.M - m, cols_left = g.N - n;
   if (rows_left <= 0 || cols_left <= 0) return;
@@ -393,22 +383,40 @@ __device__ __forceinline__ void epilogue(const GemmArgs& g, void* cbase, void* c
     void* o2 = origin2 + (long)i * 32 * ld * 2;
     void* o3 = origin3 ? origin3 + (long)i * 32 * ld * 2 : nullptr;
     const long rl = rows_left - i * 32;
+    f32x16 row[TN];
+    rows(ic, row);
     switch (variant) {
-      case 0: store_tile_row<TN, kOutF32, false, false>(acc[i], o, ld, lane, rl, cols_left); break;
-      case 1: store_tile_row<TN, kOutF32, false, true>(acc[i], o, ld, lane, rl, cols_left); break;
-      case 2: store_tile_row<TN, kOutF32, true, false>(acc[i], o, ld, lane, rl, cols_left); break;
-      case 3: store_tile_row<TN, kOutF32, true, true>(acc[i], o, ld, lane, rl, cols_left); break;
-      case 4: store_tile_row_wide<TN, kOutBf16, false>(acc[i], stage, o, ld, lane, nullptr, bias, reinterpret_cast<unsigned short*>(o3), relu_c); break;
-      case 5: store_tile_row<TN, kOutBf16, false, true>(acc[i], o, ld, lane, rl, cols_left, nullptr, bias, reinterpret_cast<unsigned short*>(o3), relu_c); break;
-      case 6: store_tile_row_wide<TN, kOutBf16, true>(acc[i], stage, o, ld, lane); break;
-      case 7: store_tile_row<TN, kOutBf16, true, true>(acc[i], o, ld, lane, rl, cols_left); break;
-      case 8: store_tile_row_wide<TN, kOutF32Copy, false>(acc[i], stage, o, ld, lane, o2); break;
-      case 9: store_tile_row<TN, kOutF32Copy, false, true>(acc[i], o, ld, lane, rl, cols_left, o2); break;
-      case 10: store_tile_row_wide<TN, kOutF32Copy, true>(acc[i], stage, o, ld, lane, o2); break;
-      default: store_tile_row<TN, kOutF32Copy, true, true>(acc[i], o, ld, lane, rl, cols_left, o2); break;
+      case 0: store_tile_row<TN, kOutF32, false, false>(row, o, ld, lane, rl, cols_left); break;
+      case 1: store_tile_row<TN, kOutF32, false, true>(row, o, ld, lane, rl, cols_left); break;
+      case 2: store_tile_row<TN, kOutF32, true, false>(row, o, ld, lane, rl, cols_left); break;
+      case 3: store_tile_row<TN, kOutF32, true, true>(row, o, ld, lane, rl, cols_left); break;
+      case 4: store_tile_row_wide<TN, kOutBf16, false>(row, stage, o, ld, lane, nullptr, bias, reinterpret_cast<unsigned short*>(o3), relu_c); break;
+      case 5: store_tile_row<TN, kOutBf16, false, true>(row, o, ld, lane, rl, cols_left, nullptr, bias, reinterpret_cast<unsigned short*>(o3), relu_c); break;
+      case 6: store_tile_row_wide<TN, kOutBf16, true>(row, stage, o, ld, lane); break;
+      case 7: store_tile_row<TN, kOutBf16, true, true>(row, o, ld, lane, rl, cols_left); break;
+      case 8: store_tile_row_wide<TN, kOutF32Copy, false>(row, stage, o, ld, lane, o2); break;
+      case 9: store_tile_row<TN, kOutF32Copy, false, true>(row, o, ld, lane, rl, cols_left, o2); break;
+      case 10: store_tile_row_wide<TN, kOutF32Copy, true>(row, stage, o, ld, lane, o2); break;
+      default: store_tile_row<TN, kOutF32Copy, true, true>(row, o, ld, lane, rl, cols_left, o2); break;
     }
     __builtin_amdgcn_sched_barrier(0);
   });
+}
+
+// The epilogue of 32 x 32 tiles.  A row is pinned to accumulation registers until its turn: without that the register
+// allocator may move all accumulators of the block into ordinary registers right after the main loop and spill most.
+template <int TM, int TN>
+__device__ __forceinline__ void epilogue(const GemmArgs& g, void* cbase, void* c2base, f32x16 (&acc)[TM][TN], long m, long n, long co, int lane,
+                                         float* stage) {
+  static_assert(TN == 1 || TN == 2 || TN == 4, "tile rows of 1, 2 or 4 tiles");
+  auto rows = [&](auto ic, f32x16 (&row)[TN]) OCN_LAMBDA_INLINE {
+    f32x16(&from)[TN] = acc[decltype(ic)::value];
+    if constexpr (TN == 1) asm volatile("" : "+a"(from[0]));
+    else asm volatile("" : "+a"(from[0]), "+a"(from[1]));
+    if constexpr (TN == 4) asm volatile("" : "+a"(from[2]), "+a"(from[3]));
+    static_for<TN>([&](auto jc) OCN_LAMBDA_INLINE { row[decltype(jc)::value] = from[decltype(jc)::value]; });
+  };
+  epilogue<TM, TN>(g, cbase, c2base, rows, m, n, co, lane, stage);
 }
 
 // Sums the split-K partials in split order (deterministic) and applies them to C.

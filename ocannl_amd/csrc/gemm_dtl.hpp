@@ -12,13 +12,20 @@
 //     bytes, CPR = chunks per row: the ds_read_b128 of 16 consecutive rows at one k touch 16
 //     different 16-byte bank groups.
 //   row-contiguous operand, tile held [k][row] as it lies in memory, k-line = ROWS * 2 bytes:
-//     chunk c of k-line kl sits at position c ^ ((kl & 3) << 2) (ROWS >= 128) or
-//     c ^ (((kl >> 1) & 1) << 2) (ROWS = 64): the four k-lines that one ds_read_b64_tr_b16 of 32
-//     lanes touches land in four different 64-byte bank groups.
+//     chunk c of k-line kl sits at position c ^ ((kl & 3) << 2) ^ ((kl >> 3 & 1) << 1) (ROWS >= 128) or
+//     c ^ ((kl >> 1 & 1) << 2) ^ ((kl >> 3 & 1) << 1) (ROWS = 64): the eight k-lines (0 .. 3, 8 .. 11) that one
+//     ds_read_b64_tr_b16 of 32 lanes touches, 32 bytes of each, land in eight different 32-byte bank groups.
 // The 1 KB blocks of a tile are dealt to the four waves round robin (block b to wave b % 4), which
 // makes the swizzle term of a lane independent of the block: one 32-bit lane offset per operand.
 //
-// Pipeline (one barrier per K step, placed ahead of the LAST 16-k sub-step of the step): at that
+// v_mfma_f32_16x16x32_bf16: in a loop of matrix instructions alone it sustains 2.08 PFLOP/s where v_mfma_f32_32x32x16_bf16
+// sustains 1.80, from the same bytes of fragments.  Its results are brought
+// into the order of 32 x 32 tiles, in which the epilogue stores them, by one exchange of 16-lane rows per register: of
+// the column halves in lanes, and of the second and third four rows by where the fragments of A start (kPerm).
+// 8192 x 4096 x 4096: 221 -> 207 us (1.33 PFLOP/s), B row-contiguous 216 -> 207, both, 4096 x 4096 x 8192: 202 either way.
+// (Loads issued by the four waves in turn instead of together: 223 -> 229.)
+//
+// Pipeline (one barrier per K step, placed ahead of the LAST 32-k sub-step of the step): at that
 // point every wave has issued all fragment reads of the previous step, so its stage is free: the
 // loads of K step ks + NS - 1 go there, and the first fragments of step ks + 1 (whose stage the
 // wait ahead of the barrier has seen land) are read under the MFMAs of the last sub-step -- the
@@ -70,40 +77,46 @@ struct DtlTile {
 
   // per-lane byte offset into global memory of the chunk this lane fetches in the wave's first block
   // (`ld`: elements between rows / k-lines)
-  static __device__ __forceinline__ unsigned lane_goff(int wave, int lane, long ld) {
+  static __device__ __forceinline__ int turn(int kl) {
+    return (ROWS >= 128 ? (kl & 3) << 2 : (kl >> 1 & 1) << 2) ^ (kl >> 3 & 1) << 1;
+  }
+  // (a 256-row tile's k-lines 8 apart have different places: `odd` loads)
+  static constexpr bool kTwo = !KC && kOpLines == 8;
+  static_assert(KC || kOpLines % 8 == 0, "one or two places for all loads of a lane");
+  static __device__ __forceinline__ unsigned lane_goff(int wave, int lane, long ld, int odd) {
     if constexpr (KC) {
       const int r = kRPB * wave + lane / kCPR;
       const int c = (lane % kCPR) ^ ((r / kRP) & (kCPR - 1));
       return (unsigned)((r * ld + c * 8) * 2);
     } else {
       const int kl = kLPB * wave + lane / kCPL;
-      const int sw = ROWS >= 128 ? (kl & 3) << 2 : ((kl >> 1) & 1) << 2;
-      const int c = (lane % kCPL) ^ sw;
+      const int c = (lane % kCPL) ^ turn(kl + (kTwo ? odd * 8 : 0));
       return (unsigned)((kl * ld + c * 8) * 2);
     }
   }
 
-  // per-lane byte offset of the MFMA fragment of 32-row block 0, sub-step 0, inside the tile; `w0`:
-  // first row of the wave's block of rows
+  // per-lane byte offset of the MFMA fragment of 16-row block 0, sub-step 0, inside the tile; `w0`: first row of the
+  // wave's block of rows; `kPerm`: rows 4 .. 7 and 8 .. 11 of a block change places
+  template <bool kPerm>
   static __device__ __forceinline__ unsigned lane_frag(int lane, int w0) {
+    const int g = lane >> 4;
+    auto place = [](int q) { return kPerm ? (q >> 1 | q << 1) & 3 : q; };
     if constexpr (KC) {
-      const int r = lane & 31;
-      const int sw = (r / kRP) & (kCPR - 1);
-      return (unsigned)((w0 + r) * kRowBytes + (((lane >> 5) ^ sw) * 16));
+      const int r = place(lane >> 2 & 3) * 4 + (lane & 3);
+      return (unsigned)((w0 + r) * kRowBytes + ((g ^ ((r / kRP) & (kCPR - 1))) * 16));
     } else {
-      const int p = lane & 15;
-      const int sw = ROWS >= 128 ? (p >> 2) & 3 : (p >> 3) & 1;
-      return (unsigned)(((lane >> 5) * 8 + (p >> 2)) * kLineBytes + ((w0 * 2 + ((lane >> 4) & 1) * 32 + (p & 3) * 8) ^ (sw * 64)));
+      const int kl = g * 8 + (lane >> 2 & 3);
+      return (unsigned)(kl * kLineBytes + ((w0 * 2 + place(lane & 3) * 8) ^ (turn(kl) * 16)));
     }
   }
 
-  // fragment of 32-row block `blk`, 16-k sub-step `kk`; `tile`: the tile's first byte in LDS
+  // fragment of 16-row block `blk`, 32-k sub-step `kk`; `tile`: the tile's first byte in LDS
   template <int BLK, int KK>
   static __device__ __forceinline__ bf16x8 fragment(const unsigned char* tile, unsigned frag) {
     if constexpr (KC) {
-      return *reinterpret_cast<const bf16x8*>(tile + (frag ^ (unsigned)(KK * 32)) + BLK * 32 * kRowBytes);
+      return *reinterpret_cast<const bf16x8*>(tile + (frag ^ (unsigned)(KK * 64)) + BLK * 16 * kRowBytes);
     } else {
-      return tr_fragment(reinterpret_cast<const unsigned short*>(tile + (frag ^ (unsigned)(BLK * 64)) + KK * 16 * kLineBytes), kLineBytes / 2);
+      return tr_fragment(reinterpret_cast<const unsigned short*>(tile + (frag ^ (unsigned)(BLK * 32)) + KK * 32 * kLineBytes), kLineBytes / 2);
     }
   }
 };
@@ -111,7 +124,9 @@ struct DtlTile {
 template <int BM, int BN, int BK, int NS>
 constexpr size_t dtl_smem() { return (size_t)NS * (BM + BN) * BK * 2; }
 
-template <int BM, int BN, int BK, int NS, bool A_KC, bool B_KC>
+// kOdd: K steps of a split beyond the last NS - 1, modulo two (launch_dtl_layout picks it; a branch here would have the
+// register allocator move all accumulators)
+template <int BM, int BN, int BK, int NS, bool A_KC, bool B_KC, bool kOdd>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, (BM * BN >= 256 * 256) ? 1 : 2)))
 gemm_bf16_dtl_kernel(const GemmArgs g) {
   constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 32, TN = WN / 32;
@@ -119,7 +134,8 @@ gemm_bf16_dtl_kernel(const GemmArgs g) {
   using TB = DtlTile<BN, BK, B_KC>;
   constexpr int kStage = TA::kBytes + TB::kBytes;
   constexpr int kOps = TA::kOps + TB::kOps;
-  constexpr int kSub = BK / 16, kPer = TM * TN, kR = TM + TN;
+  constexpr int IM = WM / 16, JN = WN / 16;                // 16 x 16 blocks of a wave
+  constexpr int kSub = BK / 32, kPer = IM * JN;
   static_assert(NS >= 3, "the barrier ahead of the last sub-step needs three stages");
   static_assert((NS - 2) * kOps < 64, "loads in flight fit the counter");
   extern __shared__ __align__(16) unsigned short smem[];
@@ -152,7 +168,8 @@ gemm_bf16_dtl_kernel(const GemmArgs g) {
   const unsigned short* b_src = uniform_ptr(static_cast<const unsigned short*>(bbase) + bo + (B_KC ? n0 * ldb + sbeg * BK : sbeg * BK * ldb + n0));
   const long a_adv = A_KC ? BK : BK * lda, b_adv = B_KC ? BK : BK * ldb;
   const long a_op = (long)TA::kOpLines * lda, b_op = (long)TB::kOpLines * ldb;   // elements between a wave's loads
-  const unsigned a_goff = TA::lane_goff(wave, lane, lda), b_goff = TB::lane_goff(wave, lane, ldb);
+  const unsigned a_goff[2] = {TA::lane_goff(wave, lane, lda, 0), TA::lane_goff(wave, lane, lda, 1)};
+  const unsigned b_goff[2] = {TB::lane_goff(wave, lane, ldb, 0), TB::lane_goff(wave, lane, ldb, 1)};
   unsigned fetch_lds = lds0 + wave * 1024;   // LDS byte address of this wave's first block in the stage being fetched
   int fetch_stage = 0;
   auto advance_fetch = [&]() OCN_LAMBDA_INLINE {
@@ -163,23 +180,26 @@ gemm_bf16_dtl_kernel(const GemmArgs g) {
   // load number `o` of the stage being fetched (compile-time): A's blocks, then B's
   auto fetch_op = [&](auto oc) OCN_LAMBDA_INLINE {
     constexpr int o = decltype(oc)::value;
-    if constexpr (o < TA::kOps) dtl_load16(a_src + o * a_op, a_goff, fetch_lds + o * 4096);
-    else dtl_load16(b_src + (o - TA::kOps) * b_op, b_goff, fetch_lds + TA::kBytes + (o - TA::kOps) * 4096);
+    if constexpr (o < TA::kOps) dtl_load16(a_src + o * a_op, a_goff[TA::kTwo ? o & 1 : 0], fetch_lds + o * 4096);
+    else dtl_load16(b_src + (o - TA::kOps) * b_op, b_goff[TB::kTwo ? (o - TA::kOps) & 1 : 0], fetch_lds + TA::kBytes + (o - TA::kOps) * 4096);
   };
 
-  const unsigned a_frag = TA::lane_frag(lane, wm0), b_frag = TB::lane_frag(lane, wn0);
-  f32x16 acc[TM][TN];
-  static_for<TM>([&](auto ic) OCN_LAMBDA_INLINE {
-    static_for<TN>([&](auto jc) OCN_LAMBDA_INLINE {
-      static_for<16>([&](auto ec) OCN_LAMBDA_INLINE { acc[decltype(ic)::value][decltype(jc)::value][decltype(ec)::value] = 0.0f; });
-    });
+  const unsigned a_frag = TA::template lane_frag<true>(lane, wm0), b_frag = TB::template lane_frag<false>(lane, wn0);
+  f32x4 acc[IM][JN];
+  static_for<IM>([&](auto ic) OCN_LAMBDA_INLINE {
+    static_for<JN>([&](auto jc) OCN_LAMBDA_INLINE { acc[decltype(ic)::value][decltype(jc)::value] = f32x4{0, 0, 0, 0}; });
   });
-  bf16x8 af[2][TM], bf[2][TN];
-  // fragment number r (A's blocks, then B's) of sub-step kk from the stage starting at `st`
-  auto read_frag = [&](const unsigned char* st, auto kkc, auto rc) OCN_LAMBDA_INLINE {
-    constexpr int kk = decltype(kkc)::value, r = decltype(rc)::value, fb = kk & 1;
-    if constexpr (r < TM) af[fb][r] = TA::template fragment<r, kk>(st, a_frag);
-    else bf[fb][r - TM] = TB::template fragment<r - TM, kk>(st + TA::kBytes, b_frag);
+  // The products of a sub-step go row by row of blocks.  B's fragments serve all rows and have two sets; a fragment of A
+  // is done with after its row, and the next sub-step's takes its place while the row after it is multiplied -- the last
+  // row's during the first row of its own sub-step.
+  bf16x8 af[IM], bf[2][JN];
+  auto read_a = [&](const unsigned char* st, auto kkc, auto rc) OCN_LAMBDA_INLINE {
+    constexpr int kk = decltype(kkc)::value, r = decltype(rc)::value;
+    af[r] = TA::template fragment<r, kk>(st, a_frag);
+  };
+  auto read_b = [&](const unsigned char* st, auto kkc, auto rc, auto fbc) OCN_LAMBDA_INLINE {
+    constexpr int kk = decltype(kkc)::value, r = decltype(rc)::value;
+    bf[decltype(fbc)::value][r] = TB::template fragment<r, kk>(st + TA::kBytes, b_frag);
   };
 
   // The kOps loads of a stage are spread evenly over the kAll MFMAs that follow the barrier that
@@ -199,11 +219,12 @@ gemm_bf16_dtl_kernel(const GemmArgs g) {
   // sub-step, wait until at most kWait loads are in flight (the next stage has landed) and meet the
   // other waves; then, under the MFMAs of the last sub-step, issue the tail part of a further stage
   // (kTail) and read the first fragments of the next stage (kNext), which starts at `nx`.
-  auto step = [&](const unsigned char* st, const unsigned char* nx, auto head_c, auto wait_c, auto tail_c, auto next_c) OCN_LAMBDA_INLINE {
+  auto step = [&](const unsigned char* st, const unsigned char* nx, auto head_c, auto wait_c, auto tail_c, auto next_c, auto par_c) OCN_LAMBDA_INLINE {
     constexpr int kWait = decltype(wait_c)::value;
     constexpr bool kHead = decltype(head_c)::value, kTail = decltype(tail_c)::value, kNext = decltype(next_c)::value;
     static_for<kSub>([&](auto kkc) OCN_LAMBDA_INLINE {
-      constexpr int kk = decltype(kkc)::value, fb = kk & 1;
+      constexpr int kk = decltype(kkc)::value, fb = (kk + decltype(par_c)::value) & 1;
+      using Next = std::integral_constant<int, 1 - fb>;
       constexpr bool last = kk + 1 == kSub;
       if constexpr (last) {
         if constexpr (kHead) advance_fetch();
@@ -215,22 +236,21 @@ gemm_bf16_dtl_kernel(const GemmArgs g) {
         }
       }
       static_for<kPer>([&](auto mc) OCN_LAMBDA_INLINE {
-        constexpr int idx = decltype(mc)::value, i = idx / TN, j = idx % TN;
-        constexpr int r0 = idx * kR / kPer, r1 = (idx + 1) * kR / kPer;
-        if constexpr (!last) {
-          static_for<r1 - r0>([&](auto rc) OCN_LAMBDA_INLINE {
-            read_frag(st, std::integral_constant<int, kk + 1>{}, std::integral_constant<int, r0 + decltype(rc)::value>{});
+        constexpr int idx = decltype(mc)::value, i = idx / JN, j = idx % JN;
+        // the next sub-step lies in this stage or in the next
+        const unsigned char* const from = last ? nx : st;
+        using To = std::integral_constant<int, last ? 0 : kk + 1>;
+        if constexpr (i == 0 && j == 0) read_a(st, kkc, std::integral_constant<int, IM - 1>{});
+        if constexpr (!last || kNext) {
+          if constexpr (i > 0 && j == 0) read_a(from, To{}, std::integral_constant<int, i - 1>{});
+          static_for<JN>([&](auto rc) OCN_LAMBDA_INLINE {
+            if constexpr (decltype(rc)::value * kPer / JN + JN / 2 == idx) read_b(from, To{}, rc, Next{});
           });
-          if constexpr (kHead) fetch_at(std::integral_constant<int, (kk + 1) * kPer + idx>{});
-        } else {
-          if constexpr (kNext) {
-            static_for<r1 - r0>([&](auto rc) OCN_LAMBDA_INLINE {
-              read_frag(nx, std::integral_constant<int, 0>{}, std::integral_constant<int, r0 + decltype(rc)::value>{});
-            });
-          }
-          if constexpr (kTail) fetch_at(std::integral_constant<int, idx>{});
         }
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[fb][i], bf[fb][j], acc[i][j], 0, 0, 0);
+        if constexpr (!last) {
+          if constexpr (kHead) fetch_at(std::integral_constant<int, (kk + 1) * kPer + idx>{});
+        } else if constexpr (kTail) fetch_at(std::integral_constant<int, idx>{});
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], bf[fb][j], acc[i][j], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
       });
     });
@@ -240,9 +260,12 @@ gemm_bf16_dtl_kernel(const GemmArgs g) {
     static_for<kOps>([&](auto oc) OCN_LAMBDA_INLINE { fetch_op(oc); });
     advance_fetch();
   };
-  auto first_frags = [&](const unsigned char* st) OCN_LAMBDA_INLINE {
-    static_for<kR>([&](auto rc) OCN_LAMBDA_INLINE { read_frag(st, std::integral_constant<int, 0>{}, rc); });
+  auto first_frags = [&](const unsigned char* st, auto fbc) OCN_LAMBDA_INLINE {
+    static_for<IM - 1>([&](auto rc) OCN_LAMBDA_INLINE { read_a(st, std::integral_constant<int, 0>{}, rc); });
+    static_for<JN>([&](auto rc) OCN_LAMBDA_INLINE { read_b(st, std::integral_constant<int, 0>{}, rc, fbc); });
   };
+  using P0 = std::integral_constant<int, 0>;
+  using P1 = std::integral_constant<int, 1>;
 
   if (ksteps >= NS - 1) {
     // prologue: stages 0 .. NS - 3, then what the tail of a step does: wait for stage 0, barrier,
@@ -252,15 +275,23 @@ gemm_bf16_dtl_kernel(const GemmArgs g) {
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
     static_for<kPer>([&](auto wc) OCN_LAMBDA_INLINE { fetch_at(wc); });   // tail part of stage NS - 2
-    first_frags(lds);
     int cur = 0;   // stage of the step being multiplied
     auto stage_ptr = [&](int s) OCN_LAMBDA_INLINE { return lds + s * kStage; };
     auto next_of = [&](int s) OCN_LAMBDA_INLINE { return s + 1 == NS ? 0 : s + 1; };
-    int ks = 0;
-    for (; ks + NS - 1 < ksteps; ++ks) {
+    auto turn = [&](auto par_c) OCN_LAMBDA_INLINE {
       const int nxt = next_of(cur);
-      step(stage_ptr(cur), stage_ptr(nxt), Y{}, std::integral_constant<int, (NS - 3) * kOps>{}, Y{}, Y{});
+      step(stage_ptr(cur), stage_ptr(nxt), Y{}, std::integral_constant<int, (NS - 3) * kOps>{}, Y{}, Y{}, par_c);
       cur = nxt;
+    };
+    // steps of an odd number of sub-steps take the fragment sets in turn: they go in pairs, an odd one (kOdd) last
+    int turns = ksteps - (NS - 1);
+    if constexpr (kSub % 2 == 0) {
+      first_frags(lds, P0{});
+      for (; turns > 0; --turns) turn(P0{});
+    } else {
+      first_frags(lds, P0{});
+      for (turns >>= 1; turns > 0; --turns) { turn(P0{}); turn(P1{}); }
+      if constexpr (kOdd) turn(P0{});
     }
     // NS - 1 steps are left: the first completes the last stage's fetch, then nothing more to fetch.
     // With `rem` steps left (this one included), the stages after the next one that are still in
@@ -268,12 +299,13 @@ gemm_bf16_dtl_kernel(const GemmArgs g) {
     static_for<NS - 1>([&](auto tc) OCN_LAMBDA_INLINE {
       constexpr int rem = NS - 1 - decltype(tc)::value;
       using Head = std::integral_constant<bool, rem == NS - 1>;
+      using Par = std::integral_constant<int, (kSub * decltype(tc)::value + (kSub % 2 && kOdd)) & 1>;
       const int nxt = next_of(cur);
       if constexpr (rem > 1) {
         constexpr int fl = (rem - 2) < (NS - 3) ? (rem - 2) : (NS - 3);
-        step(stage_ptr(cur), stage_ptr(nxt), Head{}, std::integral_constant<int, fl * kOps>{}, N{}, Y{});
+        step(stage_ptr(cur), stage_ptr(nxt), Head{}, std::integral_constant<int, fl * kOps>{}, N{}, Y{}, Par{});
       } else {
-        step(stage_ptr(cur), stage_ptr(nxt), Head{}, std::integral_constant<int, -1>{}, N{}, N{});
+        step(stage_ptr(cur), stage_ptr(nxt), Head{}, std::integral_constant<int, -1>{}, N{}, N{}, Par{});
       }
       cur = nxt;
     });
@@ -286,7 +318,23 @@ gemm_bf16_dtl_kernel(const GemmArgs g) {
   __builtin_amdgcn_sched_barrier(0);
   constexpr int kStageFloats = 32 * (TN * 32 + 4);
   static_assert((size_t)4 * kStageFloats * 4 <= dtl_smem<BM, BN, BK, NS>(), "epilogue staging fits the operand stages");
-  epilogue<TM, TN>(g, cbase, c2base, acc, m0 + wm0, n0 + wn0, co, lane, reinterpret_cast<float*>(smem) + wave * kStageFloats);
+  // row i of 32 x 32 tiles out of its 16 x 16 blocks
+  auto tiles = [&](auto ic, f32x16 (&row)[TN]) OCN_LAMBDA_INLINE {
+    constexpr int i = decltype(ic)::value;
+    static_for<2>([&](auto hc) OCN_LAMBDA_INLINE {
+      static_for<TN>([&](auto jc) OCN_LAMBDA_INLINE {
+        constexpr int h = decltype(hc)::value, j = decltype(jc)::value;
+        asm volatile("" : "+a"(acc[2 * i + h][2 * j]), "+a"(acc[2 * i + h][2 * j + 1]));   // (in accumulation registers until here)
+        static_for<4>([&](auto ec) OCN_LAMBDA_INLINE {
+          constexpr int e = decltype(ec)::value;
+          const auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(acc[2 * i + h][2 * j][e]), __float_as_uint(acc[2 * i + h][2 * j + 1][e]), false, false);
+          row[j][8 * h + e] = __uint_as_float(x[0]);
+          row[j][8 * h + 4 + e] = __uint_as_float(x[1]);
+        });
+      });
+    });
+  };
+  epilogue<TM, TN>(g, cbase, c2base, tiles, m0 + wm0, n0 + wn0, co, lane, reinterpret_cast<float*>(smem) + wave * kStageFloats);
 }
 
 }  // namespace
