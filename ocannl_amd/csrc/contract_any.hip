@@ -79,9 +79,10 @@ int direct_splits(const GemmDesc& d) {
   const long t32 = ((d.M + 31) / 32) * ((d.N + 31) / 32) * any_entries(d);
   const bool f32 = any_is_f32(d), both_kc = any_kc(d.a) && any_kc(d.b);
   const long members = 1 + (long)d.group.size();
-  if (d.K <= 64 || d.K > 4096 || !any_regular(d)) return 0;
+  const int64_t all_k = d.K * (int64_t)(1 + d.more.size());
+  if (all_k <= 64 || all_k > 4096 || !any_regular(d)) return 0;
   if (t32 > (f32 && !both_kc ? 512 : 256) && t32 / members > (f32 ? 128 : 64)) return 0;
-  if (!f32 && both_kc && d.K > 256) return 0;
+  if (!f32 && both_kc && all_k > 256) return 0;
   auto odd = [&](const GemmOperand& o) {
     int64_t all = o.offset;
     for (auto& t : o.static_terms) all |= t.second;
@@ -90,6 +91,7 @@ int direct_splits(const GemmDesc& d) {
     return o.prec == Prec::Bfloat16 && any_kc(o) && (all & 1);
   };
   if (odd(d.a) || odd(d.b)) return 0;
+  if (!d.more.empty()) return f32 || d.c.prec != Prec::Single ? 0 : 1;
   int splits = 1;
   if (d.epi_bias < 0 && d.epi_relu < 0) while (splits * 2 * t32 <= 512 && d.K / (splits * 2) >= (f32 ? 768 : 1536)) splits *= 2;
   return splits;
@@ -149,7 +151,8 @@ const char* contract_any_name(const GemmDesc& d) {
   const AnyShape s = any_shape(d);
   const char* tf[2] = {"false", "true"};
   const char *ak = tf[any_kc(d.a)], *bk = tf[any_kc(d.b)], *ab = tf[d.a.prec == Prec::Bfloat16], *bb = tf[d.b.prec == Prec::Bfloat16];
-  if (s.direct) snprintf(buf, sizeof buf, "gemm_%s_kernel_any_direct<%s, %s, %s, %s>", any_is_f32(d) ? "f32" : "bf16", ak, bk, ab, bb);
+  if (s.direct) snprintf(buf, sizeof buf, "gemm_%s_kernel_any_direct<%s, %s, %s, %s, %d, %s>", any_is_f32(d) ? "f32" : "bf16", ak, bk, ab, bb,
+                         any_is_f32(d) || !d.more.empty() ? 2 : 3, tf[!d.more.empty()]);
   else if (!any_is_f32(d)) snprintf(buf, sizeof buf, "gemm_bf16_kernel_any<%d, %d, %s, %s>", s.bm, s.bn, ak, bk);
   else snprintf(buf, sizeof buf, "gemm_f32_kernel_any<%d, %d, %s, %s, %s, %s, %s>", s.bm, s.bn, ak, bk, ab, bb, tf[s.parts]);
   return buf;
@@ -185,10 +188,12 @@ hipError_t launch_contract_any(const GemmDesc& g, const GemmArgs& in, void* work
   AnyPtrs p{};
   p.a[0] = in.a; p.b[0] = in.b; p.c[0] = in.c; p.c2[0] = in.c2;
   for (int i = 1; i < in.ngroups; ++i) { p.a[i] = in.a_more[i - 1]; p.b[i] = in.b_more[i - 1]; p.c[i] = in.c_more[i - 1]; p.c2[i] = in.c2_more[i - 1]; }
+  p.pairs = in.npairs;
+  for (int i = 1; i < in.npairs; ++i) { p.a[i] = in.a_more[i - 1]; p.b[i] = in.b_more[i - 1]; }
   p.ws = static_cast<float*>(workspace);
   p.ep = {static_cast<const unsigned short*>(in.bias), in.relu_out ? static_cast<const char*>(in.relu_out) - static_cast<const char*>(in.c) : 0, in.relu_c};
   const long entries = (long)q.batches * q.members, tiles = (long)d.tiles_m * d.tiles_n * entries;
-  if (tiles <= 0 || tiles > 0x3FFFFFFFL || entries > 65535 || in.npairs != 1 || (sh.splits > 1 && !p.ws)) return hipErrorInvalidValue;
+  if (tiles <= 0 || tiles > 0x3FFFFFFFL || entries > 65535 || in.npairs < 1 || in.npairs > 4 || (in.npairs > 1 && (!sh.direct || in.ngroups > 1)) || (sh.splits > 1 && !p.ws)) return hipErrorInvalidValue;
   const dim3 grid((unsigned)((tiles + 7) / 8 * 8), (unsigned)sh.splits, 1);
   const bool akc = any_kc(g.a), bkc = any_kc(g.b), f32 = any_is_f32(g);
   hipError_t e = sh.direct ? launch_direct(akc, bkc, grid, d, &q, &p, s)

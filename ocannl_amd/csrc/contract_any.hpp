@@ -19,6 +19,7 @@ struct AnyPtrs {
   const void* b[4];
   void* c[4];
   void* c2[4];
+  int pairs;                  // a chain into one C (contract_direct.hip only): operands a[i], b[i] in turn
   float* ws;
   OcnAnyEpilogue ep;
 };

@@ -16,7 +16,8 @@
 // 594 x 320 (190 tiles) by K, tile with LDS stages before -> now: fp32 10.4 + 0.011 us a k -> 5 + 0.0065; bf16 with a
 // row-contiguous operand 4.5 + 0.005 -> 4.2 + 0.003.  A transformer step of 594 rows with 320 to 1280 channels and mixed
 // products 528 -> 475 us.  Tiles of 64 x 64 in this form take 1.5 us more to start and to meet; eight wavefronts instead of
-// four gained nothing (K = 1001 bf16 7.1 -> 7.4 us, fp32 11.2 -> 11.3).
+// four gained nothing (K = 1001 bf16 7.1 -> 7.4 us, fp32 11.2 -> 11.3).  Chains of three products into one C, 594 x 320 x 320 each:
+// 24.9 us on fifteen 128 x 128 tiles, 11.0 here.
 #include <hip/hip_runtime.h>
 
 #include "contract_any.hpp"
@@ -166,10 +167,11 @@ struct DirectOperand {
 constexpr int kDirectTile = 16 * R, kDirectStride = kDirectTile + 4;   // floats of a row of partial sums
 
 // Grid as in any_body (contract_any.hpp).
-template <int W, bool A_KC, bool B_KC, bool ABF, bool BBF>
+// PF: steps in flight; CHAIN: several operand pairs into one C (bf16 operands).
+template <int W, bool A_KC, bool B_KC, bool ABF, bool BBF, int PF, bool CHAIN>
 __device__ __forceinline__ void direct_body(const OcnAnyDesc& d, const AnyBatch& q, const AnyPtrs& p) {
   constexpr bool F32 = !(ABF && BBF);
-  constexpr int BT = kDirectTile, LS = kDirectStride, PF = F32 ? 2 : 3;
+  constexpr int BT = kDirectTile, LS = kDirectStride;
   using OA = DirectOperand<A_KC, ABF>;
   using OB = DirectOperand<B_KC, BBF>;
   extern __shared__ __align__(16) float smem_direct[];
@@ -231,10 +233,11 @@ __device__ __forceinline__ void direct_body(const OcnAnyDesc& d, const AnyBatch&
       }
     }
   };
+  const void *pa = a, *pb = b;
   auto load = [&](typename OA::Set& x, typename OB::Set& y, int step, auto tail, auto single) __attribute__((always_inline)) {
     constexpr bool T = decltype(tail)::value, K1 = decltype(single)::value;
-    oa.template load<T, K1>(x, d, d.a, a, kbeg + step * 32, kend, lane);
-    ob.template load<T, K1>(y, d, d.b, b, kbeg + step * 32, kend, lane);
+    oa.template load<T, K1>(x, d, d.a, pa, kbeg + step * 32, kend, lane);
+    ob.template load<T, K1>(y, d, d.b, pb, kbeg + step * 32, kend, lane);
   };
   using Yes = OcnAnyYes;
   using No = OcnAnyNo;
@@ -308,6 +311,15 @@ __device__ __forceinline__ void direct_body(const OcnAnyDesc& d, const AnyBatch&
   }
   clear();
   if (d.dk.n == 1) sum(Yes{}, No{}); else sum(No{}, No{});
+  if constexpr (CHAIN) {
+    // (at the same offsets in the tensors of every pair)
+#pragma unroll 1
+    for (int pair = 1; pair < p.pairs; ++pair) {
+      pa = static_cast<const char*>(pair == 1 ? p.a[1] : pair == 2 ? p.a[2] : p.a[3]) + (static_cast<const char*>(a) - static_cast<const char*>(p.a[0]));
+      pb = static_cast<const char*>(pair == 1 ? p.b[1] : pair == 2 ? p.b[2] : p.b[3]) + (static_cast<const char*>(b) - static_cast<const char*>(p.b[0]));
+      if (d.dk.n == 1) sum(Yes{}, No{}); else sum(No{}, No{});
+    }
+  }
   reduce();
   if constexpr (F32) {
     float nan = 0.0f;
@@ -349,21 +361,21 @@ __device__ __forceinline__ void direct_body(const OcnAnyDesc& d, const AnyBatch&
   }
 }
 
-template <bool A_KC, bool B_KC, bool ABF, bool BBF>
+template <bool A_KC, bool B_KC, bool ABF, bool BBF, int PF, bool CHAIN>
 __global__ void __launch_bounds__(64 * kDirectWaves) gemm_bf16_kernel_any_direct(const OcnAnyDesc d, const AnyBatch q, const AnyPtrs p) {
-  direct_body<kDirectWaves, A_KC, B_KC, ABF, BBF>(d, q, p);
+  direct_body<kDirectWaves, A_KC, B_KC, ABF, BBF, PF, CHAIN>(d, q, p);
 }
-template <bool A_KC, bool B_KC, bool ABF, bool BBF>
+template <bool A_KC, bool B_KC, bool ABF, bool BBF, int PF, bool CHAIN>
 __global__ void __launch_bounds__(64 * kDirectWaves) gemm_f32_kernel_any_direct(const OcnAnyDesc d, const AnyBatch q, const AnyPtrs p) {
-  direct_body<kDirectWaves, A_KC, B_KC, ABF, BBF>(d, q, p);
+  direct_body<kDirectWaves, A_KC, B_KC, ABF, BBF, PF, CHAIN>(d, q, p);
 }
 
 template <bool A_KC, bool B_KC, bool ABF, bool BBF>
 hipError_t go_direct(dim3 grid, const OcnAnyDesc& d, const AnyBatch& q, const AnyPtrs& p, hipStream_t s) {
   constexpr int smem = kDirectWaves * kDirectTile * kDirectStride * 4;
   void (*kernel)(OcnAnyDesc, AnyBatch, AnyPtrs);
-  if constexpr (ABF && BBF) kernel = gemm_bf16_kernel_any_direct<A_KC, B_KC, ABF, BBF>;
-  else kernel = gemm_f32_kernel_any_direct<A_KC, B_KC, ABF, BBF>;
+  if constexpr (ABF && BBF) kernel = p.pairs > 1 ? gemm_bf16_kernel_any_direct<A_KC, B_KC, ABF, BBF, 2, true> : gemm_bf16_kernel_any_direct<A_KC, B_KC, ABF, BBF, 3, false>;
+  else kernel = gemm_f32_kernel_any_direct<A_KC, B_KC, ABF, BBF, 2, false>;
   hipLaunchKernelGGL(kernel, grid, dim3(64 * kDirectWaves), smem, s, d, q, p);
   return hipGetLastError();
 }

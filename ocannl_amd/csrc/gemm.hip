@@ -380,6 +380,7 @@ void as_any_shape(GemmDesc& g) {
   auto digits = [](GemmOperand& o) { o.row_stride[2] = o.s_row; o.k_stride[2] = o.s_k; };
   digits(g.a); digits(g.b); digits(g.c);
   for (auto& m : g.group) { digits(m.a); digits(m.b); digits(m.c); }
+  for (auto& p : g.more) { digits(p.first); digits(p.second); }
   g.m_ext[2] = g.M; g.n_ext[2] = g.N; g.k_ext[2] = g.K;
   g.any = true;
 }
@@ -395,15 +396,17 @@ void as_any_shape(GemmDesc& g) {
 // 18 against 12; 2048 fp32 52 against 59, bf16 21 against 20; 8192 fp32 157 against 225, bf16 44 against 66.  From 256
 // tiles on the larger tile wins (8000 x 1000 x 1000 bf16, both gradients too: 122 against 173 us).
 // A workspace that would take the routine beyond the static scratch array, where the small tile's does not, is no choice.
-// Few enough tiles for contract_direct.hip: that, whatever the layout (512 x 512 x 1024 in fp32 12 us, 30 on 64 x 64 tiles).
+// Few enough tiles for contract_direct.hip: that, whatever the layout (512 x 512 x 1024 in fp32 12 us, 30 on 64 x 64 tiles),
+// and chains too (three products of 594 x 320 x 320, 15 tiles of 128 x 128: 24.9 -> 11.0 us).
 bool gemm_prefers_any(const GemmDesc& d, uint64_t room) {
-  if (d.any || !d.more.empty() || d.a.prec != d.b.prec || !contract_any_fits(d)) return false;
+  if (d.any || d.a.prec != d.b.prec || !contract_any_fits(d)) return false;
+  GemmDesc few = d;
+  as_any_shape(few);
+  if (!d.more.empty()) return contract_any_direct(few);
   const int64_t t128 = (int64_t)((d.M + 127) / 128) * ((d.N + 127) / 128) * batch_count(d);
   if (t128 >= 256) return false;
   const bool f32 = d.a.prec == Prec::Single;
   if (!f32 && dtl_shape(d).bm != 0) return false;
-  GemmDesc few = d;
-  as_any_shape(few);
   if (contract_any_direct(few) && contract_any_workspace_bytes(few) <= room) return true;
   if (gemm_workspace_bytes(d) > room && contract_any_workspace_bytes(d) <= room) return true;
   const TileConfig c = tile_config(d);

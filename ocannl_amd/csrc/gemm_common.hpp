@@ -348,7 +348,7 @@ __device__ __forceinline__ void store_tile_row_wide(f32x16 (&acc)[TN], float* st
 // registers (hoisting all 256 accumulator reads above one up-front branch spills them).
 // `stage`: this wave's own LDS area of at least 32 * (TN * 32 + 4) floats, free once the main loop
 // has passed its last barrier.
-// `rows(i, row)`: makes row i of tiles in ordinary registers.
+// `rows(i, room)`: row i of tiles, made in `room` where it has to be made.
 template <int TM, int TN, typename Rows>
 __device__ __forceinline__ void epilogue(const GemmArgs& g, void* cbase, void* c2base, Rows&& rows, long m, long n, long co, int lane,
                                          float* stage) {
@@ -383,8 +383,8 @@ __device__ __forceinline__ void epilogue(const GemmArgs& g, void* cbase, void* c
     void* o2 = origin2 + (long)i * 32 * ld * 2;
     void* o3 = origin3 ? origin3 + (long)i * 32 * ld * 2 : nullptr;
     const long rl = rows_left - i * 32;
-    f32x16 row[TN];
-    rows(ic, row);
+    f32x16 room[TN];
+    f32x16(&row)[TN] = rows(ic, room);
     switch (variant) {
       case 0: store_tile_row<TN, kOutF32, false, false>(row, o, ld, lane, rl, cols_left); break;
       case 1: store_tile_row<TN, kOutF32, false, true>(row, o, ld, lane, rl, cols_left); break;
@@ -409,12 +409,12 @@ template <int TM, int TN>
 __device__ __forceinline__ void epilogue(const GemmArgs& g, void* cbase, void* c2base, f32x16 (&acc)[TM][TN], long m, long n, long co, int lane,
                                          float* stage) {
   static_assert(TN == 1 || TN == 2 || TN == 4, "tile rows of 1, 2 or 4 tiles");
-  auto rows = [&](auto ic, f32x16 (&row)[TN]) OCN_LAMBDA_INLINE {
+  auto rows = [&](auto ic, f32x16 (&)[TN]) OCN_LAMBDA_INLINE -> f32x16 (&)[TN] {
     f32x16(&from)[TN] = acc[decltype(ic)::value];
     if constexpr (TN == 1) asm volatile("" : "+a"(from[0]));
     else asm volatile("" : "+a"(from[0]), "+a"(from[1]));
     if constexpr (TN == 4) asm volatile("" : "+a"(from[2]), "+a"(from[3]));
-    static_for<TN>([&](auto jc) OCN_LAMBDA_INLINE { row[decltype(jc)::value] = from[decltype(jc)::value]; });
+    return from;
   };
   epilogue<TM, TN>(g, cbase, c2base, rows, m, n, co, lane, stage);
 }

@@ -319,7 +319,7 @@ gemm_bf16_dtl_kernel(const GemmArgs g) {
   constexpr int kStageFloats = 32 * (TN * 32 + 4);
   static_assert((size_t)4 * kStageFloats * 4 <= dtl_smem<BM, BN, BK, NS>(), "epilogue staging fits the operand stages");
   // row i of 32 x 32 tiles out of its 16 x 16 blocks
-  auto tiles = [&](auto ic, f32x16 (&row)[TN]) OCN_LAMBDA_INLINE {
+  auto tiles = [&](auto ic, f32x16 (&row)[TN]) OCN_LAMBDA_INLINE -> f32x16 (&)[TN] {
     constexpr int i = decltype(ic)::value;
     static_for<2>([&](auto hc) OCN_LAMBDA_INLINE {
       static_for<TN>([&](auto jc) OCN_LAMBDA_INLINE {
@@ -333,6 +333,7 @@ gemm_bf16_dtl_kernel(const GemmArgs g) {
         });
       });
     });
+    return row;
   };
   epilogue<TM, TN>(g, cbase, c2base, tiles, m0 + wm0, n0 + wn0, co, lane, reinterpret_cast<float*>(smem) + wave * kStageFloats);
 }
