@@ -33,6 +33,8 @@ namespace ocannl {
 
 // gemm_dtl.hip: the direct-to-LDS instance of that shape (one of those dtl_shape() names).
 hipError_t launch_gemm_dtl(int bm, int bn, int bk, int ns, bool akc, bool bkc, const GemmArgs& a, hipStream_t s, hipEvent_t ev);
+// gemm_dtl_chain.hip: the same for several operand pairs into one C
+hipError_t launch_gemm_dtl_chain(int bm, int bn, int bk, int ns, bool akc, bool bkc, const GemmArgs& a, hipStream_t s, hipEvent_t ev);
 // gemm_f32.hip: fp32 operands, 256 x 256 (big) or 128 x 128 tiles.
 hipError_t launch_gemm_f32(bool big, bool akc, bool bkc, const GemmArgs& a, hipStream_t s, hipEvent_t ev);
 
@@ -345,20 +347,28 @@ bool b_kcontig(const GemmDesc& d) { return d.b.s_k == 1 || d.K == 1; }
 // workgroups per compute unit, measured 2 % of a transformer step against five stages of 64 k).
 struct DtlShape { int bm = 0, bn = 0, bk = 0, ns = 0; };
 
+// Chains (one pair's K after the other's) from this many workgroups on, the fewest measured; fewer run on contract_direct.hip
+// or the register-staged loop.  Three products, register-staged -> direct to LDS, both k-contiguous (row-contiguous): 1024 x
+// 512 x 512 (32 workgroups) 19.1 -> 14.0 (19.8 -> 15.6) us, 4096 x 512 x 512 20.0 -> 14.8 (20.8 -> 16.4), 8192 x 512 x 512 24.1
+// -> 18.2 (24.6 -> 19.3), 8192 x 1024 x 1024 73 -> 62 (75 -> 51).
+constexpr long kChainWorkgroups = 32;
+
 DtlShape dtl_shape(const GemmDesc& d) {
   DtlShape none, s;
-  if (d.a.prec != Prec::Bfloat16 || d.b.prec != Prec::Bfloat16 || !d.more.empty()) return none;
+  if (d.a.prec != Prec::Bfloat16 || d.b.prec != Prec::Bfloat16) return none;
   const TileConfig c = tile_config(d);
+  const long pairs = 1 + (long)d.more.size();
   if (c.big) s = {256, 256, 32, 4};
   else if (c.narrow) s = {128, 64, 32, 4};
   else {
     const long t128 = ((d.M + 127) / 128) * ((d.N + 127) / 128) * batch_count(d);
+    if (pairs > 1 && t128 * c.splits < kChainWorkgroups) return none;
     if (t128 * c.splits <= 256) s = {128, 128, 64, 5};
     else s = {128, 128, 32, 4};
   }
   if (d.M % s.bm || d.N % s.bn || d.K % s.bk) return none;
   const long steps = d.K / s.bk;
-  if (steps % c.splits || steps / c.splits < s.ns - 1) return none;
+  if (steps % c.splits || steps / c.splits * pairs < s.ns - 1) return none;
   return s;
 }
 
@@ -370,7 +380,7 @@ bool dtl_operands_ok(const GemmArgs& a, bool akc, bool bkc) {
   if (!aligned(a.a) || !aligned(a.b) || lda % 8 || ldb % 8 || lda <= 0 || ldb <= 0 || lda >= (1 << 24) || ldb >= (1 << 24)) return false;
   if ((akc ? a.a_k : a.a_row) != 1 || (bkc ? a.b_k : a.b_row) != 1) return false;
   for (int i = 0; i < a.nbatch; ++i) if (a.a_batch[i] % 8 || a.b_batch[i] % 8) return false;
-  for (int g = 1; g < a.ngroups; ++g) if (!aligned(a.a_more[g - 1]) || !aligned(a.b_more[g - 1])) return false;
+  for (int g = 1; g < a.ngroups || g < a.npairs; ++g) if (!aligned(a.a_more[g - 1]) || !aligned(a.b_more[g - 1])) return false;
   return true;
 }
 
@@ -478,8 +488,8 @@ hipError_t launch_gemm(const GemmDesc& d, const GemmArgs& a_in, void* workspace,
   if (a.npairs > 1 && (af || bf)) return hipErrorInvalidValue;   // chains: bf16 operands only
   if (!af && !bf) {
     const DtlShape ds = dtl_shape(d);
-    if (ds.bm && a.npairs == 1 && dtl_operands_ok(a, akc, bkc)) {
-      return launch_gemm_dtl(ds.bm, ds.bn, ds.bk, ds.ns, akc, bkc, a, s, ev);
+    if (ds.bm && dtl_operands_ok(a, akc, bkc)) {
+      return (a.npairs > 1 ? launch_gemm_dtl_chain : launch_gemm_dtl)(ds.bm, ds.bn, ds.bk, ds.ns, akc, bkc, a, s, ev);
     }
     if (a.npairs > 1) return launch_bf16_layout<128, 128, unsigned short, unsigned short, 2, true>(akc, bkc, a, s, ev);
     if (big) return launch_bf16_layout<256, 256, unsigned short, unsigned short>(akc, bkc, a, s, ev);

@@ -126,7 +126,9 @@ constexpr size_t dtl_smem() { return (size_t)NS * (BM + BN) * BK * 2; }
 
 // kOdd: K steps of a split beyond the last NS - 1, modulo two (launch_dtl_layout picks it; a branch here would have the
 // register allocator move all accumulators)
-template <int BM, int BN, int BK, int NS, bool A_KC, bool B_KC, bool kOdd>
+// kChain: several operand pairs into one C, one pair's K after the other's: the fetch goes on to the next pair's tensors and
+// nothing else of the pipeline knows
+template <int BM, int BN, int BK, int NS, bool A_KC, bool B_KC, bool kOdd, bool kChain>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, (BM * BN >= 256 * 256) ? 1 : 2)))
 gemm_bf16_dtl_kernel(const GemmArgs g) {
   constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 32, TN = WN / 32;
@@ -160,7 +162,7 @@ gemm_bf16_dtl_kernel(const GemmArgs g) {
   const long per_split = (all_steps + g.splits - 1) / g.splits;
   const long sbeg = (long)blockIdx.y * per_split;
   const long send = sbeg + per_split < all_steps ? sbeg + per_split : all_steps;
-  const int ksteps = send > sbeg ? (int)(send - sbeg) : 0;
+  const int pair_steps = send > sbeg ? (int)(send - sbeg) : 0, ksteps = kChain ? pair_steps * g.npairs : pair_steps;
 
   // uniform source of the next stage to fetch (first element of the tile at that K step), advanced per stage
   // (the batch decoding divides in vector registers: the addresses are uniform, say so)
@@ -172,8 +174,20 @@ gemm_bf16_dtl_kernel(const GemmArgs g) {
   const unsigned b_goff[2] = {TB::lane_goff(wave, lane, ldb, 0), TB::lane_goff(wave, lane, ldb, 1)};
   unsigned fetch_lds = lds0 + wave * 1024;   // LDS byte address of this wave's first block in the stage being fetched
   int fetch_stage = 0;
+  // chains (never grouped): the place of a source in its tensor, steps of this pair still to fetch, pairs gone on to
+  const long a_at = kChain ? a_src - static_cast<const unsigned short*>(g.a) : 0, b_at = kChain ? b_src - static_cast<const unsigned short*>(g.b) : 0;
+  int pair_left = pair_steps, pair = 0;
   auto advance_fetch = [&]() OCN_LAMBDA_INLINE {
     a_src += a_adv; b_src += b_adv;
+    if constexpr (kChain) {
+      // (selections and no branch; behind the last pair nothing is fetched)
+      const bool wrap = --pair_left == 0;
+      const unsigned short* const an = static_cast<const unsigned short*>(pair == 0 ? g.a_more[0] : pair == 1 ? g.a_more[1] : g.a_more[2]) + a_at;
+      const unsigned short* const bn = static_cast<const unsigned short*>(pair == 0 ? g.b_more[0] : pair == 1 ? g.b_more[1] : g.b_more[2]) + b_at;
+      a_src = wrap ? an : a_src; b_src = wrap ? bn : b_src;
+      pair_left = wrap ? pair_steps : pair_left;
+      pair += wrap;
+    }
     ++fetch_stage; fetch_lds += kStage;
     if (fetch_stage == NS) { fetch_stage = 0; fetch_lds -= NS * kStage; }
   };
@@ -336,6 +350,23 @@ gemm_bf16_dtl_kernel(const GemmArgs g) {
     return row;
   };
   epilogue<TM, TN>(g, cbase, c2base, tiles, m0 + wm0, n0 + wn0, co, lane, reinterpret_cast<float*>(smem) + wave * kStageFloats);
+}
+
+template <int BM, int BN, int BK, int NS, bool kOdd, bool kChain>
+hipError_t launch_dtl_layout(bool akc, bool bkc, const GemmArgs& a, hipStream_t s, hipEvent_t ev) {
+  constexpr size_t smem = dtl_smem<BM, BN, BK, NS>();
+  if (akc && bkc) return launch(gemm_bf16_dtl_kernel<BM, BN, BK, NS, true, true, kOdd, kChain>, smem, BM, BN, a, s, ev);
+  if (akc && !bkc) return launch(gemm_bf16_dtl_kernel<BM, BN, BK, NS, true, false, kOdd, kChain>, smem, BM, BN, a, s, ev);
+  if (!akc && bkc) return launch(gemm_bf16_dtl_kernel<BM, BN, BK, NS, false, true, kOdd, kChain>, smem, BM, BN, a, s, ev);
+  return launch(gemm_bf16_dtl_kernel<BM, BN, BK, NS, false, false, kOdd, kChain>, smem, BM, BN, a, s, ev);
+}
+template <int BM, int BN, int BK, int NS, bool kChain>
+hipError_t launch_dtl_steps(bool akc, bool bkc, const GemmArgs& a, hipStream_t s, hipEvent_t ev) {
+  // (a split's K is a whole number of steps: dtl_shape)
+  if constexpr (BK == 32) {
+    if ((a.K / BK / a.splits * a.npairs - (NS - 1)) % 2) return launch_dtl_layout<BM, BN, BK, NS, true, kChain>(akc, bkc, a, s, ev);
+  }
+  return launch_dtl_layout<BM, BN, BK, NS, false, kChain>(akc, bkc, a, s, ev);
 }
 
 }  // namespace

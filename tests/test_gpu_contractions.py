@@ -304,6 +304,34 @@ def test_chain_of_products_into_one_result_is_one_launch(shape, layout, accumula
         hip.close()
 
 
+@pytest.mark.parametrize("a_kc,b_kc", [(True, True), (True, False), (False, True), (False, False)])
+@pytest.mark.parametrize("shape,pairs,tile", [
+    ((2048, 1024, 128), 2, "128, 128, 64, 5"),    # the pipeline's own length: no turn of its loop
+    ((2048, 1024, 64), 4, "128, 128, 64, 5"),     # a pair a step
+    ((1024, 512, 192), 3, "128, 128, 64, 5"),     # the fewest workgroups
+    ((1024, 1024, 1024), 3, "128, 128, 64, 5"),   # K split in two, each split through every pair
+    ((2304, 2048, 64), 3, "128, 128, 32, 4"),     # more tiles than compute units, an odd number of steps in the loop
+    ((2304, 2048, 96), 3, "128, 128, 32, 4"),     # and an even one
+])
+def test_chains_of_many_tiles_are_fetched_straight_into_lds(shape, pairs, tile, a_kc, b_kc):
+    M, N, K = shape
+    L.reset_symbols(0)
+    As = [L.Node(1 + p, f"a{p}", "bfloat16", (M, K) if a_kc else (K, M)) for p in range(pairs)]
+    Bs = [L.Node(5 + p, f"b{p}", "bfloat16", (N, K) if b_kc else (K, N)) for p in range(pairs)]
+    C = L.Node(9, "c", "single", (M, N))
+    r = L.Routine("chain", [L.ZeroOut(C)] + [_product_nest(a, b, C, M, N, K, a_kc, b_kc) for a, b in zip(As, Bs)])
+    rng = np.random.default_rng(12)
+    init = {x.id: W.as_prec(rng.standard_normal(x.dims).astype(np.float32), "bfloat16") for x in As + Bs}
+    want = sum(_f64(init[a.id], "bfloat16", a_kc) @ _f64(init[b.id], "bfloat16", b_kc).T for a, b in zip(As, Bs))
+    hip = HipRun(r, init, "min_mfma_flops=1")
+    assert [k["name"] for k in hip.code.kernels()] == [f"gemm_bf16_dtl_kernel<{tile}, {str(a_kc).lower()}, {str(b_kc).lower()}>"]
+    for _ in range(2):
+        hip.step()
+        # (fp32 sums of exact products of bf16 values: half a unit in the last place an addition, as a random walk)
+        assert np.max(np.abs(hip.get(C) - want)) <= 2e-6 * max(1.0, np.sqrt(pairs * K) / 8) * np.max(np.abs(want))
+    hip.close()
+
+
 def test_operand_rewritten_between_two_products_is_not_read_from_a_stale_copy():
     from test_capi_cpu import _stale_copy_routine
     r, n = _stale_copy_routine()
