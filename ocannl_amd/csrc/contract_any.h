@@ -88,11 +88,20 @@ __device__ __forceinline__ int ocn_digit_off(const OcnDigitVal& v, const int (&s
 // not do (see ocn_any_tile), as fp32, a bf16 source widened.
 constexpr int kOcnBf16 = 0, kOcnWhole = 1, kOcnParts = 2, kOcnPart = 3;
 
+// Operands multiplied in parts are taken kOcnScale times as large, a bf16 one beside them too, and the sums kOcnUnscale times: no
+// part of any fp32 value is then a subnormal bf16, next to which the matrix cores keep fewer bits of a product.
+constexpr float kOcnScale = 0x1p23f, kOcnUnscale = 0x1p-46f;
+
 // Two values rounded to bf16 (to nearest even), x in the low half.
 __device__ __forceinline__ unsigned ocn_bf16_pair(float x, float y) {
   typedef float f32x2 __attribute__((ext_vector_type(2)));
   typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
   return __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{x, y}), bf16x2));
+}
+
+// Two bf16 values, kOcnScale times as large (exactly).
+__device__ __forceinline__ unsigned ocn_bf16_scaled(unsigned w) {
+  return ocn_bf16_pair(__uint_as_float(w << 16) * kOcnScale, __uint_as_float(w & 0xFFFF0000u) * kOcnScale);
 }
 
 // ROWS x BK tile of one operand: global -> registers -> LDS, 256 threads.  WIN: see OcnAnyDesc (1: this is A, 2: B).
@@ -126,10 +135,8 @@ struct OcnAnyStage {
   int off[KC ? CH : 1];       // KC: row offset of each chunk; else the offset of this thread's rows (chunk start)
   int u0[WIN == 1 ? CH : 1], u1[WIN == 1 ? CH : 1];
   int shift;                  // !KC: elements by which the chunk starts early (0 .. V)
-  unsigned tiny;              // parts: least 2 |bits| - 1 stored so far (zero: the largest unsigned)
 
   __device__ __forceinline__ void init(const OcnAnyOperand& o, const OcnDigits& dr, int row0, int rows, int tid) {
-    tiny = ~0u;
     if constexpr (KC) {
       shift = 0;
 #pragma unroll
@@ -267,7 +274,7 @@ struct OcnAnyStage {
   }
   // `edge`: rows of the tile run past the end; TAIL: so may k
   template <bool TAIL, bool WIDEN>
-  __device__ __forceinline__ void store(const Set& s, Elem* lds, int tid, bool edge) {
+  __device__ __forceinline__ void store(const Set& s, Elem* lds, int tid, bool edge) const {
 #pragma unroll
     for (int j = 0; j < CH; ++j) {
       Chunk c = s.c[j];
@@ -285,13 +292,13 @@ struct OcnAnyStage {
   }
   // part P of a chunk to its plane; what is left of the values stays in the chunk
   template <int P>
-  __device__ __forceinline__ void put(Chunk& c, Elem* to) {
-    if constexpr (MODE == kOcnPart) *reinterpret_cast<ocn_u32x2*>(to) = ocn_u32x2{c.u.x, c.u.y};
+  static __device__ __forceinline__ void put(Chunk& c, Elem* to) {
+    if constexpr (MODE == kOcnPart) *reinterpret_cast<ocn_u32x2*>(to) = ocn_u32x2{ocn_bf16_scaled(c.u.x), ocn_bf16_scaled(c.u.y)};
     else {
       ocn_f32x4& r = c.f;
       if constexpr (P == 0) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) { const unsigned t = (__float_as_uint(r[q]) << 1) - 1u; tiny = t < tiny ? t : tiny; }
+        for (int q = 0; q < 4; ++q) r[q] *= kOcnScale;
       }
       const unsigned x = ocn_bf16_pair(r.x, r.y), y = ocn_bf16_pair(r.z, r.w);
       *reinterpret_cast<ocn_u32x2*>(to + P * PLANE) = ocn_u32x2{x, y};
@@ -309,7 +316,7 @@ struct OcnAnyStage {
     }
   }
   template <int U>
-  __device__ __forceinline__ void unit(Set& s, Elem* lds, int tid) {
+  __device__ __forceinline__ void unit(Set& s, Elem* lds, int tid) const {
     constexpr int J = U / (UNITS / CH), P = U % (UNITS / CH);
     if constexpr (WIN != 0 && P == 0) { if (!(s.mask >> J & 1u)) s.c[J].u = ocn_u32x4{0, 0, 0, 0}; }
     put<P>(s.c[J], lds + place(tid) + J * LINES * STRIDE);
@@ -391,8 +398,8 @@ struct OcnAnyEpilogue {
 //
 // PARTS: an fp32 operand is multiplied as the sum of three bf16 values, which it is exactly, on the bf16 matrix cores: six of the
 // nine products of two such operands (the others are below 2^-24 of the whole), all three with a bf16 operand.  Tiles
-// with values below 2^-102, whose third part may be no normal bf16, or with results that are not finite (an infinity
-// has no remainder) are multiplied again with fp32 instructions.
+// with results that are not finite (an infinity has no remainder; sums from 2^81 on and values from 2^104 on overflow) are
+// multiplied again with fp32 instructions (1777 x 771 x 1001, one in every tile: 86 us, 35 without, 43 on those instructions alone).
 template <int BM, int BN, bool A_KC, bool B_KC, bool ABF, bool BBF, bool WIN, int PF, bool PARTS>
 __device__ __forceinline__ void ocn_any_tile(const OcnAnyDesc& d, const void* a, const void* b, void* c, void* c2, float* ws, const OcnAnyEpilogue& ep,
                                              int tm, int tn, int split, int r0, int r1, unsigned char* smem) {
@@ -623,8 +630,14 @@ __device__ __forceinline__ void ocn_any_tile(const OcnAnyDesc& d, const void* a,
       for (int j = 0; j < TN; ++j)
 #pragma unroll
         for (int e = 0; e < 16; ++e) nan = __builtin_fmaf(acc[i][j][e], 0.0f, nan);
-    constexpr unsigned kTiny = 25u << 24;   // of 2^-102
-    if (__syncthreads_or(nan != nan || sa.tiny < kTiny || sb.tiny < kTiny)) {
+    if (!__syncthreads_or(nan != nan)) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) acc[i][j][e] *= kOcnUnscale;
+    } else {
       WA wa; WB wb;
       wa.init(d.a, d.dm, m0, d.M, tid);
       wb.init(d.b, d.dn, n0, d.N, tid);

@@ -39,10 +39,8 @@ struct DirectOperand {
   struct Set { unsigned w[KC ? R : 8][kWords]; };
   int off[KC ? R : 1];
   int shift;        // !KC: rows by which the chunk starts early
-  unsigned tiny;    // fp32: least 2 |bits| - 1 so far (zero: the largest unsigned)
 
   __device__ __forceinline__ void init(const OcnAnyOperand& o, const OcnDigits& dr, int row0, int rows, int lane) {
-    tiny = ~0u;
     shift = 0;
     if constexpr (KC) {
 #pragma unroll
@@ -135,22 +133,21 @@ struct DirectOperand {
       return (KC ? j & 1 : b & 1) ? __uint_as_float(x & 0xFFFF0000u) : __uint_as_float(x << 16);
     }
   }
-  // block b as matrix operands: its bf16 values, or the three parts of its fp32 values
-  __device__ __forceinline__ void fragments(const Set& s, int b, bf16x8 (&f)[BF ? 1 : 3]) {
+  // block b as matrix operands: its bf16 values (SCALED: beside an operand in parts), or the three parts of its fp32 values
+  template <bool SCALED>
+  static __device__ __forceinline__ void fragments(const Set& s, int b, bf16x8 (&f)[BF ? 1 : 3]) {
     unsigned u[4];
     if constexpr (BF) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
+      for (int q = 0; q < 4; ++q) {
         u[q] = KC ? s.w[b][q] : __builtin_amdgcn_perm(s.w[2 * q + 1][b / 2], s.w[2 * q][b / 2], b & 1 ? 0x07060302u : 0x05040100u);
+        if constexpr (SCALED) u[q] = ocn_bf16_scaled(u[q]);
+      }
       f[0] = __builtin_bit_cast(bf16x8, u);
     } else {
       float r[8];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        r[j] = value(s, b, j);
-        const unsigned t = (__float_as_uint(r[j]) << 1) - 1u;
-        tiny = t < tiny ? t : tiny;
-      }
+      for (int j = 0; j < 8; ++j) r[j] = value(s, b, j) * kOcnScale;
 #pragma unroll
       for (int p = 0; p < 3; ++p) {
 #pragma unroll
@@ -217,11 +214,11 @@ __device__ __forceinline__ void direct_body(const OcnAnyDesc& d, const AnyBatch&
       constexpr int NA = ABF ? 1 : 3, NB = BBF ? 1 : 3;
       bf16x8 fb[R][NB];
 #pragma unroll
-      for (int j = 0; j < R; ++j) ob.fragments(y, j, fb[j]);
+      for (int j = 0; j < R; ++j) OB::template fragments<F32>(y, j, fb[j]);
 #pragma unroll
       for (int i = 0; i < R; ++i) {
         bf16x8 fa[NA];
-        oa.fragments(x, i, fa);
+        OA::template fragments<F32>(x, i, fa);
 #pragma unroll
         for (int s = NA == 1 && NB == 1 ? 0 : 2; s >= 0; --s)       // small products first
 #pragma unroll
@@ -325,11 +322,13 @@ __device__ __forceinline__ void direct_body(const OcnAnyDesc& d, const AnyBatch&
     float nan = 0.0f;
 #pragma unroll
     for (int x = 0; x < RW / RL; ++x) nan = __builtin_fmaf(v[x], 0.0f, nan);
-    constexpr unsigned kTiny = 25u << 24;   // of 2^-102
-    if (__syncthreads_or(nan != nan || oa.tiny < kTiny || ob.tiny < kTiny)) {
+    if (__syncthreads_or(nan != nan)) {
       clear();
       sum(No{}, Yes{});
       reduce();
+    } else {
+#pragma unroll
+      for (int x = 0; x < RW / RL; ++x) v[x] *= kOcnUnscale;
     }
   }
   if (n >= d.N) return;

@@ -8,15 +8,17 @@
 // 64: 1.1e-7 (1.4e-7), 1024: 4.7e-7 (5.6e-7), 4096: 1.00e-6 (1.18e-6); positive values, K = 4096: 5.3e-7 (8.4e-7);
 // values spread over e^(3 sigma): 7.0e-7 (1.41e-6).
 //
-// What that does not cover is multiplied again with fp32 instructions, tile by tile: values below 2^-102, whose lo
-// part may be no normal bf16 (watched on the way to LDS), and results that are not finite -- an infinity has no
-// remainder, and a value above the largest bf16 rounds to one.
+// Both operands are taken 2^23 times as large and the sums 2^-46 times: no part of any fp32 value, subnormal ones included, is
+// then a subnormal bf16, next to which the matrix cores keep fewer bits of a product.  What that does not cover is
+// multiplied again with fp32 instructions, tile by tile: results that are not finite -- an infinity has no remainder, and
+// sums from 2^81 on and values from 2^104 on overflow.  That pass hides nothing: 4096 x 4096 x 4096 with such a value in
+// every tile 1.62 ms, 0.63 without one, 1.04 where all tiles ran on fp32 instructions.
 //
 // What bounds it: the matrix cores at the clock they sustain: 8192 x 4096 x 4096 in 1.36 ms is 1.21 PFLOP/s of bf16
 // products (an MFMA-only loop: 1.40), 202 TFLOP/s of fp32 ones; with v_mfma_f32_32x32x2_f32, which this replaces, 2.12 ms,
 // 82 % of what that instruction can do.  One operand row-contiguous 1.38 (2.18), both, 4096 x 4096 x 8192: 1.36 (2.16);
 // 2048 x 2048 x 2048 on 128 x 128 tiles 120 us (174).  A step moves 48 KB into LDS and 96 KB of fragments out of it in
-// the 3072 cycles of its products, and splits 32 values a thread in about 180 vector instructions: room enough beside
+// the 3072 cycles of its products, and splits 32 values a thread in about 210 vector instructions: room enough beside
 // the products, so the tile converts its values itself and no pass over the operands does.
 // Four wavefronts of 128 x 128, one to a SIMD; eight of 128 x 64 read more fragments: forward and both gradients of the
 // first product 3.83 ms against 3.75.
@@ -29,7 +31,7 @@ namespace ocannl {
 namespace {
 
 constexpr int kSK = 16;          // k of a step: one matrix instruction per product
-constexpr int kTinyExp = 25;     // biased exponent of 2^-102
+constexpr float kScale = 0x1p23f, kUnscale = 0x1p-46f;
 
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
@@ -49,7 +51,6 @@ struct F32Stage {
   const float* at[KC ? kChunks : 1];   // rows of this thread's chunks, at k = 0
   int k;                               // first chunk's k in step 0
   int put;                             // and its place in a plane
-  unsigned tiny;                       // least 2 |bits| - 1 so far (zero: the largest unsigned)
 
   __device__ __forceinline__ void init(const float* base, long ld, long row0, long rows, int tid) {
     const int line = tid / kPerLine, c = tid % kPerLine;
@@ -67,7 +68,6 @@ struct F32Stage {
       k = line;
       put = line * kStride + ((c >> 1) ^ (line & 3) << 2) * 8 + (c & 1) * 4;
     }
-    tiny = ~0u;
   }
   // chunk j of the step that starts at k0, of K
   template <int J>
@@ -87,7 +87,7 @@ struct F32Stage {
     f32x4& r = regs[J];
     if constexpr (P == 0) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q) { const unsigned t = (__float_as_uint(r[q]) << 1) - 1u; tiny = t < tiny ? t : tiny; }
+      for (int q = 0; q < 4; ++q) r[q] *= kScale;
     }
     const u32x2 p = u32x2{pack2(r.x, r.y), pack2(r.z, r.w)};
     if constexpr (P < 2)
@@ -267,8 +267,9 @@ gemm_f32_kernel(const GemmArgs g) {
       });
     });
   });
-  const bool again = nan != nan || sa.tiny < ((unsigned)kTinyExp << 24) || sb.tiny < ((unsigned)kTinyExp << 24);
-  if (__syncthreads_or(again)) {
+  float unscale = kUnscale;
+  if (__syncthreads_or(nan != nan)) {
+    unscale = 1.0f;
     clear();
     float* const as = reinterpret_cast<float*>(smem);
     float* const bs = as + SA::kWhole;
@@ -299,7 +300,15 @@ gemm_f32_kernel(const GemmArgs g) {
     }
     __syncthreads();
   }
-  epilogue<TM, TN>(g, cbase, c2base, acc, m0 + wm0, n0 + wn0, co, lane, reinterpret_cast<float*>(smem) + wave * 32 * (TN * 32 + 4));
+  auto rows = [&](auto ic, f32x16 (&row)[TN]) OCN_LAMBDA_INLINE -> f32x16 (&)[TN] {
+    static_for<TN>([&](auto jc) OCN_LAMBDA_INLINE {
+      constexpr int i = decltype(ic)::value, j = decltype(jc)::value;
+      asm volatile("" : "+a"(acc[i][j]));   // (in accumulation registers until here)
+      static_for<16>([&](auto ec) OCN_LAMBDA_INLINE { row[j][decltype(ec)::value] = acc[i][j][decltype(ec)::value] * unscale; });
+    });
+    return row;
+  };
+  epilogue<TM, TN>(g, cbase, c2base, rows, m0 + wm0, n0 + wn0, co, lane, reinterpret_cast<float*>(smem) + wave * 32 * (TN * 32 + 4));
 }
 
 template <int BM, int BN, int GM, int GN, bool A_KC, bool B_KC>

@@ -1,7 +1,8 @@
 // Runs a generated kernel of one 256-thread contraction tile on the host, for tests that need no GPU: the threads of a
 // workgroup are fibers that take turns at barriers and matrix instructions, every tensor ends where a page that cannot
 // be touched begins.  Include ahead of the kernel's source; the test supplies `host_kernel(void** tensors)`.
-//   usage: program BLOCKS FILE BYTES...   (the tensors lie in FILE one after the other and are written back to it)
+//   usage: program BLOCKS FILE BYTES...   (the tensors lie in FILE one after the other and are written back to it;
+//   prints how many fp32 matrix instructions the threads went through)
 #include <sys/mman.h>
 #include <ucontext.h>
 
@@ -65,7 +66,8 @@ template <typename V> static V host_transposed(const void* at) {
   return v;
 }
 #define __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, x, y, z) host_mfma_bf16(a, b, c)
-template <typename C> static C host_mfma_f32(float a, float b, C c) { return host_mfma(&a, &b, 1, c); }
+static long host_f32_products;
+template <typename C> static C host_mfma_f32(float a, float b, C c) { ++host_f32_products; return host_mfma(&a, &b, 1, c); }
 #define __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, x, y, z) host_mfma_f32(a, b, c)
 #define __builtin_amdgcn_ds_read_tr16_b64_v4i16(p) host_transposed<s16x4>((const void*)(p))
 // fp32 -> bf16 bits, to nearest even
@@ -136,6 +138,6 @@ int main(int argc, char** argv) {
   rewind(f);
   for (int i = 0; i < n; ++i) fwrite(p[i], 1, strtoull(argv[3 + i], nullptr, 10), f);
   fclose(f);
-  puts("done");
+  printf("%ld\n", host_f32_products);
   return 0;
 }

@@ -128,7 +128,8 @@ CLANG = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin", "c
 
 
 def _on_the_host(tmp_path, code, values):
-    """The one kernel of `code` in a host program (host_workgroup.h): the tensors by name, as it leaves them."""
+    """The one kernel of `code` in a host program (host_workgroup.h): the tensors by name, as it leaves them, and under
+    "f32_products" the fp32 matrix instructions it went through."""
     source = code.source()
     tile, kernel = source[source.index("template <bool C, typename A"):], source[source.index('extern "C" __global__'):]
     name, params = re.match(r'extern "C" __global__ void __launch_bounds__\(256\) (\w+)\(([^)]*)\)', kernel).groups()
@@ -141,8 +142,8 @@ def _on_the_host(tmp_path, code, values):
     arrays = [np.ascontiguousarray(values[n]) for n in names]
     (tmp_path / "tensors").write_bytes(b"".join(a.tobytes() for a in arrays))
     blocks = 8 * int(re.search(r"blockIdx.x % 8u\) \* (\d+)", kernel).group(1))
-    subprocess.run([tmp_path / "kernel", str(blocks), tmp_path / "tensors"] + [str(a.nbytes) for a in arrays], check=True, timeout=120, stdout=subprocess.DEVNULL)
-    raw, out, at = (tmp_path / "tensors").read_bytes(), {}, 0
+    p = subprocess.run([tmp_path / "kernel", str(blocks), tmp_path / "tensors"] + [str(a.nbytes) for a in arrays], check=True, timeout=120, stdout=subprocess.PIPE)
+    raw, out, at = (tmp_path / "tensors").read_bytes(), {"f32_products": int(p.stdout)}, 0
     for n, a in zip(names, arrays):
         out[n] = np.frombuffer(raw, a.dtype, a.size, at).reshape(a.shape)
         at += a.nbytes
@@ -224,3 +225,23 @@ def test_a_weight_counts_only_where_its_tap_reaches(taps, stride, ic, prec, zero
     with np.errstate(invalid="ignore"):
         ref = want(values)
     _same_numbers(_on_the_host(tmp_path, B.compile(r, "min_mfma_flops=1"), init)["dx"], ref, 4e-6)
+
+
+@pytest.mark.skipif(not os.path.exists(CLANG), reason="needs the ROCm compiler")
+@pytest.mark.parametrize("prec", ["single", "bfloat16"])
+@pytest.mark.parametrize("value,again", [(2.0 ** -149, False), (2.0 ** -111, False), (2.0 ** 70, False), (2.0 ** 105, True), (np.inf, True)])
+def test_small_values_are_multiplied_once(value, again, prec, tmp_path):
+    # an fp32 gradient of y of 288 products per cell, multiplied in bf16 parts: what soft-max tails hold costs no second pass
+    r, (w, dy, dx), want = input_gradient((3, 3), (1, 1), prec, False, b=1, oh=4, ow=4)
+    dy.prec = "single"
+    rng = np.random.default_rng(8)
+    init = {n.ident: W.as_prec(rng.standard_normal(n.dims).astype(np.float32), n.prec) for n in (w, dy, dx)}
+    init["dy"].flat[::7] = value
+    code = B.compile(r, "min_mfma_flops=1")
+    assert ", true, 2, true>(d_" in code.source()
+    out = _on_the_host(tmp_path, code, init)
+    assert (out["f32_products"] > 0) == again
+    with np.errstate(invalid="ignore"):
+        ref = want({n.ident: W.to_float(init[n.ident], n.prec).astype(np.float64) for n in (w, dy, dx)})
+    got, fine = out["dx"].astype(np.float64), np.isfinite(ref) & (np.abs(ref) < 2.0 ** 127)
+    assert np.max(np.abs(got[fine] - ref[fine]), initial=0) <= 4e-6 * np.max(np.abs(ref[fine]), initial=0)   # (as above)

@@ -224,6 +224,32 @@ def test_few_tiles_share_k_among_wavefronts(M, N, K, batch, precs, layout):
 
 
 @pytest.mark.parametrize("layout", [(True, True), (False, False), (True, False)])
+@pytest.mark.parametrize("precs,form", [(("single", "single"), "f32_kernel_any<"), (("single", "single"), "f32_kernel_any_direct<"), (("single", "single"), "f32_kernel<"),
+                                        (("single", "bfloat16"), "f32_kernel_any<"), (("single", "bfloat16"), "f32_kernel_any_direct<"),
+                                        (("bfloat16", "single"), "f32_kernel_any<"), (("bfloat16", "single"), "f32_kernel_any_direct<")])
+@pytest.mark.parametrize("sa,sb", [(-142, 40), (-130, 20), (-60, -60), (30, -128), (0, 0)])
+def test_single_products_in_bf16_parts(sa, sb, precs, form, layout):
+    """One non-zero value in a row of A, of around 2^sa (subnormal ones too), so that a cell is one product: as exact as
+    an fp32 product, whatever the parts' exponents."""
+    M, N, K = (70, 66, 132) if "direct" in form else (1032, 1100, 152) if form.endswith("kernel<") else (1031, 1099, 151)
+    r, A, B, C = _routine(M, N, K, *precs, "single", *layout, False)
+    rng = np.random.default_rng(6)
+    a, b = np.zeros((M, K), np.float32), np.ldexp(rng.standard_normal((N, K)), sb).astype(np.float32)
+    a[np.arange(M), rng.integers(K, size=M)] = np.ldexp(rng.standard_normal(M), sa).astype(np.float32)
+    t = lambda x, kc, p: W.as_prec(np.ascontiguousarray(x if kc else x.T), p)
+    hip = HipRun(r, {1: t(a, layout[0], precs[0]), 2: t(b, layout[1], precs[1])}, "min_mfma_flops=1;bf16_copies=0" + (";any=0" if form.endswith("kernel<") else ""))
+    assert form in hip.code.kernels()[-1]["name"], hip.code.kernels()
+    hip.step()
+    got = hip.get(C).astype(np.float64)
+    hip.close()
+    f = lambda x, p: W.to_float(W.as_prec(x, p), p).astype(np.float64)
+    want = f(a, precs[0]) @ f(b, precs[1]).T
+    # the six part products (or three) are added one after the other, each sum off by less than 2^-23 of the result; the
+    # three left out are below 2^-24 of it together; the result itself may be subnormal
+    assert np.all(np.abs(got - want) <= 7 * 2.0 ** -23 * np.abs(want) + 2.0 ** -149)
+
+
+@pytest.mark.parametrize("layout", [(True, True), (False, False), (True, False)])
 @pytest.mark.parametrize("precs", [("single", "single"), ("single", "bfloat16"), ("bfloat16", "single")])
 @pytest.mark.parametrize("M,N,K", [(70, 66, 131), (1031, 1099, 150), (30, 9000, 150), (2049, 4099, 135)])
 @pytest.mark.parametrize("what", ["tiny", "special"])
