@@ -365,9 +365,6 @@ DtlShape dtl_shape(const GemmDesc& d) {
     if (pairs > 1 && t128 * c.splits < kChainWorkgroups) return none;
     if (t128 * c.splits <= 256) s = {128, 128, 64, 5};
     else s = {128, 128, 32, 4};
-    // K = 64, batched products of attention above all: two steps, three stages (48 KB).  Their stores bound them: 256 x 1024 x
-    // 1024, fp32 results, 244 us register-staged, 237 so (256 x 256 x 256: 24 either way).  Fewer tiles: gemm_prefers_any.
-    if (t128 >= 256 && pairs == 1 && d.K == 64) s = {128, 128, 32, 3};
   }
   if (d.M % s.bm || d.N % s.bn || d.K % s.bk) return none;
   const long steps = d.K / s.bk;

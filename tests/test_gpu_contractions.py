@@ -112,7 +112,7 @@ def test_batched(layout):
 @pytest.mark.parametrize("c_prec,accumulate", [("single", True), ("bfloat16", False)])
 def test_two_steps_of_k(shape, batch, a_kc, b_kc, c_prec, accumulate):
     name = _check(*shape, 64, "bfloat16", "bfloat16", c_prec, a_kc, b_kc, accumulate, batch=batch, seed=6)
-    assert name.startswith("gemm_bf16_dtl_kernel<128, 128, 32, 3,"), name
+    assert name.startswith("gemm_bf16_kernel<128, 128,"), name
 
 
 def test_split_k_is_deterministic():
