@@ -93,7 +93,7 @@ int direct_splits(const GemmDesc& d) {
   if (odd(d.a) || odd(d.b)) return 0;
   if (!d.more.empty()) return f32 || d.c.prec != Prec::Single ? 0 : 1;
   int splits = 1;
-  if (d.epi_bias < 0 && d.epi_relu < 0) while (splits * 2 * t32 <= 512 && d.K / (splits * 2) >= (f32 ? 768 : 1536)) splits *= 2;
+  if (!d.unsplit && d.epi_bias < 0 && d.epi_relu < 0) while (splits * 2 * t32 <= 512 && d.K / (splits * 2) >= (f32 ? 768 : 1536)) splits *= 2;
   return splits;
 }
 
@@ -138,6 +138,10 @@ bool contract_any_fits(const GemmDesc& d) {
 }
 
 bool contract_any_direct(const GemmDesc& d) { return direct_splits(d) > 0; }
+
+void contract_any_settle(GemmDesc& d, uint64_t room) {
+  if (d.any && direct_splits(d) > 1 && contract_any_workspace_bytes(d) > room) d.unsplit = true;
+}
 
 int64_t contract_any_area(const GemmDesc& d, bool& alone) {
   const AnyShape s = staged_shape(d);

@@ -2558,8 +2558,9 @@ Plan make_plan(Routine& r, const PlanOptions& requested) {
     constexpr uint64_t limit = OCANNL_HIP_STATIC_SCRATCH_BYTES;
     const uint64_t room = local <= limit ? limit - local : ~0ull;
     for (auto& ph : plan.phases) {
-      if (ph.kind != Phase::Contraction || !gemm_prefers_any(ph.gemm, room)) continue;
-      as_any_shape(ph.gemm);
+      if (ph.kind != Phase::Contraction) continue;
+      if (gemm_prefers_any(ph.gemm, room)) as_any_shape(ph.gemm);
+      contract_any_settle(ph.gemm, room);
     }
   }
   if (opt.enable_serial_group) serialise_tiny(r, plan);

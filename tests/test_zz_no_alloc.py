@@ -79,6 +79,29 @@ def test_static_scratch_run_equals_the_allocating_run_twice_in_a_row():
             h.close()
 
 
+@pytest.mark.parametrize("M,K", [(32, 2048), (31, 2047)])
+def test_few_tiles_split_k_only_where_the_array_has_room(M, K):
+    # 200 products of one 32 x 32 tile each: two splits of K would take 1.6 MB, beside local tensors of 31 MiB too many
+    L.reset_symbols(0)
+    a = L.Node(1, "a", "single", (200, M, K)); b = L.Node(2, "b", "single", (200, M, K)); c = L.Node(3, "c", "single", (200, M, M))
+    n = 31 << 18
+    src, t, out = L.Node(4, "src", "single", (n,)), L.Node(5, "t", "single", (n,), mode="local"), L.Node(6, "out", "single", (n,))
+    z, i, j, k, p, q = (L.fresh_symbol() for _ in range(6))
+    at = (L.It(z), L.It(i), L.It(j))
+    body = L.Set(c, at, L.Ternop("fma", L.Get(a, (L.It(z), L.It(i), L.It(k))), L.Get(b, (L.It(z), L.It(j), L.It(k))), L.Get(c, at)))
+    for sym, ext in ((k, K), (j, M), (i, M), (z, 200)):
+        body = L.For(sym, 0, ext - 1, [body])
+    copy = lambda s, x, y: L.For(s, 0, n - 1, [L.Set(x, (L.It(s),), L.Unop("neg", L.Get(y, (L.It(s),))))])
+    r = L.Routine("one_tile_each", [L.ZeroOut(c), body, copy(p, t, src), copy(q, out, t)])
+    rng = np.random.default_rng(M)
+    init = {x.id: rng.standard_normal(x.dims).astype(np.float32) for x in (a, b, src)}
+    assert any("_any_direct<" in x["name"] for x in B.compile(r, "min_mfma_flops=1").kernels())
+    ref, got = _both_ways(r, init, (c, out))
+    assert all(np.array_equal(x, y) for x, y in zip(ref, got)) and np.array_equal(ref[1], init[4])
+    want = init[1].astype(np.float64) @ init[2].astype(np.float64).transpose(0, 2, 1)
+    assert np.max(np.abs(ref[0] - want)) <= 2e-6 * max(1.0, np.sqrt(K) / 8) * np.max(np.abs(want))
+
+
 def test_static_scratch_refuses_a_routine_beyond_the_array():
     # a routine-local tensor of 48 MiB: more than the 32 MiB array
     L.reset_symbols(0)
