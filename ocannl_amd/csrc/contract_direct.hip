@@ -10,8 +10,9 @@
 //     two blocks {even rows} and {odd rows}: 16 lanes read consecutive bytes, and no transposition is left to do but
 //     pairing the halves of bf16 words.
 //
-// An fp32 operand is multiplied as the sum of three bf16 values (see contract_any.h); tiles that this does not cover are
-// multiplied again with v_mfma_f32_16x16x4_f32, whose k = j, 8 + j, 16 + j, 24 + j are what the lanes hold at place j.
+// An fp32 operand is multiplied as the sum of three bf16 values (see contract_any.h); tiles that this does not cover, those
+// with subnormal values of a bf16 operand beside it among them, are multiplied again with v_mfma_f32_16x16x4_f32, whose k =
+// j, 8 + j, 16 + j, 24 + j are what the lanes hold at place j (594 x 320 x 320 10.3 -> 14.3 us).
 //
 // 594 x 320 (190 tiles) by K, tile with LDS stages before -> now: fp32 10.4 + 0.011 us a k -> 5 + 0.0065; bf16 with a
 // row-contiguous operand 4.5 + 0.005 -> 4.2 + 0.003.  A transformer step of 594 rows with 320 to 1280 channels and mixed
@@ -28,6 +29,16 @@ namespace {
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
+// Subnormal values of a bf16 operand beside one in parts: the least 2 |bits| - 1 of each half of its words (zero: the largest).
+// Three instructions a word, where scaling the operand would take five: 2 % of a launch instead of 4 (a batch of five 180 x 26
+// x 870 8.0 us without either, 8.6, 8.9).
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ unsigned watch(unsigned least, unsigned w) {
+  const u16x2 twice = __builtin_bit_cast(u16x2, w) * (unsigned short)2;
+  return __builtin_bit_cast(unsigned, __builtin_elementwise_min(__builtin_bit_cast(u16x2, least), (u16x2)(twice - (unsigned short)1)));
+}
+__device__ __forceinline__ bool subnormal(unsigned least) { return (least & 0xFFFFu) < 0xFFu || least >> 16 < 0xFFu; }
+
 // One operand of a wavefront's step.
 constexpr int R = 2;              // blocks of 16 rows of a tile
 constexpr int kDirectWaves = 4;   // wavefronts that share K
@@ -39,9 +50,11 @@ struct DirectOperand {
   struct Set { unsigned w[KC ? R : 8][kWords]; };
   int off[KC ? R : 1];
   int shift;        // !KC: rows by which the chunk starts early
+  unsigned least;   // of watch()
 
   __device__ __forceinline__ void init(const OcnAnyOperand& o, const OcnDigits& dr, int row0, int rows, int lane) {
     shift = 0;
+    least = ~0u;
     if constexpr (KC) {
 #pragma unroll
       for (int i = 0; i < R; ++i) {
@@ -133,15 +146,15 @@ struct DirectOperand {
       return (KC ? j & 1 : b & 1) ? __uint_as_float(x & 0xFFFF0000u) : __uint_as_float(x << 16);
     }
   }
-  // block b as matrix operands: its bf16 values (SCALED: beside an operand in parts), or the three parts of its fp32 values
-  template <bool SCALED>
-  static __device__ __forceinline__ void fragments(const Set& s, int b, bf16x8 (&f)[BF ? 1 : 3]) {
+  // block b as matrix operands: its bf16 values (WATCH: beside an operand in parts), or the three parts of its fp32 values
+  template <bool WATCH>
+  __device__ __forceinline__ void fragments(const Set& s, int b, bf16x8 (&f)[BF ? 1 : 3]) {
     unsigned u[4];
     if constexpr (BF) {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         u[q] = KC ? s.w[b][q] : __builtin_amdgcn_perm(s.w[2 * q + 1][b / 2], s.w[2 * q][b / 2], b & 1 ? 0x07060302u : 0x05040100u);
-        if constexpr (SCALED) u[q] = ocn_bf16_scaled(u[q]);
+        if constexpr (WATCH) least = watch(least, u[q]);
       }
       f[0] = __builtin_bit_cast(bf16x8, u);
     } else {
@@ -214,11 +227,11 @@ __device__ __forceinline__ void direct_body(const OcnAnyDesc& d, const AnyBatch&
       constexpr int NA = ABF ? 1 : 3, NB = BBF ? 1 : 3;
       bf16x8 fb[R][NB];
 #pragma unroll
-      for (int j = 0; j < R; ++j) OB::template fragments<F32>(y, j, fb[j]);
+      for (int j = 0; j < R; ++j) ob.template fragments<F32>(y, j, fb[j]);
 #pragma unroll
       for (int i = 0; i < R; ++i) {
         bf16x8 fa[NA];
-        OA::template fragments<F32>(x, i, fa);
+        oa.template fragments<F32>(x, i, fa);
 #pragma unroll
         for (int s = NA == 1 && NB == 1 ? 0 : 2; s >= 0; --s)       // small products first
 #pragma unroll
@@ -322,13 +335,13 @@ __device__ __forceinline__ void direct_body(const OcnAnyDesc& d, const AnyBatch&
     float nan = 0.0f;
 #pragma unroll
     for (int x = 0; x < RW / RL; ++x) nan = __builtin_fmaf(v[x], 0.0f, nan);
-    if (__syncthreads_or(nan != nan)) {
+    if (__syncthreads_or(nan != nan || subnormal(oa.least) || subnormal(ob.least))) {
       clear();
       sum(No{}, Yes{});
       reduce();
     } else {
 #pragma unroll
-      for (int x = 0; x < RW / RL; ++x) v[x] *= kOcnUnscale;
+      for (int x = 0; x < RW / RL; ++x) v[x] *= ABF || BBF ? 1.0f / kOcnScale : kOcnUnscale;
     }
   }
   if (n >= d.N) return;
