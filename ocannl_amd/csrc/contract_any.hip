@@ -66,23 +66,30 @@ long any_entries(const GemmDesc& d) {
 }
 
 // Do 32 x 32 tiles whose wavefronts share K and read their operands straight from memory (contract_direct.hip) take it, and
-// in how many splits?  They read twice the operands per product that 64 x 64 tiles do and cost 5 us + 6.5 ns a k in fp32
-// (4.2 + 3 in bf16) where a compute unit has one of them, against 6 + 16 (4.5 + 5): so up to one tile a unit, and up to
-// two in fp32 where an operand is row-contiguous.  594 x 320, start -> now, both row-contiguous: K = 320 fp32 11.8 -> 7.4
-// us, bf16 6.1 -> 5.6; K = 1001 20.1 -> 11.2 and 10.6 -> 7.1; 594 x 640 x 1001 (380 tiles) fp32 21.3 -> 16.4, bf16 10.6 ->
-// 9.6 but x 320 6.2 -> 6.9.  Two k-contiguous bf16 operands touch 32 rows with every load and lose from K = 320 on (5.4 ->
-// 5.7); rows at odd elements, which the vector memory path takes apart, at once (K = 1001 9.5 -> 12.9).  Short sums are all
-// start (K = 27 fp32 4.4 -> 4.8) and beyond 4096 the traffic tells (594 x 320 x 4096 bf16, k-contiguous 13.7 -> 17.9).
-// Members of a grouped launch that are few enough by themselves for four of them to fit are taken however many there are:
-// grouped or apart, they are then summed in the same order.  A split has to give back the launch that sums the splits.
+// in how many splits?  They read twice the operands per product that 64 x 64 tiles do, so up to one tile a compute unit, and
+// long sums only where splits are free for them.  Measured (staged tile -> these, us) over products, batches and groups
+// of 16 to 768 tiles, K of 66 to 4096 and all layouts:
+//   fp32, up to 256 tiles: K = 128 7.2 -> 6.1 to 6.8, 512 14 -> 9 to 10, 1024 18 -> 13 to 15, 2048 20 -> 19 with a row-contiguous
+//     operand, but 19 -> 22 without one (1800: 18 to 21 -> 19), and 3072 24 -> 25 to 29; in splits, 128 tiles, 2 x 1024 19
+//     -> 17, 2 x 1500 23 -> 18, but 2 x 1536, where the staged tile has eight, 18 -> 20; 64 tiles, 4 x 1024 20 -> 17.
+//   257 to 512 tiles, a row-contiguous operand: K = 512 16 -> 13, 1024 20 -> 18, 1500 25 -> 23, 2048 26 -> 29; with one operand
+//     k-contiguous 81 6.6 -> 6.1, 128 7.5 -> 7.9, 131 8.6 -> 8.0, 200 10.3 -> 8.6.
+//   bf16, up to 256 tiles, a row-contiguous operand: K = 128 5.5 -> 5.3, 1024 10 -> 7 to 8, 2560 16 -> 13, 3056 18 -> 13, but
+//     3072, where the staged tile has four splits, 14 -> 15; in two, 128 tiles, 13.2 -> 13.0 there and 14.5 -> 14.3 at 4096.  k-contiguous operands touch 32 rows with every
+//     load: K = 160 5.6 -> 5.1, 320 5.4 -> 5.7; rows 128 bytes apart or a multiple of that collide, K = 128 5.3 -> 5.5, 256 5.7
+//     -> 5.5.  Rows at odd elements, which the vector memory path takes apart, lose at once (K = 1001 9.5 -> 12.9).
+//   One or two tiles to an entry of a batch, where a staged tile is mostly padding: at any K (200 x 32 x 32 x 4000 fp32 79 ->
+//     44, bf16 34 -> 24).
+// A grouped launch goes by all of its tiles, so its members may be summed in another order than apart.  Not so up to 128 tiles
+// each and 512 of K: k-contiguous fp32 products keep to these tiles then, at 8.7, 11.5 and 15.6 us for K = 128, 256, 512
+// against 7.4, 9.6 and 14.2.
 int direct_splits(const GemmDesc& d) {
-  const long t32 = ((d.M + 31) / 32) * ((d.N + 31) / 32) * any_entries(d);
-  const bool f32 = any_is_f32(d), both_kc = any_kc(d.a) && any_kc(d.b);
-  const long members = 1 + (long)d.group.size();
+  const long members = 1 + (long)d.group.size(), tiles = ((d.M + 31) / 32) * ((d.N + 31) / 32) * any_entries(d);
+  const bool f32 = any_is_f32(d), both_kc = any_kc(d.a) && any_kc(d.b), one_kc = any_kc(d.a) != any_kc(d.b);
   const int64_t all_k = d.K * (int64_t)(1 + d.more.size());
-  if (all_k <= 64 || all_k > 4096 || !any_regular(d)) return 0;
-  if (t32 > (f32 && !both_kc ? 512 : 256) && t32 / members > (f32 ? 128 : 64)) return 0;
-  if (!f32 && both_kc && all_k > 256) return 0;
+  if (all_k <= 64 || all_k > 4096 || tiles > (f32 ? 512 : 256) || !any_regular(d)) return 0;
+  if (tiles > 256 && (both_kc ? tiles / members > 128 || all_k > 512 : all_k > 1536 || (one_kc && !any_mixed(d) && all_k > 96 && all_k <= 128))) return 0;
+  if (!f32 && both_kc && (all_k > 256 || (d.more.empty() && all_k < 256 && (d.a.row_stride[2] % 64 == 0 || d.b.row_stride[2] % 64 == 0)))) return 0;
   auto odd = [&](const GemmOperand& o) {
     int64_t all = o.offset;
     for (auto& t : o.static_terms) all |= t.second;
@@ -93,8 +100,10 @@ int direct_splits(const GemmDesc& d) {
   if (odd(d.a) || odd(d.b)) return 0;
   if (!d.more.empty()) return f32 || d.c.prec != Prec::Single ? 0 : 1;
   int splits = 1;
-  if (!d.unsplit && d.epi_bias < 0 && d.epi_relu < 0) while (splits * 2 * t32 <= 512 && d.K / (splits * 2) >= (f32 ? 768 : 1536)) splits *= 2;
-  return splits;
+  if (!d.unsplit && d.epi_bias < 0 && d.epi_relu < 0) while (splits * 2 * tiles <= 256 && d.K / (splits * 2) >= (f32 ? 768 : 1536)) splits *= 2;
+  const bool padding = std::min(d.M, d.N) <= 32 && std::max(d.M, d.N) <= 64;
+  const int64_t most = !f32 ? 3071 : splits > 1 ? 1535 : both_kc && !any_mixed(d) ? 1800 : 2048;
+  return padding || d.unsplit || d.K / splits <= most ? splits : 0;
 }
 
 // 128 x 128 tiles when they fill the chip twice over, else 64 x 64 (128 x 32 or 32 x 128 when one extent is at most
@@ -140,7 +149,9 @@ bool contract_any_fits(const GemmDesc& d) {
 bool contract_any_direct(const GemmDesc& d) { return direct_splits(d) > 0; }
 
 void contract_any_settle(GemmDesc& d, uint64_t room) {
-  if (d.any && direct_splits(d) > 1 && contract_any_workspace_bytes(d) > room) d.unsplit = true;
+  if (!d.any || contract_any_workspace_bytes(d) <= room) return;
+  d.unsplit = true;
+  if (contract_any_workspace_bytes(d) > room) d.unsplit = false;
 }
 
 int64_t contract_any_area(const GemmDesc& d, bool& alone) {

@@ -418,7 +418,10 @@ bool gemm_prefers_any(const GemmDesc& d, uint64_t room) {
   const bool f32 = d.a.prec == Prec::Single;
   if (!f32 && dtl_shape(d).bm != 0) return false;
   if (contract_any_direct(few)) return true;   // (its splits: contract_any_settle)
-  if (gemm_workspace_bytes(d) > room && contract_any_workspace_bytes(d) <= room) return true;
+  if (gemm_workspace_bytes(d) > room) {
+    contract_any_settle(few, room);
+    if (contract_any_workspace_bytes(few) <= room) return true;
+  }
   const TileConfig c = tile_config(d);
   const int64_t staged = (t128 * c.splits + 255) / 256 * 128 * (c.narrow ? 64 : 128) / c.splits;
   bool alone;

@@ -79,7 +79,8 @@ bool contract_any_fits(const GemmDesc& desc);
 int64_t contract_any_area(const GemmDesc& desc, bool& alone);
 // Is it few enough tiles for contract_direct.hip?
 bool contract_any_direct(const GemmDesc& desc);
-// Such a contraction does without K splits whose workspace is larger than `room`.
+// One whose K splits would take more workspace than `room` goes unsplit to the tiles of contract_direct.hip, if they are few
+// enough.
 void contract_any_settle(GemmDesc& desc, uint64_t room);
 hipError_t launch_contract_any(const GemmDesc& desc, const GemmArgs& args, void* workspace, hipStream_t stream, hipEvent_t after_main);
 size_t contract_any_workspace_bytes(const GemmDesc& desc);

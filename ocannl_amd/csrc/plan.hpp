@@ -42,7 +42,7 @@ struct GemmDesc {
   // then numbers of up to three digits (the loop symbols of the class that do not merge, slowest first; unused
   // leading digits have extent 1), s_row / s_k are not used, and a mixed product is computed in fp32.
   bool any = false;
-  // Set by contract_any_settle: the tiles whose wavefronts share K keep K whole, for want of room for a workspace.
+  // Set by contract_any_settle: the tiles whose wavefronts share K take it and keep K whole, for want of room for a workspace.
   bool unsplit = false;
   int m_digits = 1, n_digits = 1, k_digits = 1;
   int64_t m_ext[3] = {1, 1, 1}, n_ext[3] = {1, 1, 1}, k_ext[3] = {1, 1, 1};

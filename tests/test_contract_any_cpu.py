@@ -60,6 +60,46 @@ def test_a_workspace_does_not_take_a_routine_beyond_the_static_scratch(local_mib
     assert ("kernel_any<64, 64" in name) == small
 
 
+def _products(M, N, K, precs, a_kc, b_kc, batch=1, members=1):
+    L.reset_symbols(0)
+    z, m, n, k = (L.fresh_symbol() for _ in range(4))
+    at = lambda r, s, kc: (L.It(z),) + ((L.It(r), L.It(s)) if kc else (L.It(s), L.It(r)))
+    a, body = L.Node(1, "a", precs[0], (batch, M, K) if a_kc else (batch, K, M)), []
+    for g in range(members):
+        b = L.Node(2 + 2 * g, f"b{g}", precs[1], (batch, N, K) if b_kc else (batch, K, N)); c = L.Node(3 + 2 * g, f"c{g}", "single", (batch, M, N))
+        nest = L.Set(c, at(m, n, True), L.Ternop("fma", L.Get(a, at(m, k, a_kc)), L.Get(b, at(n, k, b_kc)), L.Get(c, at(m, n, True))))
+        for sym, ext in ((k, K), (n, N), (m, M), (z, batch)):
+            nest = L.For(sym, 0, ext - 1, [nest])
+        body += [L.ZeroOut(c), nest]
+    return L.Routine("products", body)
+
+
+F, H = "single", "bfloat16"
+
+
+@pytest.mark.parametrize("M,N,K,precs,layout,batch,members,direct", [
+    # one tile a compute unit, and one more; long sums in fp32, unsplit, two splits, four
+    (511, 511, 1000, (F, F), (True, True), 1, 1, True), (545, 481, 1000, (F, F), (True, True), 1, 1, False), (511, 511, 1800, (F, F), (True, True), 1, 1, True),
+    (511, 511, 1801, (F, F), (True, True), 1, 1, False), (511, 511, 2048, (F, F), (True, False), 1, 1, True), (511, 511, 2049, (F, F), (True, False), 1, 1, False),
+    (255, 511, 3071, (F, F), (True, True), 1, 1, True), (255, 511, 3072, (F, F), (True, True), 1, 1, False), (255, 255, 4096, (F, F), (True, True), 1, 1, True),
+    # up to two a unit, with a row-contiguous operand
+    (511, 1023, 1536, (F, F), (True, False), 1, 1, True), (511, 1023, 1537, (F, F), (True, False), 1, 1, False), (511, 1055, 512, (F, F), (True, False), 1, 1, False),
+    (511, 1023, 96, (F, F), (True, False), 1, 1, True), (511, 1023, 128, (F, F), (True, False), 1, 1, False), (511, 1023, 128, (F, F), (False, False), 1, 1, True),
+    # bf16
+    (511, 511, 3071, (H, H), (False, False), 1, 1, True), (511, 511, 3072, (H, H), (False, False), 1, 1, False), (255, 511, 4096, (H, H), (False, False), 1, 1, True),
+    (511, 545, 512, (H, H), (False, False), 1, 1, False), (300, 300, 160, (H, H), (True, True), 1, 1, True), (300, 300, 128, (H, H), (True, True), 1, 1, False),
+    (300, 300, 256, (H, H), (True, True), 1, 1, True), (300, 300, 260, (H, H), (True, True), 1, 1, False), (301, 301, 510, (H, F), (True, True), 1, 1, True),
+    # batches of one tile, which is mostly padding of a staged one; groups go by all of their tiles
+    (31, 31, 4000, (F, F), (True, True), 200, 1, True), (63, 31, 4000, (F, F), (True, True), 128, 1, True), (95, 31, 4000, (F, F), (True, True), 60, 1, False),
+    (256, 256, 4096, (F, F), (True, True), 1, 1, True), (256, 256, 4096, (F, F), (True, True), 1, 4, False), (256, 512, 2048, (F, F), (True, True), 1, 1, True),
+    (256, 512, 2048, (F, F), (True, True), 1, 2, False), (512, 256, 512, (F, F), (True, True), 1, 4, True), (512, 256, 520, (F, F), (True, True), 1, 4, False)])
+def test_few_tiles_share_k_where_that_is_measured_to_be_faster(M, N, K, precs, layout, batch, members, direct):
+    code = B.compile(_products(M, N, K, precs, *layout, batch, members), "min_mfma_flops=1;bf16_copies=0")
+    name, = {k["name"] for k in code.kernels() if k["kind"] == "mfma"}
+    assert ("_any_direct<" in name) == direct, name
+    assert direct or "kernel_any<" in name, name
+
+
 def test_sums_of_more_terms_than_32_bits_count_are_left_alone():
     # k in two digits over operands of few elements: x[i + j] * w[i + j], 2^31 terms and more
     def names(I, J):

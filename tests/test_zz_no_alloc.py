@@ -79,17 +79,18 @@ def test_static_scratch_run_equals_the_allocating_run_twice_in_a_row():
             h.close()
 
 
-@pytest.mark.parametrize("M,K", [(32, 2048), (31, 2047)])
-def test_few_tiles_split_k_only_where_the_array_has_room(M, K):
-    # 200 products of one 32 x 32 tile each: two splits of K would take 1.6 MB, beside local tensors of 31 MiB too many
+@pytest.mark.parametrize("Z,M,N,K", [(120, 32, 32, 2048), (120, 31, 31, 2047), (2, 296, 296, 4000)])
+def test_few_tiles_split_k_only_where_the_array_has_room(Z, M, N, K):
+    # 120 products of one 32 x 32 tile each: two splits of K would take 0.9 MB, beside local tensors of 31.5 MiB too many;
+    # two of 100 tiles: of so long a sum the staged tiles would take them, in eight splits
     L.reset_symbols(0)
-    a = L.Node(1, "a", "single", (200, M, K)); b = L.Node(2, "b", "single", (200, M, K)); c = L.Node(3, "c", "single", (200, M, M))
-    n = 31 << 18
+    a = L.Node(1, "a", "single", (Z, M, K)); b = L.Node(2, "b", "single", (Z, N, K)); c = L.Node(3, "c", "single", (Z, M, N))
+    n = 63 << 17
     src, t, out = L.Node(4, "src", "single", (n,)), L.Node(5, "t", "single", (n,), mode="local"), L.Node(6, "out", "single", (n,))
     z, i, j, k, p, q = (L.fresh_symbol() for _ in range(6))
     at = (L.It(z), L.It(i), L.It(j))
     body = L.Set(c, at, L.Ternop("fma", L.Get(a, (L.It(z), L.It(i), L.It(k))), L.Get(b, (L.It(z), L.It(j), L.It(k))), L.Get(c, at)))
-    for sym, ext in ((k, K), (j, M), (i, M), (z, 200)):
+    for sym, ext in ((k, K), (j, N), (i, M), (z, Z)):
         body = L.For(sym, 0, ext - 1, [body])
     copy = lambda s, x, y: L.For(s, 0, n - 1, [L.Set(x, (L.It(s),), L.Unop("neg", L.Get(y, (L.It(s),))))])
     r = L.Routine("one_tile_each", [L.ZeroOut(c), body, copy(p, t, src), copy(q, out, t)])
