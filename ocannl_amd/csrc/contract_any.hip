@@ -113,12 +113,13 @@ int direct_splits(const GemmDesc& d) {
 // through 4096 x 4096, four splits: 13.6 us).
 AnyShape staged_shape(const GemmDesc& d) {
   const long nb = any_entries(d);
-  AnyShape s{64, 64, 1, any_is_f32(d) && d.K >= kPartsFrom, false};
+  AnyShape s{64, 64, 1, false, false};
   if (any_mixed(d)) {}   // (the one tile built for a bf16 and an fp32 operand)
   else if (d.N <= 32) { s.bm = 128; s.bn = 32; }
   else if (d.M <= 32) { s.bm = 32; s.bn = 128; }
   else if (d.M > 64 && d.N > 64 && ((d.M + 127) / 128) * ((d.N + 127) / 128) * nb >= 512) s.bm = s.bn = 128;
   const long tiles = ((d.M + s.bm - 1) / s.bm) * ((d.N + s.bn - 1) / s.bn) * nb;
+  s.parts = any_is_f32(d) && d.K >= (tiles > 256 ? kPartsFrom : kPartsFromAlone);
   if (tiles < 192 && d.epi_bias < 0 && d.epi_relu < 0) while ((long)s.splits * 2 * tiles <= 512 && d.K / (s.splits * 2) >= (any_is_f32(d) ? 384 : 768)) s.splits *= 2;
   return s;
 }

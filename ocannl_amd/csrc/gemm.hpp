@@ -66,10 +66,11 @@ bool gemm_prefers_any(const GemmDesc& desc, uint64_t room);
 // Makes it one of any shape: extents and strides as digits.
 void as_any_shape(GemmDesc& desc);
 
-// Least K at which an fp32 operand of a contraction of any shape is multiplied in bf16 parts: below, what parts save is less
-// than what they cost, a vote on whether to multiply again (260 x 132 x 16 4.4 us as fp32, 5.2 in parts; 1023 x 1023 x 198
-// 9.4, 9.5).
-constexpr int64_t kPartsFrom = 129;
+// Least K at which an fp32 operand of a contraction of any shape is multiplied in bf16 parts, and the same where no compute
+// unit has a second tile: below, what parts save is less than what they cost, a vote on whether to multiply again (260 x 132
+// x 16 4.4 us as fp32, 5.2 in parts).  2001 x 2001 x 130 (1024 tiles) 22 to 25 us as fp32, 20 to 21 in parts; 1023 x 1023 (256) x 130
+// 8.6 to 9.5 and 8.8 to 9.8, x 198 10.6 to 11.9 and 10.5 to 11.7, x 300 13.8 to 16.1 and 12.2 to 13.8.
+constexpr int64_t kPartsFrom = 129, kPartsFromAlone = 193;
 
 // contract_any.hip: the same for contractions with `desc.any` set (launch_gemm and its siblings forward to these).
 // Do the extents and the element offsets within one batch entry fit the 32-bit arithmetic of contract_any.h?
