@@ -8,9 +8,11 @@
 // order: padding between rows is not available, so bank conflicts are avoided by choosing WHICH
 // 16-byte chunk of the tile a lane fetches (an XOR swizzle of the chunk position):
 //   K-contiguous operand, tile held [row][k], row = BK * 2 bytes (64 or 128):
-//     chunk c of row r sits at position c ^ ((r / RP) & (CPR - 1)) of its row, RP = rows per 256
-//     bytes, CPR = chunks per row: the ds_read_b128 of 16 consecutive rows at one k touch 16
-//     different 16-byte bank groups.
+//     chunk c of row r sits at position c ^ row_turn(r) of its row.  A ds_read_b128 serves 16 lanes at once, lanes 0 .. 3,
+//     12 .. 15, 20 .. 23 and 24 .. 27 of 32, or the rest of them: eight rows each at two neighbouring chunks.  row_turn
+//     gives these 16 different 16-byte bank groups of 256 bytes (the static_assert below).  With r / 4 as the turn of
+//     64-byte rows half of all LDS cycles of 8192 x 4096 x 4096 were conflicts (16.8 of 33.6 million, none now; 226 us
+//     either way: the matrix cores' clock bounds it).
 //   row-contiguous operand, tile held [k][row] as it lies in memory, k-line = ROWS * 2 bytes:
 //     chunk c of k-line kl sits at position c ^ ((kl & 3) << 2) ^ ((kl >> 3 & 1) << 1) (ROWS >= 128) or
 //     c ^ ((kl >> 1 & 1) << 2) ^ ((kl >> 3 & 1) << 1) (ROWS = 64): the eight k-lines (0 .. 3, 8 .. 11) that one
@@ -23,6 +25,8 @@
 // into the order of 32 x 32 tiles, in which the epilogue stores them, by one exchange of 16-lane rows per register: of
 // the column halves in lanes, and of the second and third four rows by where the fragments of A start (kPerm).
 // 8192 x 4096 x 4096: 221 -> 207 us (1.33 PFLOP/s), B row-contiguous 216 -> 207, both, 4096 x 4096 x 8192: 202 either way.
+// Few workgroups with a row-contiguous operand lose: 512 x 512 x 512 9.7 -> 9.9 us, both 10.1; 256 x 256 x 3072 13.7 -> 14.1,
+// both 14.4.
 // (Loads issued by the four waves in turn instead of together: 223 -> 229.)
 //
 // Pipeline (one barrier per K step, placed ahead of the LAST 32-k sub-step of the step): at that
@@ -72,6 +76,22 @@ struct DtlTile {
   static_assert(KC || ROWS == 64 || ROWS == 128 || ROWS == 256, "k-lines of 128, 256 or 512 bytes");
   static_assert(BK == 32 || BK == 64, "rows of 64 or 128 bytes");
 
+  static constexpr int row_turn(int r) { return kCPR == 8 ? r / 2 & 7 : ((r >> 2 ^ r >> 3) & 1) << 1 | (r >> 3 & 1); }
+  // row of its 16-row block that a lane's fragment holds; `perm`: rows 4 .. 7 and 8 .. 11 change places
+  static constexpr int frag_row(int lane, bool perm) { return (perm ? (lane >> 3 & 1) | (lane >> 1 & 2) : lane >> 2 & 3) * 4 + (lane & 3); }
+  static constexpr bool no_conflict() {
+    for (int perm = 0; perm < 2; ++perm)
+      for (int part = 0; part < 4; ++part) {
+        unsigned seen = 0;
+        for (int i = 0; i < 16; ++i) {
+          const int q[2][4] = {{0, 3, 5, 6}, {1, 2, 4, 7}}, lane = (part >> 1) * 32 + q[part & 1][i >> 2] * 4 + (i & 3), r = frag_row(lane, perm);
+          seen |= 1u << (r % kRP * kCPR + ((lane >> 4) ^ row_turn(r)));
+        }
+        if (seen != 0xFFFFu) return false;
+      }
+    return true;
+  }
+
   // rows (KC) or k-lines (!KC) between the blocks that consecutive loads of one wave fetch
   static constexpr int kOpLines = (KC ? kRPB : kLPB) * 4;
 
@@ -86,7 +106,7 @@ struct DtlTile {
   static __device__ __forceinline__ unsigned lane_goff(int wave, int lane, long ld, int odd) {
     if constexpr (KC) {
       const int r = kRPB * wave + lane / kCPR;
-      const int c = (lane % kCPR) ^ ((r / kRP) & (kCPR - 1));
+      const int c = (lane % kCPR) ^ row_turn(r);
       return (unsigned)((r * ld + c * 8) * 2);
     } else {
       const int kl = kLPB * wave + lane / kCPL;
@@ -100,13 +120,13 @@ struct DtlTile {
   template <bool kPerm>
   static __device__ __forceinline__ unsigned lane_frag(int lane, int w0) {
     const int g = lane >> 4;
-    auto place = [](int q) { return kPerm ? (q >> 1 | q << 1) & 3 : q; };
     if constexpr (KC) {
-      const int r = place(lane >> 2 & 3) * 4 + (lane & 3);
-      return (unsigned)((w0 + r) * kRowBytes + ((g ^ ((r / kRP) & (kCPR - 1))) * 16));
+      static_assert(no_conflict(), "16 lanes of a fragment read meet all banks");
+      const int r = frag_row(lane, kPerm);
+      return (unsigned)((w0 + r) * kRowBytes + ((g ^ row_turn(r)) * 16));
     } else {
-      const int kl = g * 8 + (lane >> 2 & 3);
-      return (unsigned)(kl * kLineBytes + ((w0 * 2 + place(lane & 3) * 8) ^ (turn(kl) * 16)));
+      const int kl = g * 8 + (lane >> 2 & 3), q = lane & 3;
+      return (unsigned)(kl * kLineBytes + ((w0 * 2 + (kPerm ? (q >> 1 | q << 1) & 3 : q) * 8) ^ (turn(kl) * 16)));
     }
   }
 
