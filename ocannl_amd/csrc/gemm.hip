@@ -442,7 +442,8 @@ const char* gemm_kernel_name(const GemmDesc& d) {
   if (af && bf)
     snprintf(buf, sizeof buf, "gemm_f32_kernel<%d, %d, 2, 2, %s, %s>", tile, tile, tf[a_kcontig(d)], tf[b_kcontig(d)]);
   else if (ds.bm)   // (operands that turn out misaligned at launch take the register-staged kernel instead)
-    snprintf(buf, sizeof buf, "gemm_bf16_dtl_kernel<%d, %d, %d, %d, %s, %s>", ds.bm, ds.bn, ds.bk, ds.ns, tf[a_kcontig(d)], tf[b_kcontig(d)]);
+    snprintf(buf, sizeof buf, "gemm_bf16_dtl_kernel<%d, %d, %d, %d, %s, %s, %s, %s>", ds.bm, ds.bn, ds.bk, ds.ns, tf[a_kcontig(d)], tf[b_kcontig(d)],
+             tf[dtl_odd(ds.bk, ds.ns, d.K, split_count(d), 1 + (int)d.more.size())], tf[!d.more.empty()]);
   else
     snprintf(buf, sizeof buf, "gemm_bf16_kernel<%d, %d, %s, %s, %s, %s, %d, %s>", tile, tile_n, af ? "float" : "unsigned short",
              bf ? "float" : "unsigned short", tf[a_kcontig(d)], tf[b_kcontig(d)], prefetch_depth(d), tf[!d.more.empty()]);

@@ -57,6 +57,10 @@ hipError_t launch_gemm(const GemmDesc& desc, const GemmArgs& args, void* workspa
 // Bytes of split-K workspace this contraction needs (0 when K is not split).
 size_t gemm_workspace_bytes(const GemmDesc& desc);
 
+// Direct-to-LDS kernel with one sub-step a step: is the number of K steps of a split (a whole number each) beyond the last
+// ns - 1 odd?  It runs them in pairs.
+constexpr bool dtl_odd(int64_t bk, int64_t ns, int64_t K, int64_t splits, int64_t pairs) { return bk == 32 && (K / bk / splits * pairs - (ns - 1)) % 2 != 0; }
+
 // Name of the instance launch_gemm would pick (for kernel_info and profiles).
 const char* gemm_kernel_name(const GemmDesc& desc);
 

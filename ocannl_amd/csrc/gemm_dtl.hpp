@@ -144,8 +144,8 @@ struct DtlTile {
 template <int BM, int BN, int BK, int NS>
 constexpr size_t dtl_smem() { return (size_t)NS * (BM + BN) * BK * 2; }
 
-// kOdd: K steps of a split beyond the last NS - 1, modulo two (launch_dtl_layout picks it; a branch here would have the
-// register allocator move all accumulators)
+// kOdd: K steps of a split beyond the last NS - 1, modulo two (dtl_odd; a branch here would have the register allocator move
+// all accumulators)
 // kChain: several operand pairs into one C, one pair's K after the other's: the fetch goes on to the next pair's tensors and
 // nothing else of the pipeline knows
 template <int BM, int BN, int BK, int NS, bool A_KC, bool B_KC, bool kOdd, bool kChain>
@@ -382,9 +382,8 @@ hipError_t launch_dtl_layout(bool akc, bool bkc, const GemmArgs& a, hipStream_t 
 }
 template <int BM, int BN, int BK, int NS, bool kChain>
 hipError_t launch_dtl_steps(bool akc, bool bkc, const GemmArgs& a, hipStream_t s, hipEvent_t ev) {
-  // (a split's K is a whole number of steps: dtl_shape)
   if constexpr (BK == 32) {
-    if ((a.K / BK / a.splits * a.npairs - (NS - 1)) % 2) return launch_dtl_layout<BM, BN, BK, NS, true, kChain>(akc, bkc, a, s, ev);
+    if (dtl_odd(BK, NS, a.K, a.splits, a.npairs)) return launch_dtl_layout<BM, BN, BK, NS, true, kChain>(akc, bkc, a, s, ev);
   }
   return launch_dtl_layout<BM, BN, BK, NS, false, kChain>(akc, bkc, a, s, ev);
 }
