@@ -4,6 +4,7 @@ fp32; an fp32 operand keeps all its bits (a mixed product is computed in fp32)."
 import numpy as np
 import pytest
 
+from ocannl_amd import backend
 from ocannl_amd import llir as L
 from ocannl_amd import workloads as W
 from parity import HipRun, OracleRun
@@ -41,9 +42,12 @@ def _run(r, nodes, out, want, accumulate, k, seed=0):
     hip.close()
 
 
-def _product(M, N, K, a_prec, b_prec, c_prec, a_kc, b_kc, accumulate, batch=0, seed=0):
+def _product(M, N, K, a_prec, b_prec, c_prec, a_kc, b_kc, accumulate, batch=0, seed=0, direct=None):
     r, A, B, C = _routine(M, N, K, a_prec, b_prec, c_prec, a_kc, b_kc, accumulate, batch)
     t = lambda x, kc: x if kc else np.swapaxes(x, -1, -2)
+    if direct is not None:
+        names = [k["name"] for k in backend.compile(r, "min_mfma_flops=1").kernels() if k["kind"] == "mfma"]
+        assert len(names) == 1 and ("_any_direct<" in names[0]) == direct, names
     _run(r, dict(a=A, b=B, c=C), "c", lambda f: t(f["a"], a_kc) @ np.swapaxes(t(f["b"], b_kc), -1, -2), accumulate, K, seed)
 
 
@@ -199,7 +203,7 @@ def test_bias_and_relu_of_every_batch_entry(shape, one_statement):
     rng = np.random.default_rng(M)
     init = {t.value.id: W.as_prec((rng.standard_normal(t.value.dims) / np.sqrt(K if t is w else 1)).astype(np.float32), "bfloat16") for t in (x, w, bias)}
     folded, apart = HipRun(r, init, "min_mfma_flops=1"), HipRun(r, init, "min_mfma_flops=1;epilogues=0;fused=0")
-    assert [k["name"][:20] for k in folded.code.kernels()] == ["gemm_bf16_kernel_any"] and len(apart.code.kernels()) > 1
+    assert [k["name"].split("<")[0] for k in folded.code.kernels()] == ["gemm_bf16_kernel_any" + ("_direct" if K > 64 else "")] and len(apart.code.kernels()) > 1
     folded.step(); apart.step()
     f = {t: W.to_float(init[t.value.id], "bfloat16").astype(np.float64) for t in (x, w, bias)}
     want = np.einsum("zbi,zoi->zbo", f[x], f[w]) + f[bias]
@@ -220,7 +224,38 @@ def _forms(kernels):
 @pytest.mark.parametrize("M,N,K,batch", [(40, 30, 66, 0), (33, 18, 97, 5), (16, 8, 127, 0), (70, 66, 200, 7), (34, 130, 3100, 0)])
 def test_few_tiles_share_k_among_wavefronts(M, N, K, batch, precs, layout):
     # one step of K for some wavefronts and none for others, a partial step, rows past the end, batch entries, K splits
-    _product(M, N, K, *precs, *layout, accumulate=K % 2 == 0, batch=batch, seed=K)
+    # (rows of bf16 at odd elements, and long sums of two k-contiguous bf16 operands, go to staged tiles)
+    bf16 = precs[:2] == ("bfloat16", "bfloat16")
+    staged = any(p == "bfloat16" and kc and K % 2 for p, kc in zip(precs, layout)) or (bf16 and all(layout) and K > 256)
+    _product(M, N, K, *precs, *layout, accumulate=K % 2 == 0, batch=batch, seed=K, direct=not staged)
+
+
+@pytest.mark.parametrize("accumulate", [False, True])
+@pytest.mark.parametrize("precs", [("bfloat16", "bfloat16", "bfloat16"), ("single", "single", "bfloat16"), ("single", "bfloat16", "bfloat16")])
+def test_few_tiles_store_bf16(precs, accumulate):
+    _product(71, 66, 202, *precs, True, False, accumulate=accumulate, seed=7, direct=True)
+
+
+@pytest.mark.parametrize("layout", [(True, True), (True, False), (False, True)])
+@pytest.mark.parametrize("precs", [("bfloat16", "bfloat16"), ("single", "bfloat16"), ("bfloat16", "single")])
+@pytest.mark.parametrize("K", [73, 97, 131, 191])
+def test_few_tiles_with_an_odd_end_of_k(K, precs, layout):
+    # sums over the first K columns of rows of K + 1, so that bf16 rows start at even elements and the last chunk is shifted
+    # by an odd number of halves
+    M, N = 70, 66
+    L.reset_symbols(0)
+    a = L.Node(1, "a", precs[0], (M, K + 1) if layout[0] else (K + 1, M)); b = L.Node(2, "b", precs[1], (N, K + 1) if layout[1] else (K + 1, N))
+    c = L.Node(3, "c", "single", (M, N))
+    m, n, k = (L.fresh_symbol() for _ in range(3))
+    at = lambda r, kc: (L.It(r), L.It(k)) if kc else (L.It(k), L.It(r))
+    body = L.Set(c, (L.It(m), L.It(n)), L.Ternop("fma", L.Get(a, at(m, layout[0])), L.Get(b, at(n, layout[1])), L.Get(c, (L.It(m), L.It(n)))))
+    for sym, ext in ((k, K), (n, N), (m, M)):
+        body = L.For(sym, 0, ext - 1, [body])
+    r = L.Routine("odd_end", [L.ZeroOut(c), body])
+    name, = [x["name"] for x in backend.compile(r, "min_mfma_flops=1").kernels() if x["kind"] == "mfma"]
+    assert "_any_direct<" in name, name
+    t = lambda x, kc: x[:, :K] if kc else x[:K].T
+    _run(r, dict(a=a, b=b, c=c), "c", lambda f: t(f["a"], layout[0]) @ t(f["b"], layout[1]).T, False, K, K)
 
 
 @pytest.mark.parametrize("layout", [(True, True), (False, False), (True, False)])
