@@ -51,6 +51,19 @@ def build_workload(name: str):
     raise SystemExit(f"unknown workload {name}")
 
 
+def matrix_peak(kernel: str) -> float:
+    """Products per second (TFLOP/s) of the matrix instructions that a contraction kernel runs on: an fp32 operand is
+    multiplied as three bf16 values, six bf16 products to one of two fp32 operands and three beside a bf16 one; short sums
+    of the tile for any shape (last argument false) use fp32 instructions."""
+    if "gemm_f32" not in kernel:
+        return PEAKS["mfma_bf16"]
+    args = kernel[kernel.index("<") + 1:-1].split(", ")
+    if "_any" in kernel and "_direct" not in kernel and args[-1] == "false":
+        return PEAKS["mfma_f32"]
+    mixed = "_any" in kernel and "true" in (args[2:4] if "_direct" in kernel else args[4:6])
+    return PEAKS["mfma_bf16"] / (3 if mixed else 6)
+
+
 def measured_traffic(workload: str, kernel: str):
     """HBM bytes per launch of `kernel` from the committed rocprofv3 counter summary of this
     workload (profiles/<workload>_step_hbm_traffic.txt), or None when there is none."""
@@ -209,8 +222,7 @@ def measure(workload: str, steps: int, warmup: int, options=None, kernel_table: 
     if bound == "mfma":
         per_launch = sum(kernels[i]["flops"] for i in sampled) / len(sampled)   # (of the launches that were bracketed)
         achieved = per_launch / (avg_ms * 1e-3) / 1e12
-        f32 = "gemm_f32" in dom_name
-        peak = PEAKS["mfma_f32"] if f32 else PEAKS["mfma_bf16"]
+        peak = matrix_peak(dom_name)
         roof = {"bound": "mfma", "kernel": dom_name, "achieved": achieved, "peak": peak, "unit": "TFLOP/s",
                 "frac": achieved / peak, "traffic": measured_traffic(workload, dom_name),
                 "launches_per_step": len(dom_idx),
