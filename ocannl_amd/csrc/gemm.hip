@@ -365,6 +365,11 @@ DtlShape dtl_shape(const GemmDesc& d) {
     if (pairs > 1 && t128 * c.splits < kChainWorkgroups) return none;
     if (t128 * c.splits <= 256) s = {128, 128, 64, 5};
     else s = {128, 128, 32, 4};
+    // K = 64, batched products of attention above all: two steps, three stages (48 KB), for at most 1024 tiles, two rounds of
+    // two a unit.  Register-staged -> so, four layouts, fp32 and bf16 results: batches of 256 x 256, 256 of them 21 -> 20.5 and
+    // 19.8 -> 19.1 us, but 1024 of them 67 -> 70 and 57 -> 60; 128 x 1024, 256 of them (2048 tiles) 40 -> 42 and 31 -> 33; 2048 x
+    // 2048 10.4 -> 10.0 and 8.9 -> 8.6.  Fewer tiles: gemm_prefers_any.
+    if (t128 >= 256 && t128 <= 1024 && pairs == 1 && d.K == 64) s = {128, 128, 32, 3};
   }
   if (d.M % s.bm || d.N % s.bn || d.K % s.bk) return none;
   const long steps = d.K / s.bk;

@@ -108,11 +108,11 @@ def test_batched(layout):
 
 
 @pytest.mark.parametrize("a_kc,b_kc", [(True, True), (True, False), (False, True), (False, False)])
-@pytest.mark.parametrize("shape,batch", [((256, 256), 64), ((2048, 2048), 0), ((128, 128), 257)])
+@pytest.mark.parametrize("shape,batch", [((256, 256), 64), ((2048, 2048), 0), ((128, 128), 257), ((128, 128), 1024), ((128, 128), 1025)])
 @pytest.mark.parametrize("c_prec,accumulate", [("single", True), ("bfloat16", False)])
 def test_two_steps_of_k(shape, batch, a_kc, b_kc, c_prec, accumulate):
     name = _check(*shape, 64, "bfloat16", "bfloat16", c_prec, a_kc, b_kc, accumulate, batch=batch, seed=6)
-    assert name.startswith("gemm_bf16_kernel<128, 128,"), name
+    assert name.startswith("gemm_bf16_kernel<128, 128," if batch == 1025 else "gemm_bf16_dtl_kernel<128, 128, 32, 3,"), name
 
 
 def test_split_k_is_deterministic():
