@@ -230,7 +230,18 @@ enum : int { kOutF32 = 0, kOutBf16 = 1, kOutF32Copy = 2 };
 // bf16 bits <-> float, as the generated code converts them
 __device__ __forceinline__ float bf2f(unsigned b) { return __uint_as_float(b << 16); }
 
-template <int TN, int OUT, bool ACC, bool CHECK>
+// Holds a row of tiles in accumulation registers up to here: without that the register allocator may move all accumulators
+// of a block into ordinary registers right after the main loop and spill most.
+template <int TN>
+__device__ __forceinline__ void pin_row(f32x16 (&row)[TN]) {
+  static_assert(TN == 1 || TN == 2 || TN == 4, "tile rows of 1, 2 or 4 tiles");
+  if constexpr (TN == 1) asm volatile("" : "+a"(row[0]));
+  else asm volatile("" : "+a"(row[0]), "+a"(row[1]));
+  if constexpr (TN == 4) asm volatile("" : "+a"(row[2]), "+a"(row[3]));
+}
+
+// PIN: the row is one of accumulators
+template <int TN, int OUT, bool ACC, bool CHECK, bool PIN>
 __device__ __forceinline__ void store_tile_row(f32x16 (&acc)[TN], void* origin, long ld, int lane,
                                                long rows_left, long cols_left, void* origin2 = nullptr,
                                                const unsigned short* bias = nullptr, unsigned short* relu_out = nullptr,
@@ -240,6 +251,7 @@ __device__ __forceinline__ void store_tile_row(f32x16 (&acc)[TN], void* origin, 
   unsigned short* const base2 = static_cast<unsigned short*>(origin2);
   const unsigned col = lane & 31, rb = (lane >> 5) * 4;
   const unsigned loff = rb * (unsigned)ld + col;
+  if constexpr (PIN) pin_row<TN>(acc);
   float old[ACC ? TN : 1][16];
   if (ACC) {
     static_for<TN>([&](auto jc) OCN_LAMBDA_INLINE {
@@ -283,11 +295,12 @@ __device__ __forceinline__ void store_tile_row(f32x16 (&acc)[TN], void* origin, 
 // fp32 or eight bf16 results) next to its neighbours' -- an eighth (a quarter) of the store
 // instructions of the direct form, each covering whole cache lines.  `stage` holds 32 * (TN * 32 + 4)
 // floats of this wave's own; LDS operations of one wave complete in order, so no barrier is needed.
-template <int TN, int OUT, bool ACC>
+template <int TN, int OUT, bool ACC, bool PIN>
 __device__ __forceinline__ void store_tile_row_wide(f32x16 (&acc)[TN], float* stage, void* origin, long ld, int lane,
                                                     void* origin2 = nullptr, const unsigned short* bias = nullptr,
                                                     unsigned short* relu_out = nullptr, bool relu_c = false) {
   constexpr int CW = TN * 32, LS = CW + 4;
+  if constexpr (PIN) pin_row<TN>(acc);
   float* const wr = stage + ((lane >> 5) * 4) * LS + (lane & 31);
   static_for<TN>([&](auto jc) OCN_LAMBDA_INLINE {
     static_for<16>([&](auto ec) OCN_LAMBDA_INLINE {
@@ -349,7 +362,7 @@ __device__ __forceinline__ void store_tile_row_wide(f32x16 (&acc)[TN], float* st
 // `stage`: this wave's own LDS area of at least 32 * (TN * 32 + 4) floats, free once the main loop
 // has passed its last barrier.
 // `rows(i, room)`: row i of tiles, made in `room` where it has to be made.
-template <int TM, int TN, typename Rows>
+template <int TM, int TN, bool PIN = false, typename Rows>
 __device__ __forceinline__ void epilogue(const GemmArgs& g, void* cbase, void* c2base, Rows&& rows, long m, long n, long co, int lane,
                                          float* stage) {
   const long rows_left = g.M - m, cols_left = g.N - n;
@@ -386,37 +399,30 @@ __device__ __forceinline__ void epilogue(const GemmArgs& g, void* cbase, void* c
     f32x16 room[TN];
     f32x16(&row)[TN] = rows(ic, room);
     switch (variant) {
-      case 0: store_tile_row<TN, kOutF32, false, false>(row, o, ld, lane, rl, cols_left); break;
-      case 1: store_tile_row<TN, kOutF32, false, true>(row, o, ld, lane, rl, cols_left); break;
-      case 2: store_tile_row<TN, kOutF32, true, false>(row, o, ld, lane, rl, cols_left); break;
-      case 3: store_tile_row<TN, kOutF32, true, true>(row, o, ld, lane, rl, cols_left); break;
-      case 4: store_tile_row_wide<TN, kOutBf16, false>(row, stage, o, ld, lane, nullptr, bias, reinterpret_cast<unsigned short*>(o3), relu_c); break;
-      case 5: store_tile_row<TN, kOutBf16, false, true>(row, o, ld, lane, rl, cols_left, nullptr, bias, reinterpret_cast<unsigned short*>(o3), relu_c); break;
-      case 6: store_tile_row_wide<TN, kOutBf16, true>(row, stage, o, ld, lane); break;
-      case 7: store_tile_row<TN, kOutBf16, true, true>(row, o, ld, lane, rl, cols_left); break;
-      case 8: store_tile_row_wide<TN, kOutF32Copy, false>(row, stage, o, ld, lane, o2); break;
-      case 9: store_tile_row<TN, kOutF32Copy, false, true>(row, o, ld, lane, rl, cols_left, o2); break;
-      case 10: store_tile_row_wide<TN, kOutF32Copy, true>(row, stage, o, ld, lane, o2); break;
-      default: store_tile_row<TN, kOutF32Copy, true, true>(row, o, ld, lane, rl, cols_left, o2); break;
+      case 0: store_tile_row<TN, kOutF32, false, false, PIN>(row, o, ld, lane, rl, cols_left); break;
+      case 1: store_tile_row<TN, kOutF32, false, true, PIN>(row, o, ld, lane, rl, cols_left); break;
+      case 2: store_tile_row<TN, kOutF32, true, false, PIN>(row, o, ld, lane, rl, cols_left); break;
+      case 3: store_tile_row<TN, kOutF32, true, true, PIN>(row, o, ld, lane, rl, cols_left); break;
+      case 4: store_tile_row_wide<TN, kOutBf16, false, PIN>(row, stage, o, ld, lane, nullptr, bias, reinterpret_cast<unsigned short*>(o3), relu_c); break;
+      case 5: store_tile_row<TN, kOutBf16, false, true, PIN>(row, o, ld, lane, rl, cols_left, nullptr, bias, reinterpret_cast<unsigned short*>(o3), relu_c); break;
+      case 6: store_tile_row_wide<TN, kOutBf16, true, PIN>(row, stage, o, ld, lane); break;
+      case 7: store_tile_row<TN, kOutBf16, true, true, PIN>(row, o, ld, lane, rl, cols_left); break;
+      case 8: store_tile_row_wide<TN, kOutF32Copy, false, PIN>(row, stage, o, ld, lane, o2); break;
+      case 9: store_tile_row<TN, kOutF32Copy, false, true, PIN>(row, o, ld, lane, rl, cols_left, o2); break;
+      case 10: store_tile_row_wide<TN, kOutF32Copy, true, PIN>(row, stage, o, ld, lane, o2); break;
+      default: store_tile_row<TN, kOutF32Copy, true, true, PIN>(row, o, ld, lane, rl, cols_left, o2); break;
     }
     __builtin_amdgcn_sched_barrier(0);
   });
 }
 
-// The epilogue of 32 x 32 tiles.  A row is pinned to accumulation registers until its turn: without that the register
-// allocator may move all accumulators of the block into ordinary registers right after the main loop and spill most.
+// The epilogue of 32 x 32 tiles.  Their rows are pinned where they are stored: pinned ahead of the choice of the store, fp32
+// results of 512 x 512 x 64 in batches of 256 took 82 us instead of 74.
 template <int TM, int TN>
 __device__ __forceinline__ void epilogue(const GemmArgs& g, void* cbase, void* c2base, f32x16 (&acc)[TM][TN], long m, long n, long co, int lane,
                                          float* stage) {
-  static_assert(TN == 1 || TN == 2 || TN == 4, "tile rows of 1, 2 or 4 tiles");
-  auto rows = [&](auto ic, f32x16 (&)[TN]) OCN_LAMBDA_INLINE -> f32x16 (&)[TN] {
-    f32x16(&from)[TN] = acc[decltype(ic)::value];
-    if constexpr (TN == 1) asm volatile("" : "+a"(from[0]));
-    else asm volatile("" : "+a"(from[0]), "+a"(from[1]));
-    if constexpr (TN == 4) asm volatile("" : "+a"(from[2]), "+a"(from[3]));
-    return from;
-  };
-  epilogue<TM, TN>(g, cbase, c2base, rows, m, n, co, lane, stage);
+  auto rows = [&](auto ic, f32x16 (&)[TN]) OCN_LAMBDA_INLINE -> f32x16 (&)[TN] { return acc[decltype(ic)::value]; };
+  epilogue<TM, TN, true>(g, cbase, c2base, rows, m, n, co, lane, stage);
 }
 
 // Sums the split-K partials in split order (deterministic) and applies them to C.
