@@ -20,8 +20,8 @@
 // The 1 KB blocks of a tile are dealt to the four waves round robin (block b to wave b % 4), which
 // makes the swizzle term of a lane independent of the block: one 32-bit lane offset per operand.
 //
-// v_mfma_f32_16x16x32_bf16: in a loop of matrix instructions alone it sustains 2.08 PFLOP/s where v_mfma_f32_32x32x16_bf16
-// sustains 1.80, from the same bytes of fragments.  Its results are brought
+// v_mfma_f32_16x16x32_bf16: in a loop of matrix instructions alone, normally distributed operands in registers, it sustains
+// 1.97 PFLOP/s where v_mfma_f32_32x32x16_bf16 sustains 1.76 (zeros: 2.39, 2.42), from the same bytes of fragments.  Its results are brought
 // into the order of 32 x 32 tiles, in which the epilogue stores them, by one exchange of 16-lane rows per register: of
 // the column halves in lanes, and of the second and third four rows by where the fragments of A start (kPerm).
 // 8192 x 4096 x 4096: 221 -> 207 us (1.33 PFLOP/s), B row-contiguous 216 -> 207, both, 4096 x 4096 x 8192: 202 either way.

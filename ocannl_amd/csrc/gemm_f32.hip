@@ -14,8 +14,9 @@
 // sums from 2^81 on and values from 2^104 on overflow.  That pass hides nothing: 4096 x 4096 x 4096 with such a value in
 // every tile 1.62 ms, 0.63 without one, 1.04 where all tiles ran on fp32 instructions.
 //
-// What bounds it: the matrix cores at the clock they sustain: 8192 x 4096 x 4096 in 1.36 ms is 1.21 PFLOP/s of bf16
-// products (an MFMA-only loop: 1.40), 202 TFLOP/s of fp32 ones; with v_mfma_f32_32x32x2_f32, which this replaces, 2.12 ms,
+// What bounds it: the matrix cores: 8192 x 4096 x 4096 in 1.36 ms is 1.21 PFLOP/s of bf16 products, 202 TFLOP/s of fp32
+// ones; they are busy in 62 % of the cycles, a loop of their instruction alone sustains 1.76 PFLOP/s on normally distributed
+// operands and a library's bf16 product of 8192^3 1.48; with v_mfma_f32_32x32x2_f32, which this replaces, 2.12 ms,
 // 82 % of what that instruction can do.  One operand row-contiguous 1.38 (2.18), both, 4096 x 4096 x 8192: 1.36 (2.16);
 // 2048 x 2048 x 2048 on 128 x 128 tiles 120 us (174).  A step moves 48 KB into LDS and 96 KB of fragments out of it in
 // the 3072 cycles of its products, and splits 32 values a thread in about 210 vector instructions: room enough beside
